@@ -1,0 +1,224 @@
+"""The calls whose speed this repository is judged by: what a user of the Canon conv1d package has it do.
+
+``listed()`` holds the fixed cases, ``draw()`` further ones of the same ranges.  ``prepare()`` makes what a program
+has in hand before the call (inputs, layer, mask, cache tensors), ``run()`` makes the one call.  The shapes are those
+of the 18-layer Viby model (hidden 640; q 640 + k 160 + v 160; gate and up 1728 each; width 4), of the package's
+tests and of its benchmark.
+"""
+import math
+import os
+import sys
+import types
+
+import torch
+
+sys.path.insert(0, os.path.abspath("viby-model_amd"))
+
+from causal_conv1d import causal_conv1d_fn, causal_conv1d_update  # noqa: E402
+from causal_conv1d.canon import CanonLayer  # noqa: E402
+
+WIDTH = 4
+DTYPES = {"bf16": torch.bfloat16, "fp16": torch.float16, "fp32": torch.float32}
+LAYERS = 18   # slots a model's cache keeps per Canon site
+
+# Most elements of one tensor in a drawn case: forward calls, calls with a backward.
+MOST_FORWARD = 28 << 20
+MOST_TRAIN = 28 << 20
+
+
+def listed():
+    return [
+        # one sequence being generated, one Canon-A layer: the call a model makes 72 times per token
+        dict(name="step_one_sequence", kind="step", dtype="bf16", B=1, C=640, act=False),
+        # decode of a large batch at the widest Canon site, shift-register state
+        dict(name="update_batch", kind="update", dtype="bf16", B=256, C=3456, S=3, mode="shift", act=False),
+        # a serving loop whose sequences own rows of one state pool, Canon-B
+        dict(name="update_pool", kind="update", dtype="bf16", B=96, C=960, S=4, mode="pool", act=True),
+        # the prompt of a single chat turn: odd length, state captured for the decode that follows
+        dict(name="prompt_one_sequence", kind="prompt", dtype="bf16", B=1, L=77, C=640, act=False, mask=False),
+        # a padded batch of prompts through Canon-A, state captured
+        dict(name="prompt_batch", kind="prompt", dtype="bf16", B=8, L=1024, C=640, act=False, mask=True),
+        # q, k and v as their projections leave them, prefill of sixteen sequences
+        dict(name="parts_qkv", kind="parts", dtype="bf16", B=16, L=1024, C=640, C2=160, n=3, act=False),
+        # the benchmark's headline shape in the layout it is quoted in
+        dict(name="fn_headline", kind="fn", dtype="bf16", layout="time", B=8, L=1024, C=3456, act=False, mask=False),
+        # fp32, time-contiguous, a length that is no multiple of anything, with SiLU
+        dict(name="fn_odd_length", kind="fn", dtype="fp32", layout="time", B=4, L=1023, C=960, act=True, mask=False),
+        # the ragged right-padded batch: the largest forward
+        dict(name="fn_ragged_batch", kind="fn", dtype="bf16", layout="channel", B=32, L=1024, C=3456, act=False, mask=True),
+        # a training step of Canon-D as the trainer runs it: bf16 activations, fp32 parameters, padding mask
+        dict(name="train_wide", kind="train", dtype="bf16", weights="fp32", layout="channel", B=32, L=1024, C=3456,
+             act=False, mask=True),
+        # ... of Canon-A with SiLU; the trainer's inputs are one token shorter than its sequence length
+        dict(name="train_hidden", kind="train", dtype="bf16", weights="same", layout="channel", B=16, L=511, C=640,
+             act=True, mask=True),
+        # ... on documents packed into long rows (seq_idx)
+        dict(name="train_packed", kind="packed", dtype="bf16", weights="same", B=2, L=8192, C=3456, act=True),
+    ]
+
+
+def _log_int(rng, lo, hi):
+    return max(lo, min(hi, int(math.exp(rng.uniform(math.log(lo), math.log(hi + 1))))))
+
+
+def _channels(rng, lo=64, hi=3456):
+    """Mostly multiples of 32 as models have them, one in six an odd number."""
+    c = _log_int(rng, lo, hi)
+    return c | 1 if rng.random() < 1 / 6 else max(32, c // 32 * 32)
+
+
+def _sizes(rng, most, longest=4096):
+    c, l = _channels(rng), _log_int(rng, 2, longest)
+    b = _log_int(rng, 1, 32)
+    while b > 1 and b * c * l > most:
+        b //= 2
+    return dict(B=b, L=min(l, max(2, most // (b * c))), C=c)
+
+
+def draw(rng):
+    kind = rng.choice(["step", "update", "prompt", "parts", "fn", "train", "packed"])
+    act = rng.random() < 0.4
+    dtype = rng.choices(["bf16", "fp16", "fp32"], [6, 1, 2])[0]
+    if kind == "step":
+        return dict(kind=kind, dtype="bf16", B=_log_int(rng, 1, 256), C=_channels(rng), act=act)
+    if kind == "update":
+        return dict(kind=kind, dtype=dtype, B=_log_int(rng, 1, 512), C=_channels(rng), S=rng.choice([3, 4, 8]),
+                    mode=rng.choice(["shift", "shift", "pool", "ring"]), act=act)
+    if kind == "prompt":
+        return dict(kind=kind, dtype="bf16", act=act, mask=rng.random() < 0.5, **_sizes(rng, MOST_FORWARD))
+    if kind == "parts":
+        s = _sizes(rng, MOST_FORWARD // 2)
+        c = max(64, s["C"] // 32 * 32)
+        two = rng.random() < 0.5     # gate and up, or q, k and v
+        return dict(kind=kind, dtype="bf16", B=s["B"], L=s["L"], C=c, C2=c if two else c // 4, n=2 if two else 3, act=act)
+    weights = rng.choice(["same", "fp32"])
+    if kind == "packed":
+        l, c = _log_int(rng, 256, 8192), _channels(rng) // 32 * 32
+        return dict(kind=kind, dtype="bf16", weights=weights, B=rng.choice([1, 1, 2]), L=min(l, MOST_TRAIN // (2 * c)), C=c,
+                    act=act)
+    layout = rng.choice(["channel", "time"])
+    if kind == "fn":
+        return dict(kind=kind, dtype=dtype, layout=layout, act=act, mask=rng.random() < 0.4, **_sizes(rng, MOST_FORWARD))
+    return dict(kind=kind, dtype=dtype, weights=weights, layout=layout, act=act, mask=rng.random() < 0.6,
+                **_sizes(rng, MOST_TRAIN))
+
+
+class _Config:
+    canon_kernel, canon_bias = WIDTH, True
+
+    def __init__(self, act):
+        self.canon_activation = act
+
+
+def prepare(case, seed):
+    dev = "cuda"
+    g = torch.Generator(device=dev).manual_seed(int(seed))
+    kind, dtype = case["kind"], DTYPES[case["dtype"]]
+    B, C, L = case["B"], case["C"], case.get("L", 1)
+
+    def normal(*shape, scale=1.0, of=None):
+        return (torch.randn(*shape, generator=g, device=dev) * scale).to(of or dtype)
+
+    parts = [C] + [case["C2"]] * (case["n"] - 1) if kind == "parts" else [C]
+    D = sum(parts)
+    s = types.SimpleNamespace(case=case, act="silu" if case["act"] else None, mask=None)
+    wtype = torch.float32 if case.get("weights") == "fp32" else dtype
+    weight, bias = normal(D, WIDTH, scale=0.02, of=wtype), normal(D, scale=0.01, of=wtype)
+
+    if case.get("mask"):
+        # right-padded rows, as a tokenizer or a trainer hands them over (int64)
+        lens = torch.randint(max(1, L // 8), L + 1, (B, 1), generator=g, device=dev)
+        s.mask = (torch.arange(L, device=dev) < lens).long()
+
+    if kind in ("step", "prompt", "parts"):
+        s.layer = CanonLayer(D, _Config(case["act"]), "a").to(dev, dtype).requires_grad_(False)
+        s.layer.weight.copy_(weight.unsqueeze(1))
+        s.layer.bias_param.copy_(bias)
+        if kind == "parts":
+            s.x = [normal(B, L, d) for d in parts]
+        else:
+            s.x = normal(B, L, C)
+        if kind == "step":
+            s.mask = torch.ones(B, 512, dtype=torch.int64, device=dev)
+            s.cache = types.SimpleNamespace(_max_layers=LAYERS)
+            s.cache.canon_cache_a = [None] * LAYERS
+            s.cache.canon_cache_a[0] = normal(B, C, 8)
+        return s
+
+    s.weight, s.bias = weight, bias
+    if kind == "update":
+        s.x = normal(B, C)
+        s.options = {}
+        rows = B
+        if case["mode"] == "pool":
+            rows = B + B // 3 + 1
+            s.options["conv_state_indices"] = torch.randperm(rows, generator=g, device=dev)[:B].to(torch.int32)
+        elif case["mode"] == "ring":
+            s.options["cache_seqlens"] = torch.randint(0, 4096, (B,), generator=g, device=dev, dtype=torch.int32)
+        s.state = normal(rows, C, case["S"])
+        return s
+
+    if case.get("layout") == "time":
+        s.x = normal(B, C, L)
+    else:
+        s.x = normal(B, L, C).transpose(1, 2)
+    if kind in ("train", "packed"):
+        s.dout = torch.empty_like(s.x).copy_(normal(B, C, L))
+        for t in (s.x, s.weight, s.bias):
+            t.requires_grad_()
+    s.seq_idx = None
+    if kind == "packed":
+        # documents of 32 to 1024 tokens, one after the other
+        first = torch.cumsum(torch.randint(32, 1025, (B, L // 32 + 1), generator=g, device=dev), 1)
+        s.seq_idx = (torch.arange(L, device=dev).view(1, L, 1) >= first.unsqueeze(1)).sum(-1).to(torch.int32)
+    return s
+
+
+def run(s):
+    kind = s.case["kind"]
+    if kind == "step":
+        with torch.no_grad():
+            return s.layer(s.x, s.mask, s.cache, 0), s.cache.canon_cache_a[0]
+    if kind in ("prompt", "parts"):
+        cache = types.SimpleNamespace(_max_layers=LAYERS)
+        with torch.no_grad():
+            forward = s.layer if kind == "prompt" else s.layer.forward_parts
+            return forward(s.x, s.mask, cache, 0), cache.canon_cache_a[0]
+    if kind == "update":
+        with torch.no_grad():
+            return causal_conv1d_update(s.x, s.state, s.weight, s.bias, s.act, residual=True, **s.options), s.state
+    if kind == "fn":
+        with torch.no_grad():
+            return causal_conv1d_fn(s.x, s.weight, s.bias, activation=s.act, attention_mask=s.mask)
+    y = causal_conv1d_fn(s.x, s.weight, s.bias, seq_idx=s.seq_idx, activation=s.act, attention_mask=s.mask,
+                         residual=kind == "train")
+    return (y.detach(), *torch.autograd.grad(y, (s.x, s.weight, s.bias), s.dout))
+
+
+def work(case):
+    """Each input read once, each output written once (a backward reads x a second time: it is another pass)."""
+    kind, size = case["kind"], 4 if case["dtype"] == "fp32" else 2
+    B, L = case["B"], case.get("L", 1)
+    C = case["C"] + case["C2"] * (case["n"] - 1) if kind == "parts" else case["C"]
+    wsize = 4 if case.get("weights") == "fp32" else size
+    taps = C * (WIDTH + 1) * wsize
+    if kind in ("step", "update"):
+        S = case.get("S", 8)
+        per_row = WIDTH + 2 if case.get("mode") == "ring" else 2 * S + 2
+        return {"bytes": B * C * per_row * size + taps, "flops": 2 * WIDTH * B * C}
+    n = B * C * L
+    extra = taps + (8 * B * L if case.get("mask") else 0) + (4 * B * L if kind == "packed" else 0)
+    if kind in ("prompt", "parts"):
+        extra += 8 * B * C * size   # the captured state
+    if kind in ("train", "packed"):
+        return {"bytes": 5 * n * size + 2 * extra + taps, "flops": 4 * 2 * WIDTH * n}
+    return {"bytes": 2 * n * size + extra, "flops": 2 * WIDTH * n}
+
+
+def tolerance(case):
+    """Four times what the calls differ by from the same arithmetic in 64 bits: the rounding of the storage type
+    (measured over forty cases: bf16 1.7e-3 in the 2-norm and 3.9e-3 at most, fp32 1.1e-7 and 3.7e-7; fp16 has three
+    more bits than bf16), with room for fp32 sums over more steps than those."""
+    if case["dtype"] == "fp32":
+        return {"rel": 1e-6, "max": 1e-5}
+    return {"rel": 7e-3, "max": 1.6e-2} if case["dtype"] == "bf16" else {"rel": 9e-4, "max": 2e-3}
