@@ -195,6 +195,68 @@ def run(s):
     return (y.detach(), *torch.autograd.grad(y, (s.x, s.weight, s.bias), s.dout))
 
 
+def exact(case, seed):
+    """What run() returns, from the definition: plain torch in 64 bits on the same inputs (about three seconds for the
+    largest case)."""
+    s = prepare(case, seed)
+    kind, L = case["kind"], case.get("L", 1)
+
+    def act(v):
+        return torch.nn.functional.silu(v) if case["act"] else v
+
+    def back(x, k):
+        """x of k steps earlier, zero before the row's start."""
+        return x if k == 0 else torch.nn.functional.pad(x, (k, 0))[..., :x.shape[-1]]
+
+    def conv(x, weight, bias, seq=None):
+        total = 0
+        for k in range(WIDTH):
+            v = back(x, k)
+            if seq is not None and k:
+                v = v * (back(seq + 1, k) == seq + 1).unsqueeze(1)
+            total = total + v * weight[:, WIDTH - 1 - k, None]
+        return act(total + bias[:, None])
+
+    if kind in ("step", "prompt", "parts"):
+        weight, bias = s.layer.weight.double().squeeze(1), s.layer.bias_param.double()
+    else:
+        weight, bias = s.weight.detach().double(), s.bias.detach().double()
+
+    if kind in ("step", "update"):
+        x = (s.x[:, 0] if kind == "step" else s.x).double()
+        full = (s.cache.canon_cache_a[0] if kind == "step" else s.state).double()
+        options = s.options if kind == "update" else {}
+        rows = options["conv_state_indices"].long() if "conv_state_indices" in options else slice(None)
+        state = full[rows]
+        S = state.shape[-1]
+        if "cache_seqlens" in options:   # a ring: the token's place is its number modulo the length
+            at = options["cache_seqlens"].long() % S
+            place = ((at[:, None] - WIDTH + 1 + torch.arange(WIDTH - 1, device=x.device)) % S).unsqueeze(1)
+            history = state.gather(2, place.expand(-1, state.shape[1], -1))
+            after = state.scatter(2, at.view(-1, 1, 1).expand(-1, state.shape[1], 1), x.unsqueeze(-1))
+        else:
+            history, after = state[..., S - WIDTH + 1:], torch.cat([state[..., 1:], x.unsqueeze(-1)], -1)
+        y = x + act((torch.cat([history, x.unsqueeze(-1)], -1) * weight).sum(-1) + bias)
+        full[rows] = after
+        return y.unsqueeze(1) if kind == "step" else y, full
+
+    mask = 1.0 if s.mask is None else s.mask.double().unsqueeze(1)
+    if kind in ("prompt", "parts"):
+        x = (torch.cat(s.x, -1) if kind == "parts" else s.x).double().transpose(1, 2) * mask
+        y = (x + conv(x, weight, bias)).transpose(1, 2)
+        state = torch.nn.functional.pad(x, (8, 0))[..., L:]
+        return tuple(y.split([p.shape[-1] for p in s.x], -1)) if kind == "parts" else y, state
+    if kind == "fn":
+        return conv(s.x.double() * mask, weight, bias)
+    x = s.x.detach().double().requires_grad_()
+    weight.requires_grad_()
+    bias.requires_grad_()
+    y = conv(x * mask, weight, bias, s.seq_idx)
+    if kind == "train":
+        y = y + x * mask
+    return (y.detach(), *torch.autograd.grad(y, (x, weight, bias), s.dout.double()))
+
+
 def work(case):
     """Each input read once, each output written once (a backward reads x a second time: it is another pass)."""
     kind, size = case["kind"], 4 if case["dtype"] == "fp32" else 2
