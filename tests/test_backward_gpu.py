@@ -324,6 +324,30 @@ def test_backward_of_packed_sequences(cc, dtype, layout):
                 check(db, rdb, dtype, what + " dbias", sum_terms=B * L)
 
 
+@pytest.mark.parametrize("dtype,act,masked", [(torch.bfloat16, "silu", False), (torch.bfloat16, None, True), (torch.float32, "silu", True)])
+def test_backward_of_packed_sequences_in_chunks_of_several_tiles(cc, dtype, act, masked):
+    """Enough columns that one block walks a whole row (three tiles of 32 steps and a part of one): boundaries between
+    slabs, waves and tiles, sequences of one step, and whole tiles without a boundary."""
+    g = torch.Generator().manual_seed(77)
+    B, C, L = 96, 1024 if dtype != torch.float32 else 512, 101
+    x = torch.randn(B, C, L, generator=g).to(dtype)
+    w = (torch.randn(C, 4, generator=g) * 0.5).to(dtype)
+    b = (torch.randn(C, generator=g) * 0.2).to(dtype)
+    dout = torch.randn(B, C, L, generator=g).to(dtype)
+    seq = packed_seq_idx(B, L, g, 64)
+    for row, cuts in enumerate(([32], [8, 16, 24], [31, 33], [64, 65, 66, 67], [29, 61, 93], [99, 100], [])):
+        seq[row] = 0
+        for c in cuts:
+            seq[row, c:] += 1
+    mask = right_padded_mask([max(1, L - i) for i in range(B)], L) if masked else None
+    dx, dw, db, out = gpu_grads(cc, x, w, b, dout, "blc", mask, act, "masked", seq_idx=seq)
+    rdx, rdw, rdb, rout = conv1d_grads(x, w, b, dout, mask, act, "masked", seq_idx=seq)
+    check(out, rout, dtype, "out")
+    check(dx, rdx, dtype, "dx")
+    check(dw, rdw, dtype, "dweight", sum_terms=B * L)
+    check(db, rdb, dtype, "dbias", sum_terms=B * L)
+
+
 def test_backward_of_packed_sequences_equals_the_sequences_on_their_own(cc):
     """Oracle-free: the gradients of a packed row are those of its sequences run as separate calls
     (dx cut out per sequence, dweight / dbias summed over them)."""

@@ -619,11 +619,11 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     a.b_pair = p->bias && ((uintptr_t)p->bias & 3u) == 0 && (p->w_dtype == CANON_DTYPE_F32 || p->channels % 2 == 0);
     a.m_vec = mask_run_aligned(p->mask, p->mask_dtype, p->mask_stride_b, p->mask_stride_l, p->x_dtype);
     const bool ptrs16 = aligned16(p->x) && aligned16(p->dout) && aligned16(p->dx);
-    // packed sequences: only the walk kernel gates taps by sequence index.  States (the history before t = 0, the
-    // gradient of the captured final state): the walk kernel and the channel-contiguous one.
-    const bool packed = force_generic || p->seq_idx != nullptr;
+    // packed sequences and states (the history before t = 0, the gradient of the captured final state): the walk
+    // kernel and the channel-contiguous one
+    const bool packed = p->seq_idx != nullptr;
     const bool states = p->initial_state != nullptr || p->dfinal_state != nullptr;
-    const bool rows = !packed && !states && ptrs16 && a.x_sl == 1 && a.g_sl == 1 && a.d_sl == 1 && a.L % E == 0 && a.L / E >= 16 &&
+    const bool rows = !force_generic && !packed && !states && ptrs16 && a.x_sl == 1 && a.g_sl == 1 && a.d_sl == 1 && a.L % E == 0 && a.L / E >= 16 &&
                       a.x_sb % E == 0 && a.x_sc % E == 0 && a.g_sb % E == 0 && a.g_sc % E == 0 &&
                       a.d_sb % E == 0 && a.d_sc % E == 0 &&
                       // the kernel receives the batch and channel strides of x and dout in vectors, as 32-bit leading scalars
@@ -663,7 +663,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     // channel-contiguous tensors: a group of kBwdVecBytes of adjacent channels per lane
     const int E8 = kBwdVecBytes / elem_bytes(p->x_dtype);
     const bool ptrs8 = (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & (uintptr_t)(kBwdVecBytes - 1)) == 0;
-    const bool vec = !packed && a.x_sc == 1 && a.g_sc == 1 && a.d_sc == 1 && a.C % E8 == 0 && a.x_sl != 1 &&
+    const bool vec = !force_generic && a.x_sc == 1 && a.g_sc == 1 && a.d_sc == 1 && a.C % E8 == 0 && a.x_sl != 1 &&
                      a.x_sb % E8 == 0 && a.x_sl % E8 == 0 && a.g_sb % E8 == 0 && a.g_sl % E8 == 0 &&
                      a.d_sb % E8 == 0 && a.d_sl % E8 == 0 && ptrs8;
     if (vec) {
@@ -699,7 +699,11 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
             }
         }
         const uint64_t blocks = (uint64_t)a.B * nchunk * nct;
-        if (blocks < (1ull << 31)) {
+        // Packed rows: the walk kernel cuts long rows into fewer partial sets when there are many channels, so a scratch
+        // that holds its sets may be too small for these; such a call keeps the walk kernel.
+        const int64_t need = (int64_t)a.B * nchunk * a.C * 5 * (int64_t)sizeof(float);
+        const bool short_scratch = packed && check_pointers && p->workspace_bytes < need;
+        if (blocks < (1ull << 31) && !short_scratch) {
             plan->kind = BWD_BLC_VEC;
             a.nvec = nvec; a.nct = nct; a.chunk = chunk; a.nchunk = nchunk;
             a.nsets = a.B * nchunk;
@@ -973,6 +977,8 @@ CANON_API int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *st
     q.workspace_bytes = kStaticScratchBytes;
     BwdPlan pl;
     rc = plan_bwd(&q, &pl, false);
+    if (rc == CANON_OK && pl.workspace_bytes > kStaticScratchBytes && p->seq_idx)
+        rc = plan_bwd(&q, &pl, false, true);   // fewer partial sets; plan_bwd makes the same choice at the launch
     if (rc != CANON_OK) return rc;
     if (pl.workspace_bytes > kStaticScratchBytes)
         return fail(CANON_ERR_UNSUPPORTED,
@@ -1013,6 +1019,8 @@ CANON_API const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p)
 {
     BwdPlan pl;
     if (plan_bwd(p, &pl, false) != CANON_OK) return nullptr;
+    // (packed rows keep the name callers know for them, whichever kernel gates their taps)
+    if (p->seq_idx) return "bwd_generic";
     return pl.kind == BWD_BLC_VEC ? "bwd_blc_vec" : pl.kind == BWD_BCL_VEC ? "bwd_bcl_vec" : "bwd_generic";
 }
 

@@ -344,16 +344,34 @@ __device__ __forceinline__ void bwd_dz(const float (*w)[W], const float *bias, c
     }
 }
 
+// ... where rows of the window may belong to another packed sequence (keep: whether they belong to this step's)
+template <int W, int E, bool ACT>
+__device__ __forceinline__ void bwd_dz_gated(const float (*w)[W], const float *bias, const float *x0, const float *x1,
+                                             const float *x2, const float *x3, bool keep0, bool keep1, bool keep2,
+                                             const float *g, float *dz)
+{
+    float y[3][E];
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        y[0][e] = keep0 ? x0[e] : 0.0f;
+        y[1][e] = keep1 ? x1[e] : 0.0f;
+        y[2][e] = keep2 ? x2[e] : 0.0f;
+    }
+    bwd_dz<W, E, ACT>(w, bias, y[0], y[1], y[2], x3, g, dz);
+}
+
 // The sweep over one slab, last step first.  X / H hold xm in storage bits, dzh the dz of the
 // first three steps (already zero past the end of the sequence), dzf the dz of the three steps
 // after the slab.  FULL: all R steps exist.  FIN: some steps of the slab were captured into the final state
 // (slot t - fin_first for t >= fin_first = L - S_out) and get that slot's gradient, read at `fin` (the lane's
 // first channel of slot 0) where it is needed: at most S_out steps per sequence.
-template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E>
+// SEQ: rows of several packed sequences in reach; q[j] is the sequence index of slab row j - 3 (rows -3 .. R+2).
+template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E, bool SEQ = false>
 __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W], const float *bias, const BVT *X,
                                           const BVT *H, const BVT *G, const float *mm, const float (*dzh)[E],
                                           float (*dzf)[E], float (*dw)[W], float *dbs, char *dxp, int64_t ds, int rows,
-                                          bool active, const char *fin = nullptr, int64_t fin_first_row = 0)
+                                          bool active, const char *fin = nullptr, int64_t fin_first_row = 0,
+                                          const int32_t *q = nullptr)
 {
     float xw[4][E];   // xm of rows r-3 .. r
 #pragma unroll
@@ -367,8 +385,23 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
     for (int r = R - 1; r >= 0; --r) {
         float g[E], dz[E], o[E];
         unpack_half<DT>(G[r], g);
+        // the window and the three later dz as this row sees them: rows of another sequence read as zero
+        float xg[SEQ ? 3 : 1][E], dg[SEQ ? 3 : 1][E];
+        if constexpr (SEQ) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const bool before = q[r + k] == q[r + 3], after = q[r + 4 + k] == q[r + 3];
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    xg[k][e] = before ? xw[k][e] : 0.0f;
+                    dg[k][e] = after ? dzf[k][e] : 0.0f;
+                }
+            }
+        }
+        const float (*xv)[E] = SEQ ? xg : xw;      // rows r-3, r-2, r-1
+        const float (*dv)[E] = SEQ ? dg : dzf;     // dz of rows r+1, r+2, r+3
         if (r >= 3 || !ACT) {
-            bwd_dz<W, E, ACT>(w, bias, xw[0], xw[1], xw[2], xw[3], g, dz);
+            bwd_dz<W, E, ACT>(w, bias, xv[0], xv[1], xv[2], xw[3], g, dz);
             if constexpr (!FULL) {
 #pragma unroll
                 for (int e = 0; e < E; ++e) dz[e] = r < rows ? dz[e] : 0.0f;
@@ -380,12 +413,13 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             float acc = w[e][W - 1] * dz[e];
-            acc = fmaf(w[e][W - 2], dzf[0][e], acc);
-            if constexpr (W >= 3) acc = fmaf(w[e][W - 3], dzf[1][e], acc);
-            if constexpr (W == 4) acc = fmaf(w[e][0], dzf[2][e], acc);
+            acc = fmaf(w[e][W - 2], dv[0][e], acc);
+            if constexpr (W >= 3) acc = fmaf(w[e][W - 3], dv[1][e], acc);
+            if constexpr (W == 4) acc = fmaf(w[e][0], dv[2][e], acc);
             o[e] = acc;
 #pragma unroll
-            for (int k = 0; k < W; ++k) dw[e][k] = fmaf(dz[e], xw[(4 - W) + k][e], dw[e][k]);
+            for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], xv[(4 - W) + k][e], dw[e][k]);
+            dw[e][W - 1] = fmaf(dz[e], xw[3][e], dw[e][W - 1]);
             dbs[e] += dz[e];
             dzf[2][e] = dzf[1][e];
             dzf[1][e] = dzf[0][e];
@@ -432,9 +466,17 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 // STATES: the call has an initial state or the gradient of a captured final state.  Its own instances: as
 // run-time branches of one kernel the three pieces of code cost every call 30 registers and 100 scalar spills
 // (B 8, C 3456, L 1024 without states: 38 -> 41 us).
-template <int DT, int W, bool MASK, bool ACT, bool STATES>
+//
+// SEQ: the call carries sequence indices of packed rows (seq_idx; no states then).  They are staged in LDS like the
+// mask.  A slab whose reach (three rows before it to three after) lies in one sequence, which is nearly every slab
+// of rows packed from documents of hundreds of tokens, takes the ordinary sweep after one ballot; only a slab with a
+// boundary in reach takes the sweep that gates each tap.  The walk kernel, which gates every row and reads two bytes
+// per lane, took 192 us at B 2, C 3456, L 8192, bf16, SiLU (the whole training
+// call 233.0 us with it, 131.4 us with this one).
+template <int DT, int W, bool MASK, bool ACT, bool STATES, bool SEQ = false>
 __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 {
+    static_assert(!(STATES && SEQ), "seq_idx excludes states");
     constexpr int BY = Elem<DT>::bytes;
     constexpr int E = kBwdVecBytes / BY;
     constexpr int R = kBwdSlab, NW = kBwdWaves;
@@ -450,6 +492,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     // time loop (after the first store to dx) the compiler can no longer use scalar loads for them, and
     // as vector loads in the tile's load group they cost 20 % of the kernel.
     __shared__ float smask[MASK ? kBwdMaxChunk + 6 : 1];
+    __shared__ int32_t sseq[SEQ ? kBwdMaxChunk + 6 : 1];   // sequence indices of the same steps
 
     // blockIdx = (b * nchunk + ch) * nct + ct : channel tile fastest, i.e. memory order
     const uint32_t bc = fdiv(blockIdx.x, a.div_nct);
@@ -473,11 +516,12 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     RawTaps<E> rawt;
     fetch_taps<W, E>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c0, rawt);
     float w[E][W], bias[E];
-    if constexpr (MASK) {
+    if constexpr (MASK || SEQ) {
         for (uint32_t i = threadIdx.x; i < a.chunk + 6u; i += 64u * NW) {
             int64_t t = t_chunk - 3 + (int64_t)i;
             t = t < 0 ? 0 : (t > Lm1 ? Lm1 : t);
-            smask[i] = load_mask(a.mask, (int64_t)b * a.m_sb + t * a.m_sl, a.mask_dtype);
+            if constexpr (MASK) smask[i] = load_mask(a.mask, (int64_t)b * a.m_sb + t * a.m_sl, a.mask_dtype);
+            if constexpr (SEQ) sseq[i] = a.seq[(int64_t)b * a.q_sb + t * a.q_sl];
         }
         __syncthreads();
     }
@@ -541,7 +585,13 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
             for (int j = 0; j < 3; ++j) {
                 float g[E], d[E];
                 unpack_half<DT>(GE[j], g);
-                bwd_dz<W, E, ACT>(w, bias, xt[j], xt[j + 1], xt[j + 2], xt[j + 3], g, d);
+                if constexpr (SEQ) {
+                    const int32_t *q = sseq + a.chunk;      // steps te-3 .. te+2
+                    bwd_dz_gated<W, E, ACT>(w, bias, xt[j], xt[j + 1], xt[j + 2], xt[j + 3], q[j] == q[j + 3],
+                                            q[j + 1] == q[j + 3], q[j + 2] == q[j + 3], g, d);
+                } else {
+                    bwd_dz<W, E, ACT>(w, bias, xt[j], xt[j + 1], xt[j + 2], xt[j + 3], g, d);
+                }
                 const bool inside = te + j <= Lm1;
 #pragma unroll
                 for (int e = 0; e < E; ++e) headdz[0][j][e][lane] = inside ? d[e] : 0.0f;
@@ -588,6 +638,13 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
             const uint32_t first = ((uint32_t)it * NW + wv) * R;   // index of step t0 - 3 in smask
 #pragma unroll
             for (int j = 0; j < R + 3; ++j) mm[j] = smask[first + j];
+        }
+        // SEQ: indices of steps t0-3 .. t0+R+2, one per lane, and whether they are all the same
+        int32_t q_lane = 0;
+        bool one_seq = true;
+        if constexpr (SEQ) {
+            q_lane = sseq[((uint32_t)it * NW + wv) * R + (uint32_t)(lane < R + 6 ? lane : R + 5)];
+            one_seq = __builtin_amdgcn_ballot_w64(q_lane != __builtin_amdgcn_readfirstlane(q_lane)) == 0;
         }
 
         // dz of the three steps after the slab; the last wave's are the previous iteration's head of wave 0
@@ -672,7 +729,15 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
                 for (int j = 0; j < 3; ++j) {
                     float g[E];
                     unpack_half<DT>(G[j], g);
-                    bwd_dz<W, E, ACT>(w, bias, xq[j], xq[j + 1], xq[j + 2], xq[j + 3], g, dzh[j]);
+                    if (SEQ && !one_seq) {
+                        const int32_t own = __builtin_amdgcn_readlane(q_lane, j + 3);
+                        bwd_dz_gated<W, E, ACT>(w, bias, xq[j], xq[j + 1], xq[j + 2], xq[j + 3],
+                                                __builtin_amdgcn_readlane(q_lane, j) == own,
+                                                __builtin_amdgcn_readlane(q_lane, j + 1) == own,
+                                                __builtin_amdgcn_readlane(q_lane, j + 2) == own, g, dzh[j]);
+                    } else {
+                        bwd_dz<W, E, ACT>(w, bias, xq[j], xq[j + 1], xq[j + 2], xq[j + 3], g, dzh[j]);
+                    }
 #pragma unroll
                     for (int e = 0; e < E; ++e) {
                         dzh[j][e] = j < rows ? dzh[j][e] : 0.0f;
@@ -696,6 +761,12 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
             const char *fin = a.dfin + ((int64_t)b * a.k_sb + (int64_t)c0 * a.k_sc) * BY;
             bwd_sweep<DT, W, MASK, ACT, false, true, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows,
                                                            active, fin, fin_first - t0);
+        } else if (SEQ && !one_seq) {
+            int32_t q[R + 6];
+#pragma unroll
+            for (int j = 0; j < R + 6; ++j) q[j] = __builtin_amdgcn_readlane(q_lane, j);
+            bwd_sweep<DT, W, MASK, ACT, false, false, R, E, SEQ>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows,
+                                                                 active, nullptr, 0, q);
         } else if (rows == R)
             bwd_sweep<DT, W, MASK, ACT, true, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows, active);
         else
@@ -1304,7 +1375,10 @@ template <int DT, int W, bool MASK> void launch_bwd_m(const BwdPlan &pl, hipStre
     } else if (pl.kind == BWD_BLC_VEC)
     {
         const bool states = pl.args.init != nullptr || pl.args.dfin != nullptr;
-        if (pl.args.act) {
+        if (pl.args.seq) {
+            if (pl.args.act) hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, true, false, true>), g, b, 0, s, pl.args);
+            else hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, false, false, true>), g, b, 0, s, pl.args);
+        } else if (pl.args.act) {
             if (states) hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, true, true>), g, b, 0, s, pl.args);
             else hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, true, false>), g, b, 0, s, pl.args);
         } else {
