@@ -324,6 +324,46 @@ def test_backward_of_packed_sequences(cc, dtype, layout):
                 check(db, rdb, dtype, what + " dbias", sum_terms=B * L)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
+    """Rows that are no whole number of 16-byte vectors, or lie off 16-byte boundaries: around the shortest the
+    row kernel takes, ends inside the first, a middle and the last lane, rows of several segments (their seams), every mask type, all widths."""
+    g = torch.Generator().manual_seed(11)
+    E = 4 if dtype == torch.float32 else 8
+    masks = [None, torch.int64, torch.bool, torch.float32, torch.int32, torch.bfloat16, torch.float16]
+    cases = [(2, 5, E + 1), (3, 7, 39), (2, 5, 40), (1, 9, 41), (3, 7, 45), (2, 24, 64 * E - 1), (2, 24, 64 * E + 1), (1, 3, 128 * E + 3),
+             (2, 1030, 64 * E + E // 2), (2, 1030, 257 * E - 1), (1, 2100, 300 * E + 3), (2, 6, 16 * E), (2, 6, 80 * E)]
+    for n, (B, C, L) in enumerate(cases):
+        W, act, res = 4 - n % 3, (None, "silu")[n % 2], (False, "masked", "unmasked")[n % 3]
+        x = torch.randn(B, C, L, generator=g).to(dtype)
+        w = (torch.randn(C, W, generator=g) * 0.5).to(dtype)
+        b = (torch.randn(C, generator=g) * 0.2).to(dtype) if n % 4 else None
+        dout = torch.randn(B, C, L, generator=g).to(dtype)
+        mtype = masks[n % len(masks)]
+        mask = None
+        if mtype is not None:
+            mask = right_padded_mask([max(1, L - 3 * i) for i in range(B)], L)
+            mask[:, L // 2] = 0
+            mask = mask.to(mtype)
+        rdx, rdw, rdb, rout = conv1d_grads(x, w, b, dout, mask, act, res)
+        for offset in (0, 3):          # 3: the same rows three elements into a buffer, in rows one element longer
+            xg = x.to(DEV)
+            if offset:
+                buf = torch.zeros(offset + B * C * (L + 1), dtype=dtype, device=DEV)
+                buf[offset:].view(B, C, L + 1)[..., :L] = xg
+                xg = buf[offset:].view(B, C, L + 1)[..., :L]
+            xg = xg.detach().requires_grad_()
+            wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
+            out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
+            grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))
+            what = f"{dtype} {B}x{C}x{L} W{W} {act} {res} {mtype} offset {offset}"
+            check(out, rout, dtype, what + " out")
+            check(grads[0], rdx, dtype, what + " dx")
+            check(grads[1], rdw, dtype, what + " dweight", sum_terms=B * L)
+            if b is not None:
+                check(grads[2], rdb, dtype, what + " dbias", sum_terms=B * L)
+
+
 @pytest.mark.parametrize("dtype,act,masked", [(torch.bfloat16, "silu", False), (torch.bfloat16, None, True), (torch.float32, "silu", True)])
 def test_backward_of_packed_sequences_in_chunks_of_several_tiles(cc, dtype, act, masked):
     """Enough columns that one block walks a whole row (three tiles of 32 steps and a part of one): boundaries between

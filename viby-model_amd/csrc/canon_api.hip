@@ -165,7 +165,7 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     a.m_vec = mask_run_aligned(p->mask, p->mask_dtype, p->mask_stride_b, p->mask_stride_l, p->x_dtype);
     a.b_pair = p->bias && ((uintptr_t)p->bias & 3u) == 0 && (p->w_dtype == CANON_DTYPE_F32 || p->channels % 2 == 0);
     plan->U = 1;
-    plan->edge = false;
+    plan->ragged = false;
     plan->wpb = 4;
     plan->grid = 0;
     plan->kind = FWD_GENERIC;
@@ -182,9 +182,9 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     const bool bcl_rows = !p->seq_idx && ptr_ok && a.x_sl == 1 && a.o_sl == 1 && a.L / E >= kBclMinVectors;
     // every row starts on a 16-byte boundary and is a whole number of vectors ...
     const bool bcl_aligned = a.L % E == 0 && a.x_sb % E == 0 && a.x_sc % E == 0 && a.o_sb % E == 0 && a.o_sc % E == 0;
-    // ... or x and out share one geometry, so that a row is misaligned by the same amount in both
-    const bool bcl_edge = !bcl_aligned && a.x_sb == a.o_sb && a.x_sc == a.o_sc && a.x_sb >= 0 && a.x_sc >= 0;
-    const bool bcl_ok = bcl_rows && (bcl_aligned || bcl_edge);
+    // ... or x and out share one geometry (the kernel's ragged variant, accesses at the elements' own alignment)
+    const bool bcl_ragged = !bcl_aligned && a.x_sb == a.o_sb && a.x_sc == a.o_sc && a.x_sb >= 0 && a.x_sc >= 0;
+    const bool bcl_ok = bcl_rows && (bcl_aligned || bcl_ragged);
     const uint32_t EB = kBlcVecBytes / elem_bytes(p->x_dtype);   // channels per lane of the channel-contiguous kernel
     const bool ptr8_ok = (((uintptr_t)p->x | (uintptr_t)p->out) & (kBlcVecBytes - 1)) == 0;
     const bool blc_ok = ptr8_ok && a.x_sc == 1 && a.o_sc == 1 && a.C % EB == 0 &&
@@ -219,7 +219,7 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         return CANON_OK;
     }
     if (bcl_ok) {
-        const uint32_t nvec = a.L / E;
+        const uint32_t nvec = (a.L + E - 1) / E;
         // vectors per lane (1, 2 or 4): the fewest that reach the smallest number of segments per row while
         // >= 2048 waves stay in flight.  Every segment after a row's first re-reads its three inputs of history
         // from memory after the wave's own loads, a second round trip: rows of 144..192 vectors as three
@@ -239,7 +239,8 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         if (ntasks < (1ull << 31)) {
             plan->kind = FWD_BCL;
             plan->U = U;
-            plan->edge = !bcl_aligned;
+            plan->ragged = !bcl_aligned;
+            if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
             a.nvec = nvec; a.nseg = (uint32_t)nseg; a.ntasks = (uint32_t)ntasks;
             a.div_nseg = make_fastdiv(a.nseg); a.div_C = make_fastdiv(a.C);
                         // (measured at C 3456, L 1024, bf16: unmasked B 8 / 32 in blocks of 8 waves -0.1 / -0.9 us against 4;
@@ -611,6 +612,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     a.w_vec = p->width == 4 && p->w_stride_k == 1 && p->w_stride_c == 4 && aligned16(p->weight);
     plan->kind = BWD_GENERIC;
     plan->U = 1;
+    plan->ragged = plan->walk_too = false;
     plan->grid = 0;
     plan->workspace_bytes = 0;
     if (empty) return CANON_OK;   // the caller's dweight/dbias are zero filled by canon_conv1d_bwd
@@ -623,15 +625,24 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     // kernel and the channel-contiguous one
     const bool packed = p->seq_idx != nullptr;
     const bool states = p->initial_state != nullptr || p->dfinal_state != nullptr;
-    const bool rows = !force_generic && !packed && !states && ptrs16 && a.x_sl == 1 && a.g_sl == 1 && a.d_sl == 1 && a.L % E == 0 && a.L / E >= 16 &&
-                      a.x_sb % E == 0 && a.x_sc % E == 0 && a.g_sb % E == 0 && a.g_sc % E == 0 &&
-                      a.d_sb % E == 0 && a.d_sc % E == 0 &&
-                      // the kernel receives the batch and channel strides of x and dout in vectors, as 32-bit leading scalars
+    const bool rows_any = !force_generic && !packed && !states && a.x_sl == 1 && a.g_sl == 1 && a.d_sl == 1;
+    // whole vectors on 16-byte boundaries ...
+    const bool rows_aligned = rows_any && ptrs16 && a.L % E == 0 && a.L / E >= 16 && a.x_sb % E == 0 && a.x_sc % E == 0 &&
+                              a.g_sb % E == 0 && a.g_sc % E == 0 && a.d_sb % E == 0 && a.d_sc % E == 0;
+    // ... or not: the kernel's ragged variant (elements at their own alignment), for rows of at least kRaggedMinSteps.
+    // A wave per row costs the same whatever the row's length, the walk kernel, whose lanes lie a row apart, pays for
+    // every step: measured at 30720 rows, bf16: L 24 15.6 against 10.2 us, L 64 16.1 against 30.0, L 120 16.6 against
+    // 62.8, L 500 20.0 against 272; fp32 with mask and SiLU: L 30 17.6 against 19.6 us.
+    constexpr uint32_t kRaggedMinSteps = 40;
+    const int64_t unit = rows_aligned ? E : 1;
+    const uintptr_t elem_mask = (uintptr_t)elem_bytes(p->x_dtype) - 1;
+    const bool rows = rows_any && (rows_aligned || (a.L >= kRaggedMinSteps && (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0)) &&
+                      // the kernel receives the batch and channel strides of x and dout as 32-bit leading scalars
                       a.x_sb >= 0 && a.x_sc >= 0 && a.g_sb >= 0 && a.g_sc >= 0 &&
-                      (uint64_t)(a.x_sb / E) < (1ull << 32) && (uint64_t)(a.x_sc / E) < (1ull << 32) &&
-                      (uint64_t)(a.g_sb / E) < (1ull << 32) && (uint64_t)(a.g_sc / E) < (1ull << 32);
+                      (uint64_t)(a.x_sb / unit) < (1ull << 32) && (uint64_t)(a.x_sc / unit) < (1ull << 32) &&
+                      (uint64_t)(a.g_sb / unit) < (1ull << 32) && (uint64_t)(a.g_sc / unit) < (1ull << 32);
     if (rows) {
-        const uint32_t nvec = a.L / E;
+        const uint32_t nvec = (a.L + E - 1) / E;
         const uint64_t nrows = (uint64_t)a.B * a.C;
         // vectors per lane: the fewest that reach the smallest number of segments per row (see plan_fwd)
         int U = 1;
@@ -646,6 +657,8 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         const uint64_t nseg = (nvec + 64u * U - 1) / (64u * U);
         const uint64_t ntasks = nrows * nseg;
         if (ntasks < (1ull << 31)) {
+            plan->ragged = plan->walk_too = !rows_aligned;
+            if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
             plan->kind = BWD_BCL_VEC;
             plan->U = U;
             // field use in this kernel family: nthreads = wave tasks, nchunk = segments per row
@@ -699,12 +712,9 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
             }
         }
         const uint64_t blocks = (uint64_t)a.B * nchunk * nct;
-        // Packed rows: the walk kernel cuts long rows into fewer partial sets when there are many channels, so a scratch
-        // that holds its sets may be too small for these; such a call keeps the walk kernel.
-        const int64_t need = (int64_t)a.B * nchunk * a.C * 5 * (int64_t)sizeof(float);
-        const bool short_scratch = packed && check_pointers && p->workspace_bytes < need;
-        if (blocks < (1ull << 31) && !short_scratch) {
+        if (blocks < (1ull << 31)) {
             plan->kind = BWD_BLC_VEC;
+            plan->walk_too = packed;
             a.nvec = nvec; a.nct = nct; a.chunk = chunk; a.nchunk = nchunk;
             a.nsets = a.B * nchunk;
             a.div_nct = make_fastdiv(nct); a.div_nchunk = make_fastdiv(nchunk);
@@ -893,7 +903,17 @@ CANON_API int canon_conv1d_update(const canon_conv1d_update_params *p, void *str
 CANON_API int canon_conv1d_bwd(const canon_conv1d_bwd_params *p, void *stream)
 {
     BwdPlan pl;
-    const int rc = plan_bwd(p, &pl, true);
+    pl.walk_too = false;
+    int rc = plan_bwd(p, &pl, true);
+    if (rc != CANON_OK && pl.walk_too && p->workspace && aligned16(p->workspace)) {
+        // packed or ragged rows: the walk kernel cuts long rows into fewer partial sets where there are many channels,
+        // so a scratch that is too small for the plan's kernel may still hold its sets
+        BwdPlan walk;
+        if (plan_bwd(p, &walk, false, true) == CANON_OK && p->workspace_bytes >= walk.workspace_bytes) {
+            pl = walk;
+            rc = CANON_OK;
+        }
+    }
     if (rc != CANON_OK) return rc;
     hipStream_t s = (hipStream_t)stream;
     if (pl.grid == 0) {
@@ -977,8 +997,8 @@ CANON_API int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *st
     q.workspace_bytes = kStaticScratchBytes;
     BwdPlan pl;
     rc = plan_bwd(&q, &pl, false);
-    if (rc == CANON_OK && pl.workspace_bytes > kStaticScratchBytes && p->seq_idx)
-        rc = plan_bwd(&q, &pl, false, true);   // fewer partial sets; plan_bwd makes the same choice at the launch
+    if (rc == CANON_OK && pl.workspace_bytes > kStaticScratchBytes && pl.walk_too)
+        rc = plan_bwd(&q, &pl, false, true);   // what canon_conv1d_bwd falls back to
     if (rc != CANON_OK) return rc;
     if (pl.workspace_bytes > kStaticScratchBytes)
         return fail(CANON_ERR_UNSUPPORTED,
@@ -1019,8 +1039,8 @@ CANON_API const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p)
 {
     BwdPlan pl;
     if (plan_bwd(p, &pl, false) != CANON_OK) return nullptr;
-    // (packed rows keep the name callers know for them, whichever kernel gates their taps)
-    if (p->seq_idx) return "bwd_generic";
+    // (packed and ragged rows keep the name callers know for them, whichever kernel takes them)
+    if (pl.walk_too) return "bwd_generic";
     return pl.kind == BWD_BLC_VEC ? "bwd_blc_vec" : pl.kind == BWD_BCL_VEC ? "bwd_bcl_vec" : "bwd_generic";
 }
 

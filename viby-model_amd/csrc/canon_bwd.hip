@@ -863,11 +863,14 @@ __device__ __forceinline__ float wave_sum(float v)
 // registers with the wave (kernel-argument preload), so the loads are issued without a read of the argument block in
 // front of them, as in the forward kernel.  g_sb / g_sc: the strides of dout when they differ from x's, else a copy
 // of x's; `divC_s`: s1 | s2 << 1 of the division by C.
-template <int DT, int W, int U, bool MASK>
+// RAGGED: rows of any length from E and any alignment, as in the forward kernel (`len` is then the length in elements
+// and the strides are in elements, else both are in vectors).  Such rows took the walk kernel, whose lanes lie a row
+// apart: B 8, C 960, L 1021, bf16 162 -> 12.0 us, as fast as whole vectors (L 1024: 12.5 us with a mask).
+template <int DT, int W, int U, bool MASK, bool RAGGED>
 __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, const char *g_base, uint32_t x_sb32,
                                                             uint32_t x_sc32, uint32_t g_sb32, uint32_t g_sc32,
                                                             uint32_t nthreads, uint32_t nchunk, uint32_t C, uint32_t divC_m,
-                                                            uint32_t divC_s, uint32_t nvec, const BwdArgs a)
+                                                            uint32_t divC_s, uint32_t len, const BwdArgs a)
 {
     constexpr int E = Elem<DT>::per_vec;
     constexpr int BY = Elem<DT>::bytes;
@@ -882,9 +885,10 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
     const uint32_t b = fdiv(row, FastDiv{C, divC_m, divC_s & 1u, divC_s >> 1});
     const uint32_t c = row - b * C;
 
-    // (strides in vectors of E elements: the planner takes this kernel only for rows that start on 16-byte boundaries)
-    const char *xrow = x_base + ((int64_t)b * x_sb32 + (int64_t)c * x_sc32) * 16;
-    const char *grow = g_base + ((int64_t)b * g_sb32 + (int64_t)c * g_sc32) * 16;
+    constexpr int UNIT = RAGGED ? BY : 16;   // bytes the strides count in
+    const char *xrow = x_base + ((int64_t)b * x_sb32 + (int64_t)c * x_sc32) * UNIT;
+    const char *grow = g_base + ((int64_t)b * g_sb32 + (int64_t)c * g_sc32) * UNIT;
+    const uint32_t nvec = len;
     char *drow = a.dx + ((int64_t)b * a.d_sb + (int64_t)c * a.d_sc) * BY;
     const uint32_t v0 = seg * (64u * U) + lane;
 
@@ -892,9 +896,15 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint32_t v = v0 + u * 64u;
-        const uint32_t vc = v < nvec ? v : nvec - 1u;
-        X[u] = load_vec<kBwdStream>(xrow + (int64_t)vc * 16);
-        G[u] = load_vec<kBwdStream>(grow + (int64_t)vc * 16);
+        if constexpr (RAGGED) {
+            const int64_t off = (int64_t)row_clamp<E>(v * E, len) * BY;
+            X[u] = load_vec_any<kBwdStream>(xrow + off);
+            G[u] = load_vec_any<kBwdStream>(grow + off);
+        } else {
+            const uint32_t vc = v < nvec ? v : nvec - 1u;
+            X[u] = load_vec<kBwdStream>(xrow + (int64_t)vc * 16);
+            G[u] = load_vec<kBwdStream>(grow + (int64_t)vc * 16);
+        }
     }
     RawTaps<1> raw;
     fetch_taps_uniform<W>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, a.b_pair != 0, c, raw);
@@ -904,9 +914,22 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t v = v0 + u * 64u;
-            mbase[u] = b * a.m_sb + (int64_t)(v < nvec ? v : nvec - 1u) * E * a.m_sl;
+            const uint32_t first = RAGGED ? row_clamp<E>(v * E, len) : (v < nvec ? v : nvec - 1u) * E;
+            mbase[u] = b * a.m_sb + (int64_t)first * a.m_sl;
         }
         load_mask_vec<E, U>(a.mask, mbase, a.m_sl, a.mask_dtype, a.m_vec != 0, M);
+    }
+    if constexpr (RAGGED) {
+        // the wave that holds the end of the row undoes the move of its last vectors (zeros past the end)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t gap = row_gap<E>((v0 + u * 64u) * E, len);
+            if (__builtin_amdgcn_ballot_w64(gap != 0) != 0) {
+                X[u] = shift_down<DT>(X[u], gap);
+                G[u] = shift_down<DT>(G[u], gap);
+                if constexpr (MASK) shift_down<E>(M[u], gap);
+            }
+        }
     }
     float w[1][W], bvv[1];
     decode_taps<DT, W, 1>(raw, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bvv);
@@ -958,7 +981,8 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
     for (int k = 0; k < W; ++k) dwl[k] = 0.0f;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        const bool valid = v0 + u * 64u < nvec;
+        const uint32_t first = (v0 + u * 64u) * E;
+        const bool valid = RAGGED ? first + E <= len : v0 + u * 64u < nvec;   // the whole vector
         float xr[E], xm_store[MASK ? E : 1];
         float *xm = MASK ? xm_store : xr;
         unpack_vec<DT>(X[u], xr);
@@ -994,7 +1018,7 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
         }
         if (!valid) {
 #pragma unroll
-            for (int j = 0; j < E; ++j) dz[u][j] = 0.0f;
+            for (int j = 0; j < E; ++j) dz[u][j] = RAGGED && first + j < len ? dz[u][j] : 0.0f;
         }
 #pragma unroll
         for (int j = 0; j < E; ++j) {
@@ -1039,7 +1063,8 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
 #pragma unroll
             for (int j = 0; j < E; ++j) o[j] += gg[u][j];
         }
-        if (v < nvec) store_vec<kBwdStream>(drow + (int64_t)v * 16, pack_vec<DT>(o));
+        if constexpr (RAGGED) store_row_vec<DT, kBwdStream>(drow, v * E, len, o);
+        else if (v < nvec) store_vec<kBwdStream>(drow + (int64_t)v * 16, pack_vec<DT>(o));
     }
 
     // the wave's dweight / dbias -> partial[(b * nseg + seg) * C + c][5]
@@ -1356,22 +1381,29 @@ __global__ __launch_bounds__(256) void canon_update_bwd_vec_kernel(const UpdBwdA
 // ---------------------------------------------------------------------------
 namespace {
 
+template <int DT, int W, bool MASK, bool RAGGED> void launch_bwd_bcl(const BwdPlan &pl, hipStream_t s)
+{
+    const dim3 g(pl.grid), b(256);
+    const BwdArgs &A = pl.args;
+    constexpr int64_t EV = RAGGED ? 1 : Elem<DT>::per_vec;   // strides and length in elements, or in vectors
+    switch (pl.U) {
+#define CANON_BWD_BCL_LAUNCH(UU)                                                                                         \
+    hipLaunchKernelGGL((canon_bwd_bcl_kernel<DT, W, UU, MASK, RAGGED>), g, b, 0, s, A.x, A.dy, (uint32_t)(A.x_sb / EV),  \
+                       (uint32_t)(A.x_sc / EV), (uint32_t)(A.g_sb / EV), (uint32_t)(A.g_sc / EV), A.nthreads, A.nchunk,  \
+                       A.C, A.div_nvec.m, A.div_nvec.s1 | A.div_nvec.s2 << 1, A.L / (uint32_t)EV, A)
+    case 4: CANON_BWD_BCL_LAUNCH(4); break;
+    case 2: CANON_BWD_BCL_LAUNCH(2); break;
+    default: CANON_BWD_BCL_LAUNCH(1); break;
+#undef CANON_BWD_BCL_LAUNCH
+    }
+}
+
 template <int DT, int W, bool MASK> void launch_bwd_m(const BwdPlan &pl, hipStream_t s)
 {
     const dim3 g(pl.grid), b(256);
     if (pl.kind == BWD_BCL_VEC) {
-        const BwdArgs &A = pl.args;
-        constexpr int64_t EV = Elem<DT>::per_vec;
-        switch (pl.U) {
-#define CANON_BWD_BCL_LAUNCH(UU)                                                                                         \
-    hipLaunchKernelGGL((canon_bwd_bcl_kernel<DT, W, UU, MASK>), g, b, 0, s, A.x, A.dy, (uint32_t)(A.x_sb / EV),         \
-                       (uint32_t)(A.x_sc / EV), (uint32_t)(A.g_sb / EV), (uint32_t)(A.g_sc / EV), A.nthreads, A.nchunk,  \
-                       A.C, A.div_nvec.m, A.div_nvec.s1 | A.div_nvec.s2 << 1, A.L / (uint32_t)EV, A)
-        case 4: CANON_BWD_BCL_LAUNCH(4); break;
-        case 2: CANON_BWD_BCL_LAUNCH(2); break;
-        default: CANON_BWD_BCL_LAUNCH(1); break;
-#undef CANON_BWD_BCL_LAUNCH
-        }
+        if (pl.ragged) launch_bwd_bcl<DT, W, MASK, true>(pl, s);
+        else launch_bwd_bcl<DT, W, MASK, false>(pl, s);
     } else if (pl.kind == BWD_BLC_VEC)
     {
         const bool states = pl.args.init != nullptr || pl.args.dfin != nullptr;

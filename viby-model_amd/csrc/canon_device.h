@@ -170,6 +170,71 @@ template <bool NT> __device__ __forceinline__ void store_vec(void *p, const uint
     else *(u32x4_t *)p = q;
 }
 
+// The same at any address an element may have.  Global accesses of 16 bytes need no more than their elements'
+// alignment on this target, and the compiler emits the same one instruction; what a misaligned wave pays is one more
+// cache line per kilobyte.
+typedef unsigned int u32_any_t __attribute__((aligned(1)));
+typedef unsigned int u32x2_any_t __attribute__((ext_vector_type(2), aligned(1)));
+typedef unsigned int u32x4_any_t __attribute__((ext_vector_type(4), aligned(1)));
+template <bool NT> __device__ __forceinline__ uint4 load_vec_any(const void *p)
+{
+    const u32x4_any_t *q = (const u32x4_any_t *)p;
+    u32x4_any_t v;
+    if constexpr (NT) v = __builtin_nontemporal_load(q);
+    else v = *q;
+    return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+template <bool NT> __device__ __forceinline__ void store_vec_any(void *p, const uint4 &v)
+{
+    const u32x4_any_t q = {v.x, v.y, v.z, v.w};
+    if constexpr (NT) __builtin_nontemporal_store(q, (u32x4_any_t *)p);
+    else *(u32x4_any_t *)p = q;
+}
+
+// Rows that are no whole number of 16-byte vectors: every lane loads a full vector, the one that would pass the end of
+// the row the row's last E elements instead (lanes past the end too), so all loads are issued without a branch and
+// stay inside the row.  row_gap: by how many elements the vector at element `first` of a row of L was moved back
+// (E or more: nothing of it lies in the row); the shift that undoes it and fills up with zeros:
+template <int E> __device__ __forceinline__ uint32_t row_clamp(uint32_t first, uint32_t L) { return first + E <= L ? first : L - E; }
+template <int E> __device__ __forceinline__ uint32_t row_gap(uint32_t first, uint32_t L) { return first + E <= L ? 0u : first + E - L; }
+template <int DT> __device__ __forceinline__ uint4 shift_down(uint4 v, uint32_t gap)
+{
+    constexpr uint32_t E = Elem<DT>::per_vec, PW = 4 / Elem<DT>::bytes;   // PW: elements per word
+    if (gap & (2 * PW)) v = make_uint4(v.z, v.w, 0, 0);
+    if (gap & PW) v = make_uint4(v.y, v.z, v.w, 0);
+    if (PW == 2 && (gap & 1u))
+        v = make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, 16), __builtin_amdgcn_alignbit(v.z, v.y, 16),
+                       __builtin_amdgcn_alignbit(v.w, v.z, 16), v.w >> 16);
+    if (gap >= E) v = make_uint4(0, 0, 0, 0);
+    return v;
+}
+template <int E> __device__ __forceinline__ void shift_down(float *m, uint32_t gap)
+{
+#pragma unroll
+    for (uint32_t n = 1; n < (uint32_t)E; n *= 2) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            const float up = j + (int)n < E ? m[j + (int)n < E ? j + n : 0] : 0.0f;
+            m[j] = (gap & n) ? up : m[j];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < E; ++j) m[j] = gap >= (uint32_t)E ? 0.0f : m[j];
+}
+// ... and the store: the row's last vector element by element
+template <int DT, bool NT> __device__ __forceinline__ void store_row_vec(char *row, uint32_t first, uint32_t L, const float *o)
+{
+    constexpr int E = Elem<DT>::per_vec;
+    if (first + E <= L) {
+        store_vec_any<NT>(row + (int64_t)first * Elem<DT>::bytes, pack_vec<DT>(o));
+    } else if (first < L) {
+#pragma unroll
+        for (int j = 0; j < E - 1; ++j)
+            if (first + j < L) store1<DT>(row, (int64_t)first + j, o[j]);
+    }
+}
+
 // (float) of N 64-bit integers given as word pairs.  When every value of the whole wave fits 32 bits (the
 // usual 0/1 mask) it is one conversion instruction each; otherwise the full conversions run one after the
 // other.  Written as per-value selects, the N full conversions are scheduled side by side and their
@@ -445,9 +510,9 @@ __device__ __forceinline__ void load_seq_rows(const int32_t *p, int64_t row_base
 // U runs of N (4 or 8) consecutive mask entries, run u starting at element
 // base[u].  The element-type switch sits outside the loops and every case is
 // straight-line code, so all loads are issued back to back and waited for
-// once.  `vec` (decided on the host) says the entries are contiguous and each
-// run is aligned to its own size: it is fetched with a few wide loads instead
-// of N narrow ones.
+// once.  `vec` (decided on the host) says the entries are contiguous: a run is
+// fetched with a few wide loads instead of N narrow ones (U8 runs and rows of
+// whole vectors: aligned to their own size as well).
 template <int N, int U>
 __device__ __forceinline__ void load_mask_vec(const void *p, const int64_t *base, int64_t stride, int dt, bool vec,
                                               float (*m)[N])
@@ -459,7 +524,7 @@ __device__ __forceinline__ void load_mask_vec(const void *p, const int64_t *base
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int i = 0; i < N / 4; ++i) q[u][i] = ((const uint32_t *)((const uint8_t *)p + base[u]))[i];
+                for (int i = 0; i < N / 4; ++i) q[u][i] = ((const u32_any_t *)((const uint8_t *)p + base[u]))[i];
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -471,7 +536,7 @@ __device__ __forceinline__ void load_mask_vec(const void *p, const int64_t *base
             for (int u = 0; u < U; ++u) {   // one vector at a time, as for int64 below
                 uint4 q[N / 4 > 0 ? N / 4 : 1];   // (N < 4 never takes the vector path)
 #pragma unroll
-                for (int i = 0; i < N / 4; ++i) q[i] = ((const uint4 *)((const int32_t *)p + base[u]))[i];
+                for (int i = 0; i < N / 4; ++i) q[i] = load_vec_any<false>((const char *)((const int32_t *)p + base[u]) + 16 * i);
 #pragma unroll
                 for (int i = 0; i < N / 4; ++i) {
                     m[u][4 * i] = (float)(int32_t)q[i].x; m[u][4 * i + 1] = (float)(int32_t)q[i].y;
@@ -488,7 +553,7 @@ __device__ __forceinline__ void load_mask_vec(const void *p, const int64_t *base
             for (int u = 0; u < U; ++u) {
                 uint4 q[N / 2 > 0 ? N / 2 : 1];
 #pragma unroll
-                for (int i = 0; i < N / 2; ++i) q[i] = ((const uint4 *)((const int64_t *)p + base[u]))[i];
+                for (int i = 0; i < N / 2; ++i) q[i] = load_vec_any<false>((const char *)((const int64_t *)p + base[u]) + 16 * i);
                 uint32_t lo[N], hi[N];
 #pragma unroll
                 for (int i = 0; i < N / 2; ++i) {
@@ -505,7 +570,7 @@ __device__ __forceinline__ void load_mask_vec(const void *p, const int64_t *base
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int i = 0; i < N / 4; ++i) q[u][i] = ((const uint4 *)((const float *)p + base[u]))[i];
+                for (int i = 0; i < N / 4; ++i) q[u][i] = load_vec_any<false>((const char *)((const float *)p + base[u]) + 16 * i);
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -520,10 +585,10 @@ __device__ __forceinline__ void load_mask_vec(const void *p, const int64_t *base
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if constexpr (N == 8) {
-                    const uint4 v = *(const uint4 *)((const uint16_t *)p + base[u]);
+                    const uint4 v = load_vec_any<false>((const uint16_t *)p + base[u]);
                     q[u][0] = v.x; q[u][1] = v.y; q[u][2 % (N / 2)] = v.z; q[u][3 % (N / 2)] = v.w;
                 } else {
-                    const uint2 v = *(const uint2 *)((const uint16_t *)p + base[u]);
+                    const u32x2_any_t v = *(const u32x2_any_t *)((const uint16_t *)p + base[u]);
                     q[u][0] = v.x; q[u][1] = v.y;
                 }
             }

@@ -31,66 +31,10 @@ namespace canon {
 // unmasked path is ~130 VALU instructions per 2 KB row and hides under the
 // memory time.
 // ---------------------------------------------------------------------------
-// One element of the row computed on its own (the few elements of a row that do not fill an aligned
-// 16-byte vector, see EDGE below): scalar loads of its window, same arithmetic.  The loads are
-// issued with the row's vector loads (bcl_edge_issue) and consumed after the vector work
-// (bcl_edge_finish), so they cost the wave no round trip of their own.
-struct EdgeWindow {
-    float x[4];   // raw x[t-3 .. t] (0 where t-3+k < 0 and there is no initial state)
-    float m[4];   // their mask entries
-};
-
-template <int DT, int W, bool MASK>
-__device__ __forceinline__ void bcl_edge_issue(const FwdArgs &a, const char *xrow, uint32_t b, uint32_t c, int64_t t,
-                                               EdgeWindow &e)
-{
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        e.x[k] = 0.0f;
-        e.m[k] = 1.0f;
-    }
-#pragma unroll
-    for (int k = 4 - W; k < 4; ++k) {
-        const int64_t tt = t - 3 + k;
-        if (tt >= 0) e.x[k] = load1<DT>(xrow, tt);
-        else if (a.init) e.x[k] = load1<DT>(a.init, b * a.i_sb + c * a.i_sc + (a.S_in + tt) * a.i_ss);
-    }
-    if constexpr (MASK) {
-        // the four entries as one run from max(t-3, 0) (rows are at least 16 vectors long)
-        const int64_t first = t - 3 > 0 ? t - 3 : 0;
-        const int shift = (int)(first - (t - 3));   // 0 .. 3 window slots lie before the row
-        int64_t base[1] = {b * a.m_sb + first * a.m_sl};
-        float run[1][4];
-        load_mask_vec<4, 1>(a.mask, base, a.m_sl, a.mask_dtype, false, run);
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int j = k - shift;
-            e.m[k] = j == 0 ? run[0][0] : j == 1 ? run[0][1] : j == 2 ? run[0][2] : j == 3 ? run[0][3] : 1.0f;
-        }
-    }
-}
-
-template <int DT, int W, bool MASK>
-__device__ __forceinline__ void bcl_edge_finish(const FwdArgs &a, const float (*w)[W], float bv, char *orow, int64_t t,
-                                                const EdgeWindow &e)
-{
-    float win[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        win[k] = e.x[k];
-        if constexpr (MASK) {
-            if (t - 3 + k >= 0) win[k] = mul_round<DT>(e.x[k], e.m[k]);   // history from the initial state is not masked
-        }
-    }
-    float acc = bv;
-#pragma unroll
-    for (int k = 0; k < W; ++k) acc = fmaf(w[0][k], win[(4 - W) + k], acc);
-    store1<DT>(orow, t, finish<DT>(acc, a.act, a.res_mode, a.eager, win[3], e.x[3]));
-}
-
 // Activation, residual and store of one 16-byte vector of accumulators.
-template <int DT, bool MASK, bool EAGER>
-__device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const float *xr, const float *xm, char *dst, bool write)
+template <int DT, bool MASK, bool EAGER, bool RAGGED = false>
+__device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const float *xr, const float *xm, char *dst, bool write,
+                                               uint32_t first = 0, uint32_t L = 0)
 {
     constexpr int E = Elem<DT>::per_vec;
     activate<DT, E>(o, a.act != 0, EAGER);
@@ -101,13 +45,16 @@ __device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const
 #pragma unroll
         for (int j = 0; j < E; ++j) o[j] += xm[j];
     }
-    if (write) store_vec<true>(dst, pack_vec<DT>(o));
+    if constexpr (RAGGED) store_row_vec<DT, true>(dst, first, L, o);   // (dst: the row)
+    else if (write) store_vec<true>(dst, pack_vec<DT>(o));
 }
 
-// EDGE: the rows are contiguous in time but do not start on 16-byte boundaries (a length or a
-// row stride that is not a multiple of E).  The aligned middle of every row runs through the
-// same vector code, shifted by `head` elements; the up to E-1 elements before it and after it
-// are computed one per lane by the waves that own the first and the last segment.
+// RAGGED: the rows are contiguous in time but are no whole number of 16-byte vectors or do not start on 16-byte
+// boundaries (a length or a row stride that is not a multiple of E).  The same code with accesses at the elements'
+// own alignment; the row's last vector is loaded from the row's last E elements and shifted into place (see row_gap),
+// and stored element by element.  (Instead of an aligned middle with the elements before and after it computed one
+// per lane, whose mask had to be read entry by entry: B 8, C 960, L 1021, bf16 8.6 -> 8.3 us, with a mask 18.7 -> 10.5;
+// B 32, L 500 19.7 -> 15.2 us; fp32, SiLU, B 4, C 960, L 1023 7.6 -> 6.6 us.)
 //
 // The scalars in front of the argument block are what a wave needs to request its row.  Scalar kernel
 // arguments at the head of the list arrive in registers with the wave (kernel-argument preload: the library is
@@ -119,11 +66,11 @@ __device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const
 // `wpb`: waves per block, 1, 4 or 8 (the waves are independent; large unmasked launches run 0.5-1 % faster in
 // blocks of 8: 19.6 -> 19.5 us at B 8, 70.0 -> 69.1 us at B 32; 16 are 7 % slower; with a mask 8 are 6-9 % slower
 // and single waves 1-2 % faster than blocks of 4).
-template <int DT, int W, int U, bool MASK, bool BIG, bool EDGE = false>
+template <int DT, int W, int U, bool MASK, bool BIG, bool RAGGED = false>
 __global__ __launch_bounds__(64 * kBclMaxWaves) void canon_fwd_bcl_kernel(const char *x_base, int64_t x_sb, int64_t x_sc,
                                                                           uint32_t ntasks, uint32_t nseg, uint32_t C,
                                                                           uint32_t divC_m, uint32_t divC_s1, uint32_t divC_s2,
-                                                                          uint32_t nvec_row, uint32_t wpb, const FwdArgs a)
+                                                                          uint32_t len, uint32_t wpb, const FwdArgs a)
 {
     constexpr int E = Elem<DT>::per_vec;
     const int lane = threadIdx.x & 63;
@@ -145,41 +92,27 @@ __global__ __launch_bounds__(64 * kBclMaxWaves) void canon_fwd_bcl_kernel(const 
     const char *xrow = x_base + row_off * Elem<DT>::bytes;
     char *orow = a.out + ((int64_t)b * a.o_sb + (int64_t)c * a.o_sc) * Elem<DT>::bytes;
     const uint32_t v0 = seg * (64u * U) + lane;
-    // head: elements of the row before its first aligned vector; nvec: aligned vectors of this row
-    uint32_t head = 0, nvec = nvec_row;
-    if constexpr (EDGE) {
-        head = (uint32_t)((E - (row_off % E)) % E);
-        if (head > a.L) head = a.L;
-        nvec = (a.L - head) / E;
-    }
-    const char *xvec = xrow + (int64_t)head * Elem<DT>::bytes;   // 16-byte aligned
-    char *ovec = orow + (int64_t)head * Elem<DT>::bytes;
+    // `len`: vectors per row, or elements per row of ragged rows
+    const uint32_t nvec = len;
 
     // row data first (the long latency), then the taps (scalar-cache hits)
     uint4 X[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint32_t v = v0 + u * 64u;
-        X[u] = make_uint4(0, 0, 0, 0);
-        if (v < nvec) X[u] = load_vec<true>(xvec + (int64_t)v * 16);
+        if constexpr (RAGGED) {
+            X[u] = load_vec_any<true>(xrow + (int64_t)row_clamp<E>(v * E, len) * Elem<DT>::bytes);
+        } else {
+            X[u] = make_uint4(0, 0, 0, 0);
+            if (v < nvec) X[u] = load_vec<true>(xrow + (int64_t)v * 16);
+        }
     }
     // a later segment's history: the vector before the segment, requested by lane 0 together with the segment itself
     // (the wave of the segment before requests the same vector at about the same time)
     uint4 P = make_uint4(0, 0, 0, 0);
-    constexpr bool kPrevVector = !MASK && !EDGE;
+    constexpr bool kPrevVector = !MASK;
     if constexpr (kPrevVector) {
-        if (seg > 0 && lane == 0) P = load_vec<false>(xvec + ((int64_t)v0 - 1) * 16);
-    }
-
-    // EDGE: lanes 0 .. head-1 of the first segment take the elements before the first vector,
-    // lanes 32 .. 32+tail-1 of the last segment the elements after the last one
-    EdgeWindow edge;
-    int64_t edge_t = -1;
-    if constexpr (EDGE) {
-        const uint32_t tail = a.L - head - nvec * E;
-        if (seg == 0 && (uint32_t)lane < head) edge_t = lane;
-        if (seg == a.nseg - 1 && lane >= 32 && (uint32_t)(lane - 32) < tail) edge_t = (int64_t)head + (int64_t)nvec * E + (lane - 32);
-        if (edge_t >= 0) bcl_edge_issue<DT, W, MASK>(a, xrow, b, c, edge_t, edge);
+        if (seg > 0 && lane == 0) P = load_vec_any<false>(xrow + ((int64_t)v0 - 1) * 16);
     }
 
     RawTaps<1> raw;
@@ -195,21 +128,30 @@ __global__ __launch_bounds__(64 * kBclMaxWaves) void canon_fwd_bcl_kernel(const 
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t v = v0 + u * 64u;
-            // idle lanes shadow the last vector (a row without any aligned vector reads from its start)
-            const int64_t vv = v < nvec ? v : (nvec ? nvec - 1u : 0u);
-            mbase[u] = b * a.m_sb + ((int64_t)head + vv * E) * a.m_sl;
-            if constexpr (EDGE) {
-                if (nvec == 0) mbase[u] = b * a.m_sb;
-            }
+            // idle lanes shadow the last vector
+            const uint32_t first = RAGGED ? row_clamp<E>(v * E, len) : (v < nvec ? v : nvec - 1u) * E;
+            mbase[u] = b * a.m_sb + (int64_t)first * a.m_sl;
         }
-        load_mask_vec<E, U>(a.mask, mbase, a.m_sl, a.mask_dtype, !EDGE && a.m_vec != 0, M);
+        load_mask_vec<E, U>(a.mask, mbase, a.m_sl, a.mask_dtype, a.m_vec != 0, M);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float xr[E], xm[E];
             unpack_vec<DT>(X[u], xr);
 #pragma unroll
             for (int j = 0; j < E; ++j) xm[j] = mul_round<DT>(xr[j], M[u][j]);
-            XM[u] = pack_vec<DT>(xm);   // exact: the products are already rounded to the storage type
+            XM[u] = pack_vec<DT>(xm);   // (ragged rows: moved into place with X, below)  exact: the products are already rounded to the storage type
+        }
+    }
+
+    if constexpr (RAGGED) {
+        // the wave that holds the end of the row undoes the move of its last vectors
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t gap = row_gap<E>((v0 + u * 64u) * E, len);
+            if (__builtin_amdgcn_ballot_w64(gap != 0) != 0) {
+                X[u] = shift_down<DT>(X[u], gap);
+                if constexpr (MASK) XM[u] = shift_down<DT>(XM[u], gap);
+            }
         }
     }
 
@@ -226,19 +168,15 @@ __global__ __launch_bounds__(64 * kBclMaxWaves) void canon_fwd_bcl_kernel(const 
         for (int j = 0; j < 3; ++j)
             if (j >= 3 - (W - 1)) carry[j] = pv[E - 3 + j];
     } else if (lane == 0) {
-        if (seg > 0 || (EDGE && head > 0)) {
-            const int64_t t0 = (int64_t)head + (int64_t)v0 * E;
+        if (seg > 0) {
+            const int64_t t0 = (int64_t)v0 * E;
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const int64_t t = t0 - 3 + j;
                 if (j < 3 - (W - 1)) continue;
-                if (t >= 0) {
-                    float v = load1<DT>(xrow, t);
-                    if constexpr (MASK) v = mul_round<DT>(v, load_mask(a.mask, b * a.m_sb + t * a.m_sl, a.mask_dtype));
-                    carry[j] = v;
-                } else if (a.init) {
-                    carry[j] = load1<DT>(a.init, b * a.i_sb + c * a.i_sc + (a.S_in + t) * a.i_ss);
-                }
+                float v = load1<DT>(xrow, t);
+                if constexpr (MASK) v = mul_round<DT>(v, load_mask(a.mask, b * a.m_sb + t * a.m_sl, a.mask_dtype));
+                carry[j] = v;
             }
         } else if (a.init) {
 #pragma unroll
@@ -278,12 +216,9 @@ __global__ __launch_bounds__(64 * kBclMaxWaves) void canon_fwd_bcl_kernel(const 
         }
         // the rounding mode is branched on around the whole epilogue, store included, so that the eager module's
         // extra roundings are not evaluated and then discarded (selects) on the usual path
-        if (a.eager) bcl_finish_vec<DT, MASK, true>(a, o, xr, xm, ovec + (int64_t)v * 16, v < nvec);
-        else bcl_finish_vec<DT, MASK, false>(a, o, xr, xm, ovec + (int64_t)v * 16, v < nvec);
-    }
-
-    if constexpr (EDGE) {
-        if (edge_t >= 0) bcl_edge_finish<DT, W, MASK>(a, w, bv, orow, edge_t, edge);
+        char *dst = RAGGED ? orow : orow + (int64_t)v * 16;
+        if (a.eager) bcl_finish_vec<DT, MASK, true, RAGGED>(a, o, xr, xm, dst, v < nvec, v * E, len);
+        else bcl_finish_vec<DT, MASK, false, RAGGED>(a, o, xr, xm, dst, v < nvec, v * E, len);
     }
 
     if (a.fin && seg == a.nseg - 1) capture_row_state<DT>(a, b, c, lane);
@@ -1066,15 +1001,15 @@ __global__ __launch_bounds__(256) void canon_fwd_generic_kernel(const FwdArgs a)
 // ---------------------------------------------------------------------------
 namespace {
 
-template <int DT, int W, bool MASK, bool BIG, bool EDGE> void launch_bcl_e(const FwdPlan &pl, hipStream_t s)
+template <int DT, int W, bool MASK, bool BIG, bool RAGGED> void launch_bcl_r(const FwdPlan &pl, hipStream_t s)
 {
     const FwdArgs &a = pl.args;
     const uint32_t wpb = pl.wpb;
     const dim3 g(pl.grid), b(64 * wpb);
     switch (pl.U) {
 #define CANON_BCL_LAUNCH(UU)                                                                                             \
-    hipLaunchKernelGGL((canon_fwd_bcl_kernel<DT, W, UU, MASK, BIG, EDGE>), g, b, 0, s, a.x, a.x_sb, a.x_sc, a.ntasks, a.nseg, \
-                       a.C, a.div_C.m, a.div_C.s1, a.div_C.s2, a.nvec, wpb, a)
+    hipLaunchKernelGGL((canon_fwd_bcl_kernel<DT, W, UU, MASK, BIG, RAGGED>), g, b, 0, s, a.x, a.x_sb, a.x_sc, a.ntasks, a.nseg, \
+                       a.C, a.div_C.m, a.div_C.s1, a.div_C.s2, RAGGED ? a.L : a.nvec, wpb, a)
     case 4: CANON_BCL_LAUNCH(4); break;
     case 2: CANON_BCL_LAUNCH(2); break;
     default: CANON_BCL_LAUNCH(1); break;
@@ -1084,8 +1019,8 @@ template <int DT, int W, bool MASK, bool BIG, bool EDGE> void launch_bcl_e(const
 
 template <int DT, int W, bool MASK, bool BIG> void launch_bcl(const FwdPlan &pl, hipStream_t s)
 {
-    if (pl.edge) launch_bcl_e<DT, W, MASK, BIG, true>(pl, s);
-    else launch_bcl_e<DT, W, MASK, BIG, false>(pl, s);
+    if (pl.ragged) launch_bcl_r<DT, W, MASK, BIG, true>(pl, s);
+    else launch_bcl_r<DT, W, MASK, BIG, false>(pl, s);
 }
 
 template <int DT, int W, bool MASK, bool BIG> void launch_fwd_vec(const FwdPlan &pl, hipStream_t s)

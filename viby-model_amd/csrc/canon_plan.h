@@ -238,7 +238,7 @@ constexpr uint32_t kBclBigLaunch = 16384;
 struct FwdPlan {
     FwdKind kind;
     int U;
-    bool edge;   // bcl: rows do not start on 16-byte boundaries
+    bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
     uint32_t wpb; // bcl: waves per block
     int rows;    // blc: time steps per wave (kBlcRows or kBlcRowsShort)
     FwdArgs args;
@@ -269,6 +269,8 @@ struct UpdPartsPlan {
 struct BwdPlan {
     BwdKind kind;
     int U;
+    bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
+    bool walk_too;   // a call that the walk kernel takes instead when the scratch is too small for this kernel's sets
     BwdArgs args;
     uint32_t grid;
     int64_t workspace_bytes;
