@@ -202,7 +202,8 @@ typedef struct canon_conv1d_bwd_params {
     int32_t width;
     int32_t activation;
     int32_t residual_mode;
-    int32_t reserved0;
+    int32_t grad_dtype;             /* element type of dweight and dbias: CANON_DTYPE_BF16 / _F16 (the fp32 sum rounded
+                                       once), anything else: fp32 */
     int64_t batch, channels, seqlen;
     const void *x;
     int64_t x_stride_b, x_stride_c, x_stride_l;
@@ -215,8 +216,8 @@ typedef struct canon_conv1d_bwd_params {
     const void *bias;               /* or NULL */
     const void *mask;               /* or NULL */
     int64_t mask_stride_b, mask_stride_l;
-    float *dweight;                 /* [channels, width] contiguous fp32 */
-    float *dbias;                   /* [channels] fp32, or NULL */
+    void *dweight;                  /* [channels, width] contiguous, fp32 or grad_dtype */
+    void *dbias;                    /* [channels], of the same type, or NULL */
     void *workspace;                /* canon_conv1d_bwd_workspace_bytes() bytes, 16-byte aligned */
     int64_t workspace_bytes;
     const int32_t *seq_idx;         /* [batch, seqlen] or NULL: the forward's packed-sequence indices */

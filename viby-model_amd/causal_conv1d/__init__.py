@@ -363,20 +363,19 @@ class _CanonConvFn(torch.autograd.Function):
             dout = torch.zeros_like(x)
         act, res = ctx.flags
         channels, width = weight.shape
-        dweight = torch.empty(channels, width, dtype=torch.float32, device=x.device)
-        dbias = torch.empty(channels, dtype=torch.float32, device=x.device) if bias is not None else None
+        dweight = torch.empty(channels, width, dtype=weight.dtype, device=x.device)
+        dbias = torch.empty(channels, dtype=weight.dtype, device=x.device) if bias is not None else None
         dinit = None
         if initial_states is not None and ctx.needs_input_grad[9]:
             dinit = torch.empty_like(initial_states)
         dx = _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx, initial_states, dinit, dfinal)
-        return (dx, dweight.to(weight.dtype), dbias.to(bias.dtype) if bias is not None else None,
-                None, None, None, None, None, None, dinit)
+        return dx, dweight, dbias, None, None, None, None, None, None, dinit
 
 
 def _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx=None, initial_states=None,
                 dinit=None, dfinal=None) -> torch.Tensor:
     """One backward launch (+ the fixed-order reduction): returns dx with x's strides and fills the
-    fp32 ``dweight`` (channels, W) / ``dbias`` (channels,) given (rows of larger tensors are fine)."""
+    ``dweight`` (channels, W) / ``dbias`` (channels,) given, both of one type (rows of larger tensors are fine)."""
     if dout.dtype != x.dtype:
         dout = dout.to(x.dtype)
     if dout.stride() != x.stride():
@@ -424,6 +423,7 @@ def _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx=N
         p.final_len = dfinal.shape[2]
     p.dweight = dweight.data_ptr()
     p.dbias = dbias.data_ptr() if dbias is not None else None
+    p.grad_dtype = _lib.DTYPE_CODE[dweight.dtype]
     L = _lib.lib()
     nbytes = L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(p))
     if nbytes < 0:
@@ -902,8 +902,8 @@ class _CanonConvPartsFn(torch.autograd.Function):
         dfinal = grads[len(xs)] if has_final else None
         channels, width = weight.shape
         dev = xs[0].device
-        dweight = torch.empty(channels, width, dtype=torch.float32, device=dev)
-        dbias = torch.empty(channels, dtype=torch.float32, device=dev) if bias is not None else None
+        dweight = torch.empty(channels, width, dtype=weight.dtype, device=dev)
+        dbias = torch.empty(channels, dtype=weight.dtype, device=dev) if bias is not None else None
         dinit = None
         if initial_states is not None and ctx.needs_input_grad[7]:
             dinit = torch.empty_like(initial_states)
@@ -918,8 +918,7 @@ class _CanonConvPartsFn(torch.autograd.Function):
                                    dinit[:, c0:c1] if dinit is not None else None,
                                    dfinal[:, c0:c1] if dfinal is not None else None))
             c0 = c1
-        return (dweight.to(weight.dtype), dbias.to(bias.dtype) if bias is not None else None,
-                None, None, None, None, None, dinit, *dxs)
+        return dweight, dbias, None, None, None, None, None, dinit, *dxs
 
 
 def causal_conv1d_update_parts(
@@ -1064,8 +1063,10 @@ def _op_bwd(x: torch.Tensor, dout: torch.Tensor, weight: torch.Tensor, bias: Opt
             dfinal: Optional[torch.Tensor], act: int, res: int
             ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     channels, width = weight.shape
-    dweight = torch.empty(channels, width, dtype=torch.float32, device=x.device)
-    dbias = torch.empty(channels if bias is not None else 0, dtype=torch.float32, device=x.device)
+    # (the operator can be called with a bias of another type than the weight's: fp32 sums then)
+    gtype = weight.dtype if bias is None or bias.dtype == weight.dtype else torch.float32
+    dweight = torch.empty(channels, width, dtype=gtype, device=x.device)
+    dbias = torch.empty(channels if bias is not None else 0, dtype=gtype, device=x.device)
     dinit = torch.empty_like(initial_states) if initial_states is not None else x.new_empty((x.shape[0], channels, 0))
     dx = _launch_bwd(x, dout, weight, bias, mask, dweight, dbias if bias is not None else None, act, res, seq_idx,
                      initial_states, dinit if initial_states is not None else None, dfinal)

@@ -66,7 +66,7 @@ class BwdParams(ctypes.Structure):
     _fields_ = [
         ("struct_size", _u32),
         ("x_dtype", _i32), ("w_dtype", _i32), ("mask_dtype", _i32),
-        ("width", _i32), ("activation", _i32), ("residual_mode", _i32), ("reserved0", _i32),
+        ("width", _i32), ("activation", _i32), ("residual_mode", _i32), ("grad_dtype", _i32),
         ("batch", _i64), ("channels", _i64), ("seqlen", _i64),
         ("x", _vp), ("x_stride_b", _i64), ("x_stride_c", _i64), ("x_stride_l", _i64),
         ("dout", _vp), ("dout_stride_b", _i64), ("dout_stride_c", _i64), ("dout_stride_l", _i64),

@@ -609,6 +609,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     a.B = (uint32_t)p->batch; a.C = (uint32_t)p->channels; a.L = (uint32_t)p->seqlen;
     a.W = p->width; a.w_dtype = p->w_dtype; a.mask_dtype = p->mask_dtype;
     a.act = p->activation; a.res_mode = p->residual_mode;
+    a.grad_dtype = p->grad_dtype == CANON_DTYPE_BF16 || p->grad_dtype == CANON_DTYPE_F16 ? p->grad_dtype : CANON_DTYPE_F32;
     a.w_vec = p->width == 4 && p->w_stride_k == 1 && p->w_stride_c == 4 && aligned16(p->weight);
     plan->kind = BWD_GENERIC;
     plan->U = 1;
@@ -920,8 +921,9 @@ CANON_API int canon_conv1d_bwd(const canon_conv1d_bwd_params *p, void *stream)
         // nothing to sum: the gradients of the parameters are zero
         // (a fill kernel rather than a memset, so that the call can be captured into a HIP graph)
         if (p->channels > 0) {
-            launch_zero(p->dweight, (uint32_t)(p->channels * p->width), s);
-            if (p->dbias) launch_zero(p->dbias, (uint32_t)p->channels, s);
+            const int bytes = elem_bytes(pl.args.grad_dtype);
+            launch_zero(p->dweight, (uint32_t)(p->channels * p->width), bytes, s);
+            if (p->dbias) launch_zero(p->dbias, (uint32_t)p->channels, bytes, s);
             return check_launch("canon_conv1d_bwd");
         }
         return CANON_OK;
@@ -1018,8 +1020,8 @@ CANON_API int canon_conv1d_update_bwd(const canon_conv1d_update_bwd_params *p, v
     if (pl.grid_c == 0) {
         // an empty batch: the parameter gradients are zero (fill kernels, so that the call can be captured)
         if (p->channels > 0 && p->dweight) {
-            launch_zero(p->dweight, (uint32_t)(p->channels * p->width), s);
-            if (p->dbias) launch_zero(p->dbias, (uint32_t)p->channels, s);
+            launch_zero(p->dweight, (uint32_t)(p->channels * p->width), 4, s);
+            if (p->dbias) launch_zero(p->dbias, (uint32_t)p->channels, 4, s);
             return check_launch("canon_conv1d_update_bwd");
         }
         return CANON_OK;

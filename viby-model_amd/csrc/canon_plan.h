@@ -112,8 +112,8 @@ struct BwdArgs {
     const void *bias;
     const void *mask;
     float *partial;
-    float *dweight;
-    float *dbias;
+    void *dweight;        // of type grad_dtype
+    void *dbias;
     const int32_t *seq;   // packed-sequence indices [B, L] or nullptr (walk kernel only)
     int64_t q_sb, q_sl;
     const char *init;     // inputs before t = 0, [B, C, S_in], or nullptr (walk and channel-contiguous kernels)
@@ -128,6 +128,7 @@ struct BwdArgs {
     int64_t m_sb, m_sl;
     uint32_t B, C, L;
     int32_t W, w_dtype, mask_dtype, act, res_mode, w_vec, b_pair, m_vec;
+    int32_t grad_dtype;
     uint32_t nvec;      // channel groups per row (C / E)
     uint32_t nchunk;    // time chunks per sequence
     uint32_t chunk;     // time steps per chunk
@@ -290,7 +291,7 @@ void launch_update(const UpdPlan &pl, int x_dtype, hipStream_t s);
 void launch_update_parts(const UpdPartsPlan &pp, int x_dtype, hipStream_t s);
 void launch_bwd(const BwdPlan &pl, int x_dtype, hipStream_t s);          // dx + partial sets, then the reduction
 void launch_update_bwd(const UpdBwdPlan &pl, int x_dtype, hipStream_t s);   // dx, dstate + partial sets, then the reduction
-void launch_zero(float *p, uint32_t n, hipStream_t s);                    // fill kernel (graph-capture safe)
+void launch_zero(void *p, uint32_t n, int elem_bytes, hipStream_t s);     // fill kernel (graph-capture safe); 2 or 4
 // Make the runtime load this translation unit's code object onto the current device now (it would otherwise do so
 // at the unit's first launch): hipSuccess or the runtime's error.
 hipError_t preload_fwd();
