@@ -324,6 +324,59 @@ def test_backward_of_packed_sequences(cc, dtype, layout):
                 check(db, rdb, dtype, what + " dbias", sum_terms=B * L)
 
 
+@pytest.mark.parametrize("kind,B,C,L,static,scratch", [
+    ("channel", 96, 1024, 640, True, None),      # 480 partial sets would not fit the static scratch, 96 do
+    ("channel", 96, 1024, 200, False, 96),       # ... nor a caller's own scratch of one set per sequence
+    ("packed", 96, 1024, 640, True, None),
+    ("packed", 96, 1024, 200, False, 96),
+    ("time", 132, 1000, 2100, False, 132)])      # rows of two segments, scratch for the walk kernel's one chunk per row
+def test_backward_with_a_scratch_for_fewer_partial_sets(cc, kind, B, C, L, static, scratch):
+    """A scratch too small for the sets of the kernel's usual split gets fewer sets, not a refusal: same dx bits, sums
+    in another order (each of B * L terms added in fp32 within a set: 1e-4 of the tensor's scale, as everywhere here)."""
+    import ctypes
+
+    from causal_conv1d import _lib
+    g = torch.Generator(device=DEV).manual_seed(5)
+    shape = (B, C, L) if kind == "time" else (B, L, C)
+    x, dout = (torch.randn(shape, device=DEV, generator=g, dtype=torch.bfloat16) for _ in range(2))
+    if kind != "time":
+        x, dout = x.transpose(1, 2), dout.transpose(1, 2)
+    w, b = torch.randn(C, 4, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+    seq = (torch.arange(L, device=DEV, dtype=torch.int32) // 37).repeat(B, 1) if kind == "packed" else None
+
+    def params(nbytes):
+        dx, dw, db = torch.empty_like(x), torch.empty(C, 4, device=DEV), torch.empty(C, device=DEV)
+        p = _lib.BwdParams(struct_size=ctypes.sizeof(_lib.BwdParams), x_dtype=1, w_dtype=0, width=4, activation=1,
+                           residual_mode=1, batch=B, channels=C, seqlen=L)
+        for name, t in (("x", x), ("dout", dout), ("dx", dx)):
+            setattr(p, name, t.data_ptr())
+            for axis, stride in zip("bcl", t.stride()):
+                setattr(p, f"{name}_stride_{axis}", stride)
+        p.weight, p.w_stride_c, p.w_stride_k, p.bias = w.data_ptr(), 4, 1, b.data_ptr()
+        p.dweight, p.dbias = dw.data_ptr(), db.data_ptr()
+        if seq is not None:
+            p.seq_idx, p.seq_stride_b, p.seq_stride_l = seq.data_ptr(), L, 1
+        space = torch.empty(nbytes, dtype=torch.uint8, device=DEV)
+        p.workspace, p.workspace_bytes = space.data_ptr(), nbytes
+        return p, dx, dw, db, space
+
+    lib, stream = _lib.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    need = lib.canon_conv1d_bwd_workspace_bytes(ctypes.byref(params(16)[0]))
+    small = scratch * C * 20 if scratch else 16
+    assert need > (8 << 20 if static else small)
+    full, few = params(need), params(small)
+    assert lib.canon_conv1d_bwd(ctypes.byref(full[0]), stream) == 0
+    call = lib.canon_conv1d_bwd_static if static else lib.canon_conv1d_bwd
+    assert call(ctypes.byref(few[0]), stream) == 0, lib.canon_conv1d_last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(full[1], few[1])
+    for i in (2, 3):
+        assert (full[i] - few[i]).abs().max().item() <= 1e-4 * full[i].abs().max().item()
+    if not static:
+        few[0].workspace_bytes = small - 4
+        assert lib.canon_conv1d_bwd(ctypes.byref(few[0]), stream) == _lib.ERR_INVALID_ARGUMENT
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
     """Rows that are no whole number of 16-byte vectors, or lie off 16-byte boundaries: around the shortest the

@@ -3,6 +3,7 @@
 // include/canon_conv1d.h.  No kernels in this file; the only device object is
 // the static scratch array of canon_conv1d_bwd_static.
 #include <stdarg.h>
+#include <algorithm>
 #include <mutex>
 #include <stdint.h>
 #include <stdio.h>
@@ -543,7 +544,42 @@ int plan_update_parts(const canon_conv1d_update_params *p, const canon_conv1d_pa
 // ---------------------------------------------------------------------------
 // check_pointers: the call itself (x, dout, dx, weight, dweight and the workspace must be there).  Without it
 // (queries) NULL pointers pass and count as aligned.  force_generic: plan the strided kernel whatever the layout.
-int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointers, bool force_generic = false)
+// How the channel-contiguous backward cuts a sequence: n chunks of len steps (whole tiles) of at most `longest`, the
+// fewest that give one and a half blocks per CU.  A block walks every tile of its chunk, so the chunks are cut equal
+// (chunks of a fixed length would leave the last one mostly empty, L = 520 as 512 + 8), and a slightly larger count
+// that cuts the tiles evenly is taken where there is one.
+struct BwdChunks {
+    uint32_t n, len;
+};
+
+BwdChunks bwd_chunks(uint32_t B, uint32_t L, uint32_t nct, uint32_t longest)
+{
+    const uint32_t tile = kBwdSlab * kBwdWaves;
+    const uint32_t tiles = (L + tile - 1) / tile;
+    BwdChunks c = {tiles, tile};
+    bool found = false;
+    for (uint32_t n = 1; n <= tiles; ++n) {
+        const uint32_t len = ((L + n - 1) / n + tile - 1) / tile * tile;
+        if (len > longest) continue;
+        const uint32_t used = (L + len - 1) / len;               // chunks of that length that hold steps
+        const bool enough = 2ull * B * used * nct >= 256ull * kBwdHalfBlocksPerCU || n == tiles;
+        if (!found && enough) {
+            found = true;
+            c = {used, len};
+            if (tiles % used == 0) break;
+            continue;
+        }
+        if (found && (n >= 2 * c.n || len < 2 * tile)) break;
+        if (found && used == n && tiles % n == 0) {
+            c = {used, len};
+            break;
+        }
+    }
+    return c;
+}
+
+// scratch: bytes of scratch the call will have, where that is known before its pointers are (-1: not)
+int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointers, bool force_generic = false, int64_t scratch = -1)
 {
     if (!p) return fail(CANON_ERR_INVALID_ARGUMENT, "params is NULL");
     if (p->struct_size != sizeof(canon_conv1d_bwd_params))
@@ -674,53 +710,40 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
             return CANON_OK;
         }
     }
-    // channel-contiguous tensors: a group of kBwdVecBytes of adjacent channels per lane
-    const int E8 = kBwdVecBytes / elem_bytes(p->x_dtype);
-    const bool ptrs8 = (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & (uintptr_t)(kBwdVecBytes - 1)) == 0;
+    // channel-contiguous tensors on 8-byte boundaries, rows of whole 8-byte groups
+    const int E8 = 8 / elem_bytes(p->x_dtype);
+    const bool ptrs8 = (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & 7u) == 0;
     const bool vec = !force_generic && a.x_sc == 1 && a.g_sc == 1 && a.d_sc == 1 && a.C % E8 == 0 && a.x_sl != 1 &&
                      a.x_sb % E8 == 0 && a.x_sl % E8 == 0 && a.g_sb % E8 == 0 && a.g_sl % E8 == 0 &&
-                     a.d_sb % E8 == 0 && a.d_sl % E8 == 0 && ptrs8;
+                     a.d_sb % E8 == 0 && a.d_sl % E8 == 0 && ptrs8 &&
+                     // rows are addressed by 32-bit scalar offsets inside a slab's buffer resources
+                     a.x_sl > 0 && a.g_sl > 0 && a.d_sl > 0 &&
+                     (uint64_t)(kBwdSlab + 3) * (uint64_t)std::max({a.x_sl, a.g_sl, a.d_sl}) * elem_bytes(p->x_dtype) + 1024 < (1ull << 31);
     if (vec) {
-        const uint32_t tile = kBwdSlab * kBwdWaves;
-        const uint32_t nvec = a.C / E8;
+        const uint32_t nvec = a.C / kBwdLaneChannels;
         const uint32_t nct = (nvec + 63) / 64;
-        // time steps per block: as long as possible (few partial sets to write and to add up, taps and
-        // chunk-end work amortised) while the grid still has one and a half blocks per CU.  The sequence is
-        // cut into the fewest equal chunks (whole tiles) that give such a grid: a block walks every tile of
-        // its chunk, so chunks of a fixed length would leave the last one mostly empty (L = 520 as 512 + 8).
-        const uint32_t max_chunks = (a.L + tile - 1) / tile;   // = tiles per sequence
-        uint32_t nchunk = max_chunks, chunk = tile;
-        bool found = false;
-        for (uint32_t n = 1; n <= max_chunks; ++n) {
-            const uint32_t len = ((a.L + n - 1) / n + tile - 1) / tile * tile;
-            if (len > (uint32_t)kBwdMaxChunk) continue;
-            const uint32_t used = (a.L + len - 1) / len;               // chunks of that length that hold steps
-            const bool enough = 2ull * a.B * used * nct >= 256ull * kBwdHalfBlocksPerCU || n == max_chunks;
-            if (!found && enough) {
-                found = true;
-                nchunk = used;
-                chunk = len;
-                if (max_chunks % used == 0) break;
-                continue;
-            }
-            // the first count that is enough leaves a short last chunk: a slightly larger count that cuts the
-            // tiles evenly runs 5-10 % faster (B4 L1024: 8 chunks of 4 tiles 24.9 us, 7 of 5 tiles 27.1 us)
-            if (found && (n >= 2 * nchunk || len < 2 * tile)) break;
-            if (found && used == n && max_chunks % n == 0) {
-                nchunk = used;
-                chunk = len;
-                break;
+        const int64_t set_bytes = (int64_t)a.C * 5 * (int64_t)sizeof(float);
+        // Chunks of kBwdChunk steps, shorter where the grid would not have one and a half blocks per CU.  A scratch with
+        // no room for their partial sets (a caller's own, or the library's static one) gets the longest chunks that fill
+        // the grid.
+        BwdChunks ch = bwd_chunks(a.B, a.L, nct, kBwdChunk);
+        plan->workspace_bytes = (int64_t)a.B * ch.n * set_bytes;
+        const int64_t room = check_pointers ? p->workspace_bytes : scratch;
+        if (room >= 0 && plan->workspace_bytes > room) {
+            const BwdChunks longest = bwd_chunks(a.B, a.L, nct, kBwdMaxChunk);
+            if ((int64_t)a.B * longest.n * set_bytes <= room) {
+                ch = longest;
+                plan->workspace_bytes = (int64_t)a.B * ch.n * set_bytes;
             }
         }
-        const uint64_t blocks = (uint64_t)a.B * nchunk * nct;
+        const uint64_t blocks = (uint64_t)a.B * ch.n * nct;
         if (blocks < (1ull << 31)) {
             plan->kind = BWD_BLC_VEC;
             plan->walk_too = packed;
-            a.nvec = nvec; a.nct = nct; a.chunk = chunk; a.nchunk = nchunk;
-            a.nsets = a.B * nchunk;
-            a.div_nct = make_fastdiv(nct); a.div_nchunk = make_fastdiv(nchunk);
+            a.nvec = nvec; a.nct = nct; a.chunk = ch.len; a.nchunk = ch.n;
+            a.nsets = a.B * ch.n;
+            a.div_nct = make_fastdiv(nct); a.div_nchunk = make_fastdiv(ch.n);
             plan->grid = (uint32_t)blocks;
-            plan->workspace_bytes = (int64_t)a.nsets * a.C * 5 * (int64_t)sizeof(float);
             if (check_pointers && (!p->workspace || !aligned16(p->workspace) || p->workspace_bytes < plan->workspace_bytes))
                 return fail(CANON_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned and at least %lld bytes (got %lld)",
                             (long long)plan->workspace_bytes, (long long)p->workspace_bytes);
@@ -998,7 +1021,7 @@ CANON_API int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *st
     q.workspace = ptr;
     q.workspace_bytes = kStaticScratchBytes;
     BwdPlan pl;
-    rc = plan_bwd(&q, &pl, false);
+    rc = plan_bwd(&q, &pl, false, false, kStaticScratchBytes);
     if (rc == CANON_OK && pl.workspace_bytes > kStaticScratchBytes && pl.walk_too)
         rc = plan_bwd(&q, &pl, false, true);   // what canon_conv1d_bwd falls back to
     if (rc != CANON_OK) return rc;

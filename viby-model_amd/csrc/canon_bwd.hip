@@ -275,8 +275,8 @@ __global__ __launch_bounds__(256) void canon_bwd_walk_kernel(const BwdArgs a)
 // ---------------------------------------------------------------------------
 // backward, channel-contiguous tensors ([B, L, C] viewed as [B, C, L]).
 //
-// A block is four waves; a lane owns the channels of one 8-byte group (4 x
-// 16-bit or 2 x fp32), a wave a slab of kBwdSlab consecutive time steps of a
+// A block is four waves; a lane owns two adjacent channels (kBwdLaneChannels),
+// a wave a slab of kBwdSlab consecutive time steps of a
 // 64-lane channel tile, the four waves four consecutive slabs, and the block
 // walks over the `chunk` time steps of its chunk one such 32-step tile at a
 // time, keeping its dweight / dbias sums in registers.
@@ -291,35 +291,52 @@ __global__ __launch_bounds__(256) void canon_bwd_walk_kernel(const BwdArgs a)
 //   dz[t] = dout[t] * act'(z[t]),  dx[t] = sum_k w[k] * dz[t + (W-1) - k]
 // At the end the four waves' sums are added in a fixed order through LDS and
 // written as one partial set entry per channel.
+//
+// What bounds it: requests in flight.  The sums, taps, window and carried dz
+// of a channel stay in registers through the sweep, about thirty of them, so
+// the channels a lane owns decide how many waves a CU holds: with four
+// channels (8 bytes of a 16-bit row) 170-200 registers, two blocks per CU;
+// with two 81-95, five or six.  And chunks of 128 steps where the grid alone
+// would allow up to 1024: a CU then has new blocks to start while others drain,
+// for one partial set (20 bytes per channel) per 768 bytes of rows read and
+// written.  With both, us per call with the reduction, four channels -> two,
+// L 1024, bf16: B 32 C 3456 masked 145.2 -> 125.2, with SiLU 166.9 -> 128.5;
+// B 8 C 3456 38.7 -> 37.6, with SiLU 47.1 -> 41.0; B 16 C 640 L 511 SiLU masked
+// 19.0 -> 17.1; B 8 C 640 14.9 -> 12.8; packed rows B 2 C 3456 L 8192 SiLU
+// 91.3 -> 77.8; fp32 (two channels before as well) B 8 C 3456 70.1 -> 66.3.
+// Chunks of 192 steps: within 1 %; of 256: 2-13 % slower from B 4 C 3456 on.
 // ---------------------------------------------------------------------------
 // x and dout are read once and dx is written once: streamed (non-temporal) accesses, as in the forward kernels
 // (measured at B 8, C 3456, L 1024, bf16: 40.7 -> 37.8 us channel-contiguous, 33.6 -> 30.9 us time-contiguous).
 constexpr bool kBwdStream = true;
-using BV = VecIO<kBwdVecBytes>;
-using BVT = BV::type;   // a lane's piece of one row
-template <int DT> __device__ __forceinline__ void unpack_half(const BVT &v, float *f) { BV::template unpack<DT>(v, f); }
-template <int DT> __device__ __forceinline__ BVT pack_half(const float *f) { return BV::template pack<DT>(f); }
+template <int DT> using BwdIO = VecIO<kBwdLaneChannels * Elem<DT>::bytes>;
+template <int DT> using BwdVec = typename BwdIO<DT>::type;   // a lane's piece of one row
+template <int DT> __device__ __forceinline__ void unpack_lane(const BwdVec<DT> &v, float *f) { BwdIO<DT>::template unpack<DT>(v, f); }
+template <int DT> __device__ __forceinline__ BwdVec<DT> pack_lane(const float *f) { return BwdIO<DT>::template pack<DT>(f); }
 
 // One raw row -> the bits of xm = x * mask in the storage type (zero when the row does not exist)
+constexpr uint32_t kMaskOne = 0x3F800000u;   // 1.0f
 template <int DT, bool MASK>
-__device__ __forceinline__ BVT bwd_mask_row(const BVT &raw, float m, bool exists)
+__device__ __forceinline__ BwdVec<DT> bwd_mask_row(const BwdVec<DT> &raw, uint32_t m_bits, bool exists)
 {
-    constexpr int E = kBwdVecBytes / Elem<DT>::bytes;
-    BVT v = raw;
+    constexpr int E = kBwdLaneChannels;
+    BwdVec<DT> v = raw;
     if constexpr (MASK) {
-      // m is the same for the whole wave and 1 for every valid token of a padded batch: x * 1 is x, bit for bit
-      if (m != 1.0f) {
+      // m is the same for the whole wave (its bits are in a scalar register: a scalar branch) and 1 for every valid
+      // token of a padded batch: x * 1 is x, bit for bit
+      if (m_bits != kMaskOne) {
+        const float m = bits_f(m_bits);
         float f[E];
-        unpack_half<DT>(raw, f);
+        unpack_lane<DT>(raw, f);
 #pragma unroll
         for (int e = 0; e < E; ++e) {
             f[e] *= m;
             if constexpr (DT == CANON_DTYPE_F16) asm volatile("" : "+v"(f[e]));   // see mul_round
         }
-        v = pack_half<DT>(f);
+        v = pack_lane<DT>(f);
       }
     }
-    if (!exists) v = BV::zero();
+    if (!exists) v = BwdIO<DT>::zero();
     return v;
 }
 
@@ -367,15 +384,15 @@ __device__ __forceinline__ void bwd_dz_gated(const float (*w)[W], const float *b
 // first channel of slot 0) where it is needed: at most S_out steps per sequence.
 // SEQ: rows of several packed sequences in reach; q[j] is the sequence index of slab row j - 3 (rows -3 .. R+2).
 template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E, bool SEQ = false>
-__device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W], const float *bias, const BVT *X,
-                                          const BVT *H, const BVT *G, const float *mm, const float (*dzh)[E],
-                                          float (*dzf)[E], float (*dw)[W], float *dbs, char *dxp, int64_t ds, int rows,
-                                          bool active, const char *fin = nullptr, int64_t fin_first_row = 0,
+__device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W], const float *bias, const BwdVec<DT> *X,
+                                          const BwdVec<DT> *H, const BwdVec<DT> *G, const uint32_t *mm, const float (*dzh)[E],
+                                          float (*dzf)[E], float (*dw)[W], float *dbs, __amdgpu_buffer_rsrc_t rd, uint32_t voff,
+                                          uint32_t ds, int rows, const char *fin = nullptr, int64_t fin_first_row = 0,
                                           const int32_t *q = nullptr)
 {
     float xw[4][E];   // xm of rows r-3 .. r
 #pragma unroll
-    for (int k = 0; k < 4; ++k) unpack_half<DT>(X[R - 4 + k], xw[k]);
+    for (int k = 0; k < 4; ++k) unpack_lane<DT>(X[R - 4 + k], xw[k]);
     // The residual's gradient is added before the mask multiply (masked residual) or after it (unmasked); with
     // nothing in between the two are the same sum.  Real branches (the empty asm keeps the compiler from turning
     // them into an add and a select per element and mode: 12 of 75 VALU instructions per row).
@@ -384,7 +401,7 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {
         float g[E], dz[E], o[E];
-        unpack_half<DT>(G[r], g);
+        unpack_lane<DT>(G[r], g);
         // the window and the three later dz as this row sees them: rows of another sequence read as zero
         float xg[SEQ ? 3 : 1][E], dg[SEQ ? 3 : 1][E];
         if constexpr (SEQ) {
@@ -439,9 +456,9 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
             }
         }
         if constexpr (MASK) {
-            if (mm[3 + r] != 1.0f) {
+            if (mm[3 + r] != kMaskOne) {
 #pragma unroll
-                for (int e = 0; e < E; ++e) o[e] *= mm[3 + r];
+                for (int e = 0; e < E; ++e) o[e] *= bits_f(mm[3 + r]);
             }
         }
         if (res_post) {
@@ -449,7 +466,9 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 #pragma unroll
             for (int e = 0; e < E; ++e) o[e] += g[e];
         }
-        if ((FULL || r < rows) && active) BV::store<kBwdStream>(dxp + r * ds, pack_half<DT>(o));
+        if (FULL || r < rows) BufIO<kBwdLaneChannels * Elem<DT>::bytes>::template store<kAuxStream>(pack_lane<DT>(o), rd, voff, (uint32_t)r * ds);
+        // row by row: interleaved, the eight rows of a slab hold ten more registers and gain nothing
+        __builtin_amdgcn_sched_barrier(0);
         if (r > 0) {
             // slide the window one step back: the new oldest row is r - 4
 #pragma unroll
@@ -458,7 +477,7 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
                 xw[2][e] = xw[1][e];
                 xw[1][e] = xw[0][e];
             }
-            unpack_half<DT>(r - 4 >= 0 ? X[r - 4 >= 0 ? r - 4 : 0] : H[r - 1 < 3 ? r - 1 : 0], xw[0]);
+            unpack_lane<DT>(r - 4 >= 0 ? X[r - 4 >= 0 ? r - 4 : 0] : H[r - 1 < 3 ? r - 1 : 0], xw[0]);
         }
     }
 }
@@ -478,16 +497,28 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 {
     static_assert(!(STATES && SEQ), "seq_idx excludes states");
     constexpr int BY = Elem<DT>::bytes;
-    constexpr int E = kBwdVecBytes / BY;
+    constexpr int E = kBwdLaneChannels, VB = E * BY;
     constexpr int R = kBwdSlab, NW = kBwdWaves;
     // With an activation: tailx / headdz, two barriers per tile (dz of a slab's head needs the previous
     // wave's tail first).  Without one dz IS dout, so the head is handed over as raw rows (headg) together
     // with the tail, one barrier per tile, both double-buffered (a fast wave publishes the next tile while
     // a slow one still reads this one).
-    __shared__ BVT tailx[ACT ? 1 : 2][NW][3][64];            // last three xm rows of each wave's slab (storage bits)
-    __shared__ float headdz[ACT ? NW : 1][3][ACT ? E : 1][64];  // dz of the first three steps of each wave's slab
-    __shared__ BVT headg[2][ACT ? 1 : NW][3][64];            // ACT == false: the first three dout rows of each slab
-    __shared__ float red[NW - 1][5 * E][64];      // dweight / dbias sums of waves 1..3
+    // The sums that leave the block after its last tile lie in the same memory: 44 -> 29 KB of LDS with a mask, which
+    // lets the register count, not LDS, decide how many blocks a CU holds.
+    struct Exchange {
+        BwdVec<DT> tailx[ACT ? 1 : 2][NW][3][64];            // last three xm rows of each wave's slab (storage bits)
+        float headdz[ACT ? NW : 1][3][ACT ? E : 1][64];  // dz of the first three steps of each wave's slab
+        BwdVec<DT> headg[ACT ? 1 : 2][ACT ? 1 : NW][3][64];  // ACT == false: the first three dout rows of each slab
+    };
+    union Shared {
+        Exchange x;
+        float red[NW - 1][5 * E][64];                 // dweight / dbias sums of waves 1..3
+    };
+    __shared__ Shared shared;
+    auto &tailx = shared.x.tailx;
+    auto &headdz = shared.x.headdz;
+    auto &headg = shared.x.headg;
+    auto &red = shared.red;
     // mask entries of steps t_chunk-3 .. t_chunk+chunk+2 as floats.  Staged once per block: inside the
     // time loop (after the first store to dx) the compiler can no longer use scalar loads for them, and
     // as vector loads in the tile's load group they cost 20 % of the kernel.
@@ -505,10 +536,19 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     const bool active = cv < a.nvec;
     const uint32_t c0 = (active ? cv : a.nvec - 1u) * E;   // idle lanes shadow the last group: loads need no predicate
 
-    const char *xb = a.x + ((int64_t)b * a.x_sb + c0) * BY;
+    // The wave's rows are reached through buffer resources, one per tensor and tile: the lane is a 32-bit vector offset,
+    // the row a scalar one.  (As 64-bit pointers per lane the nineteen row addresses of a tile alone held 38 registers.)
+    // Lanes without channels are out of every resource's range: they load zeros and store nothing.
+    using IO = BufIO<VB>;
+    const uint32_t cv0 = ct * 64u, nl = a.nvec - cv0 < 64u ? a.nvec - cv0 : 64u;
+    const uint32_t voff = active ? (uint32_t)lane * VB : 0x80000000u;
+    const char *xb0 = a.x + ((int64_t)b * a.x_sb + (int64_t)cv0 * E) * BY;
+    const char *gb0 = a.dy + ((int64_t)b * a.g_sb + (int64_t)cv0 * E) * BY;
+    char *db0 = a.dx + ((int64_t)b * a.d_sb + (int64_t)cv0 * E) * BY;
+    const char *xb = a.x + ((int64_t)b * a.x_sb + c0) * BY;      // this lane's, for the rows past the chunk
     const char *gb = a.dy + ((int64_t)b * a.g_sb + c0) * BY;
-    char *db_ = a.dx + ((int64_t)b * a.d_sb + c0) * BY;
     const int64_t xs = a.x_sl * BY, gs = a.g_sl * BY, ds = a.d_sl * BY;
+    const uint32_t xs32 = (uint32_t)xs, gs32 = (uint32_t)gs, ds32 = (uint32_t)ds;
     const int64_t Lm1 = (int64_t)a.L - 1;
     const int64_t t_chunk = (int64_t)ch * a.chunk;
     const int ntiles = (int)(a.chunk / (uint32_t)(R * NW));
@@ -538,53 +578,53 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     if constexpr (!ACT) {
         // no activation: the three dz after the chunk are three rows of dout, kept by the last wave
         const int64_t te = t_chunk + (int64_t)a.chunk;
-        BVT GE[3];
+        BwdVec<DT> GE[3];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) GE[j] = BV::zero();
+        for (int j = 0; j < 3; ++j) GE[j] = BwdIO<DT>::zero();
         if (wv == NW - 1) {
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                if (te + j <= Lm1) GE[j] = BV::load<false>(gb + (te + j) * gs);
+                if (te + j <= Lm1) GE[j] = BwdIO<DT>::template load<false>(gb + (te + j) * gs);
         }
         decode_taps<DT, W, E>(rawt, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
 #pragma unroll
-        for (int j = 0; j < 3; ++j) unpack_half<DT>(GE[j], dzf[j]);
+        for (int j = 0; j < 3; ++j) unpack_lane<DT>(GE[j], dzf[j]);
     } else {
         const int64_t te = t_chunk + (int64_t)a.chunk;   // first step after the chunk (at least 32)
-        BVT XE[6], GE[3];
-        float me[6];
+        BwdVec<DT> XE[6], GE[3];
+        uint32_t me[6];
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
-            XE[j] = BV::zero();
-            me[j] = 1.0f;
+            XE[j] = BwdIO<DT>::zero();
+            me[j] = kMaskOne;
         }
 #pragma unroll
-        for (int j = 0; j < 3; ++j) GE[j] = BV::zero();
+        for (int j = 0; j < 3; ++j) GE[j] = BwdIO<DT>::zero();
         if (wv == NW - 1 && te <= Lm1) {
 #pragma unroll
             for (int j = 0; j < 6; ++j) {
                 const int64_t t = te - 3 + j;
-                XE[j] = BV::load<false>(xb + (t < Lm1 ? t : Lm1) * xs);
+                XE[j] = BwdIO<DT>::template load<false>(xb + (t < Lm1 ? t : Lm1) * xs);
             }
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const int64_t t = te + j;
-                GE[j] = BV::load<false>(gb + (t < Lm1 ? t : Lm1) * gs);
+                GE[j] = BwdIO<DT>::template load<false>(gb + (t < Lm1 ? t : Lm1) * gs);
             }
             if constexpr (MASK) {
 #pragma unroll
-                for (int j = 0; j < 6; ++j) me[j] = smask[a.chunk + j];   // steps te-3 .. te+2
+                for (int j = 0; j < 6; ++j) me[j] = f_bits(smask[a.chunk + j]);   // steps te-3 .. te+2
             }
         }
         decode_taps<DT, W, E>(rawt, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
         if (wv == NW - 1) {
             float xt[6][E];
 #pragma unroll
-            for (int j = 0; j < 6; ++j) unpack_half<DT>(bwd_mask_row<DT, MASK>(XE[j], me[j], te - 3 + j <= Lm1), xt[j]);
+            for (int j = 0; j < 6; ++j) unpack_lane<DT>(bwd_mask_row<DT, MASK>(XE[j], me[j], te - 3 + j <= Lm1), xt[j]);
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 float g[E], d[E];
-                unpack_half<DT>(GE[j], g);
+                unpack_lane<DT>(GE[j], g);
                 if constexpr (SEQ) {
                     const int32_t *q = sseq + a.chunk;      // steps te-3 .. te+2
                     bwd_dz_gated<W, E, ACT>(w, bias, xt[j], xt[j + 1], xt[j + 2], xt[j + 3], q[j] == q[j + 3],
@@ -615,29 +655,35 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
         // ---- all loads of the tile.  Requesting the next tile's rows while this one is worked on was measured
         // three times (before, and after, this tile's rows are waited for; with two register sets taken in turn
         // and wait counts that leave the next tile's loads in flight): 3-5 % slower, 40-60 more registers.
-        BVT X[R], G[R], H[3];
+        // (the x resource starts three rows before the slab; a row past the end of the sequence is the slab's last row
+        // again, loaded and never used, and a slab without rows has resources without a range)
+        const uint32_t xrec = rows == 0 ? 0u : (uint32_t)(R + 2) * xs32 + nl * VB;
+        const uint32_t grec = rows == 0 ? 0u : (uint32_t)(R - 1) * gs32 + nl * VB;
+        const uint32_t drec = rows == 0 ? 0u : (uint32_t)(R - 1) * ds32 + nl * VB;
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(xb0 + (t0 - 3) * xs), 0, (int)xrec, kBufFlags);
+        const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void *)(gb0 + t0 * gs), 0, (int)grec, kBufFlags);
+        const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void *)(db0 + t0 * ds), 0, (int)drec, kBufFlags);
+        BwdVec<DT> X[R], G[R], H[3];
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int64_t t = t0 + r < Lm1 ? t0 + r : Lm1;
-            X[r] = BV::load<kBwdStream>(xb + t * xs);
-            G[r] = BV::load<kBwdStream>(gb + t * gs);
+            const uint32_t rr = r < rows ? (uint32_t)r : (rows > 0 ? (uint32_t)(rows - 1) : 0u);
+            X[r] = IO::template load<kAuxStream>(rx, voff, (rr + 3u) * xs32);
+            G[r] = IO::template load<kAuxStream>(rg, voff, rr * gs32);
         }
 #pragma unroll
-        for (int j = 0; j < 3; ++j) H[j] = BV::zero();
-        if (wv == 0) {
+        for (int j = 0; j < 3; ++j) H[j] = BwdIO<DT>::zero();
+        if (wv == 0 && t0 > 0) {     // (t0 is a multiple of the tile: all three rows exist)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int64_t t = t0 - 3 + j;
-                if (t >= 0) H[j] = BV::load<false>(xb + (t < Lm1 ? t : Lm1) * xs);
-            }
+            for (int j = 0; j < 3; ++j) H[j] = IO::template load<kAuxPlain>(rx, voff, (uint32_t)j * xs32);
         }
-        float mm[R + 3];   // mask of steps t0-3 .. t0+R-1
+        uint32_t mm[R + 3];   // mask of steps t0-3 .. t0+R-1 (bits, in scalar registers: one LDS read, then lane by lane)
 #pragma unroll
-        for (int j = 0; j < R + 3; ++j) mm[j] = 1.0f;
+        for (int j = 0; j < R + 3; ++j) mm[j] = kMaskOne;
         if constexpr (MASK) {
             const uint32_t first = ((uint32_t)it * NW + wv) * R;   // index of step t0 - 3 in smask
+            const uint32_t m_lane = f_bits(smask[first + (uint32_t)(lane < R + 2 ? lane : R + 2)]);
 #pragma unroll
-            for (int j = 0; j < R + 3; ++j) mm[j] = smask[first + j];
+            for (int j = 0; j < R + 3; ++j) mm[j] = (uint32_t)__builtin_amdgcn_readlane((int)m_lane, j);
         }
         // SEQ: indices of steps t0-3 .. t0+R+2, one per lane, and whether they are all the same
         int32_t q_lane = 0;
@@ -659,7 +705,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
         } else {
             if (wv == NW - 1 && it != ntiles - 1) {   // (the chunk's last tile: the rows loaded before the loop)
 #pragma unroll
-                for (int j = 0; j < 3; ++j) unpack_half<DT>(headg[pb ^ 1][0][j][lane], dzf[j]);
+                for (int j = 0; j < 3; ++j) unpack_lane<DT>(headg[pb ^ 1][0][j][lane], dzf[j]);
             }
         }
 
@@ -684,7 +730,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 #pragma unroll
                 for (int e = 0; e < E; ++e)
                     f[e] = load1<DT>(a.init, (int64_t)b * a.i_sb + (int64_t)(c0 + e) * a.i_sc + (int64_t)s_ * a.i_ss);
-                H[j] = pack_half<DT>(f);
+                H[j] = pack_lane<DT>(f);
             }
         }
         if constexpr (!ACT) {
@@ -692,7 +738,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 tailx[pb][wv][j][lane] = X[R - 3 + j];
-                headg[pb][wv][j][lane] = j < rows ? G[j] : BV::zero();
+                headg[pb][wv][j][lane] = j < rows ? G[j] : BwdIO<DT>::zero();
             }
             __syncthreads();
             if (wv > 0) {
@@ -701,7 +747,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
             }
             if (wv < NW - 1) {
 #pragma unroll
-                for (int j = 0; j < 3; ++j) unpack_half<DT>(headg[pb][wv + 1][j][lane], dzf[j]);
+                for (int j = 0; j < 3; ++j) unpack_lane<DT>(headg[pb][wv + 1][j][lane], dzf[j]);
             }
         }
         float dzh[3][E];
@@ -722,13 +768,13 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
             {
                 float xq[6][E];   // xm of rows -3 .. 2
 #pragma unroll
-                for (int k = 0; k < 3; ++k) unpack_half<DT>(H[k], xq[k]);
+                for (int k = 0; k < 3; ++k) unpack_lane<DT>(H[k], xq[k]);
 #pragma unroll
-                for (int k = 0; k < 3; ++k) unpack_half<DT>(X[k], xq[3 + k]);
+                for (int k = 0; k < 3; ++k) unpack_lane<DT>(X[k], xq[3 + k]);
 #pragma unroll
                 for (int j = 0; j < 3; ++j) {
                     float g[E];
-                    unpack_half<DT>(G[j], g);
+                    unpack_lane<DT>(G[j], g);
                     if (SEQ && !one_seq) {
                         const int32_t own = __builtin_amdgcn_readlane(q_lane, j + 3);
                         bwd_dz_gated<W, E, ACT>(w, bias, xq[j], xq[j + 1], xq[j + 2], xq[j + 3],
@@ -759,18 +805,18 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
         if (STATES && a.dfin && t0 + rows > fin_first) {
             // slot 0 of the final state's gradient holds step fin_first
             const char *fin = a.dfin + ((int64_t)b * a.k_sb + (int64_t)c0 * a.k_sc) * BY;
-            bwd_sweep<DT, W, MASK, ACT, false, true, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows,
-                                                           active, fin, fin_first - t0);
+            bwd_sweep<DT, W, MASK, ACT, false, true, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
+                                                           fin, fin_first - t0);
         } else if (SEQ && !one_seq) {
             int32_t q[R + 6];
 #pragma unroll
             for (int j = 0; j < R + 6; ++j) q[j] = __builtin_amdgcn_readlane(q_lane, j);
-            bwd_sweep<DT, W, MASK, ACT, false, false, R, E, SEQ>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows,
-                                                                 active, nullptr, 0, q);
+            bwd_sweep<DT, W, MASK, ACT, false, false, R, E, SEQ>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
+                                                                 nullptr, 0, q);
         } else if (rows == R)
-            bwd_sweep<DT, W, MASK, ACT, true, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows, active);
+            bwd_sweep<DT, W, MASK, ACT, true, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows);
         else
-            bwd_sweep<DT, W, MASK, ACT, false, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, db_ + t0 * ds, ds, rows, active);
+            bwd_sweep<DT, W, MASK, ACT, false, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows);
     }
 
     if (STATES && a.dinit && ch == 0 && wv == 0 && active) {
@@ -796,6 +842,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     }
 
     // ---- the four waves' sums, added in the order 0, 1, 2, 3 -----------------------------
+    __syncthreads();   // (every wave has read its neighbours' rows of the last tile)
     if (wv > 0) {
 #pragma unroll
         for (int e = 0; e < E; ++e) {

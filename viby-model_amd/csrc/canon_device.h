@@ -451,6 +451,16 @@ constexpr int kAuxPlain = 0, kAuxStream = 2 /* nt */, kAuxStreamThrough = 2 | 16
 template <bool BIG> constexpr int store_policy() { return BIG ? kAuxStreamThrough : kAuxStream; }
 
 template <int VB> struct BufIO;
+template <> struct BufIO<4> {
+    template <int AUX> static __device__ __forceinline__ uint32_t load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff)
+    {
+        return (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, AUX);
+    }
+    template <int AUX> static __device__ __forceinline__ void store(uint32_t v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff)
+    {
+        __builtin_amdgcn_raw_buffer_store_b32(v, r, (int)voff, (int)soff, AUX);
+    }
+};
 template <> struct BufIO<8> {
     template <int AUX> static __device__ __forceinline__ uint2 load(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff)
     {

@@ -193,12 +193,13 @@ constexpr int kBlcVecBytes = 8;   // bytes per lane and access: 8 measured 4-9 %
 #define CANON_BWD_SLAB 8
 #endif
 constexpr int kBwdSlab = CANON_BWD_SLAB;    // time steps per wave and tile
-#ifndef CANON_BWD_VEC_BYTES
-#define CANON_BWD_VEC_BYTES 8
+constexpr int kBwdLaneChannels = 2;         // adjacent channels per lane in the channel-contiguous backward
+#ifndef CANON_BWD_CHUNK
+#define CANON_BWD_CHUNK 128
 #endif
-constexpr int kBwdVecBytes = CANON_BWD_VEC_BYTES;   // bytes per lane and row in the channel-contiguous backward
+constexpr uint32_t kBwdChunk = CANON_BWD_CHUNK;   // most time steps a block of it walks while the scratch has room for the sets
 constexpr int kBwdWaves = 4;
-constexpr int kBwdMaxChunk = 32 * kBwdSlab * kBwdWaves;   // most time steps one block of the channel-contiguous backward walks
+constexpr int kBwdMaxChunk = 32 * kBwdSlab * kBwdWaves;   // ... and at all
 enum FwdKind { FWD_BCL, FWD_BCL_SHORT, FWD_BLC, FWD_GENERIC };
 #ifndef CANON_BCL_MAX_U
 #define CANON_BCL_MAX_U 4
