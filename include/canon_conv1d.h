@@ -346,6 +346,9 @@ int canon_conv1d_init(void);
 /* Enqueue on `stream` (a hipStream_t; NULL = the default stream). */
 int canon_conv1d_fwd(const canon_conv1d_fwd_params *p, void *stream);
 int canon_conv1d_update(const canon_conv1d_update_params *p, void *stream);
+/* The same, except that the output row of a skipped entry (its conv_state_indices value lies outside the pool) is
+ * written with zeros, where canon_conv1d_update leaves it as it is. */
+int canon_conv1d_update_zero_skipped(const canon_conv1d_update_params *p, void *stream);
 int canon_conv1d_bwd(const canon_conv1d_bwd_params *p, void *stream);
 int canon_conv1d_update_bwd(const canon_conv1d_update_bwd_params *p, void *stream);
 

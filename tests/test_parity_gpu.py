@@ -769,6 +769,38 @@ def test_update_ring_buffer_and_state_pool(cc, dtype):
             assert torch.equal(bits(ring_gpu), bits(ring_ref)), what
 
 
+@pytest.mark.parametrize("dtype,B,C,S,ring", [(torch.bfloat16, 5, 264, 4, False), (torch.bfloat16, 600, 640, 4, False), (torch.float32, 5, 20, 8, False),
+                                              (torch.float16, 4, 33, 4, False), (torch.bfloat16, 5, 264, 4, True)])
+def test_output_rows_of_skipped_pool_entries(cc, dtype, B, C, S, ring):
+    """canon_conv1d_update leaves the output row of an entry outside the pool alone, canon_conv1d_update_zero_skipped
+    writes zeros there; everything else is the same."""
+    import ctypes
+
+    from causal_conv1d import _lib
+    g = torch.Generator().manual_seed(3)
+    pool = torch.randn(B + 2, C, S, generator=g).to(dtype).to(DEV)
+    x, w = torch.randn(B, C, generator=g).to(dtype).to(DEV), torch.randn(C, 4, generator=g).to(dtype).to(DEV)
+    idx = torch.randperm(B + 2, generator=g)[:B].to(torch.int32)
+    idx[1], idx[B - 1] = -1, B + 2
+    idx, lens = idx.to(DEV), torch.arange(B, dtype=torch.int32, device=DEV)
+    skipped = torch.zeros(B, dtype=torch.bool, device=DEV)
+    skipped[1] = skipped[B - 1] = True
+    outs, pools = [], []
+    for fn in (_lib.lib().canon_conv1d_update, _lib.lib().canon_conv1d_update_zero_skipped):
+        out, state = torch.full((B, C), 7.0, dtype=dtype, device=DEV), pool.clone()
+        p = cc._fill_update(x, out, state, w, None, None, 0, 1, 0)
+        p.conv_state_indices, p.state_rows = idx.data_ptr(), B + 2
+        if ring:
+            p.cache_seqlens = lens.data_ptr()
+        assert fn(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        torch.cuda.synchronize()
+        outs.append(out)
+        pools.append(state)
+    assert torch.equal(pools[0], pools[1]) and not torch.equal(pools[0], pool)
+    assert torch.equal(outs[0][~skipped], outs[1][~skipped])
+    assert bool((outs[0][skipped] == 7.0).all()) and bool((bits(outs[1][skipped]) == 0).all())
+
+
 def test_randomised_shapes_layouts_and_options(cc):
     """300 seeded random calls across layouts (time-contiguous, channel-contiguous, both as slices of larger
     tensors), sizes around every vector / tile boundary, dtypes, widths and options, each against the oracle."""

@@ -651,9 +651,8 @@ def _remember_update(key, block) -> None:
 
 
 def _launch_update(x2, conv_state, weight, bias, token_mask, cache_seqlens, conv_state_indices, act, res, rnd):
-    # entries of a state pool whose index lies outside the pool are skipped by the kernel: their output rows are zeros
-    alloc = torch.empty if conv_state_indices is None else torch.zeros
-    out = alloc(tuple(x2.shape), dtype=x2.dtype, device=x2.device)
+    # (entries of a state pool whose index lies outside the pool are skipped: the kernel writes their output rows, zeros)
+    out = torch.empty(tuple(x2.shape), dtype=x2.dtype, device=x2.device)
     if out.numel():
         p = _fill_update(x2, out, conv_state, weight, bias, token_mask, act, res, rnd)
         if cache_seqlens is not None:
@@ -661,7 +660,7 @@ def _launch_update(x2, conv_state, weight, bias, token_mask, cache_seqlens, conv
         if conv_state_indices is not None:
             p.conv_state_indices = conv_state_indices.data_ptr()
             p.state_rows = conv_state.shape[0]
-        rc = _call(_lib.lib().canon_conv1d_update, x2.device, ctypes.byref(p))
+        rc = _call(_lib.lib().canon_conv1d_update_zero_skipped, x2.device, ctypes.byref(p))
         _lib.check(rc, "causal_conv1d_update")
     return out
 

@@ -121,6 +121,7 @@ EXPORTS = (
     "canon_conv1d_last_error",
     "canon_conv1d_fwd",
     "canon_conv1d_update",
+    "canon_conv1d_update_zero_skipped",
     "canon_conv1d_init",
     "canon_conv1d_fwd_plan",
     "canon_conv1d_fwd_plan_waves",
@@ -157,6 +158,8 @@ def lib() -> ctypes.CDLL:
         L.canon_conv1d_fwd.argtypes = [ctypes.POINTER(FwdParams), _vp]
         L.canon_conv1d_update.restype = ctypes.c_int
         L.canon_conv1d_update.argtypes = [ctypes.POINTER(UpdateParams), _vp]
+        L.canon_conv1d_update_zero_skipped.restype = ctypes.c_int
+        L.canon_conv1d_update_zero_skipped.argtypes = [ctypes.POINTER(UpdateParams), _vp]
         L.canon_conv1d_init.restype = ctypes.c_int
         L.canon_conv1d_init.argtypes = []
         L.canon_conv1d_fwd_plan_waves.restype = ctypes.c_int

@@ -913,15 +913,26 @@ CANON_API int canon_conv1d_fwd(const canon_conv1d_fwd_params *p, void *stream)
     return check_launch("canon_conv1d_fwd");
 }
 
-CANON_API int canon_conv1d_update(const canon_conv1d_update_params *p, void *stream)
+static int launch_update_call(const canon_conv1d_update_params *p, void *stream, bool zero_skipped, const char *who)
 {
     UpdPlan pl;
     const int rc = plan_update(p, &pl);
     if (rc != CANON_OK) return rc;
     if (pl.grid == 0) return CANON_OK;
+    pl.args.zero_skipped = zero_skipped;
     hipStream_t s = (hipStream_t)stream;
     launch_update(pl, p->x_dtype, s);
-    return check_launch("canon_conv1d_update");
+    return check_launch(who);
+}
+
+CANON_API int canon_conv1d_update(const canon_conv1d_update_params *p, void *stream)
+{
+    return launch_update_call(p, stream, false, "canon_conv1d_update");
+}
+
+CANON_API int canon_conv1d_update_zero_skipped(const canon_conv1d_update_params *p, void *stream)
+{
+    return launch_update_call(p, stream, true, "canon_conv1d_update_zero_skipped");
 }
 
 CANON_API int canon_conv1d_bwd(const canon_conv1d_bwd_params *p, void *stream)

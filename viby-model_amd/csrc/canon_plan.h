@@ -92,6 +92,7 @@ struct UpdArgs {
     int64_t w_sc, w_sk;
     int32_t w_vec;
     uint32_t state_rows;      // rows of the state pool (0: not stated, indices are only checked for a negative value)
+    int32_t zero_skipped;     // the output row of an entry whose index lies outside the pool is written (zeros)
     // the rest: strided kernel, ring buffer, launch geometry
     const int32_t *seqlens;   // circular-buffer mode: conv_state is written at seqlens[b] % S, not shifted
     int64_t x_sc, o_sc;
