@@ -1,0 +1,174 @@
+"""The native host path against the general one: the same calls with the native module answering None throughout
+(then every argument block is filled field by field in Python), outputs and errors alike."""
+import types
+
+import pytest
+import torch
+
+from helpers import bits
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module")
+def cc():
+    import causal_conv1d
+    return causal_conv1d
+
+
+def both(cc, monkeypatch, call):
+    """call() through the native module and without it: the two results, or the two exceptions as text."""
+    results = []
+    none = types.SimpleNamespace(**{name: (lambda *a: None) for name in
+                                    ("try_fwd", "try_fwd_parts", "try_update_modes", "try_decode_step", "launch_fwd", "launch_bwd")})
+    for native in (cc._lib.native(), none):
+        with monkeypatch.context() as m:
+            m.setattr(cc._lib, "native", lambda native=native: native)
+            try:
+                results.append(call())
+            except Exception as e:
+                results.append(f"{type(e).__name__}: {e}")
+    return results
+
+
+def flat(r):
+    return [t for x in r for t in flat(x)] if isinstance(r, (tuple, list)) else [r]
+
+
+def assert_same(got, want, what):
+    if isinstance(want, str) or isinstance(got, str):
+        assert got == want, what
+        return
+    for a, b in zip(flat(got), flat(want), strict=True):
+        assert a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype, what
+        assert torch.equal(bits(a), bits(b)), what
+
+
+def layouts(B, C, L, dtype, g):
+    x = torch.randn(B, L, C, device=DEV, generator=g).to(dtype)
+    yield "channel", x.transpose(1, 2)
+    yield "time", x.transpose(1, 2).contiguous()
+    yield "slice", torch.cat([x, x], -1)[..., 3:3 + C].transpose(1, 2)
+    yield "batch inside", x.permute(2, 0, 1).contiguous().permute(1, 0, 2)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_prefill_and_backward(cc, monkeypatch, dtype):
+    g = torch.Generator(device=DEV).manual_seed(1)
+    n = 0
+    for B, C, L in [(1, 24, 1), (2, 33, 77), (3, 64, 130)]:
+        for name, x in layouts(B, C, L, dtype, g):
+            for wtype in (dtype, torch.float32):
+                W = 2 + n % 3
+                w = torch.randn(C, W, device=DEV, generator=g).to(wtype)
+                w = w if n % 2 else w.t().contiguous().t()
+                b = None if n % 3 == 0 else torch.randn(C, device=DEV, generator=g).to(wtype if n % 4 else torch.float32)
+                mask = (None if n % 2 else (torch.rand(B, L, device=DEV, generator=g) > 0.3).to(
+                    [torch.int64, torch.bool, torch.float32, torch.int32, torch.uint8, torch.float16][n // 2 % 6]))
+                seq = torch.arange(L, device=DEV, dtype=torch.int32).div(5, rounding_mode="floor").int().repeat(B, 1)
+                init = torch.randn(B, C, 5, device=DEV, generator=g).to(dtype)
+                options = dict(activation=[None, "silu", "swish"][n % 3], residual=[False, True, "masked", "unmasked", None, 2][n % 6],
+                               rounding=["fused", "eager"][n % 2], attention_mask=mask)
+                what = (name, B, C, L, dtype, wtype, n)
+                n += 1
+                assert_same(*both(cc, monkeypatch, lambda: cc.causal_conv1d_fn(x, w, b, **options)), what)
+                assert_same(*both(cc, monkeypatch, lambda: cc.causal_conv1d_fn(x, w, b, seq, **options)), what)
+                assert_same(*both(cc, monkeypatch, lambda: cc.causal_conv1d_fn(
+                    x, w, b, initial_states=init, final_states_out=torch.zeros(B, C, 8, dtype=dtype, device=DEV), **options)), what)
+                assert_same(*both(cc, monkeypatch, lambda: cc.causal_conv1d_fn(x, w, b, return_final_states=True, **options)), what)
+                half = C // 2
+                assert_same(*both(cc, monkeypatch, lambda: cc.causal_conv1d_fn_parts(
+                    (x[:, :half], x[:, half:]), w, b, final_states_out=torch.zeros(B, C, 4, dtype=dtype, device=DEV), **options)), what)
+
+                def train():
+                    leaves = [t.detach().requires_grad_() for t in (x, w, b, init) if t is not None]
+                    it = iter(leaves)
+                    xx, ww, bb, ii = next(it), next(it), next(it) if b is not None else None, next(it)
+                    fin = torch.zeros(B, C, 3, dtype=dtype, device=DEV)
+                    y, fin = cc.causal_conv1d_fn(xx, ww, bb, initial_states=ii, final_states_out=fin, **options)
+                    return torch.autograd.grad([y, fin], leaves, [torch.ones_like(y).transpose(1, 2).contiguous().transpose(1, 2),
+                                                                  torch.ones_like(fin)])
+
+                assert_same(*both(cc, monkeypatch, train), what)
+
+
+def test_decode_over_pool_and_ring(cc, monkeypatch):
+    g = torch.Generator(device=DEV).manual_seed(2)
+    for n, (B, C, S, dtype) in enumerate([(5, 24, 4, torch.bfloat16), (3, 33, 6, torch.float32), (70, 640, 3, torch.float16)]):
+        x = torch.randn(B, C, device=DEV, generator=g).to(dtype)
+        w, b = torch.randn(C, 4, device=DEV, generator=g).to(dtype), torch.randn(C, device=DEV, generator=g).to(dtype)
+        pool = torch.randn(B + 4, C, S, device=DEV, generator=g).to(dtype)
+        idx = torch.randperm(B + 4, device=DEV, generator=g)[:B].to(torch.int32)
+        idx[0] = -1
+        lens = torch.randint(0, 99, (B,), device=DEV, generator=g, dtype=torch.int32)
+        for options in (dict(conv_state_indices=idx), dict(cache_seqlens=lens), dict(conv_state_indices=idx, cache_seqlens=lens)):
+            for mask in (None, torch.ones(B, dtype=torch.int64, device=DEV)):
+                def step():
+                    state = pool.clone() if "conv_state_indices" in options else pool[:B].clone()
+                    y = cc.causal_conv1d_update(x, state, w, b, [None, "silu"][n % 2], token_mask=mask, residual=True, **options)
+                    return y, state
+                assert_same(*both(cc, monkeypatch, step), (B, C, S, dtype, list(options)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_decode_step_of_the_layer(cc, monkeypatch, dtype):
+    g = torch.Generator(device=DEV).manual_seed(3)
+    for n, (B, C, S) in enumerate([(1, 640, 8), (3, 33, 4), (70, 64, 3), (2, 24, 6)]):
+        wide = torch.randn(B, 3, C + 1, device=DEV, generator=g).to(dtype)
+        w, b = torch.randn(C, 4, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+        w, b = (w, b) if n == 1 else (w.to(dtype), b.to(dtype))
+        start = torch.randn(B, C, S, device=DEV, generator=g).to(dtype)
+        for x in (wide[:, :1, :C].contiguous(), wide[:, 1:2, 1:], wide.transpose(1, 2).contiguous().transpose(1, 2)[:, 2:, :C]):
+            for mtype in (None, torch.int64, torch.bool, torch.float32):
+                mask = None if mtype is None else (torch.rand(B, 9, device=DEV, generator=g) > 0.5).to(mtype)[:, ::2]
+
+                def step():
+                    state = start.clone()
+                    return cc._canon_decode_step(x, state, w, b if n != 2 else None, mask, [None, "silu"][n % 2],
+                                                 ["fused", "eager"][n % 2]), state
+                assert_same(*both(cc, monkeypatch, step), (B, C, S, dtype, mtype))
+
+
+def test_refused_calls(cc, monkeypatch):
+    x, w, b = torch.randn(2, 8, 16, device=DEV), torch.randn(8, 4, device=DEV), torch.randn(8, device=DEV)
+    mask, pool = torch.ones(2, 16, device=DEV), torch.randn(4, 8, 4, device=DEV)
+    idx = torch.zeros(2, dtype=torch.int32, device=DEV)
+    fn, parts, update = cc.causal_conv1d_fn, cc.causal_conv1d_fn_parts, cc.causal_conv1d_update
+    calls = [lambda: fn(x[0], w), lambda: fn(x.double(), w), lambda: fn(x, w[:7]), lambda: fn(x, torch.randn(8, 5, device=DEV)),
+             lambda: fn(x, w.cpu()), lambda: fn(x, w, b[:7]), lambda: fn(x, w, b.cpu()), lambda: fn(x, w, b, activation="relu"),
+             lambda: fn(x, w, b, residual="other"), lambda: fn(x, w, b, rounding="other"), lambda: fn(x, w, b, attention_mask=mask[:1]),
+             lambda: fn(x, w, b, attention_mask=mask.double()), lambda: fn(x, w, b, attention_mask=mask.cpu()),
+             lambda: fn(x, w, b, idx), lambda: fn(x, w, b, torch.zeros(2, 16, device=DEV)),
+             lambda: fn(x, w, b, torch.zeros(2, 16, dtype=torch.int32, device=DEV), initial_states=x[..., :4]),
+             lambda: fn(x, w, b, initial_states=x[..., :2]), lambda: fn(x, w, b, initial_states=x[:1, :, :4]),
+             lambda: fn(x, w, b, final_states_out=x[:, :, :0]), lambda: fn(x, w, b, final_states_out=x.half()),
+             lambda: fn(x, w, b, final_states_out=torch.zeros(2, 8, 65, device=DEV)), lambda: fn(x[..., :0], w, b),
+             lambda: parts([x, x[:, :, :8]], w), lambda: parts([x] * 5, w), lambda: parts([x, x.half()], w), lambda: parts([x[:, :4]], w),
+             lambda: update(x[..., 0], pool, w, b, conv_state_indices=idx.long()), lambda: update(x[..., 0], pool, w, b, cache_seqlens=idx),
+             lambda: update(x[..., 0], pool[:, :7], w, b, conv_state_indices=idx), lambda: update(x[..., 0], pool[..., :2], w, b, conv_state_indices=idx),
+             lambda: update(x[..., 0], pool.half(), w, b, conv_state_indices=idx), lambda: update(x[..., 0], pool, w, b, conv_state_indices=idx[:1])]
+    for n, call in enumerate(calls):
+        native, general = both(cc, monkeypatch, call)
+        assert_same(native, general, n)
+
+
+def test_another_stream_and_a_captured_graph(cc):
+    x = torch.randn(2, 64, 256, device=DEV).bfloat16()
+    w = torch.randn(64, 4, device=DEV).bfloat16()
+    want = cc.causal_conv1d_fn(x, w)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        got = cc.causal_conv1d_fn(x, w)
+    side.synchronize()
+    assert torch.equal(bits(got), bits(want))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = cc.causal_conv1d_fn(x, w)
+    for i in range(3):
+        x.copy_(torch.randn(2, 64, 256, device=DEV).bfloat16())
+        want = cc.causal_conv1d_fn(x, w)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(bits(out), bits(want)), i

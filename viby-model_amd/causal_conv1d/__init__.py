@@ -281,6 +281,15 @@ def causal_conv1d_fn(
                      conv, after SiLU and after the residual add, which
                      reproduces the eager bf16/fp16 module bit for bit).
     """
+    # a plain call is checked and launched in one native step; None: anything else, errors included, from here on
+    if not torch.compiler.is_compiling() and x.is_cuda and not (return_final_states and final_states_out is None):
+        out = _lib.native().try_fwd(x, weight, bias, seq_idx, initial_states, final_states_out, activation,
+                                    attention_mask if attention_mask is None else _narrow_mask(attention_mask, x, x.numel()),
+                                    residual, rounding)
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out, "causal_conv1d_fn")
+            return out if final_states_out is None else (out, final_states_out)
     act = _activation_flag(activation)
     res = _residual_mode(residual)
     rnd = _round_mode(rounding)
@@ -321,9 +330,14 @@ def causal_conv1d_fn(
 
 
 def _launch_fwd(x, weight, bias, mask, initial_states, final_states, act, res, rnd, seq_idx=None) -> torch.Tensor:
-    out = torch.empty_like(x)
     if x.numel() == 0:
+        return torch.empty_like(x)
+    out = _lib.native().launch_fwd(x, weight, bias, mask, initial_states, final_states, act, res, rnd, seq_idx)
+    if type(out) is int:
+        _lib.check(out, "causal_conv1d_fn")
+    if out is not None:
         return out
+    out = torch.empty_like(x)      # (x on another device than the current one, or a dispatch mode)
     p = _fill_fwd(x, out, weight, bias, mask, initial_states, final_states, act, res, rnd, seq_idx)
     rc = _call(_lib.lib().canon_conv1d_fwd, x.device, ctypes.byref(p))
     _lib.check(rc, "causal_conv1d_fn")
@@ -378,6 +392,16 @@ def _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx=N
     ``dweight`` (channels, W) / ``dbias`` (channels,) given, both of one type (rows of larger tensors are fine)."""
     if dout.dtype != x.dtype:
         dout = dout.to(x.dtype)
+    if dfinal is not None and dfinal.dtype != x.dtype:
+        dfinal = dfinal.to(x.dtype)
+    if x.numel():
+        dx = _lib.native().launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx, initial_states, dinit,
+                                      dfinal)
+        if type(dx) is int:
+            _lib.check(dx, "causal_conv1d_fn backward")
+        if dx is not None:
+            return dx
+    # nothing to launch over, x on another device than the current one, or a dispatch mode
     if dout.stride() != x.stride():
         dout = torch.empty_like(x).copy_(dout)       # same layout as x: keeps the vector kernel
     dx = torch.empty_like(x)
@@ -416,8 +440,6 @@ def _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx=N
                 p.dinitial_state = dinit.data_ptr()
                 p.dinit_stride_b, p.dinit_stride_c, p.dinit_stride_s = dinit.stride()
     if dfinal is not None and x.numel():
-        if dfinal.dtype != x.dtype:
-            dfinal = dfinal.to(x.dtype)
         p.dfinal_state = dfinal.data_ptr()
         p.dfinal_stride_b, p.dfinal_stride_c, p.dfinal_stride_s = dfinal.stride()
         p.final_len = dfinal.shape[2]
@@ -522,6 +544,13 @@ def causal_conv1d_update(
             return out
     else:
         key = None
+        if not torch.compiler.is_compiling() and x.is_cuda and (cache_seqlens is not None or conv_state_indices is not None):
+            out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices,
+                                                 token_mask, residual, rounding)
+            if out is not None:
+                if type(out) is int:
+                    _lib.check(out, "causal_conv1d_update")
+                return out
     act = _activation_flag(activation)
     res = _residual_mode(residual)
     rnd = _round_mode(rounding)
@@ -598,6 +627,12 @@ def _canon_decode_step(x: torch.Tensor, conv_state: torch.Tensor, taps: torch.Te
         token_mask = attention_mask[:, -1] if attention_mask is not None else None
         return causal_conv1d_update(x[:, 0], conv_state, taps, bias, activation=activation, token_mask=token_mask,
                                     residual="unmasked", rounding=rounding).unsqueeze(1)
+    if x.is_cuda:
+        out = _lib.native().try_decode_step(x, conv_state, taps, bias, attention_mask, activation, rounding)
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out, "causal_conv1d_update")
+            return out
     key = (x.shape, x.stride(), x.dtype, x.device, conv_state.shape, conv_state.stride(), conv_state.dtype,
            conv_state.device, taps.shape, taps.stride(), taps.dtype, taps.device,
            None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device),
@@ -829,6 +864,16 @@ def causal_conv1d_fn_parts(
     the conv once); results equal the call on the concatenation bit for bit.  Differentiable:
     the backward runs once per part on that part's rows of the weights (no cat there either).
     """
+    xs = list(xs)
+    if not torch.compiler.is_compiling() and xs and xs[0].is_cuda and not (return_final_states and final_states_out is None):
+        outs = _lib.native().try_fwd_parts(
+            xs, weight, bias, initial_states, final_states_out, activation,
+            attention_mask if attention_mask is None else _narrow_mask(attention_mask, xs[0], sum(x.numel() for x in xs)),
+            residual, rounding)
+        if outs is not None:
+            if type(outs) is int:
+                _lib.check(outs, "causal_conv1d_fn_parts")
+            return outs if final_states_out is None else (outs, final_states_out)
     act = _activation_flag(activation)
     res = _residual_mode(residual)
     rnd = _round_mode(rounding)

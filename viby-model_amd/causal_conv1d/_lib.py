@@ -195,6 +195,24 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The module that takes torch tensors to the library without a Python statement per field; raises if it has not
+    been built."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise ImportError(f"causal_conv1d._native cannot be loaded ({e}): build it with "
+                              "`make -j4 -C viby-model_amd/csrc`. There is no fallback implementation.") from e
+        _native = module
+    return _native
+
+
 def check(rc: int, what: str) -> None:
     """Turn a status code into the exception the Python API documents."""
     if rc == OK:
