@@ -769,6 +769,24 @@ def test_update_ring_buffer_and_state_pool(cc, dtype):
             assert torch.equal(bits(ring_gpu), bits(ring_ref)), what
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_captured_state_of_eight_slots(cc, dtype):
+    """Eight slots leave in one go where the row has them and the slots are contiguous, one by one otherwise: lengths
+    around eight and around a slab, idle lanes, states off 16-byte boundaries and with strided slots, exactly."""
+    g = torch.Generator().manual_seed(61)
+    for n, (B, C, L) in enumerate([(1, 4, 8), (2, 260, 7), (2, 264, 9), (3, 640, 32), (2, 12, 33), (1, 520, 77), (2, 64, 1)]):
+        x = torch.randn(B, L, C, generator=g).to(dtype).to(DEV).transpose(1, 2)
+        w = torch.randn(C, 4, generator=g).to(dtype).to(DEV)
+        init = torch.randn(B, C, 5, generator=g).to(dtype).to(DEV)
+        for mask in (None, right_padded_mask([max(1, L - 2 * i) for i in range(B)], L).to(DEV)):
+            xm = x if mask is None else (x.float() * mask[:, None].float()).to(dtype)
+            want = torch.cat([torch.zeros(B, C, 8, dtype=dtype, device=DEV), init, xm], -1)[..., -8:]
+            for state in (torch.full((B, C, 8), 7.0, dtype=dtype, device=DEV), torch.full((B, C, 9), 7.0, dtype=dtype, device=DEV)[..., 1:],
+                          torch.full((B, 8, C), 7.0, dtype=dtype, device=DEV).transpose(1, 2)):
+                _, got = cc.causal_conv1d_fn(x, w, initial_states=init, final_states_out=state, attention_mask=mask)
+                assert torch.equal(got, want), (B, C, L, mask is not None, state.stride())
+
+
 @pytest.mark.parametrize("dtype,B,C,S,ring", [(torch.bfloat16, 5, 264, 4, False), (torch.bfloat16, 600, 640, 4, False), (torch.float32, 5, 20, 8, False),
                                               (torch.float16, 4, 33, 4, False), (torch.bfloat16, 5, 264, 4, True)])
 def test_output_rows_of_skipped_pool_entries(cc, dtype, B, C, S, ring):

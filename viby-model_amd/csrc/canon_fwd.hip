@@ -485,6 +485,78 @@ __device__ __forceinline__ void blc_request(const BlcLead &h, const BlcWave<VB> 
     }
 }
 
+// Captures the last S_out masked inputs of the wave's channels into the final state (the wave of the sequence's last
+// slab).  Every block of the launch has to wait for these waves: eight slots of rows that are long enough, CanonLayer's
+// state, are requested together and leave in 16-byte stores, a channel's run each.  A row at a time, with a wait and a
+// two-byte store per channel behind each, the end of the launch came eight memory round trips later: B 1, C 640, L 77
+// 5.9 -> 4.0 us, masked B 8, C 640, L 1024 10.0 -> 7.2, q / k / v at B 16, L 1024 17.1 -> 14.6.  One channel after the
+// other, in raw bits: with everything unpacked at once the kernel needed 171 registers, not 81.
+template <int DT, bool MASK, int VB>
+__device__ __forceinline__ void blc_capture(const FwdArgs &a, const BlcLead &h, const BlcWave<VB> &g, const uint32_t cshift)
+{
+    constexpr int E = VB / Elem<DT>::bytes, BY = Elem<DT>::bytes, N = 8;
+    using V = VecIO<VB>;
+    const uint32_t c = cshift + g.c0;
+    if (a.S_out == N && a.f_ss == 1 && a.L >= (uint32_t)N) {
+        const int64_t first = (int64_t)a.L - N;
+        const char *xw = h.x + ((int64_t)g.b * h.x_sb + (int64_t)g.cv0 * E) * BY + first * (int64_t)g.xs;
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)xw, 0, (int)((N - 1) * g.xs + g.nl * VB), kBufFlags);
+        typename V::type row[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) row[j] = BufIO<VB>::template load<kAuxPlain>(r, g.voff, (uint32_t)j * g.xs);
+        if constexpr (MASK) {
+            float m[N];
+            load_mask_rows_wave<N>(a.mask, (int64_t)g.b * a.m_sb, first, a.L, a.m_sl, a.mask_dtype, (int)g.lane, m);
+#pragma unroll
+            for (int j = 0; j < N; ++j) {
+                float v[E];
+                V::template unpack<DT>(row[j], v);
+#pragma unroll
+                for (int e = 0; e < E; ++e) v[e] = mul_round<DT>(v[e], m[j]);
+                row[j] = V::template pack<DT>(v);   // (exact: the products are already rounded)
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (!g.active) return;
+        char *dst = (char *)a.fin + ((int64_t)g.b * a.f_sb + (int64_t)c * a.f_sc) * BY;
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            uint32_t words[N * BY / 4] = {};
+#pragma unroll
+            for (int j = 0; j < N; ++j) Packed<DT>::put(words, j, Packed<DT>::get((const uint32_t *)&row[j], e));
+#pragma unroll
+            for (int i = 0; i < N * BY / 16; ++i)
+                store_vec_any<false>(dst + 16 * i, make_uint4(words[4 * i], words[4 * i + 1], words[4 * i + 2], words[4 * i + 3]));
+            dst += a.f_sc * BY;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        return;
+    }
+    if (!g.active) return;
+    const char *xb = h.x + ((int64_t)g.b * h.x_sb + g.c0) * BY;
+    for (int slot = 0; slot < a.S_out; ++slot) {
+        const int64_t t = (int64_t)a.L - a.S_out + slot;
+        float v[E];
+#pragma unroll
+        for (int e = 0; e < E; ++e) v[e] = 0.0f;
+        if (t >= 0) {
+            V::template unpack<DT>(V::template load<false>(xb + t * (int64_t)g.xs), v);
+            if constexpr (MASK) {
+                const float mm = load_mask(a.mask, g.b * a.m_sb + t * a.m_sl, a.mask_dtype);
+#pragma unroll
+                for (int e = 0; e < E; ++e) v[e] = mul_round<DT>(v[e], mm);
+            }
+        } else if (a.init && a.S_in + t >= 0) {
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                v[e] = load1<DT>(a.init, g.b * a.i_sb + (int64_t)(c + e) * a.i_sc + (a.S_in + t) * a.i_ss);
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e)
+            store1<DT>(a.fin, g.b * a.f_sb + (int64_t)(c + e) * a.f_sc + slot * a.f_ss, v[e]);
+    }
+}
+
 using ArgsHere = ArgsRead<FwdArgs>;
 // ... with the two pointers the taps are fetched through, which the plain kernel receives among its leading
 // scalars: large launches request the taps BEFORE the slab, from registers, so that they wait neither for the slab
@@ -554,7 +626,7 @@ __device__ __forceinline__ void blc_block_body(const ARGS &args, const BlcLead &
     const FwdArgs &a = args.get();
     const uint32_t cshift = part ? a.pair_c : 0u;   // the block's channels in tensors that cover both parts of a pair
     const uint32_t b = wave.b, lane = wave.lane, wv = wave.wv, wt = wave.wt, wc = wave.wc, cv0 = wave.cv0, nl = wave.nl, c0 = wave.c0;
-    const uint32_t voff = wave.voff, xs = wave.xs;
+    const uint32_t voff = wave.voff;
     const int64_t t0 = wave.t0;
     const int rows = wave.rows;
     const bool active = wave.active;
@@ -665,30 +737,7 @@ __device__ __forceinline__ void blc_block_body(const ARGS &args, const BlcLead &
         blc_rows_dispatch<DT, W, R, MASK, BIG, VB>(a, w, bias, hist, X, m, ro, voff, os, rows);
     }
 
-    if (a.fin && active && t0 + rows == (int64_t)a.L) {
-        const char *xb = h.x + ((int64_t)b * h.x_sb + c0) * BY;
-        for (int slot = 0; slot < a.S_out; ++slot) {
-            const int64_t t = (int64_t)a.L - a.S_out + slot;
-            float v[E];
-#pragma unroll
-            for (int e = 0; e < E; ++e) v[e] = 0.0f;
-            if (t >= 0) {
-                V::template unpack<DT>(V::template load<false>(xb + t * (int64_t)xs), v);
-                if constexpr (MASK) {
-                    const float mm = load_mask(a.mask, b * a.m_sb + t * a.m_sl, a.mask_dtype);
-#pragma unroll
-                    for (int e = 0; e < E; ++e) v[e] = mul_round<DT>(v[e], mm);
-                }
-            } else if (a.init && a.S_in + t >= 0) {
-#pragma unroll
-                for (int e = 0; e < E; ++e)
-                    v[e] = load1<DT>(a.init, b * a.i_sb + (int64_t)(cshift + c0 + e) * a.i_sc + (a.S_in + t) * a.i_ss);
-            }
-#pragma unroll
-            for (int e = 0; e < E; ++e)
-                store1<DT>(a.fin, b * a.f_sb + (int64_t)(cshift + c0 + e) * a.f_sc + slot * a.f_ss, v[e]);
-        }
-    }
+    if (a.fin && t0 + rows == (int64_t)a.L) blc_capture<DT, MASK, VB>(a, h, wave, cshift);
 }
 
 // The block's code once per tap layout (wave-uniform choice): the contiguous layouts are straight-line
