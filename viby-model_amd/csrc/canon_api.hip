@@ -373,7 +373,9 @@ int plan_update(const canon_conv1d_update_params *p, UpdPlan *plan)
         a.div_nvec = make_fastdiv(a.nvec);
         plan->grid = (a.nthreads + 255) / 256;
     } else {
+        a.nvec = a.C;
         a.nthreads = a.B * a.C;
+        a.div_nvec = make_fastdiv(a.C);
         plan->grid = (a.nthreads + 255) / 256;
     }
     return CANON_OK;
