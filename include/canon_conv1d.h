@@ -190,8 +190,8 @@ typedef struct canon_conv1d_update_params {
  * sequence index (the ones the forward left out) are left out of z, dxm and
  * dweight alike.
  * All arithmetic in fp32; dx is rounded once to the storage type.  dweight and
- * dbias are fp32, OVERWRITTEN (not accumulated into), and reduced in a fixed
- * order in two stages through `workspace` (no float atomics: results are
+ * dbias are summed in fp32 (stored as grad_dtype says), OVERWRITTEN (not
+ * accumulated into), and reduced in a fixed order in two stages through `workspace` (no float atomics: results are
  * reproducible run to run).
  */
 typedef struct canon_conv1d_bwd_params {
@@ -375,9 +375,10 @@ int canon_conv1d_update_parts(const canon_conv1d_update_params *p, const canon_c
  * Nothing is allocated or freed, by the library or by the runtime on its
  * behalf, once the device is set up (canon_conv1d_init, or one earlier call
  * of this function on the GPU: the first one makes the runtime load the
- * library's code object, which allocates).  A problem whose scratch exceeds
- * the buffer is rejected with
- * CANON_ERR_UNSUPPORTED (the metric shape, bf16 [8, 3456, 1024], needs 2.2 MB).
+ * library's code object, which allocates).  A problem whose partial sets exceed
+ * the buffer is cut into fewer where that is possible, else rejected with
+ * CANON_ERR_UNSUPPORTED (the metric shape, bf16 [8, 3456, 1024], uses 4.4 MB;
+ * batch 128 of it is rejected).
  * All calls on one GPU share that GPU's buffer: calls that overlap in time on
  * one GPU (different streams, different threads) race and must be serialised
  * by the caller; calls that follow each other on one stream are safe.
@@ -385,8 +386,8 @@ int canon_conv1d_update_parts(const canon_conv1d_update_params *p, const canon_c
 #define CANON_CONV1D_STATIC_SCRATCH_BYTES (8 << 20)
 int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *stream);
 
-/* Scratch bytes canon_conv1d_bwd needs for these sizes, strides and pointer
- * alignments; with x, dout or dx missing (NULL) the figure also covers the
+/* Scratch bytes canon_conv1d_bwd works with for these sizes, strides and pointer
+ * alignments (less is accepted where fewer partial sets can be cut); with x, dout or dx missing (NULL) the figure also covers the
  * kernel a misaligned pointer would select.  Negative if the arguments are
  * rejected. */
 int64_t canon_conv1d_bwd_workspace_bytes(const canon_conv1d_bwd_params *p);

@@ -263,8 +263,8 @@ def causal_conv1d_fn(
 
     seq_idx          (batch, seqlen) int32: packed variable-length sequences; positions
                      with different values do not see each other (the slot the
-                     reference leaves at None, ``model/model.py:465``).  Inference
-                     only, without initial / final states.
+                     reference leaves at None, ``model/model.py:465``).  Without
+                     initial / final states.
     initial_states   (batch, dim, >= W-1): history before t = 0 instead of zeros (differentiable).
     return_final_states / final_states_out (batch, dim, S): receives the last S
                      inputs (S = W-1 when allocated here; any S >= 1 when

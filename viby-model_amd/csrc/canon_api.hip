@@ -560,9 +560,8 @@ BwdChunks bwd_chunks(uint32_t B, uint32_t L, uint32_t nct, uint32_t longest)
     const uint32_t tiles = (L + tile - 1) / tile;
     BwdChunks c = {tiles, tile};
     bool found = false;
-    for (uint32_t n = 1; n <= tiles; ++n) {
+    for (uint32_t n = (L + longest - 1) / longest; n <= tiles; ++n) {   // (longest is whole tiles)
         const uint32_t len = ((L + n - 1) / n + tile - 1) / tile * tile;
-        if (len > longest) continue;
         const uint32_t used = (L + len - 1) / len;               // chunks of that length that hold steps
         const bool enough = 2ull * B * used * nct >= 256ull * kBwdHalfBlocksPerCU || n == tiles;
         if (!found && enough) {
