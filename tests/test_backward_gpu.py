@@ -417,6 +417,69 @@ def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
                 check(grads[2], rdb, dtype, what + " dbias", sum_terms=B * L)
 
 
+def dweight_of(x, dout, W, seq_idx=None):
+    """dweight of the call without an activation, from its definition: dout[t] times the input each tap reads, where
+    there is one of the same sequence.  (Sums of existing products only: what is not there is not multiplied by zero.)"""
+    B, C, L = x.shape
+    x64, d64 = x.double(), dout.double()
+    dw = torch.zeros(C, W, dtype=torch.float64)
+    for k in range(W):
+        back = W - 1 - k
+        if back >= L:
+            continue
+        part = x64[..., :L - back] * d64[..., back:]
+        if seq_idx is not None:
+            part = torch.where((seq_idx[:, :L - back] == seq_idx[:, back:]).unsqueeze(1), part, torch.zeros(()).double())
+        dw[:, k] = part.sum((0, 2))
+    return dw
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("route,B,C,L", [
+    ("bcl", 2, 6, 45), ("bcl", 2, 6, 1021), ("bcl", 3, 1030, 1021),        # rows that end inside a vector, 1 and 2 vectors a lane
+    ("bcl", 2, 6, 40), ("bcl", 2, 6, 136), ("bcl", 2, 6, 520), ("bcl", 2, 1030, 1536), ("bcl", 2, 6, 1024),   # idle lanes, none
+    ("bcl", 2, 6, 23), ("blc", 2, 7, 45),                                  # the walk kernel
+    ("blc", 2, 8, 3), ("blc", 2, 24, 45), ("blc", 2, 24, 40), ("blc", 2, 24, 64), ("blc", 2, 136, 1021),   # partial and empty slabs, none
+    ("packed", 2, 24, 45), ("packed", 2, 24, 40), ("packed", 2, 136, 1021), ("packed", 2, 7, 45), ("state", 2, 24, 45)])
+def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, route, B, C, L):
+    """An Inf or a NaN among a row's last inputs makes the sums of the taps that read it non-finite and no others: steps
+    past the end of a row are not there, so the window they would have must not be multiplied by a dz of zero."""
+    g = torch.Generator().manual_seed(3)
+    W = 4
+    seq = None
+    if route == "packed":
+        seq = torch.zeros(B, L, dtype=torch.int32)
+        seq[0, L // 2:] = 1
+        seq[1, L - 2:] = 1
+    for bad, back in ((float("inf"), 1), (float("-inf"), 2), (float("nan"), 1), (float("nan"), 3), (float("inf"), 4)):
+        x = torch.randn(B, C, L, generator=g).to(dtype)
+        if back <= L:
+            x[1, 0::2, L - back] = bad
+        w, b = (torch.randn(C, W, generator=g) * 0.5).to(dtype), torch.zeros(C, dtype=dtype)
+        dout = torch.randn(B, C, L, generator=g).to(dtype)
+        layout = "bcl" if route == "bcl" else "blc"
+        if route == "state":       # the sweep that adds the gradient of a captured final state
+            xg = x.to(DEV).transpose(1, 2).contiguous().transpose(1, 2).requires_grad_()
+            wg = w.to(DEV).requires_grad_()
+            out, fin = cc.causal_conv1d_fn(xg, wg, b.to(DEV), final_states_out=torch.empty(B, C, 4, dtype=dtype, device=DEV))
+            dw, = torch.autograd.grad([out, fin], wg, [dout.to(DEV), torch.ones(B, C, 4, dtype=dtype, device=DEV)])
+        else:
+            _, dw, _, _ = gpu_grads(cc, x, w, b, dout, layout, seq_idx=seq)
+        want = dweight_of(x, dout, W, seq)
+        assert torch.equal(torch.isfinite(dw.cpu()), torch.isfinite(want)), (bad, back)
+        check(dw[1::2], want[1::2], dtype, f"{bad} {back} finite channels", sum_terms=B * L)
+        # with SiLU: which taps are finite is what the walk kernel says of the same values (it takes the strided view)
+        if route != "state":
+            _, dw, _, _ = gpu_grads(cc, x, w, b, dout, layout, act="silu", seq_idx=seq)
+            xs = torch.zeros(B, C, 2 * L, dtype=dtype, device=DEV)[..., ::2]
+            xs.copy_(x)
+            xs.requires_grad_()
+            ws = w.to(DEV).requires_grad_()
+            out = cc.causal_conv1d_fn(xs, ws, b.to(DEV), activation="silu", seq_idx=None if seq is None else seq.to(DEV))
+            dws, = torch.autograd.grad(out, ws, dout.to(DEV))
+            assert torch.equal(torch.isfinite(dw), torch.isfinite(dws)), (bad, back, "silu")
+
+
 @pytest.mark.parametrize("dtype,act,masked", [(torch.bfloat16, "silu", False), (torch.bfloat16, None, True), (torch.float32, "silu", True)])
 def test_backward_of_packed_sequences_in_chunks_of_several_tiles(cc, dtype, act, masked):
     """Enough columns that one block walks a whole row (three tiles of 32 steps and a part of one): boundaries between

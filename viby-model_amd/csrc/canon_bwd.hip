@@ -434,9 +434,19 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
             if constexpr (W >= 3) acc = fmaf(w[e][W - 3], dv[1][e], acc);
             if constexpr (W == 4) acc = fmaf(w[e][0], dv[2][e], acc);
             o[e] = acc;
+        }
+        // (steps past the end of the sequence are left out, not multiplied by their dz of zero: their window holds the
+        // sequence's last inputs, and 0 * Inf is NaN)
+        if (FULL || r < rows) {
 #pragma unroll
-            for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], xv[(4 - W) + k][e], dw[e][k]);
-            dw[e][W - 1] = fmaf(dz[e], xw[3][e], dw[e][W - 1]);
+            for (int e = 0; e < E; ++e) {
+#pragma unroll
+                for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], xv[(4 - W) + k][e], dw[e][k]);
+                dw[e][W - 1] = fmaf(dz[e], xw[3][e], dw[e][W - 1]);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
             dbs[e] += dz[e];
             dzf[2][e] = dzf[1][e];
             dzf[1][e] = dzf[0][e];
@@ -1067,12 +1077,30 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
 #pragma unroll
             for (int j = 0; j < E; ++j) dz[u][j] = RAGGED && first + j < len ? dz[u][j] : 0.0f;
         }
+        // Steps past the end of the row have a dz of zero, but their window reaches back over the row's last inputs, and
+        // 0 * Inf is NaN: their window is zero as well.  Whole vectors: selects for every lane (no time measured; a branch
+        // around the sums costs up to 5 % at B 8, C 1000, L 1536 with a mask).  Ragged rows, whose last vector has steps
+        // on both sides of the end: the selects, one per step and tap, only in the wave that holds the end (B 8, C 960,
+        // L 1021 13.5 -> 13.9 us, with SiLU 15.5 -> 15.0, for every lane 16.5; B 32, L 500, where every wave holds one,
+        // 21.0 -> 21.5, with SiLU 24.0 -> 25.5).
+        if (RAGGED && __builtin_amdgcn_ballot_w64(!valid) == 0) {
 #pragma unroll
-        for (int j = 0; j < E; ++j) {
+            for (int j = 0; j < E; ++j)
 #pragma unroll
-            for (int k = 0; k < W; ++k) dwl[k] = fmaf(dz[u][j], seq[j + (4 - W) + k], dwl[k]);
-            dbl += dz[u][j];
+                for (int k = 0; k < W; ++k) dwl[k] = fmaf(dz[u][j], seq[j + (4 - W) + k], dwl[k]);
+        } else {
+            float win[E + 3];
+#pragma unroll
+            for (int i = 0; i < E + 3; ++i) win[i] = RAGGED || valid ? seq[i] : 0.0f;
+#pragma unroll
+            for (int j = 0; j < E; ++j) {
+                const bool inside = !RAGGED || first + j < len;
+#pragma unroll
+                for (int k = 0; k < W; ++k) dwl[k] = fmaf(dz[u][j], inside ? win[j + (4 - W) + k] : 0.0f, dwl[k]);
+            }
         }
+#pragma unroll
+        for (int j = 0; j < E; ++j) dbl += dz[u][j];
     }
 
     // pass 2: dx
