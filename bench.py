@@ -177,8 +177,8 @@ def bench_prefill(layout, steps, warmup, nbuf, ramp=True, shape=None, dtype=None
 
 def bench_ragged(layout, steps, warmup, nbuf, batch=32):
     """right-padded batch of 32, valid lengths uniform in [128, 1024], the padding mask multiplied
-    in before the conv and the masked residual added (out = m*x + conv(m*x) + bias).  The mask is what the
-    Python wrapper hands the kernel for a trainer's int64 mask on a problem of this size: narrowed to bf16."""
+    in before the conv and the masked residual added (out = m*x + conv(m*x) + bias).  The mask is in bf16, to which the
+    Python wrapper converts a trainer's int64 mask for time-contiguous tensors of this size."""
     import torch
     import causal_conv1d as cc
     from causal_conv1d import _lib

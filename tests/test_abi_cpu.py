@@ -407,22 +407,29 @@ def test_static_scratch_backward_checks_on_the_host():
     assert "struct_size" in last_error()
 
 
-def test_mask_narrowing_works_on_inference_tensors():
-    """An int64 padding mask is converted to x's type once and cached on its identity and version; tensors made
-    under torch.inference_mode() have no version counter, so they are converted without the cache."""
+def test_mask_narrowing():
+    """A wide integer mask of a large call is converted to x's type, for that call alone, unless the channel-contiguous
+    vector kernels take it; everything else is handed over as given.  Tensors made under torch.inference_mode(), which have no version counter, like any other."""
     import causal_conv1d as cc
     x = torch.zeros(2, 4, 8, dtype=torch.bfloat16)
     big = cc._NARROW_MIN_ELEMENTS
     mask = torch.ones(2, 8, dtype=torch.int64)
     first = cc._narrow_mask(mask, x, big)
-    assert first.dtype == torch.bfloat16 and cc._narrow_mask(mask, x, big) is first          # cached
+    assert first.dtype == torch.bfloat16 and cc._narrow_mask(mask, x, big) is not first      # nothing is kept
     assert cc._narrow_mask(mask, x, big - 1) is mask                                         # small problems: as given
+    assert cc._narrow_mask(mask, torch.zeros(2, 8, 4, dtype=torch.bfloat16).transpose(1, 2), big) is mask
+    odd = torch.zeros(2, 8, 5, dtype=torch.bfloat16).transpose(1, 2)                         # no whole 8-byte groups: strided kernel
+    assert cc._narrow_mask(mask, odd, big).dtype == torch.bfloat16
+    assert cc._narrow_mask(mask.bool(), x, big).dtype == torch.bool and cc._narrow_mask(mask.float(), x, big).dtype == torch.float32
+    assert cc._narrow_mask(mask.int(), x.float(), big).dtype == torch.int32                  # no wider than x
     with torch.inference_mode():
         imask = torch.ones(2, 8, dtype=torch.int64)
         got = cc._narrow_mask(imask, x, big)
         assert got.dtype == torch.bfloat16 and torch.equal(got.float(), imask.float())
-    mask[0, 3] = 0                                                                           # a new version: converted again
+    mask[0, 3] = 0
     assert cc._narrow_mask(mask, x, big)[0, 3].item() == 0
+    mask.data[0, 4] = 0
+    assert cc._narrow_mask(mask, x, big)[0, 4].item() == 0
 
 
 def update_bwd_params(B=256, C=3456, S=3, dtype=1, **over):

@@ -505,29 +505,64 @@ def test_errors_surface(cc):
         cc.causal_conv1d_update(x[:, :, 0], torch.zeros(2, 8, 2, device=DEV), w)
 
 
-def test_integer_mask_narrowing_is_never_stale(cc):
-    """Large problems convert an int64 mask to x.dtype once and reuse it while the same mask
-    object comes back; a changed or different mask must never hit the cached copy."""
+@pytest.mark.parametrize("layout", ["bcl", "blc"])
+def test_integer_mask_of_a_large_call_is_never_stale(cc, layout):
+    """An int64 mask on a call large enough that the time-contiguous layout has it converted to x.dtype: each call reads the
+    mask as it is then, whoever changed it (a write, a new tensor, a view, a write past the version counter), from
+    another stream and in a captured graph."""
     g = torch.Generator().manual_seed(91)
-    B, C, L = 4, 512, 1024          # 2M elements: above the narrowing threshold
+    B, C, L = 16, 1024, 1024
+    assert B * C * L >= cc._NARROW_MIN_ELEMENTS
     x = torch.randn(B, C, L, generator=g).bfloat16()
     w = torch.randn(C, 4, generator=g).bfloat16()
+    m1 = right_padded_mask([1024, 700, 300, 5] * 4, L)
+    m2 = right_padded_mask([10, 1024, 64, 999] * 4, L)
+    want = [(m, co.conv1d_fwd(x, w, None, mask=m, residual=1)) for m in (m1, m2)]
+    (_, want1), (_, want2) = want
     xg, wg = x.to(DEV), w.to(DEV)
-    m1 = right_padded_mask([1024, 700, 300, 5], L)
-    m2 = right_padded_mask([10, 1024, 64, 999], L)
+    if layout == "blc":
+        xg = xg.transpose(1, 2).contiguous().transpose(1, 2)
+
+    def call(mask):
+        return cc.causal_conv1d_fn(xg, wg, attention_mask=mask, residual=True)
+
     mg = m1.to(DEV)
-    for m_cpu in (m1, m1, m2):
-        if m_cpu is m2:
-            mg.copy_(m2.to(DEV))     # same tensor object and address, new content
-        got = cc.causal_conv1d_fn(xg, wg, attention_mask=mg, residual=True)
-        assert_parity(got, co.conv1d_fwd(x, w, None, mask=m_cpu, residual=1), exact=True, what="narrowed mask")
+    assert_parity(call(mg), want1, exact=True, what="first")
+    assert_parity(call(mg), want1, exact=True, what="again")
+    mg.copy_(m2.to(DEV))             # same tensor object and address, new content
+    assert_parity(call(mg), want2, exact=True, what="written to")
+    mg.data.copy_(m1.to(DEV))        # ... without a new version
+    assert_parity(call(mg), want1, exact=True, what="written past the version counter")
     del mg
-    other = m1.to(DEV)               # may land on the freed address
-    got = cc.causal_conv1d_fn(xg, wg, attention_mask=other, residual=True)
-    assert_parity(got, co.conv1d_fwd(x, w, None, mask=m1, residual=1), exact=True, what="narrowed mask, new tensor")
+    other = m2.to(DEV)               # may land on the freed address
+    assert_parity(call(other), want2, exact=True, what="new tensor")
     sliced = torch.cat([m2, m1], dim=1).to(DEV)[:, -L:]      # a view, as CanonLayer slices it
-    got = cc.causal_conv1d_fn(xg, wg, attention_mask=sliced, residual=True)
-    assert_parity(got, co.conv1d_fwd(x, w, None, mask=m1, residual=1), exact=True, what="narrowed mask view")
+    assert_parity(call(sliced), want1, exact=True, what="view")
+
+    # two streams, the first one busy: what it has only enqueued is nothing the second may read
+    shared = m1.to(DEV)
+    torch.cuda.synchronize()
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    with torch.cuda.stream(first):
+        torch.cuda._sleep(20_000_000)
+        y1 = call(shared)
+    with torch.cuda.stream(second):
+        y2 = call(shared)
+    torch.cuda.synchronize()
+    assert_parity(y2, want1, exact=True, what="second stream")
+    assert_parity(y1, want1, exact=True, what="first stream")
+
+    # a graph captured after calls on the same mask, and eager calls after the capture
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call(shared)
+    assert_parity(call(shared), want1, exact=True, what="eager after the capture")
+    for m_cpu, want_m in (want[1], want[0], want[1]):
+        shared.copy_(m_cpu.to(DEV))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert_parity(out, want_m, exact=True, what="replay")
+        assert_parity(call(shared), want_m, exact=True, what="eager between replays")
 
 
 # ---- packed variable-length sequences (seq_idx) --------------------------------

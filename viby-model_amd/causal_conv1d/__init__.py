@@ -111,37 +111,26 @@ def _prep_bias(weight: torch.Tensor, bias: Optional[torch.Tensor]) -> Optional[t
     return bias
 
 
-_NARROW_MIN_ELEMENTS = 1 << 20
-# (key, the source mask (kept alive so its address stays unique), converted mask); replaced as one object, so
-# threads that race here each see a consistent entry
-_narrow_cache = (None, None, None)
+_NARROW_MIN_ELEMENTS = 1 << 24
 
 
 def _narrow_mask(mask: torch.Tensor, x: torch.Tensor, numel: int) -> torch.Tensor:
-    """An integer mask wider than x's element type is converted to x.dtype once.
+    """An integer mask wider than x's element type is converted to x.dtype for a large call.
 
-    Every (batch, channel) row re-reads its batch row of the mask, so an int64
-    mask moves four times the bytes of bf16 data through the caches.  The
-    conversion is what the multiply does anyway (``x * mask`` promotes the
-    integer to x.dtype, ``model/model.py:455``; the reference wrapper casts the
-    mask the same way, ``causal_conv1d_mps/__init__.py:244-247``).  The result
-    is cached on the mask's identity because a model passes one mask to every
-    Canon call of a forward.  Small problems keep the caller's mask as is.
+    Every (batch, channel) row re-reads its batch row of the mask, so an int64 mask moves four times the bytes of
+    bf16 data through the caches; the conversion costs about 3 us (and converts as ``x * mask`` does,
+    ``model/model.py:455``; the reference wrapper casts the mask the same way,
+    ``causal_conv1d_mps/__init__.py:244-247``).  Read as it is / converted, bf16, us: time-contiguous B 16 C 640 L 1024
+    11.0 / 12.4, B 4 C 960 L 4096 17.7 / 16.5, B 8 C 3456 L 1024 24.0 / 24.4 (training in fp32 104.7 / 100.0), B 32
+    86.1 / 75.2; strided kernels (B 32 C 3455) 311 / 301, training 754 / 690.  The channel-contiguous vector kernels
+    read an entry once per wave: 73.0 / 76.8 at B 32 C 3456, so they get the mask as it is.
+    The result belongs to this call alone: a copy kept for the next one would not follow what another stream, a
+    captured graph or a write past the version counter does to the mask.  (``canon_native.cpp`` has the same rule.)
     """
-    if (mask.dtype.is_floating_point or mask.element_size() <= x.element_size()
-            or numel < _NARROW_MIN_ELEMENTS):
+    if (mask.dtype.is_floating_point or mask.element_size() <= x.element_size() or numel < _NARROW_MIN_ELEMENTS
+            or (x.stride(1) == 1 and x.stride(2) != 1 and x.shape[1] * x.element_size() % 8 == 0)):
         return mask
-    if torch.compiler.is_compiling():
-        return mask.to(x.dtype)      # one node of the traced graph; identical conversions are merged there
-    if mask.is_inference():
-        return mask.to(x.dtype)      # tensors made under torch.inference_mode() carry no version counter to key on
-    global _narrow_cache
-    key = (mask.data_ptr(), mask._version, tuple(mask.shape), mask.stride(), mask.dtype, x.dtype, mask.device)
-    entry = _narrow_cache
-    if entry[0] != key:
-        entry = (key, mask, mask.to(x.dtype))
-        _narrow_cache = entry
-    return entry[2]
+    return mask.to(x.dtype)
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # the handle without building a Stream object
@@ -284,8 +273,7 @@ def causal_conv1d_fn(
     # a plain call is checked and launched in one native step; None: anything else, errors included, from here on
     if not torch.compiler.is_compiling() and x.is_cuda and not (return_final_states and final_states_out is None):
         out = _lib.native().try_fwd(x, weight, bias, seq_idx, initial_states, final_states_out, activation,
-                                    attention_mask if attention_mask is None else _narrow_mask(attention_mask, x, x.numel()),
-                                    residual, rounding)
+                                    attention_mask, residual, rounding)
         if out is not None:
             if type(out) is int:
                 _lib.check(out, "causal_conv1d_fn")
@@ -866,10 +854,8 @@ def causal_conv1d_fn_parts(
     """
     xs = list(xs)
     if not torch.compiler.is_compiling() and xs and xs[0].is_cuda and not (return_final_states and final_states_out is None):
-        outs = _lib.native().try_fwd_parts(
-            xs, weight, bias, initial_states, final_states_out, activation,
-            attention_mask if attention_mask is None else _narrow_mask(attention_mask, xs[0], sum(x.numel() for x in xs)),
-            residual, rounding)
+        outs = _lib.native().try_fwd_parts(xs, weight, bias, initial_states, final_states_out, activation, attention_mask,
+                                           residual, rounding)
         if outs is not None:
             if type(outs) is int:
                 _lib.check(outs, "causal_conv1d_fn_parts")

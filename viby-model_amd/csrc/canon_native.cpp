@@ -216,6 +216,18 @@ bool fwd_args_ok(const Tensor &x, int64_t B, int64_t C, int64_t L, const Tensor 
     return true;
 }
 
+// What _narrow_mask does: a wide integer mask of a large call is converted, for this call, to x's type, unless the
+// channel-contiguous vector kernels take it (`kept` holds it until the launch is enqueued).
+constexpr int64_t kNarrowMinElements = 1 << 24;
+const Tensor *narrow(const Tensor *mask, const Tensor &x, int64_t numel, Tensor &kept)
+{
+    if (!mask || at::isFloatingType(mask->scalar_type()) || mask->element_size() <= x.element_size() || numel < kNarrowMinElements ||
+        (x.stride(1) == 1 && x.stride(2) != 1 && x.size(1) * x.element_size() % 8 == 0))
+        return mask;
+    kept = mask->to(x.scalar_type());
+    return &kept;
+}
+
 // (a dispatch mode sees the tensor operations of the Python path, not what happens here)
 bool no_mode() { return !c10::impl::dispatch_mode_enabled(); }
 
@@ -238,7 +250,8 @@ PyObject *try_fwd(PyObject *, PyObject *const *args, Py_ssize_t n)
                                seq->scalar_type() == at::kInt && seq->device() == x->device()));
     void *stream;
     CANON_NONE_UNLESS(stream_of(*x, &stream));
-    Tensor out = at::empty_like(*x);
+    Tensor out = at::empty_like(*x), narrowed;
+    mask = narrow(mask, *x, x->numel(), narrowed);
     const canon_conv1d_fwd_params p = fwd_params(*x, out, *weight, bias, mask, init, fin, seq, act, res, rnd);
     const int rc = without_gil([&] { return canon_conv1d_fwd(&p, stream); });
     if (rc != CANON_OK) return PyLong_FromLong(rc);
@@ -278,6 +291,8 @@ PyObject *try_fwd_parts(PyObject *, PyObject *const *args, Py_ssize_t n)
         outs[i] = at::empty_like(*xs[i]);
         parts[i] = part_of(*xs[i], outs[i]);
     }
+    Tensor narrowed;
+    mask = narrow(mask, *xs[0], xs[0]->size(0) * dim * xs[0]->size(2), narrowed);
     canon_conv1d_fwd_params p = fwd_params(*xs[0], outs[0], *weight, bias, mask, init, fin, nullptr, act, res, rnd);
     p.channels = dim;
     p.x = p.out = nullptr;
