@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define CANON_CONV1D_ABI_VERSION 9
+#define CANON_CONV1D_ABI_VERSION 10
 #define CANON_CONV1D_MIN_WIDTH 2
 #define CANON_CONV1D_MAX_WIDTH 4
 
@@ -202,8 +202,8 @@ typedef struct canon_conv1d_bwd_params {
     int32_t width;
     int32_t activation;
     int32_t residual_mode;
-    int32_t grad_dtype;             /* element type of dweight and dbias: CANON_DTYPE_BF16 / _F16 (the fp32 sum rounded
-                                       once), anything else: fp32 */
+    int32_t grad_dtype;             /* element type of dweight and dbias (CANON_DTYPE_*; the fp32 sum rounded once).
+                                       A reserved word until ABI version 9. */
     int64_t batch, channels, seqlen;
     const void *x;
     int64_t x_stride_b, x_stride_c, x_stride_l;

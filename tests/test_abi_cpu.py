@@ -360,6 +360,15 @@ def test_bwd_plan_and_workspace():
                       (dict(initial_state=FAKE_X, initial_len=3, seq_idx=FAKE_X + 0x400000), "seq_idx")]:
         assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(bwd_params(**over))) == -1, over
         assert msg in last_error(), (over, last_error())
+    # the type of dweight / dbias, a reserved word until ABI version 9: one of the three, and a header that knows it
+    assert _lib.ABI_VERSION >= 10
+    for grad_dtype in (0, 1, 2):
+        assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(bwd_params(grad_dtype=grad_dtype))) > 0
+    for grad_dtype in (3, -1, 0x7fffffff):
+        q = bwd_params(grad_dtype=grad_dtype, workspace=FAKE_W + 0x200000, workspace_bytes=1 << 30)
+        assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q)) == -1
+        assert f"unknown grad_dtype {grad_dtype}" in last_error()
+        assert L.canon_conv1d_bwd(ctypes.byref(q), None) == _lib.ERR_INVALID_ARGUMENT
     assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(bwd_params(width=9))) == -1
     assert "width 9" in last_error()
     assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(bwd_params(B=0))) == 0

@@ -588,6 +588,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
                     p->struct_size, sizeof(canon_conv1d_bwd_params));
     if (!valid_dtype(p->x_dtype) || !valid_dtype(p->w_dtype))
         return fail(CANON_ERR_INVALID_ARGUMENT, "unknown x_dtype %d or w_dtype %d", p->x_dtype, p->w_dtype);
+    if (!valid_dtype(p->grad_dtype)) return fail(CANON_ERR_INVALID_ARGUMENT, "unknown grad_dtype %d", p->grad_dtype);
     if (p->width < CANON_CONV1D_MIN_WIDTH || p->width > CANON_CONV1D_MAX_WIDTH)
         return fail(CANON_ERR_UNSUPPORTED, "width %d not supported (only widths 2..4)", p->width);
     if (p->activation != CANON_ACT_NONE && p->activation != CANON_ACT_SILU)
@@ -646,7 +647,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     a.B = (uint32_t)p->batch; a.C = (uint32_t)p->channels; a.L = (uint32_t)p->seqlen;
     a.W = p->width; a.w_dtype = p->w_dtype; a.mask_dtype = p->mask_dtype;
     a.act = p->activation; a.res_mode = p->residual_mode;
-    a.grad_dtype = p->grad_dtype == CANON_DTYPE_BF16 || p->grad_dtype == CANON_DTYPE_F16 ? p->grad_dtype : CANON_DTYPE_F32;
+    a.grad_dtype = p->grad_dtype;
     a.w_vec = p->width == 4 && p->w_stride_k == 1 && p->w_stride_c == 4 && aligned16(p->weight);
     plan->kind = BWD_GENERIC;
     plan->U = 1;
