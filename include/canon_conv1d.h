@@ -404,7 +404,9 @@ const char *canon_conv1d_fwd_plan(const canon_conv1d_fwd_params *p);
  * mask, else 4; 4 for the other vector kernels and the strided one), 0 for an empty problem, -1 if rejected. */
 int canon_conv1d_fwd_plan_waves(const canon_conv1d_fwd_params *p);
 const char *canon_conv1d_update_plan(const canon_conv1d_update_params *p);
-const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p);   /* "bwd_blc_vec" | "bwd_bcl_vec" | "bwd_generic" */
+/* "bwd_blc_vec" | "bwd_blc_vec_seq" | "bwd_bcl_vec" | "bwd_bcl_vec_ragged" | "bwd_generic": with a workspace given the
+ * kernel that runs in that many bytes, without one the kernel that runs where there is room for its partial sets */
+const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p);
 /* "blc_vec_pair" (two dense tensors of one shape: one launch of the single-tensor code), "blc_vec_parts" /
  * "update_vec_parts" (one launch over a table of parts) or "per_part" (one launch per part) */
 const char *canon_conv1d_fwd_parts_plan(const canon_conv1d_fwd_params *p, const canon_conv1d_part *parts, int32_t nparts);

@@ -337,12 +337,29 @@ def test_bwd_plan_and_workspace():
     ws = L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(p))
     assert 0 < ws <= 20 << 20 and ws % (3456 * 5 * 4) == 0        # whole partial sets, bounded scratch
     assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl"))) == b"bwd_bcl_vec"
-    assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl", L=1023))) == b"bwd_generic"
+    # time-contiguous rows off the 16-byte vectors: the row kernel's ragged variant from 40 steps on, the walk kernel below
+    for length, want in ((1023, b"bwd_bcl_vec_ragged"), (1024, b"bwd_bcl_vec"), (41, b"bwd_bcl_vec_ragged"),
+                         (40, b"bwd_bcl_vec_ragged"), (39, b"bwd_generic"), (32, b"bwd_generic"), (128, b"bwd_bcl_vec"),
+                         (127, b"bwd_bcl_vec_ragged"), (120, b"bwd_bcl_vec_ragged")):
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl", L=length))) == want, length
     assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(C=3457))) == b"bwd_generic"
-    # packed sequences: only the walk kernel gates taps by sequence index
-    for layout in ("blc", "bcl"):
-        q = bwd_params(layout=layout, seq_idx=FAKE_X + 0x400000, seq_stride_b=1024, seq_stride_l=1)
-        assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == b"bwd_generic"
+    # packed sequences: the channel-contiguous kernel gates taps by sequence index, time-contiguous rows go to the walk kernel
+    for layout, over, want in (("blc", {}, b"bwd_blc_vec_seq"), ("blc", dict(C=3457), b"bwd_generic"), ("bcl", {}, b"bwd_generic"),
+                               ("bcl", dict(L=1023), b"bwd_generic")):
+        q = bwd_params(layout=layout, seq_idx=FAKE_X + 0x400000, seq_stride_b=1024, seq_stride_l=1, **over)
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == want
+    # with a workspace given: the kernel that runs in it (packed and ragged calls go to the walk kernel, whose sets are
+    # fewer where there are many channels; the others only take fewer sets)
+    for over, want in ((dict(B=96, C=1024, L=200, seq_idx=FAKE_X + 0x400000, seq_stride_b=200, seq_stride_l=1), b"bwd_blc_vec_seq"),
+                       (dict(B=132, C=1000, L=2100, layout="bcl"), b"bwd_bcl_vec_ragged"), (dict(B=96, C=1024, L=200), b"bwd_blc_vec")):
+        q = bwd_params(**over)
+        full = L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q))
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == want
+        q.workspace = FAKE_W + 0x200000
+        for nbytes, expected in ((full, want), (q.batch * q.channels * 20, b"bwd_generic" if over.get("layout") == "bcl" else want),
+                                 (16, want)):
+            q.workspace_bytes = nbytes
+            assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == expected, (over, nbytes)
     assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(bwd_params(seq_idx=FAKE_X + 2))) == -1
     assert "seq_idx must be 4-byte aligned" in last_error()
     # an initial state / the gradient of the captured final state: the channel-contiguous kernel handles both,
@@ -391,14 +408,17 @@ def _demanded_workspace(p):
 
 def test_bwd_workspace_query_covers_misaligned_pointers():
     L = _lib.lib()
-    # time-contiguous rows with a padded row stride, x off by one element: the call takes the strided kernel,
-    # which needs more scratch than the vector kernel an aligned x would get
+    # time-contiguous rows with a padded row stride, x off by one element: the call takes the ragged variant
     for over in (dict(x=FAKE_X + 2), dict(dout=FAKE_OUT + 2), dict(dx=FAKE_STATE + 2), dict()):
         q = bwd_params(layout="bcl", x_stride_c=1032, x_stride_b=3456 * 1032, **over)
-        want_kernel = b"bwd_generic" if over else b"bwd_bcl_vec"
+        want_kernel = b"bwd_bcl_vec_ragged" if over else b"bwd_bcl_vec"
         assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == want_kernel, over
         assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q)) == _demanded_workspace(q), over
-    for over in (dict(x=FAKE_X + 4), dict(dx=FAKE_STATE + 2)):          # channel-contiguous: 8-byte lanes
+    for over in (dict(x=FAKE_X + 1), dict(dout=FAKE_OUT + 1)):          # ... not even on an element: the strided kernel
+        q = bwd_params(layout="bcl", **over)
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == b"bwd_generic"
+        assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q)) == _demanded_workspace(q), over
+    for over in (dict(x=FAKE_X + 4), dict(dx=FAKE_STATE + 2)):          # channel-contiguous: 8-byte boundaries
         q = bwd_params(**over)
         assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == b"bwd_generic"
         assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q)) == _demanded_workspace(q), over

@@ -37,6 +37,24 @@ def gpu_grads(cc, x_cpu, w, b, dout_cpu, layout, mask=None, act=None, residual=F
     return xg.grad, wg.grad, (bg.grad if bg is not None else None), out.detach()
 
 
+def plan_of(x, W=4, seq_idx=None):
+    """The kernel that the backward of a plain call on x runs (dout and dx in x's layout)."""
+    import ctypes
+
+    from causal_conv1d import _lib
+    code = _lib.DTYPE_CODE[x.dtype]
+    others = [torch.empty_like(x) for _ in range(2)]
+    p = _lib.BwdParams(struct_size=ctypes.sizeof(_lib.BwdParams), x_dtype=code, w_dtype=code, width=W, batch=x.shape[0],
+                       channels=x.shape[1], seqlen=x.shape[2])
+    for name, t in zip(("x", "dout", "dx"), (x, *others)):
+        setattr(p, name, t.data_ptr())
+        for axis, stride in zip("bcl", t.stride()):
+            setattr(p, f"{name}_stride_{axis}", stride)
+    if seq_idx is not None:
+        p.seq_idx, p.seq_stride_b, p.seq_stride_l = seq_idx.data_ptr(), *seq_idx.stride()
+    return _lib.lib().canon_conv1d_bwd_plan(ctypes.byref(p)).decode()
+
+
 def check(got, want64, dtype, what, sum_terms=1):
     """dx-like tensors: fp32 to 2e-5 of the tensor's scale; 16-bit to 1 ulp of the rounded float64
     value.  Sums over `sum_terms` products are compared relative to the magnitude of the sum."""
@@ -317,6 +335,9 @@ def test_backward_of_packed_sequences(cc, dtype, layout):
             dx, dw, db, out = gpu_grads(cc, x, w, b, dout, layout, mask, act, res, seq_idx=seq)
             rdx, rdw, rdb, rout = conv1d_grads(x, w, b, dout, mask, act, res, seq_idx=seq)
             what = f"case {case} {dtype} {layout} {B}x{C}x{L} W{W} {act} {res}"
+            if layout == "blc" and L > 1:
+                whole = C * dtype.itemsize % 8 == 0
+                assert plan_of(dx, W, seq.to(DEV)) == ("bwd_blc_vec_seq" if whole else "bwd_generic"), what
             check(out, rout, dtype, what + " out")
             check(dx, rdx, dtype, what + " dx")
             check(dw, rdw, dtype, what + " dweight", sum_terms=B * L)
@@ -361,10 +382,14 @@ def test_backward_with_a_scratch_for_fewer_partial_sets(cc, kind, B, C, L, stati
         return p, dx, dw, db, space
 
     lib, stream = _lib.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    usual = {"channel": b"bwd_blc_vec", "packed": b"bwd_blc_vec_seq", "time": b"bwd_bcl_vec_ragged"}[kind]
     need = lib.canon_conv1d_bwd_workspace_bytes(ctypes.byref(params(16)[0]))
     small = scratch * C * 20 if scratch else 16
     assert need > (8 << 20 if static else small)
     full, few = params(need), params(small)
+    assert lib.canon_conv1d_bwd_plan(ctypes.byref(full[0])) == usual
+    if not static:
+        assert lib.canon_conv1d_bwd_plan(ctypes.byref(few[0])) == (b"bwd_generic" if kind == "time" else usual)
     assert lib.canon_conv1d_bwd(ctypes.byref(full[0]), stream) == 0
     call = lib.canon_conv1d_bwd_static if static else lib.canon_conv1d_bwd
     assert call(ctypes.byref(few[0]), stream) == 0, lib.canon_conv1d_last_error()
@@ -406,6 +431,9 @@ def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
                 buf[offset:].view(B, C, L + 1)[..., :L] = xg
                 xg = buf[offset:].view(B, C, L + 1)[..., :L]
             xg = xg.detach().requires_grad_()
+            # (a slice of longer rows is no dense tensor: dout and dx are rows of their own length, which may be whole vectors)
+            assert plan_of(xg, W) == ("bwd_generic" if L < 40 else
+                                      "bwd_bcl_vec" if L % E == 0 and L >= 16 * E and not offset else "bwd_bcl_vec_ragged")
             wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
             out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
             grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))
@@ -451,6 +479,13 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
         seq = torch.zeros(B, L, dtype=torch.int32)
         seq[0, L // 2:] = 1
         seq[1, L - 2:] = 1
+    probe = torch.empty(B, C, L, dtype=dtype, device=DEV)
+    if route != "bcl":
+        probe = probe.transpose(1, 2).contiguous().transpose(1, 2)
+    E = 16 // dtype.itemsize
+    assert plan_of(probe, W, None if seq is None else seq.to(DEV)) == (
+        "bwd_generic" if (L < 40 if route == "bcl" else C * dtype.itemsize % 8) else "bwd_blc_vec_seq" if route == "packed" else
+        "bwd_blc_vec" if route != "bcl" else "bwd_bcl_vec" if L % E == 0 and L >= 16 * E else "bwd_bcl_vec_ragged")
     for bad, back in ((float("inf"), 1), (float("-inf"), 2), (float("nan"), 1), (float("nan"), 3), (float("inf"), 4)):
         x = torch.randn(B, C, L, generator=g).to(dtype)
         if back <= L:
@@ -496,6 +531,7 @@ def test_backward_of_packed_sequences_in_chunks_of_several_tiles(cc, dtype, act,
         for c in cuts:
             seq[row, c:] += 1
     mask = right_padded_mask([max(1, L - i) for i in range(B)], L) if masked else None
+    assert plan_of(x.to(DEV).transpose(1, 2).contiguous().transpose(1, 2), 4, seq.to(DEV)) == "bwd_blc_vec_seq"
     dx, dw, db, out = gpu_grads(cc, x, w, b, dout, "blc", mask, act, "masked", seq_idx=seq)
     rdx, rdw, rdb, rout = conv1d_grads(x, w, b, dout, mask, act, "masked", seq_idx=seq)
     check(out, rout, dtype, "out")

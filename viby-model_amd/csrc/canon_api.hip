@@ -937,6 +937,16 @@ CANON_API int canon_conv1d_update_zero_skipped(const canon_conv1d_update_params 
     return launch_update_call(p, stream, true, "canon_conv1d_update_zero_skipped");
 }
 
+// What canon_conv1d_bwd makes of a call with this many bytes of scratch (the usual plan where no kernel's sets fit).
+static int plan_bwd_in(const canon_conv1d_bwd_params *p, BwdPlan *plan, int64_t scratch)
+{
+    const int rc = plan_bwd(p, plan, false, false, scratch);
+    if (rc != CANON_OK || plan->workspace_bytes <= scratch || !plan->walk_too) return rc;
+    BwdPlan walk;
+    if (plan_bwd(p, &walk, false, true) == CANON_OK && walk.workspace_bytes <= scratch) *plan = walk;
+    return CANON_OK;
+}
+
 CANON_API int canon_conv1d_bwd(const canon_conv1d_bwd_params *p, void *stream)
 {
     BwdPlan pl;
@@ -1034,9 +1044,7 @@ CANON_API int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *st
     q.workspace = ptr;
     q.workspace_bytes = kStaticScratchBytes;
     BwdPlan pl;
-    rc = plan_bwd(&q, &pl, false, false, kStaticScratchBytes);
-    if (rc == CANON_OK && pl.workspace_bytes > kStaticScratchBytes && pl.walk_too)
-        rc = plan_bwd(&q, &pl, false, true);   // what canon_conv1d_bwd falls back to
+    rc = plan_bwd_in(&q, &pl, kStaticScratchBytes);
     if (rc != CANON_OK) return rc;
     if (pl.workspace_bytes > kStaticScratchBytes)
         return fail(CANON_ERR_UNSUPPORTED,
@@ -1076,10 +1084,11 @@ CANON_API int64_t canon_conv1d_update_bwd_workspace_bytes(const canon_conv1d_upd
 CANON_API const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p)
 {
     BwdPlan pl;
-    if (plan_bwd(p, &pl, false) != CANON_OK) return nullptr;
-    // (packed and ragged rows keep the name callers know for them, whichever kernel takes them)
-    if (pl.walk_too) return "bwd_generic";
-    return pl.kind == BWD_BLC_VEC ? "bwd_blc_vec" : pl.kind == BWD_BCL_VEC ? "bwd_bcl_vec" : "bwd_generic";
+    const int rc = p && p->workspace ? plan_bwd_in(p, &pl, p->workspace_bytes) : plan_bwd(p, &pl, false);
+    if (rc != CANON_OK) return nullptr;
+    if (pl.kind == BWD_BLC_VEC) return pl.args.seq ? "bwd_blc_vec_seq" : "bwd_blc_vec";
+    if (pl.kind == BWD_BCL_VEC) return pl.ragged ? "bwd_bcl_vec_ragged" : "bwd_bcl_vec";
+    return "bwd_generic";
 }
 
 CANON_API const char *canon_conv1d_fwd_plan(const canon_conv1d_fwd_params *p)
