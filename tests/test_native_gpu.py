@@ -130,6 +130,33 @@ def test_decode_step_of_the_layer(cc, monkeypatch, dtype):
                 assert_same(*both(cc, monkeypatch, step), (B, C, S, dtype, mtype))
 
 
+class Tagged(torch.Tensor):
+    """A subclass as a library on top of torch brings one: plain data, a type of its own."""
+
+
+@pytest.mark.parametrize("layout", ["channel", "time"])
+def test_tensor_subclasses_keep_their_type(cc, monkeypatch, layout):
+    """empty_like of a subclass is of that subclass: outputs and input gradients are, with the native module as without."""
+    g = torch.Generator(device=DEV).manual_seed(5)
+    x = torch.randn(2, 40, 24, device=DEV, generator=g)
+    x = x.transpose(1, 2) if layout == "channel" else x.transpose(1, 2).contiguous()
+    w, b = torch.randn(24, 4, device=DEV, generator=g), torch.randn(24, device=DEV, generator=g)
+    tagged = x.as_subclass(Tagged)
+
+    def train():
+        xx, ww = tagged.detach().requires_grad_(), w.detach().requires_grad_()
+        y = cc.causal_conv1d_fn(xx, ww, b, activation="silu", residual=True)
+        return y.detach(), torch.autograd.grad(y.as_subclass(torch.Tensor).sum(), [xx, ww])
+
+    for call in (lambda: cc.causal_conv1d_fn(tagged, w, b), train, lambda: cc._launch_fwd(tagged, w, b, None, None, None, 0, 0, 0),
+                 lambda: cc.causal_conv1d_fn_parts([tagged[:, :8], tagged[:, 8:]], w, b),
+                 lambda: cc._launch_bwd(tagged, tagged, w, b, None, torch.empty(24, 4, device=DEV), torch.empty(24, device=DEV), 0, 0)):
+        native, general = both(cc, monkeypatch, call)
+        assert_same(native, general, layout)
+        assert [type(t) for t in flat(native)] == [type(t) for t in flat(general)]
+        assert type(flat(native)[0]) is Tagged
+
+
 def test_refused_calls(cc, monkeypatch):
     x, w, b = torch.randn(2, 8, 16, device=DEV), torch.randn(8, 4, device=DEV), torch.randn(8, device=DEV)
     mask, pool = torch.ones(2, 16, device=DEV), torch.randn(4, 8, 4, device=DEV)

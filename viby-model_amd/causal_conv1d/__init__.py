@@ -325,7 +325,7 @@ def _launch_fwd(x, weight, bias, mask, initial_states, final_states, act, res, r
         _lib.check(out, "causal_conv1d_fn")
     if out is not None:
         return out
-    out = torch.empty_like(x)      # (x on another device than the current one, or a dispatch mode)
+    out = torch.empty_like(x)      # (x on another device than the current one, a tensor subclass or a dispatch mode)
     p = _fill_fwd(x, out, weight, bias, mask, initial_states, final_states, act, res, rnd, seq_idx)
     rc = _call(_lib.lib().canon_conv1d_fwd, x.device, ctypes.byref(p))
     _lib.check(rc, "causal_conv1d_fn")
@@ -389,7 +389,7 @@ def _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx=N
             _lib.check(dx, "causal_conv1d_fn backward")
         if dx is not None:
             return dx
-    # nothing to launch over, x on another device than the current one, or a dispatch mode
+    # nothing to launch over, x on another device than the current one, a tensor subclass or a dispatch mode
     if dout.stride() != x.stride():
         dout = torch.empty_like(x).copy_(dout)       # same layout as x: keeps the vector kernel
     dx = torch.empty_like(x)

@@ -3,7 +3,7 @@
 // 7 of the 18 us such a call needs on the host (B 1, C 640, L 77: the kernel runs 6 us).
 //
 // The functions come in two kinds.  launch_*: the arguments were checked by the caller; the output (a status code where
-// the launch failed) is returned.  try_*: the public calls' own arguments; they check what the Python functions check
+// the launch failed) is returned, or None as below, where the tensors are not plain.  try_*: the public calls' own arguments; they check what the Python functions check
 // and launch, or return None without having done anything when a call is not plain (gradients, another device than the
 // current one, tensor subclasses, transforms, types that need a conversion, an argument that is wrong): the Python
 // function then goes on as if it had not asked, and raises what there is to raise.
@@ -61,8 +61,6 @@ bool plain(PyObject *o, const Tensor **t)
     *t = &v;
     return true;
 }
-
-const Tensor *given(PyObject *o) { return o == Py_None ? nullptr : &THPVariable_Unpack(o); }
 
 long small_int(PyObject *o) { return PyLong_AsLong(o); }
 
@@ -380,18 +378,19 @@ PyObject *try_decode_step(PyObject *, PyObject *const *args, Py_ssize_t n)
 }
 
 // launch_fwd(x, weight, bias, mask, initial_states, final_states, act, res, rnd, seq_idx) -> output | status code, of
-// checked arguments; None when x's device is not the current one
+// checked arguments; None when x's device is not the current one or a tensor is not plain
 PyObject *launch_fwd(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
     CANON_NONE_UNLESS(n == 10 && no_mode());
-    const Tensor &x = THPVariable_Unpack(args[0]);
+    const Tensor *x, *weight, *bias, *mask, *init, *fin, *seq;
+    CANON_NONE_UNLESS(plain(args[0], &x) && plain(args[1], &weight) && plain(args[2], &bias) && plain(args[3], &mask) &&
+                      plain(args[4], &init) && plain(args[5], &fin) && plain(args[9], &seq) && x && weight);
     void *stream;
-    CANON_NONE_UNLESS(stream_of(x, &stream));
-    Tensor out = at::empty_like(x);
-    const canon_conv1d_fwd_params p =
-        fwd_params(x, out, THPVariable_Unpack(args[1]), given(args[2]), given(args[3]), given(args[4]), given(args[5]), given(args[9]),
-                   (int)small_int(args[6]), (int)small_int(args[7]), (int)small_int(args[8]));
+    CANON_NONE_UNLESS(stream_of(*x, &stream));
+    Tensor out = at::empty_like(*x);
+    const canon_conv1d_fwd_params p = fwd_params(*x, out, *weight, bias, mask, init, fin, seq, (int)small_int(args[6]),
+                                                 (int)small_int(args[7]), (int)small_int(args[8]));
     const int rc = without_gil([&] { return canon_conv1d_fwd(&p, stream); });
     if (rc != CANON_OK) return PyLong_FromLong(rc);
     return THPVariable_Wrap(std::move(out));
@@ -400,18 +399,20 @@ PyObject *launch_fwd(PyObject *, PyObject *const *args, Py_ssize_t n)
 
 // launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx, initial_states, dinit, dfinal)
 //   -> dx | status code, of checked arguments (dout and dfinal of x's type); None when x's device is not the current one
+//   or a tensor is not plain
 PyObject *launch_bwd(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
     CANON_NONE_UNLESS(n == 13 && no_mode());
-    const Tensor &x = THPVariable_Unpack(args[0]);
+    const Tensor *xp, *gp, *wp, *dwp, *bias, *mask, *dbias, *seq, *init, *dinit, *dfin;
+    CANON_NONE_UNLESS(plain(args[0], &xp) && plain(args[1], &gp) && plain(args[2], &wp) && plain(args[3], &bias) &&
+                      plain(args[4], &mask) && plain(args[5], &dwp) && plain(args[6], &dbias) && plain(args[9], &seq) &&
+                      plain(args[10], &init) && plain(args[11], &dinit) && plain(args[12], &dfin) && xp && gp && wp && dwp);
+    const Tensor &x = *xp, &weight = *wp, &dweight = *dwp;
     void *stream;
     CANON_NONE_UNLESS(stream_of(x, &stream));
-    const Tensor &weight = THPVariable_Unpack(args[2]), &dweight = THPVariable_Unpack(args[5]);
-    const Tensor *bias = given(args[3]), *mask = given(args[4]), *dbias = given(args[6]), *seq = given(args[9]), *init = given(args[10]);
-    const Tensor *dinit = given(args[11]), *dfin = given(args[12]);
     Tensor dx = at::empty_like(x);
-    Tensor dout = THPVariable_Unpack(args[1]);
+    Tensor dout = *gp;
     if (dout.strides() != x.strides()) {
         // x's own layout keeps the vector kernels (empty_like: x's strides where x is dense)
         Tensor copy = at::empty_like(x);
