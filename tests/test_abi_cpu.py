@@ -37,6 +37,25 @@ def test_library_exports_every_declared_function():
     assert L.canon_conv1d_last_error() is not None
 
 
+def test_native_module_is_used_with_the_torch_it_was_built_for(monkeypatch):
+    import warnings
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        module = _lib.native()
+    assert callable(module.try_fwd) and torch.__version__.startswith(module.torch_version)
+    # another torch: left alone, with a warning, and every function declines (the general path takes the calls)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(torch, "__version__", "1.13.1+other")
+    with pytest.warns(RuntimeWarning, match=r"not built for this torch \(1\.13\.1\): it is for torch 2"):
+        other = _lib.native()
+    assert other.try_fwd(1, 2, 3) is None and other.launch_bwd() is None and _lib.native() is other
+    # not built at all: an error
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "NATIVE_PATH", "/nowhere/_native.so")
+    with pytest.raises(ImportError, match="build it with"):
+        _lib.native()
+
+
 def test_ctypes_structs_match_the_header(tmp_path):
     lines = ['#include <stdio.h>', '#include <stddef.h>', f'#include "{HEADER}"', 'int main(void){']
     structs = (("canon_conv1d_fwd_params", FwdParams), ("canon_conv1d_update_params", UpdateParams),

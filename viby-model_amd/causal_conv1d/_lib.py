@@ -7,11 +7,14 @@ from __future__ import annotations
 
 import ctypes
 import os
+import re
+import warnings
 
 import torch  # noqa: F401  (loads the HIP runtime the library binds to)
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libcanon_conv1d.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 
 ABI_VERSION = 10
 
@@ -198,17 +201,34 @@ def lib() -> ctypes.CDLL:
 _native = None
 
 
+class _OtherTorch:
+    """In the place of a native module built for another torch: every function of it declines, so every call takes the
+    general path (ctypes), which needs nothing of torch but its Python interface."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 def native():
     """The module that takes torch tensors to the library without a Python statement per field; raises if it has not
-    been built."""
+    been built.  It is compiled against one torch's C++ interface: under another torch it is left alone, with a
+    warning, and calls cost more host time."""
     global _native
     if _native is None:
         lib()
+        if not os.path.exists(NATIVE_PATH):
+            raise ImportError(f"{NATIVE_PATH} not found: build it with `make -j4 -C viby-model_amd/csrc`. "
+                              "There is no fallback implementation.")
+        running = re.match(r"[0-9.]*[0-9]", torch.__version__).group()
         try:
             from . import _native as module
+            reason = None if module.torch_version == running else f"it is for torch {module.torch_version}"
         except ImportError as e:
-            raise ImportError(f"causal_conv1d._native cannot be loaded ({e}): build it with "
-                              "`make -j4 -C viby-model_amd/csrc`. There is no fallback implementation.") from e
+            reason = str(e)
+        if reason is not None:
+            warnings.warn(f"causal_conv1d: {NATIVE_PATH} was not built for this torch ({running}): {reason}. Calls take the "
+                          "slower general path until `make -B -C viby-model_amd/csrc` has built it again.", RuntimeWarning)
+            module = _OtherTorch()
         _native = module
     return _native
 

@@ -16,6 +16,7 @@
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include "canon_conv1d.h"
 
@@ -488,5 +489,8 @@ PyMODINIT_FUNC PyInit__native()
     g_get_device = PyObject_GetAttrString(torch_c, "_cuda_getDevice");
     Py_DECREF(torch_c);
     if (!g_raw_stream || !g_get_device) return nullptr;
-    return PyModule_Create(&module);
+    // (torch's C++ interface is another one in every release: the loader compares this before it calls anything)
+    PyObject *m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
 }
