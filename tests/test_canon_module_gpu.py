@@ -190,9 +190,10 @@ def test_unmodified_model_call_pattern():
 
 
 def test_prepared_decode_call_agrees_with_the_checked_path():
-    """The decode fast path (a signature seen once is launched from a prepared argument block): second and later
-    calls with a mask that grew, a token that is a non-contiguous view, and a trainable bias under autograd give
-    what the fully checked path gives, and the table of signatures never grows beyond its limit."""
+    """The two decode fast paths, a layer's step (checked and launched natively) and causal_conv1d_update (a signature
+    seen once is launched from a prepared argument block): first and later calls, with a mask that grew, a token that is
+    a non-contiguous view, and a trainable bias under autograd, give what the oracle gives, and the table of signatures
+    never grows beyond its limit."""
     import causal_conv1d as cc
     from oracle import canon_oracle as co
     torch.manual_seed(9)
@@ -202,6 +203,9 @@ def test_prepared_decode_call_agrees_with_the_checked_path():
     layer = make_layer(C, 4, w, b, False, dtype, "fused")
     cache = types.SimpleNamespace()
     state_ref = torch.zeros(B, C, 8, dtype=dtype)
+    known = cc._known_updates()
+    known.clear()
+    wd, bd, state_direct = w.to(DEV), b.to(DEV), torch.zeros(B, C, 8, dtype=dtype, device=DEV)
     with torch.no_grad():
         for step, width in enumerate([3, 4, 9, 9, 17]):           # the mask's length changes from call to call
             wide = torch.randn(B, 3, 2 * C).to(dtype)
@@ -210,10 +214,14 @@ def test_prepared_decode_call_agrees_with_the_checked_path():
             mask[step % B, -1] = 0
             got = layer(tok.to(DEV) if tok.is_contiguous() else wide.to(DEV)[:, 1:2, ::2], attention_mask=mask.to(DEV),
                         cache=cache, layer_idx=0)
+            direct = cc.causal_conv1d_update((tok.to(DEV) if tok.is_contiguous() else wide.to(DEV)[:, 1:2, ::2])[:, 0], state_direct,
+                                             wd, bd, token_mask=mask[:, -1].clone().to(DEV), residual="unmasked")
+            assert len(known) == min(step + 1, 2)                 # two signatures: the later steps come from their blocks
             xt = tok[:, 0] * mask[:, -1:].to(dtype)
             want = tok[:, 0] + co.conv1d_update(xt.contiguous(), state_ref, w, b)   # the residual is the unmasked token
             assert torch.equal(bits(cache.canon_cache_a[0]), bits(state_ref)), step
             assert_parity(got[:, 0], want.to(dtype), exact=False, what=f"step {step}", res=tok[:, 0])
+            assert torch.equal(bits(direct), bits(got[:, 0])) and torch.equal(bits(state_direct), bits(state_ref)), step
     # a frozen weight with a trainable bias takes the autograd path, not the prepared launch
     layer.weight.requires_grad_(False)
     layer.bias_param.requires_grad_(True)
@@ -223,7 +231,6 @@ def test_prepared_decode_call_agrees_with_the_checked_path():
     y.float().sum().backward()
     assert layer.bias_param.grad is not None and torch.isfinite(layer.bias_param.grad.float()).all()
     # the table keeps its size: new signatures push the oldest ones out
-    known = cc._known_updates()
     with torch.no_grad():
         for n in range(cc._KNOWN_UPDATES_MAX + 8):
             x = torch.zeros(1, 2 + 2 * n, dtype=dtype, device=DEV)

@@ -609,46 +609,16 @@ def _canon_decode_step(x: torch.Tensor, conv_state: torch.Tensor, taps: torch.Te
     """The single-token call of ``canon.CanonLayer`` (inference): ``x`` is the layer's (batch, 1, dim) input as it
     is, ``attention_mask`` the whole-history (batch, >= 1) mask whose LAST column scales the token, the residual
     is the unmasked token; returns (batch, 1, dim).  Same kernel and same checks as ``causal_conv1d_update`` on
-    ``x[:, 0]`` / ``attention_mask[:, -1]``, without building those views and the output's: a signature that
-    has been through ``causal_conv1d_update`` once is launched from its prepared argument block."""
-    if torch.compiler.is_compiling():
-        token_mask = attention_mask[:, -1] if attention_mask is not None else None
-        return causal_conv1d_update(x[:, 0], conv_state, taps, bias, activation=activation, token_mask=token_mask,
-                                    residual="unmasked", rounding=rounding).unsqueeze(1)
-    if x.is_cuda:
+    ``x[:, 0]`` / ``attention_mask[:, -1]``, without building those views and the output's where the call is plain."""
+    if not torch.compiler.is_compiling() and x.is_cuda:
         out = _lib.native().try_decode_step(x, conv_state, taps, bias, attention_mask, activation, rounding)
         if out is not None:
             if type(out) is int:
                 _lib.check(out, "causal_conv1d_update")
             return out
-    key = (x.shape, x.stride(), x.dtype, x.device, conv_state.shape, conv_state.stride(), conv_state.dtype,
-           conv_state.device, taps.shape, taps.stride(), taps.dtype, taps.device,
-           None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device),
-           None if attention_mask is None else (attention_mask.dim(), attention_mask.shape[0], attention_mask.stride(1),
-                                                attention_mask.dtype, attention_mask.device),
-           activation, rounding)
-    known = _known_updates()
-    p = known.get(key)
-    if p is None:
-        token_mask = attention_mask[:, -1] if attention_mask is not None else None
-        y = causal_conv1d_update(x[:, 0], conv_state, taps, bias, activation=activation, token_mask=token_mask,
-                                 residual="unmasked", rounding=rounding)
-        if y.numel() and (bias is None or (bias.dtype == taps.dtype and bias.is_contiguous())):
-            # x[:, 0] and a contiguous (batch, dim) output: the strides of every later call with this signature
-            _remember_update(key, _fill_update(x[:, 0], y, conv_state, taps, bias, token_mask, _activation_flag(activation),
-                                               _residual_mode("unmasked"), _round_mode(rounding)))
-        return y.unsqueeze(1)
-    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-    p.x, p.out, p.conv_state, p.weight = x.data_ptr(), out.data_ptr(), conv_state.data_ptr(), taps.data_ptr()
-    if bias is not None:
-        p.bias = bias.data_ptr()
-    if attention_mask is not None:
-        p.token_mask = attention_mask.data_ptr() + (attention_mask.shape[1] - 1) * attention_mask.stride(1) * attention_mask.element_size()
-        p.mask_stride_b = attention_mask.stride(0)
-    rc = _call(_lib.lib().canon_conv1d_update, x.device, ctypes.byref(p))
-    if rc:
-        _lib.check(rc, "causal_conv1d_update")
-    return out
+    token_mask = attention_mask[:, -1] if attention_mask is not None else None
+    return causal_conv1d_update(x[:, 0], conv_state, taps, bias, activation=activation, token_mask=token_mask,
+                                residual="unmasked", rounding=rounding).unsqueeze(1)
 
 
 # signature of a checked decode call -> its prepared argument block; per thread, because the block is written to

@@ -216,7 +216,7 @@ class GraphedDecodeStep:
     ``state`` further tensors the step modifies (token, position, K / V buffers, ...).
 
     The constructor runs the step once on a side stream as a warm-up (loads code objects, fills the allocator's
-    pools and the prepared-call table of the decode launches), puts every conv state and every tensor in ``state``
+    pools), puts every conv state and every tensor in ``state``
     back to what it was, and captures.  ``replay()`` then advances the model by one token; its results equal the
     step launched kernel by kernel bit for bit.  No ``hipMemsetAsync`` is recorded by the Canon launches (the
     library clears with fill kernels).
