@@ -362,6 +362,12 @@ def test_bwd_plan_and_workspace():
                          (127, b"bwd_bcl_vec_ragged"), (120, b"bwd_bcl_vec_ragged")):
         assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl", L=length))) == want, length
     assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(C=3457))) == b"bwd_generic"
+    # channel-contiguous: one row for every step (a stride of zero) is a layout like any other; rows further apart than a
+    # buffer resource reaches, or in falling order, take the walk kernel
+    for over, want in ((dict(x_stride_l=0), b"bwd_blc_vec"), (dict(dout_stride_l=0), b"bwd_blc_vec"),
+                       (dict(x_stride_l=0, dout_stride_l=0), b"bwd_blc_vec"), (dict(x_stride_l=-3456), b"bwd_generic"),
+                       (dict(dout_stride_l=1 << 27), b"bwd_generic"), (dict(dx_stride_l=1 << 26), b"bwd_blc_vec")):
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(**over))) == want, over
     # packed sequences: the channel-contiguous kernel gates taps by sequence index, time-contiguous rows go to the walk kernel
     for layout, over, want in (("blc", {}, b"bwd_blc_vec_seq"), ("blc", dict(C=3457), b"bwd_generic"), ("bcl", {}, b"bwd_generic"),
                                ("bcl", dict(L=1023), b"bwd_generic")):

@@ -402,6 +402,44 @@ def test_backward_with_a_scratch_for_fewer_partial_sets(cc, kind, B, C, L, stati
         assert lib.canon_conv1d_bwd(ctypes.byref(few[0]), stream) == _lib.ERR_INVALID_ARGUMENT
 
 
+@pytest.mark.parametrize("which", ["x", "dout", "both"])
+@pytest.mark.parametrize("act", [0, 1])
+def test_backward_of_one_row_for_every_step(cc, which, act):
+    """x or dout given as one row with a time stride of zero (C ABI): the bits of the same values written out."""
+    import ctypes
+
+    from causal_conv1d import _lib
+    g = torch.Generator(device=DEV).manual_seed(6)
+    B, C, L = 3, 136, 101
+    w, b = torch.randn(C, 4, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+    rows = {n: torch.randn(B, 1, C, device=DEV, generator=g).bfloat16() for n in ("x", "dout")}
+    full = {n: r.expand(B, L, C).contiguous() for n, r in rows.items()}
+    if which != "both":
+        other = "dout" if which == "x" else "x"
+        full[other] = torch.randn(B, L, C, device=DEV, generator=g).bfloat16()
+    results = []
+    for shared in (False, True):
+        dx, dw, db = torch.empty(B, L, C, dtype=torch.bfloat16, device=DEV), torch.empty(C, 4, device=DEV), torch.empty(C, device=DEV)
+        space = torch.empty(1 << 20, dtype=torch.uint8, device=DEV)
+        p = _lib.BwdParams(struct_size=ctypes.sizeof(_lib.BwdParams), x_dtype=1, w_dtype=0, width=4, activation=act,
+                           residual_mode=1, batch=B, channels=C, seqlen=L)
+        for name in ("x", "dout"):
+            one = shared and which in (name, "both")
+            setattr(p, name, (rows if one else full)[name].data_ptr())
+            for axis, stride in zip("bcl", (C, 1, 0) if one else (L * C, 1, C)):
+                setattr(p, f"{name}_stride_{axis}", stride)
+        p.dx, p.dx_stride_b, p.dx_stride_c, p.dx_stride_l = dx.data_ptr(), L * C, 1, C
+        p.weight, p.w_stride_c, p.w_stride_k, p.bias = w.data_ptr(), 4, 1, b.data_ptr()
+        p.dweight, p.dbias, p.workspace, p.workspace_bytes = dw.data_ptr(), db.data_ptr(), space.data_ptr(), space.numel()
+        lib = _lib.lib()
+        assert lib.canon_conv1d_bwd_plan(ctypes.byref(p)) == b"bwd_blc_vec"
+        assert lib.canon_conv1d_bwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        torch.cuda.synchronize()
+        results.append((dx, dw, db))
+    for a, c in zip(*results):
+        assert torch.equal(bits(a), bits(c))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
     """Rows that are no whole number of 16-byte vectors, or lie off 16-byte boundaries: around the shortest the

@@ -718,8 +718,9 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     const bool vec = !force_generic && a.x_sc == 1 && a.g_sc == 1 && a.d_sc == 1 && a.C % E8 == 0 && a.x_sl != 1 &&
                      a.x_sb % E8 == 0 && a.x_sl % E8 == 0 && a.g_sb % E8 == 0 && a.g_sl % E8 == 0 &&
                      a.d_sb % E8 == 0 && a.d_sl % E8 == 0 && ptrs8 &&
-                     // rows are addressed by 32-bit scalar offsets inside a slab's buffer resources
-                     a.x_sl > 0 && a.g_sl > 0 && a.d_sl > 0 &&
+                     // rows are addressed by 32-bit scalar offsets inside a slab's buffer resources (one row for every
+                     // step of x or dout is a stride of zero)
+                     a.x_sl >= 0 && a.g_sl >= 0 && a.d_sl > 0 &&
                      (uint64_t)(kBwdSlab + 3) * (uint64_t)std::max({a.x_sl, a.g_sl, a.d_sl}) * elem_bytes(p->x_dtype) + 1024 < (1ull << 31);
     if (vec) {
         const uint32_t nvec = a.C / kBwdLaneChannels;
