@@ -434,19 +434,15 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
             if constexpr (W >= 3) acc = fmaf(w[e][W - 3], dv[1][e], acc);
             if constexpr (W == 4) acc = fmaf(w[e][0], dv[2][e], acc);
             o[e] = acc;
-        }
-        // (steps past the end of the sequence are left out, not multiplied by their dz of zero: their window holds the
-        // sequence's last inputs, and 0 * Inf is NaN)
-        if (FULL || r < rows) {
+            // Steps past the end of the sequence have a dz of zero, but their window holds the sequence's last inputs, and
+            // 0 * Inf is NaN: the window is zero as well (selects), or the sums are left out (a branch).  By register
+            // count: the branch costs the ordinary instances five registers and with SiLU (95 -> 100) a wave per SIMD;
+            // the gated sweep holds 107 with it, 128 with the selects.
+            if (!SEQ || r < rows) {
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-#pragma unroll
-                for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], xv[(4 - W) + k][e], dw[e][k]);
+                for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], FULL || SEQ || r < rows ? xv[(4 - W) + k][e] : 0.0f, dw[e][k]);
                 dw[e][W - 1] = fmaf(dz[e], xw[3][e], dw[e][W - 1]);
             }
-        }
-#pragma unroll
-        for (int e = 0; e < E; ++e) {
             dbs[e] += dz[e];
             dzf[2][e] = dzf[1][e];
             dzf[1][e] = dzf[0][e];
