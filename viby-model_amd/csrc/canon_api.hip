@@ -544,8 +544,6 @@ int plan_update_parts(const canon_conv1d_update_params *p, const canon_conv1d_pa
 // ---------------------------------------------------------------------------
 // backward: planning and launch
 // ---------------------------------------------------------------------------
-// check_pointers: the call itself (x, dout, dx, weight, dweight and the workspace must be there).  Without it
-// (queries) NULL pointers pass and count as aligned.  force_generic: plan the strided kernel whatever the layout.
 // How the channel-contiguous backward cuts a sequence: n chunks of len steps (whole tiles) of at most `longest`, the
 // fewest that give one and a half blocks per CU.  A block walks every tile of its chunk, so the chunks are cut equal
 // (chunks of a fixed length would leave the last one mostly empty, L = 520 as 512 + 8), and a slightly larger count
@@ -579,6 +577,8 @@ BwdChunks bwd_chunks(uint32_t B, uint32_t L, uint32_t nct, uint32_t longest)
     return c;
 }
 
+// check_pointers: the call itself (x, dout, dx, weight, dweight and the workspace must be there).  Without it
+// (queries) NULL pointers pass and count as aligned.  force_generic: plan the strided kernel whatever the layout.
 // scratch: bytes of scratch the call will have, where that is known before its pointers are (-1: not)
 int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointers, bool force_generic = false, int64_t scratch = -1)
 {

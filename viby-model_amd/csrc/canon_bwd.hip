@@ -296,7 +296,9 @@ __global__ __launch_bounds__(256) void canon_bwd_walk_kernel(const BwdArgs a)
 // of a channel stay in registers through the sweep, about thirty of them, so
 // the channels a lane owns decide how many waves a CU holds: with four
 // channels (8 bytes of a 16-bit row) 170-200 registers, two blocks per CU;
-// with two 81-95, five or six.  And chunks of 128 steps where the grid alone
+// with two 82-100 (16-bit types, neither states nor packed rows; 93-107 with
+// packed rows, 100-123 with states; fp32 94-110, 104-123, 113-130), four or
+// five.  And chunks of 128 steps where the grid alone
 // would allow up to 1024: a CU then has new blocks to start while others drain,
 // for one partial set (20 bytes per channel) per 768 bytes of rows read and
 // written.  With both, us per call with the reduction, four channels -> two,
@@ -496,8 +498,7 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 // mask.  A slab whose reach (three rows before it to three after) lies in one sequence, which is nearly every slab
 // of rows packed from documents of hundreds of tokens, takes the ordinary sweep after one ballot; only a slab with a
 // boundary in reach takes the sweep that gates each tap.  The walk kernel, which gates every row and reads two bytes
-// per lane, took 192 us at B 2, C 3456, L 8192, bf16, SiLU (the whole training
-// call 233.0 us with it, 131.4 us with this one).
+// per lane, took 192 us at B 2, C 3456, L 8192, bf16, SiLU, this one 74 (profiled; the whole training call 233 us with it, 118 now).
 template <int DT, int W, bool MASK, bool ACT, bool STATES, bool SEQ = false>
 __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 {

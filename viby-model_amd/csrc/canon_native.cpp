@@ -1,12 +1,12 @@
 // causal_conv1d._native: the host path of the prefill, the pool / ring decode step and the backward, from torch tensors
 // to the C ABI, without a Python statement per field.  Filled through ctypes the argument block of a prefill took
-// 7 of the 18 us such a call needs on the host (B 1, C 640, L 77: the kernel runs 6 us).
+// 7 of the 18 us such a call needed on the host (CanonLayer, B 1, C 640, L 77: now 12 us, of which the kernel is 4).
 //
 // The functions come in two kinds.  launch_*: the arguments were checked by the caller; the output (a status code where
-// the launch failed) is returned, or None as below, where the tensors are not plain.  try_*: the public calls' own arguments; they check what the Python functions check
-// and launch, or return None without having done anything when a call is not plain (gradients, another device than the
-// current one, tensor subclasses, transforms, types that need a conversion, an argument that is wrong): the Python
-// function then goes on as if it had not asked, and raises what there is to raise.
+// the launch failed) is returned, or None where the tensors are not plain.  try_*: the public calls' own arguments; they
+// check what the Python functions check and launch, or return None without having done anything when a call is not plain
+// (gradients, another device than the current one, tensor subclasses, transforms, types that need a conversion, an
+// argument that is wrong): the Python function then goes on as if it had not asked, and raises what there is to raise.
 #include <Python.h>
 #include <string.h>
 

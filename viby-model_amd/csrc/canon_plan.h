@@ -115,7 +115,7 @@ struct BwdArgs {
     float *partial;
     void *dweight;        // of type grad_dtype
     void *dbias;
-    const int32_t *seq;   // packed-sequence indices [B, L] or nullptr (walk kernel only)
+    const int32_t *seq;   // packed-sequence indices [B, L] or nullptr (walk and channel-contiguous kernels)
     int64_t q_sb, q_sl;
     const char *init;     // inputs before t = 0, [B, C, S_in], or nullptr (walk and channel-contiguous kernels)
     char *dinit;          // their gradient, or nullptr
