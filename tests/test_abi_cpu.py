@@ -332,6 +332,24 @@ def test_canon_layer_module_mirrors_the_reference_class():
         layer(torch.randn(1, 4, 640))
 
 
+def test_canon_layer_taps_follow_the_weight():
+    """The (C, K) view a layer keeps outside autograd: shows in-place updates, and is made anew when the weight's storage,
+    address, size or type changes (channels cut off in place keep the address)."""
+    import types
+    from causal_conv1d.canon import CanonLayer
+    cfg = types.SimpleNamespace(canon_kernel=4, canon_bias=True, canon_activation=False)
+    layer = CanonLayer(16, cfg, "a")
+    with torch.no_grad():
+        first = layer._taps()
+        assert layer._taps() is first and tuple(first.shape) == (16, 4)
+        layer.weight.mul_(2)
+        assert torch.equal(layer._taps(), layer.weight[:, 0])
+        for change in (lambda w: w[:8], lambda w: w[::2], lambda w: w.clone(), lambda w: w.double(), lambda w: w[:, :, :3]):
+            layer.weight.data = change(layer.weight.data)
+            assert layer._taps().dtype == layer.weight.dtype and torch.equal(layer._taps(), layer.weight[:, 0])
+            assert layer._taps().stride() == layer.weight[:, 0].stride()
+
+
 def bwd_params(B=8, C=3456, L=1024, layout="blc", dtype=1, **over):
     p = BwdParams()
     p.struct_size = ctypes.sizeof(BwdParams)

@@ -68,7 +68,7 @@ class CanonLayer(nn.Module):
             self.bias_param = nn.Parameter(torch.zeros(hidden_size))
         else:
             self.register_parameter("bias_param", None)
-        self._taps_view = None   # (address of the weight, its (C, K) view): see _taps
+        self._taps_view = None   # (address and size of the weight, its (C, K) view): see _taps
 
     def reset_parameters(self) -> None:
         nn.init.kaiming_uniform_(self.weight, a=math.sqrt(5))
@@ -104,10 +104,11 @@ class CanonLayer(nn.Module):
         if torch.is_grad_enabled() and w.requires_grad:
             return w.squeeze(1)
         kept = self._taps_view
-        if kept is None or kept[0] != w.data_ptr() or kept[1].device != w.device or kept[1].dtype != w.dtype:
-            kept = (w.data_ptr(), w.detach().squeeze(1))
+        if (kept is None or kept[0] != w.data_ptr() or kept[1] != w.numel() or kept[2].dtype != w.dtype
+                or kept[2].device != w.device):
+            kept = (w.data_ptr(), w.numel(), w.detach().squeeze(1))
             self._taps_view = kept
-        return kept[1]
+        return kept[2]
 
     def forward(self, x: torch.Tensor, attention_mask: Optional[torch.Tensor] = None,
                 cache=None, layer_idx: Optional[int] = None) -> torch.Tensor:
