@@ -553,6 +553,47 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
             assert torch.equal(torch.isfinite(dw), torch.isfinite(dws)), (bad, back, "silu")
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_backward_of_short_rows_of_any_length_and_alignment(cc, dtype):
+    """Rows of 1..32 vectors share waves: every distance of the row's end from a vector's, vector counts that fill a
+    wave's lanes and that leave some idle, a last wave that is not full, rows in a buffer of longer rows, every mask
+    type; and an Inf or a NaN among a row's last inputs stays in the taps that read it (and in its channel)."""
+    g = torch.Generator().manual_seed(23)
+    E = 16 // dtype.itemsize
+    masks = [None, torch.int64, torch.bool, torch.float32, torch.int32, torch.bfloat16, torch.float16]
+    lengths = [E, E + 1, 2 * E - 1, 2 * E, *(3 * E + j for j in range(1, E)), 9 * E + 2, 10 * E + 1, 16 * E + 1, 21 * E - 1, 21 * E, 32 * E - 1, 32 * E]
+    for n, L in enumerate(lengths):
+        B, C, W, off = (1, 2, 3)[n % 3], (13, 67, 130)[n % 3], 4 - n % 3, (0, 3)[n % 2]
+        act, res, mtype = (None, "silu")[n % 4 >= 2], (False, "masked", "unmasked")[n % 3], masks[n % len(masks)]
+        x, dout = torch.randn(B, C, L, generator=g).to(dtype), torch.randn(B, C, L, generator=g).to(dtype)
+        w = (torch.randn(C, W, generator=g) * 0.5).to(dtype)
+        b = (torch.randn(C, generator=g) * 0.2).to(dtype) if n % 4 else None
+        mask = None
+        if mtype is not None:
+            mask = right_padded_mask([max(1, L - 3 * i) for i in range(B)], L)
+            mask[:, L // 2] = 0
+            mask = mask.to(mtype)
+        rdx, rdw, rdb, _ = conv1d_grads(x, w, b, dout, mask, act, res)
+        buf = torch.zeros(off + B * C * (L + off), dtype=dtype, device=DEV)
+        xg = buf[off:].view(B, C, L + off)[..., :L]
+        xg.copy_(x)
+        xg = xg.detach().requires_grad_()
+        wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
+        out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
+        grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))
+        what = f"{dtype} {B}x{C}x{L} W{W} {act} {res} {mtype} offset {off}"
+        check(grads[0], rdx, dtype, what + " dx")
+        check(grads[1], rdw, dtype, what + " dweight", sum_terms=B * L)
+        if b is not None:
+            check(grads[2], rdb, dtype, what + " dbias", sum_terms=B * L)
+        if C > 13:
+            x[B - 1, 0::2, L - 1 - n % 3] = (float("inf"), float("nan"))[n % 2]
+            _, dw, _, _ = gpu_grads(cc, x, w, torch.zeros(C, dtype=dtype), dout, "bcl", act=None)
+            want = dweight_of(x, dout, W)
+            assert torch.equal(torch.isfinite(dw.cpu()), torch.isfinite(want)), what
+            check(dw[1::2], want[1::2], dtype, what + " finite channels", sum_terms=B * L)
+
+
 @pytest.mark.parametrize("dtype,act,masked", [(torch.bfloat16, "silu", False), (torch.bfloat16, None, True), (torch.float32, "silu", True)])
 def test_backward_of_packed_sequences_in_chunks_of_several_tiles(cc, dtype, act, masked):
     """Enough columns that one block walks a whole row (three tiles of 32 steps and a part of one): boundaries between

@@ -731,6 +731,40 @@ def test_long_unmasked_time_contiguous_rows_of_several_segments(cc, dtype, shape
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_short_rows_of_any_length_and_alignment(cc, dtype):
+    """Rows of 1..32 vectors that are no whole number of vectors, or off the 16-byte grid: every distance of the row's
+    end from a vector's, vector counts that fill a wave's lanes and that leave some idle, a last wave that is not full,
+    rows in a buffer of longer rows (offset), every mask type, states."""
+    g = torch.Generator().manual_seed(17)
+    E = 16 // dtype.itemsize
+    masks = [None, torch.int64, torch.bool, torch.float32, torch.int32, torch.bfloat16, torch.float16]
+    lengths = [E, E + 1, 2 * E - 1, 2 * E, *(3 * E + j for j in range(1, E)), 9 * E + 2, 10 * E + 1, 16 * E + 1, 21 * E - 1, 21 * E + 1, 32 * E - 1]
+    for n, L in enumerate(lengths):
+        B, C, W, off = (1, 2, 3)[n % 3], (13, 67, 130)[n % 3], 4 - n % 3, (0, 3)[n % 2]
+        act, res, mtype = (None, "silu")[n % 4 == 3], (False, "masked", "unmasked")[n % 3], masks[n % len(masks)]
+        x = torch.randn(B, C, L, generator=g).to(dtype)
+        w = (torch.randn(C, W, generator=g) * 0.3).to(dtype)
+        b = (torch.randn(C, generator=g) * 0.1).to(dtype) if n % 4 else None
+        init = torch.randn(B, C, 5, generator=g).to(dtype) if n % 2 else None
+        mask = None
+        if mtype is not None:
+            mask = right_padded_mask([max(1, L - 3 * i) for i in range(B)], L)
+            mask[:, L // 2] = 0
+        buf = torch.zeros(off + B * C * (L + off), dtype=dtype, device=DEV)
+        xg = buf[off:].view(B, C, L + off)[..., :L]
+        xg.copy_(x)
+        for rounding in ("fused", "eager"):
+            want, want_fs = co.conv1d_fwd(x, w, b, mask=mask, activation=act, residual=res, initial_state=init, final_state_len=8,
+                                          round_mode=int(rounding == "eager"))
+            got, fs = run_fwd(cc, xg, w, b, act=act, mask=None if mask is None else mask.to(mtype), residual=res, init=init, S_out=8,
+                              rounding=rounding)
+            what = f"{dtype} {B}x{C}x{L} W{W} {act} {res} {mtype} offset {off} {rounding}"
+            xm = x if mask is None else (x.float() * mask[:, None, :].float()).to(dtype)
+            assert_parity(got, want, exact=act is None, what=what, res=(x if res == "unmasked" else xm) if res else None)
+            assert torch.equal(bits(fs), bits(want_fs)), what
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
 def test_short_time_contiguous_rows_share_a_wave(cc, dtype):
     """Rows of 1..32 whole vectors: 2..64 rows per wave (every power-of-two group size, vector counts on and
     off the powers of two, row counts that leave the last wave partly empty), all options, both state ends."""

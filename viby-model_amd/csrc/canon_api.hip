@@ -170,6 +170,7 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     plan->wpb = 4;
     plan->grid = 0;
     plan->kind = FWD_GENERIC;
+    plan->name = "generic";
     if (empty) return CANON_OK;
 
     const int E = 16 / elem_bytes(p->x_dtype);
@@ -200,20 +201,23 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
                         (uint64_t)(kBlcRows + 3) * (uint64_t)a.x_sl * elem_bytes(p->x_dtype) + 64 * kBlcVecBytes < (1ull << 31) &&
                         (uint64_t)(kBlcRows + 3) * (uint64_t)a.o_sl * elem_bytes(p->x_dtype) + 64 * kBlcVecBytes < (1ull << 31);
 
-    // Time-contiguous rows of at most 32 whole, aligned vectors share waves (canon_fwd_bcl_short_kernel):
-    // measured against one row per wave, the kernel below, 2.3x faster at 16 vectors per row, 1.3x at 32.
+    // Time-contiguous rows of at most 32 vectors share waves (canon_fwd_bcl_short_kernel): measured against one row
+    // per wave, the kernel below, 2.3x faster at 16 vectors per row, 1.3x at 32.
     // (Longer rows packed back to back the same way lose to the kernel below even where it leaves half of its
-    // lanes idle: 4.4-4.6 against 5.1-5.7 TB/s.)
-    const uint32_t kBclShortMaxVectors = 32;
-    if (!p->seq_idx && ptr_ok && a.x_sl == 1 && a.o_sl == 1 && bcl_aligned && a.L / E >= 1 &&
-        a.L / E <= kBclShortMaxVectors && rows < (1ull << 31)) {
-        const uint32_t nvec = a.L / E;
-        uint32_t shift = 0;
-        while ((1u << shift) < nvec) ++shift;                  // one group of lanes per row: the next power of two
-        const uint64_t groups_per_wave = 64u >> shift;
-        const uint64_t nwaves = (rows + groups_per_wave - 1) / groups_per_wave;
+    // lanes idle: 4.4-4.6 against 5.1-5.7 TB/s.)  Whole vectors on 16-byte boundaries, or from one vector on any
+    // length at the elements' own alignment (its ragged variant; below one vector, the strided kernel).
+    const bool elem_ok = (((uintptr_t)p->x | (uintptr_t)p->out) & (elem_bytes(p->x_dtype) - 1)) == 0;
+    const bool short_aligned = ptr_ok && bcl_aligned;
+    if (!p->seq_idx && a.x_sl == 1 && a.o_sl == 1 && (short_aligned || elem_ok) && a.L >= (uint32_t)E &&
+        (a.L + E - 1) / E <= kBclShortMaxVectors && rows < (1ull << 31)) {
+        const uint32_t nvec = (a.L + E - 1) / E;
+        // (the families keep their names: whole vectors, rows of at least sixteen, neither)
+        plan->name = short_aligned ? "bcl_vec_short" : bcl_ok ? "bcl_vec" : "generic";
+        plan->ragged = !short_aligned;
+        if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
+        const uint64_t nwaves = (rows + 64u / nvec - 1) / (64u / nvec);
         plan->kind = FWD_BCL_SHORT;
-        a.nvec = nvec; a.nseg = 1u << shift; a.chunk = shift; a.ntasks = (uint32_t)rows;
+        a.nvec = nvec; a.nseg = 64u / nvec; a.chunk = (65536u + nvec - 1) / nvec; a.ntasks = (uint32_t)rows;
         a.div_C = make_fastdiv(a.C);
         a.nblocks = (uint32_t)((nwaves + 3) / 4);
         plan->grid = a.nblocks;
@@ -239,6 +243,7 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         const uint64_t ntasks = rows * nseg;
         if (ntasks < (1ull << 31)) {
             plan->kind = FWD_BCL;
+            plan->name = "bcl_vec";
             plan->U = U;
             plan->ragged = !bcl_aligned;
             if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
@@ -269,6 +274,7 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         const uint64_t nblocks = (ncols + 7) / 8 * 8 * group;
         if (nblocks < (1ull << 31) - 8) {
             plan->kind = FWD_BLC;
+            plan->name = p->seq_idx ? "blc_vec_seq" : "blc_vec";
             a.nvec = nvec; a.nct = nct; a.ntt = ntt; a.ntasks = (uint32_t)ncols;
             a.nseg = ngroups; a.chunk = group;
             a.div_nct = make_fastdiv(nct); a.div_ntt = make_fastdiv(ngroups); a.div_nseg = make_fastdiv(group);
@@ -650,8 +656,9 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     a.grad_dtype = p->grad_dtype;
     a.w_vec = p->width == 4 && p->w_stride_k == 1 && p->w_stride_c == 4 && aligned16(p->weight);
     plan->kind = BWD_GENERIC;
+    plan->name = "bwd_generic";
     plan->U = 1;
-    plan->ragged = plan->walk_too = false;
+    plan->ragged = plan->short_rows = plan->walk_too = false;
     plan->grid = 0;
     plan->workspace_bytes = 0;
     if (empty) return CANON_OK;   // the caller's dweight/dbias are zero filled by canon_conv1d_bwd
@@ -680,9 +687,30 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
                       a.x_sb >= 0 && a.x_sc >= 0 && a.g_sb >= 0 && a.g_sc >= 0 &&
                       (uint64_t)(a.x_sb / unit) < (1ull << 32) && (uint64_t)(a.x_sc / unit) < (1ull << 32) &&
                       (uint64_t)(a.g_sb / unit) < (1ull << 32) && (uint64_t)(a.g_sc / unit) < (1ull << 32);
+    const uint64_t nrows = (uint64_t)a.B * a.C;
+    // rows of at most 32 vectors, down to one: several to a wave (canon_bwd_bcl_short_kernel), at any alignment
+    if (rows_any && a.L >= (uint32_t)E && (a.L + E - 1) / E <= kBclShortMaxVectors &&
+        (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0 &&
+        a.x_sb >= 0 && a.x_sc >= 0 && a.g_sb >= 0 && a.g_sc >= 0 &&      // (32-bit leading scalars, as below)
+        std::max({a.x_sb, a.x_sc, a.g_sb, a.g_sc}) < (1ll << 32)) {
+        const uint32_t nvec = (a.L + E - 1) / E;
+        const uint64_t waves = (nrows + 64u / nvec - 1) / (64u / nvec);
+        plan->kind = BWD_BCL_VEC;
+        plan->name = rows_aligned ? "bwd_bcl_vec" : rows ? "bwd_bcl_vec_ragged" : "bwd_generic";   // (the families keep their names)
+        plan->short_rows = true;
+        a.m_vec = p->mask && p->mask_stride_l == 1;
+        a.nvec = nvec; a.chunk = (65536u + nvec - 1) / nvec; a.nthreads = (uint32_t)nrows;
+        a.nchunk = 1; a.nsets = a.B;
+        a.div_nvec = make_fastdiv(a.C);
+        plan->grid = (uint32_t)((waves + 3) / 4);
+        plan->workspace_bytes = (int64_t)a.nsets * a.C * 5 * (int64_t)sizeof(float);
+        if (check_pointers && (!p->workspace || !aligned16(p->workspace) || p->workspace_bytes < plan->workspace_bytes))
+            return fail(CANON_ERR_INVALID_ARGUMENT, "workspace must be 16-byte aligned and at least %lld bytes (got %lld)",
+                        (long long)plan->workspace_bytes, (long long)p->workspace_bytes);
+        return CANON_OK;
+    }
     if (rows) {
         const uint32_t nvec = (a.L + E - 1) / E;
-        const uint64_t nrows = (uint64_t)a.B * a.C;
         // vectors per lane: the fewest that reach the smallest number of segments per row (see plan_fwd)
         int U = 1;
         uint64_t best = (nvec + 63u) / 64u;
@@ -699,6 +727,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
             plan->ragged = plan->walk_too = !rows_aligned;
             if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
             plan->kind = BWD_BCL_VEC;
+            plan->name = plan->ragged ? "bwd_bcl_vec_ragged" : "bwd_bcl_vec";
             plan->U = U;
             // field use in this kernel family: nthreads = wave tasks, nchunk = segments per row
             a.nvec = nvec; a.nchunk = (uint32_t)nseg; a.nthreads = (uint32_t)ntasks;
@@ -742,6 +771,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         const uint64_t blocks = (uint64_t)a.B * ch.n * nct;
         if (blocks < (1ull << 31)) {
             plan->kind = BWD_BLC_VEC;
+            plan->name = packed ? "bwd_blc_vec_seq" : "bwd_blc_vec";
             plan->walk_too = packed;
             a.nvec = nvec; a.nct = nct; a.chunk = ch.len; a.nchunk = ch.n;
             a.nsets = a.B * ch.n;
@@ -754,6 +784,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         }
     }
     plan->kind = BWD_GENERIC;
+    plan->name = "bwd_generic";
     a.nvec = a.C;
     // time steps per lane: about 8 waves per CU, a multiple of the look-ahead, and few enough
     // partial sets that the scratch stays below ~16 MB
@@ -1087,18 +1118,14 @@ CANON_API const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p)
     BwdPlan pl;
     const int rc = p && p->workspace ? plan_bwd_in(p, &pl, p->workspace_bytes) : plan_bwd(p, &pl, false);
     if (rc != CANON_OK) return nullptr;
-    if (pl.kind == BWD_BLC_VEC) return pl.args.seq ? "bwd_blc_vec_seq" : "bwd_blc_vec";
-    if (pl.kind == BWD_BCL_VEC) return pl.ragged ? "bwd_bcl_vec_ragged" : "bwd_bcl_vec";
-    return "bwd_generic";
+    return pl.name;
 }
 
 CANON_API const char *canon_conv1d_fwd_plan(const canon_conv1d_fwd_params *p)
 {
     FwdPlan pl;
     if (plan_fwd(p, &pl) != CANON_OK) return nullptr;
-    if (pl.kind == FWD_BLC && pl.args.seq) return "blc_vec_seq";
-    if (pl.kind == FWD_BCL_SHORT) return "bcl_vec_short";
-    return pl.kind == FWD_BCL ? "bcl_vec" : pl.kind == FWD_BLC ? "blc_vec" : "generic";
+    return pl.name;
 }
 
 CANON_API int canon_conv1d_fwd_plan_waves(const canon_conv1d_fwd_params *p)

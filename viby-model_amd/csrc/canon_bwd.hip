@@ -1151,6 +1151,172 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
     }
 }
 
+// Rows of at most 32 vectors, of any length from one vector on and any alignment: as in the forward kernel a row takes
+// as many adjacent lanes of a wave as it has vectors, and a wave as many whole rows as fit.
+// The three inputs before a lane's vector come from the lane before, the three dz after it from the lane behind, zero at
+// the row's ends; a row's sums are added over its lanes in a fixed order and are its partial set entry.
+// Leading scalars as in the kernel above (strides in elements); `packed`: vectors per row | gap << 6 | s1, s2 of the
+// division by C << 9 | (2^16 / vectors per row, rounded up) << 15 (lane / vectors is a multiply and a shift).
+//
+// What bounds it is bandwidth once the lanes are full, and the launch.  Such rows took a wave each, most of whose lanes
+// then hold nothing, or below 40 steps the walk kernel.  us per call with the reduction, bf16: B 31, C 2848, L 82 with a
+// mask 54.4 -> 25.7; B 32, C 3456: L 13 (SiLU, mask) 14.6 -> 11.0, L 39 (SiLU) 48.8 -> 14.6, L 64 47.6 -> 14.8, L 128
+// 41.0 -> 23.2, L 129 53.3 -> 31.5 (45.5 with rows in the next power of two of lanes), L 255 57 -> 44, L 256 43.5 -> 40.6
+// (27.4 at the plain copy's rate); a launch of a few rows (B 3, C 96, L 209, SiLU, mask) is one wave's life, which is
+// 0.7 us longer with two rows in it.
+template <int DT, int W, bool MASK>
+__global__ __launch_bounds__(256) void canon_bwd_bcl_short_kernel(const char *x_base, const char *g_base, uint32_t x_sb32,
+                                                                  uint32_t x_sc32, uint32_t g_sb32, uint32_t g_sc32,
+                                                                  uint32_t nrows, uint32_t C, uint32_t divC_m, uint32_t packed,
+                                                                  const BwdArgs a)
+{
+    constexpr int E = Elem<DT>::per_vec;
+    constexpr int BY = Elem<DT>::bytes;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
+    const uint32_t nvec = packed & 63u, m = packed >> 15;
+    const uint32_t rows = (64u * m) >> 16;                       // rows per wave
+    const uint32_t first_row = wave * rows;
+    if (first_row >= nrows) return;
+    const uint32_t wrow = (lane * m) >> 16;                      // row of the wave
+    const uint32_t row = first_row + wrow;
+    const bool active = wrow < rows && row < nrows;
+    const uint32_t v = active ? lane - wrow * nvec : nvec - 1u;  // vector of the row; idle lanes shadow the end of
+    const uint32_t rr = active ? row : first_row;                // the wave's first row: loads need no predicate
+    const uint32_t gap = (packed >> 6) & 7u;                     // by how much the last vector's access moves back
+    const uint32_t inside = E - gap;                             // its steps before the row's end
+    const bool last = v == nvec - 1u;
+    const uint32_t first = v * E - (last ? gap : 0u);            // first element of the lane's access
+    const uint32_t b = fdiv(rr, FastDiv{C, divC_m, (packed >> 9) & 1u, (packed >> 10) & 31u});
+    const uint32_t c = rr - b * C;
+    const char *xrow = x_base + ((int64_t)b * x_sb32 + (int64_t)c * x_sc32) * BY;
+    const char *grow = g_base + ((int64_t)b * g_sb32 + (int64_t)c * g_sc32) * BY;
+    char *drow = a.dx + ((int64_t)b * a.d_sb + (int64_t)c * a.d_sc) * BY;
+
+    uint4 X = load_vec_any<kBwdStream>(xrow + (int64_t)first * BY);
+    uint4 G = load_vec_any<kBwdStream>(grow + (int64_t)first * BY);
+    RawTaps<1> raw;
+    fetch_taps<W, 1>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c, raw);
+    float M[1][E];
+    if constexpr (MASK) {
+        const int64_t mbase[1] = {(int64_t)b * a.m_sb + (int64_t)first * a.m_sl};
+        load_mask_vec<E, 1>(a.mask, mbase, a.m_sl, a.mask_dtype, a.m_vec != 0, M);
+    }
+    float w[1][W], bvv[1];
+    decode_taps<DT, W, 1>(raw, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bvv);
+    const float bv = bvv[0];
+    if (gap != 0) {
+        X = shift_down<DT>(X, last ? gap : 0u);
+        G = shift_down<DT>(G, last ? gap : 0u);
+        if constexpr (MASK) {
+#pragma unroll
+            for (uint32_t n = 1; n < (uint32_t)E; n *= 2) {
+                if (gap & n) {
+#pragma unroll
+                    for (int j = 0; j < E; ++j) M[0][j] = last ? (j + (int)n < E ? M[0][j + (int)n < E ? j + n : 0] : 0.0f) : M[0][j];
+                }
+            }
+        }
+    }
+
+    float xr[E], g[E], xm_store[MASK ? E : 1];
+    float *xm = MASK ? xm_store : xr;
+    unpack_vec<DT>(X, xr);
+    unpack_vec<DT>(G, g);
+    if constexpr (MASK) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) xm[j] = mul_round<DT>(xr[j], M[0][j]);
+    }
+    float seq[E + 3];
+    seq[0] = wave_shift_up(xm[E - 3], 0.0f);
+    seq[1] = wave_shift_up(xm[E - 2], 0.0f);
+    seq[2] = wave_shift_up(xm[E - 1], 0.0f);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) seq[j] = v == 0 ? 0.0f : seq[j];
+#pragma unroll
+    for (int j = 0; j < E; ++j) seq[3 + j] = xm[j];
+
+    float dz[E + 3];
+#pragma unroll
+    for (int j = 0; j < E; ++j) dz[j] = g[j];
+    if (a.act) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) {
+            float z = bv;
+#pragma unroll
+            for (int k = 0; k < W; ++k) z = fmaf(w[0][k], seq[j + (4 - W) + k], z);
+            dz[j] = g[j] * silu_grad(z);
+        }
+    }
+    // Steps past the row's end, the last vector's from `inside` on, have no dz, and no window (it reaches back over the
+    // row's last inputs, and 0 * Inf is NaN): their terms are summed apart and left out in the lanes that hold the end.
+    float dwl[W], past[W], dbl = 0.0f;
+#pragma unroll
+    for (int k = 0; k < W; ++k) dwl[k] = past[k] = 0.0f;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        if ((uint32_t)j < inside) {
+#pragma unroll
+            for (int k = 0; k < W; ++k) dwl[k] = fmaf(dz[j], seq[j + (4 - W) + k], dwl[k]);
+        } else {
+            dz[j] = last ? 0.0f : dz[j];
+#pragma unroll
+            for (int k = 0; k < W; ++k) past[k] = fmaf(dz[j], seq[j + (4 - W) + k], past[k]);
+        }
+        dbl += dz[j];
+    }
+    // dz of the three steps after the vector: the next lane's first, none behind the row's last vector
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const float next = wave_shift_down(dz[j], 0.0f);
+        dz[E + j] = last ? 0.0f : next;
+    }
+    float o[E];
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        float acc = w[0][W - 1] * dz[j];
+#pragma unroll
+        for (int k = W - 2; k >= 0; --k) acc = fmaf(w[0][k], dz[j + (W - 1) - k], acc);
+        o[j] = acc;
+    }
+    if (a.res_mode == CANON_RESIDUAL_MASKED) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) o[j] += g[j];
+    }
+    if constexpr (MASK) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) o[j] *= M[0][j];
+    }
+    if (a.res_mode == CANON_RESIDUAL_UNMASKED) {
+#pragma unroll
+        for (int j = 0; j < E; ++j) o[j] += g[j];
+    }
+    uint4 out = pack_vec<DT>(o);
+    if (gap != 0) out = row_end_vec<DT>(out, gap, last);
+    if (active) store_vec_any<kBwdStream>(drow + (int64_t)first * BY, out);
+
+    float tot[5];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) tot[k] = k < W && active ? dwl[k < W ? k : 0] + (last ? 0.0f : past[k < W ? k : 0]) : 0.0f;
+    tot[4] = active ? dbl : 0.0f;
+    // after step n a lane holds the sum of the 2^n lanes from it on, as far as they are of its row
+#pragma unroll
+    for (uint32_t off = 1; off <= 16; off <<= 1) {
+        if (nvec > off) {
+#pragma unroll
+            for (int k = 0; k < 5; ++k) {
+                const float behind = __shfl_down(tot[k], off, 64);
+                tot[k] += v + off < nvec ? behind : 0.0f;
+            }
+        }
+    }
+    if (v == 0 && active) {
+        float *pp = a.partial + (int64_t)rr * 5;      // rows are numbered b * C + c
+#pragma unroll
+        for (int k = 0; k < 5; ++k) pp[k] = tot[k];
+    }
+}
+
 // dweight[c, k] / dbias[c] = sum over the partial sets, in a fixed order: a block owns 32 adjacent
 // (c, j) columns; its 8 slices each sum every 8th set in set order (fp64), then the slices are added
 // in slice order.  Reads are 128 contiguous bytes per set and slice.
@@ -1484,7 +1650,12 @@ template <int DT, int W, bool MASK> void launch_bwd_m(const BwdPlan &pl, hipStre
 {
     const dim3 g(pl.grid), b(256);
     if (pl.kind == BWD_BCL_VEC) {
-        if (pl.ragged) launch_bwd_bcl<DT, W, MASK, true>(pl, s);
+        const BwdArgs &A = pl.args;
+        if (pl.short_rows)
+            hipLaunchKernelGGL((canon_bwd_bcl_short_kernel<DT, W, MASK>), g, b, 0, s, A.x, A.dy, (uint32_t)A.x_sb, (uint32_t)A.x_sc,
+                               (uint32_t)A.g_sb, (uint32_t)A.g_sc, A.nthreads, A.C, A.div_nvec.m,
+                               A.nvec | (A.nvec * Elem<DT>::per_vec - A.L) << 6 | A.div_nvec.s1 << 9 | A.div_nvec.s2 << 10 | A.chunk << 15, A);
+        else if (pl.ragged) launch_bwd_bcl<DT, W, MASK, true>(pl, s);
         else launch_bwd_bcl<DT, W, MASK, false>(pl, s);
     } else if (pl.kind == BWD_BLC_VEC)
     {

@@ -222,6 +222,32 @@ template <int E> __device__ __forceinline__ void shift_down(float *m, uint32_t g
 #pragma unroll
     for (int j = 0; j < E; ++j) m[j] = gap >= (uint32_t)E ? 0.0f : m[j];
 }
+// The same undone for a whole row that lies in one wave (a vector per lane, `last` the lane that holds its end, `gap` the
+// same for every lane): the E elements that end the row, from the last lane's vector and the one before it, so that the
+// row's end leaves in one store as well (its first `gap` elements are the ones the lane before stores too).
+template <int DT> __device__ __forceinline__ uint4 row_end_vec(const uint4 &v, uint32_t gap, bool last)
+{
+    constexpr uint32_t E = Elem<DT>::per_vec, PW = 4 / Elem<DT>::bytes;
+    uint32_t w[8] = {v.x, v.y, v.z, v.w, v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        w[i] = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w[i], 0x138 /* wave_shr:1 */, 0xF, 0xF, false);
+    const uint32_t n = E - gap;   // (gap is 1 .. E - 1 here)
+    if (n & (2 * PW)) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) w[i] = w[i + 2];
+    }
+    if (n & PW) {
+#pragma unroll
+        for (int i = 0; i < 5; ++i) w[i] = w[i + 1];
+    }
+    if (PW == 2 && (n & 1u)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = __builtin_amdgcn_alignbit(w[i + 1], w[i], 16);
+    }
+    return last ? make_uint4(w[0], w[1], w[2], w[3]) : v;
+}
+
 // ... and the store: the row's last vector element by element
 template <int DT, bool NT> __device__ __forceinline__ void store_row_vec(char *row, uint32_t first, uint32_t L, const float *o)
 {

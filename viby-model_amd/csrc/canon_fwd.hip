@@ -31,10 +31,9 @@ namespace canon {
 // unmasked path is ~130 VALU instructions per 2 KB row and hides under the
 // memory time.
 // ---------------------------------------------------------------------------
-// Activation, residual and store of one 16-byte vector of accumulators.
-template <int DT, bool MASK, bool EAGER, bool RAGGED = false>
-__device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const float *xr, const float *xm, char *dst, bool write,
-                                               uint32_t first = 0, uint32_t L = 0)
+// Activation and residual of one vector of accumulators, ...
+template <int DT, bool MASK, bool EAGER>
+__device__ __forceinline__ void bcl_finish_values(const FwdArgs &a, float *o, const float *xr, const float *xm)
 {
     constexpr int E = Elem<DT>::per_vec;
     activate<DT, E>(o, a.act != 0, EAGER);
@@ -45,6 +44,14 @@ __device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const
 #pragma unroll
         for (int j = 0; j < E; ++j) o[j] += xm[j];
     }
+}
+
+// ... and the store of it.
+template <int DT, bool MASK, bool EAGER, bool RAGGED = false>
+__device__ __forceinline__ void bcl_finish_vec(const FwdArgs &a, float *o, const float *xr, const float *xm, char *dst, bool write,
+                                               uint32_t first = 0, uint32_t L = 0)
+{
+    bcl_finish_values<DT, MASK, EAGER>(a, o, xr, xm);
     if constexpr (RAGGED) store_row_vec<DT, true>(dst, first, L, o);   // (dst: the row)
     else if (write) store_vec<true>(dst, pack_vec<DT>(o));
 }
@@ -225,41 +232,53 @@ __global__ __launch_bounds__(64 * kBclMaxWaves) void canon_fwd_bcl_kernel(const 
 }
 
 // ---------------------------------------------------------------------------
-// prefill, time-contiguous rows of at most 32 vectors (whole vectors, 16-byte
-// aligned): a row takes P = 1, 2, 4, .. 32 adjacent lanes of a wave (the next
-// power of two from its vector count) and a wave 64 / P rows, so short prompts
-// keep most lanes busy and every access is a 16-byte one.  A lane's history is
-// its left neighbour's last three inputs (wave shift) unless it holds the
-// first vector of its row; the rows of a wave belong to different channels, so
-// each lane loads its own taps.  Field use: nseg = P, chunk = log2(P),
-// ntasks = rows (B * C), nvec = vectors per row.
+// prefill, time-contiguous rows of at most 32 vectors: a row takes as many
+// adjacent lanes of a wave as it has vectors and a wave as many whole rows as
+// fit, so short prompts keep most lanes busy and every access is a 16-byte one.
+// A lane's history is its left neighbour's last three inputs (wave shift)
+// unless it holds the first vector of its row; the rows of a wave belong to
+// different channels, so each lane loads its own taps.  Field use: nvec =
+// vectors per row, nseg = rows per wave, chunk = 2^16 / nvec rounded up (lane /
+// nvec is a multiply and a shift), ntasks = rows (B * C).
+//
+// RAGGED: rows of any length from one vector on, at their elements' alignment.
+// The row's last vector is loaded from the row's last E elements and moved into
+// place (see row_gap; the same move in every row, so scalar branches choose
+// it), and stored from there as one vector too (row_end_vec).  Such rows took
+// the strided kernel, a thread per eight steps whose accesses are two bytes
+// each, or from 16 vectors on a wave per row (us, bf16): B 31, C 2848, L 82 with
+// a mask 34.7 -> 12.3; B 32, C 3456: L 9 7.9 -> 3.5, L 39 with SiLU 16.1 -> 7.0,
+// L 100 35.6 -> 11.1, L 255 43.2 -> 22.5 (18.2 at the plain copy's rate).  Rows
+// in the next power of two of lanes instead: L 129 (17 vectors, three rows to a
+// wave, not two) 19.2 -> 15.0.
 // ---------------------------------------------------------------------------
-template <int DT, int W, bool MASK>
+template <int DT, int W, bool MASK, bool RAGGED>
 __global__ __launch_bounds__(256) void canon_fwd_bcl_short_kernel(const FwdArgs a)
 {
     constexpr int E = Elem<DT>::per_vec;
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + (threadIdx.x >> 6));
-    const uint32_t shift = a.chunk, P = a.nseg;
-    const uint32_t first_row = wave * (64u >> shift);
+    const uint32_t first_row = wave * a.nseg;
     if (first_row >= a.ntasks) return;
-    const uint32_t sub = lane & (P - 1u);
-    const uint32_t row = first_row + (lane >> shift);
-    const bool row_ok = row < a.ntasks;
-    const uint32_t rr = row_ok ? row : a.ntasks - 1u;            // idle lanes shadow the last row / vector:
-    const uint32_t v = sub < a.nvec ? sub : a.nvec - 1u;         // loads need no predicate
-    const bool active = row_ok && sub < a.nvec;
+    const uint32_t wrow = (lane * a.chunk) >> 16;                // row of the wave
+    const uint32_t row = first_row + wrow;
+    const bool active = wrow < a.nseg && row < a.ntasks;
+    const uint32_t v = active ? lane - wrow * a.nvec : a.nvec - 1u;   // vector of the row; idle lanes shadow the end of
+    const uint32_t rr = active ? row : first_row;                     // the wave's first row: loads need no predicate
+    const uint32_t gap = RAGGED ? a.nvec * E - a.L : 0u;         // by how much the last vector's access moves back
+    const bool last = v == a.nvec - 1u;
+    const uint32_t first = v * E - (last ? gap : 0u);            // first element of the lane's access
     const uint32_t b = fdiv(rr, a.div_C);
     const uint32_t c = rr - b * a.C;
     const char *xrow = a.x + ((int64_t)b * a.x_sb + (int64_t)c * a.x_sc) * Elem<DT>::bytes;
     char *orow = a.out + ((int64_t)b * a.o_sb + (int64_t)c * a.o_sc) * Elem<DT>::bytes;
 
-    const uint4 X = load_vec<true>(xrow + (int64_t)v * 16);
+    uint4 X = RAGGED ? load_vec_any<true>(xrow + (int64_t)first * Elem<DT>::bytes) : load_vec<true>(xrow + (int64_t)v * 16);
     RawTaps<1> raw;
     fetch_taps<W, 1>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c, raw);
     float M[1][E];
     if constexpr (MASK) {
-        const int64_t mbase[1] = {(int64_t)b * a.m_sb + (int64_t)v * E * a.m_sl};
+        const int64_t mbase[1] = {(int64_t)b * a.m_sb + (int64_t)first * a.m_sl};
         load_mask_vec<E, 1>(a.mask, mbase, a.m_sl, a.mask_dtype, a.m_vec != 0, M);
     }
     float w[1][W], bvv[1];
@@ -273,12 +292,16 @@ __global__ __launch_bounds__(256) void canon_fwd_bcl_short_kernel(const FwdArgs 
 #pragma unroll
         for (int j = 0; j < E; ++j) xm[j] = mul_round<DT>(xr[j], M[0][j]);
     }
+    if (RAGGED && gap != 0) {
+        if constexpr (MASK) unpack_vec<DT>(shift_down<DT>(pack_vec<DT>(xm), last ? gap : 0u), xm);   // (exact: the products are rounded already)
+        unpack_vec<DT>(shift_down<DT>(X, last ? gap : 0u), xr);
+    }
     // seq[0..2] = the three masked inputs before this vector
     float seq[E + 3];
     seq[0] = wave_shift_up(xm[E - 3], 0.0f);
     seq[1] = wave_shift_up(xm[E - 2], 0.0f);
     seq[2] = wave_shift_up(xm[E - 1], 0.0f);
-    if (sub == 0) {
+    if (v == 0) {
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
             seq[j] = 0.0f;
@@ -297,11 +320,20 @@ __global__ __launch_bounds__(256) void canon_fwd_bcl_short_kernel(const FwdArgs 
         for (int k = 0; k < W; ++k) acc = fmaf(w[0][k], seq[j + (4 - W) + k], acc);
         o[j] = acc;
     }
-    if (a.eager) bcl_finish_vec<DT, MASK, true>(a, o, xr, xm, orow + (int64_t)v * 16, active);
-    else bcl_finish_vec<DT, MASK, false>(a, o, xr, xm, orow + (int64_t)v * 16, active);
+    if constexpr (RAGGED) {
+        if (a.eager) bcl_finish_values<DT, MASK, true>(a, o, xr, xm);
+        else bcl_finish_values<DT, MASK, false>(a, o, xr, xm);
+        uint4 out = pack_vec<DT>(o);
+        if (gap != 0) out = row_end_vec<DT>(out, gap, last);
+        if (active) store_vec_any<true>(orow + (int64_t)first * Elem<DT>::bytes, out);
+    } else if (a.eager) {
+        bcl_finish_vec<DT, MASK, true>(a, o, xr, xm, orow + (int64_t)v * 16, active);
+    } else {
+        bcl_finish_vec<DT, MASK, false>(a, o, xr, xm, orow + (int64_t)v * 16, active);
+    }
 
-    if (a.fin && row_ok)
-        for (uint32_t slot = sub; slot < (uint32_t)a.S_out; slot += P) capture_row_state<DT>(a, b, c, (int)slot);
+    if (a.fin && active)
+        for (uint32_t slot = v; slot < (uint32_t)a.S_out; slot += a.nvec) capture_row_state<DT>(a, b, c, (int)slot);
 }
 
 // ---------------------------------------------------------------------------
@@ -1074,7 +1106,10 @@ template <int DT, int W, bool MASK, bool BIG> void launch_bcl(const FwdPlan &pl,
 
 template <int DT, int W, bool MASK, bool BIG> void launch_fwd_vec(const FwdPlan &pl, hipStream_t s)
 {
-    if (pl.kind == FWD_BCL_SHORT) hipLaunchKernelGGL((canon_fwd_bcl_short_kernel<DT, W, MASK>), dim3(pl.grid), dim3(256), 0, s, pl.args);
+    if (pl.kind == FWD_BCL_SHORT) {
+        if (pl.ragged) hipLaunchKernelGGL((canon_fwd_bcl_short_kernel<DT, W, MASK, true>), dim3(pl.grid), dim3(256), 0, s, pl.args);
+        else hipLaunchKernelGGL((canon_fwd_bcl_short_kernel<DT, W, MASK, false>), dim3(pl.grid), dim3(256), 0, s, pl.args);
+    }
     else if (pl.kind == FWD_BCL) launch_bcl<DT, W, MASK, BIG>(pl, s);
     else {
         const FwdArgs &a = pl.args;

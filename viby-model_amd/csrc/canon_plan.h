@@ -208,6 +208,8 @@ enum FwdKind { FWD_BCL, FWD_BCL_SHORT, FWD_BLC, FWD_GENERIC };
 constexpr int kBclMaxVectorsPerLane = CANON_BCL_MAX_U;   // most 16-byte vectors a lane of the time-contiguous kernel takes (1, 2 or 4)
 enum UpdKind { UPD_VEC, UPD_GENERIC };
 
+constexpr uint32_t kBclShortMaxVectors = 32;   // longest time-contiguous rows that share waves
+
 constexpr uint32_t kGenericChunk = 8;   // time steps per thread in the scalar kernel
 constexpr int kBlcRows = CANON_BLC_ROWS;   // time steps per wave in the channel-contiguous kernel
 // ... and in its unmasked width-4 launches that move at least kBlcShortSlabBytes (single tensor or pair): measured
@@ -240,6 +242,7 @@ constexpr uint32_t kBclBigLaunch = 16384;
 
 struct FwdPlan {
     FwdKind kind;
+    const char *name;   // what canon_conv1d_fwd_plan answers
     int U;
     bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
     uint32_t wpb; // bcl: waves per block
@@ -271,8 +274,10 @@ struct UpdPartsPlan {
 
 struct BwdPlan {
     BwdKind kind;
+    const char *name;   // what canon_conv1d_bwd_plan answers
     int U;
     bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
+    bool short_rows;   // bcl: several rows share a wave
     bool walk_too;   // a call that the walk kernel takes instead when the scratch is too small for this kernel's sets
     BwdArgs args;
     uint32_t grid;
