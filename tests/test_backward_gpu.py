@@ -554,6 +554,40 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_backward_of_channel_contiguous_rows_off_the_8_byte_grid(cc, dtype):
+    """Channel counts that are no multiple of 8 bytes, and slices of wider rows: from one lane's two channels on, around a
+    wave's 64 lanes, sequences around the slabs, the tiles and the chunks (and below the shortest the tiled kernel takes)."""
+    g = torch.Generator().manual_seed(31)
+    masks = [None, torch.int64, torch.bool, torch.bfloat16]
+    for n, (C, L) in enumerate([(2, 12), (3, 11), (3, 33), (7, 40), (127, 31), (129, 32), (129, 129), (1, 40), (257, 300), (130, 65), (961, 13), (64, 96)]):
+        B, off = (1, 3)[n % 2], (0, 1)[n % 3 == 2 or (C * dtype.itemsize) % 8 == 0]
+        act, res, mtype = (None, "silu")[n % 2], (False, "masked", "unmasked")[n % 3], masks[n % len(masks)]
+        x, dout = torch.randn(B, C, L, generator=g).to(dtype), torch.randn(B, C, L, generator=g).to(dtype)
+        w = (torch.randn(C, 4, generator=g) * 0.5).to(dtype if n % 5 else torch.float32)
+        b = (torch.randn(C, generator=g) * 0.2).to(w.dtype) if n % 4 else None
+        mask = None
+        if mtype is not None:
+            mask = right_padded_mask([max(1, L - 3 * i) for i in range(B)], L)
+            mask[:, L // 2] = 0
+            mask = mask.to(mtype)
+        wr, br = w.to(dtype), b.to(dtype) if b is not None else None          # (taps are rounded to x's type first)
+        rdx, rdw, rdb, _ = conv1d_grads(x, wr, br, dout, mask, act, res)
+        wide = torch.zeros(B, L, C + off, dtype=dtype, device=DEV)
+        xg = wide[..., off:].transpose(1, 2)
+        xg.copy_(x)
+        xg = xg.detach().requires_grad_()
+        wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
+        out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
+        dg = dout.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)
+        grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dg)
+        what = f"{dtype} {B}x{C}x{L} {act} {res} {mtype} offset {off}"
+        check(grads[0], rdx, dtype, what + " dx")
+        check(grads[1], rdw, w.dtype, what + " dweight", sum_terms=B * L)
+        if b is not None:
+            check(grads[2], rdb, w.dtype, what + " dbias", sum_terms=B * L)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_short_rows_of_any_length_and_alignment(cc, dtype):
     """Rows of 1..32 vectors share waves: every distance of the row's end from a vector's, vector counts that fill a
     wave's lanes and that leave some idle, a last wave that is not full, rows in a buffer of longer rows, every mask

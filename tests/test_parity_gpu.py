@@ -731,6 +731,44 @@ def test_long_unmasked_time_contiguous_rows_of_several_segments(cc, dtype, shape
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_channel_contiguous_rows_off_the_8_byte_grid(cc, dtype):
+    """Channel counts that are no multiple of 8 bytes, and slices of wider rows: from one lane's channels on, around a
+    wave's 64 lanes, sequences around the slabs of eight steps and the tiles of four, every mask type, states (the eight
+    slots that leave together and others), widths, both rounding modes."""
+    g = torch.Generator().manual_seed(29)
+    E = 8 // dtype.itemsize
+    masks = [None, torch.int64, torch.bool, torch.float32, torch.int32, torch.bfloat16, torch.float16]
+    channels = [E, E + 1, 2 * E - 1, 64 * E - 1, 64 * E, 64 * E + 1, 129 * E + 1, 2 * E]
+    lengths = [2, 3, 8, 9, 31, 33, 77, 257]
+    for n, (C, L) in enumerate([(c, l) for i, c in enumerate(channels) for l in lengths[i % 2::2]]):
+        B, W, off = (1, 3)[n % 2], 4 - n % 3, (0, 1, 3)[n % 3]
+        if off == 0 and C % E == 0:
+            off = 1
+        act, res, mtype = (None, "silu")[n % 4 == 3], (False, "masked", "unmasked")[n % 3], masks[n % len(masks)]
+        S_out = (8, 5)[n % 2]
+        x = torch.randn(B, C, L, generator=g).to(dtype)
+        w = (torch.randn(C, W, generator=g) * 0.3).to(dtype if n % 5 else torch.float32)
+        b = (torch.randn(C, generator=g) * 0.1).to(w.dtype) if n % 4 else None
+        init = torch.randn(B, C, 5, generator=g).to(dtype) if n % 3 == 0 else None
+        mask = None
+        if mtype is not None:
+            mask = right_padded_mask([max(1, L - 3 * i) for i in range(B)], L)
+            mask[:, L // 2] = 0
+        wide = torch.zeros(B, L, C + off, dtype=dtype, device=DEV)
+        xg = wide[..., off:].transpose(1, 2)
+        xg.copy_(x)
+        for rounding in ("fused", "eager"):
+            want, want_fs = co.conv1d_fwd(x, w, b, mask=mask, activation=act, residual=res, initial_state=init, final_state_len=S_out,
+                                          round_mode=int(rounding == "eager"))
+            got, fs = run_fwd(cc, xg, w, b, act=act, mask=None if mask is None else mask.to(mtype), residual=res, init=init, S_out=S_out,
+                              rounding=rounding)
+            what = f"{dtype} {B}x{C}x{L} W{W} {act} {res} {mtype} offset {off} {rounding}"
+            xm = x if mask is None else (x.float() * mask[:, None, :].float()).to(dtype)
+            assert_parity(got, want, exact=act is None, what=what, res=(x if res == "unmasked" else xm) if res else None)
+            assert torch.equal(bits(fs), bits(want_fs)), what
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
 def test_short_rows_of_any_length_and_alignment(cc, dtype):
     """Rows of 1..32 vectors that are no whole number of vectors, or off the 16-byte grid: every distance of the row's
     end from a vector's, vector counts that fill a wave's lanes and that leave some idle, a last wave that is not full,

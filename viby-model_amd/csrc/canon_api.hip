@@ -258,9 +258,12 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
             return CANON_OK;
         }
     }
-    if (blc_ok) {
-        const uint32_t nvec = a.C / EB;
+    // ... or off the 8-byte grid, from one lane's channels on: the same tiles with accesses at the elements' own alignment
+    const bool blc_any = !blc_ok && !p->seq_idx && elem_ok && a.x_sc == 1 && a.o_sc == 1 && a.x_sl != 1 && a.C >= EB && a.C < (1u << 29);
+    if (blc_ok || blc_any) {
+        const uint32_t nvec = (a.C + EB - 1) / EB;
         const uint32_t nct = (nvec + 64 * kBlcWC - 1) / (64 * kBlcWC);          // channel tiles per row
+        if (blc_any) blc_rows = kBlcRows;
         if (blc_rows == 0) blc_rows = blc_rows_for(p, 2ull * rows * a.L * elem_bytes(p->x_dtype));
         plan->rows = blc_rows;
         const uint32_t ntt = (a.L + kBlcWaves * blc_rows - 1) / (kBlcWaves * blc_rows);   // time tiles per sequence
@@ -273,8 +276,8 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         const uint64_t ncols = (uint64_t)a.B * ngroups * nct;
         const uint64_t nblocks = (ncols + 7) / 8 * 8 * group;
         if (nblocks < (1ull << 31) - 8) {
-            plan->kind = FWD_BLC;
-            plan->name = p->seq_idx ? "blc_vec_seq" : "blc_vec";
+            plan->kind = blc_any ? FWD_BLC_ANY : FWD_BLC;
+            plan->name = blc_any ? "generic" : p->seq_idx ? "blc_vec_seq" : "blc_vec";   // (the family keeps its name)
             a.nvec = nvec; a.nct = nct; a.ntt = ntt; a.ntasks = (uint32_t)ncols;
             a.nseg = ngroups; a.chunk = group;
             a.div_nct = make_fastdiv(nct); a.div_ntt = make_fastdiv(ngroups); a.div_nseg = make_fastdiv(group);
@@ -658,7 +661,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     plan->kind = BWD_GENERIC;
     plan->name = "bwd_generic";
     plan->U = 1;
-    plan->ragged = plan->short_rows = plan->walk_too = false;
+    plan->ragged = plan->short_rows = plan->any = plan->walk_too = false;
     plan->grid = 0;
     plan->workspace_bytes = 0;
     if (empty) return CANON_OK;   // the caller's dweight/dbias are zero filled by canon_conv1d_bwd
@@ -751,8 +754,12 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
                      // step of x or dout is a stride of zero)
                      a.x_sl >= 0 && a.g_sl >= 0 && a.d_sl > 0 &&
                      (uint64_t)(kBwdSlab + 3) * (uint64_t)std::max({a.x_sl, a.g_sl, a.d_sl}) * elem_bytes(p->x_dtype) + 1024 < (1ull << 31);
-    if (vec) {
-        const uint32_t nvec = a.C / kBwdLaneChannels;
+    // ... or off that grid: the same tiles at the elements' own alignment (neither packed nor with states, width 4)
+    const bool any = !vec && !force_generic && a.x_sc == 1 && a.g_sc == 1 && a.d_sc == 1 && a.x_sl != 1 && p->width == 4 && !packed && !states &&
+                     a.C >= (uint32_t)kBwdLaneChannels && a.C < (1u << 29) && a.L >= kBwdAnyMinSteps &&
+                     (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0;
+    if (vec || any) {
+        const uint32_t nvec = (a.C + kBwdLaneChannels - 1) / kBwdLaneChannels;
         const uint32_t nct = (nvec + 63) / 64;
         const int64_t set_bytes = (int64_t)a.C * 5 * (int64_t)sizeof(float);
         // Chunks of kBwdChunk steps, shorter where the grid would not have one and a half blocks per CU.  A scratch with
@@ -771,8 +778,9 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         const uint64_t blocks = (uint64_t)a.B * ch.n * nct;
         if (blocks < (1ull << 31)) {
             plan->kind = BWD_BLC_VEC;
-            plan->name = packed ? "bwd_blc_vec_seq" : "bwd_blc_vec";
-            plan->walk_too = packed;
+            plan->name = any ? "bwd_generic" : packed ? "bwd_blc_vec_seq" : "bwd_blc_vec";   // (the family keeps its name)
+            plan->any = any;
+            plan->walk_too = packed || any;
             a.nvec = nvec; a.nct = nct; a.chunk = ch.len; a.nchunk = ch.n;
             a.nsets = a.B * ch.n;
             a.div_nct = make_fastdiv(nct); a.div_nchunk = make_fastdiv(ch.n);

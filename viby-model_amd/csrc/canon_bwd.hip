@@ -385,12 +385,13 @@ __device__ __forceinline__ void bwd_dz_gated(const float (*w)[W], const float *b
 // (slot t - fin_first for t >= fin_first = L - S_out) and get that slot's gradient, read at `fin` (the lane's
 // first channel of slot 0) where it is needed: at most S_out steps per sequence.
 // SEQ: rows of several packed sequences in reach; q[j] is the sequence index of slab row j - 3 (rows -3 .. R+2).
-template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E, bool SEQ = false>
+// ANY: dx is written through the lane's own pointer `any` (nullptr: a lane without channels), rows a.d_sl apart.
+template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E, bool SEQ = false, bool ANY = false>
 __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W], const float *bias, const BwdVec<DT> *X,
                                           const BwdVec<DT> *H, const BwdVec<DT> *G, const uint32_t *mm, const float (*dzh)[E],
                                           float (*dzf)[E], float (*dw)[W], float *dbs, __amdgpu_buffer_rsrc_t rd, uint32_t voff,
                                           uint32_t ds, int rows, const char *fin = nullptr, int64_t fin_first_row = 0,
-                                          const int32_t *q = nullptr)
+                                          const int32_t *q = nullptr, char *any = nullptr)
 {
     float xw[4][E];   // xm of rows r-3 .. r
 #pragma unroll
@@ -474,7 +475,11 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 #pragma unroll
             for (int e = 0; e < E; ++e) o[e] += g[e];
         }
-        if (FULL || r < rows) BufIO<kBwdLaneChannels * Elem<DT>::bytes>::template store<kAuxStream>(pack_lane<DT>(o), rd, voff, (uint32_t)r * ds);
+        if constexpr (ANY) {
+            if ((FULL || r < rows) && any) store_any<kBwdLaneChannels * Elem<DT>::bytes>(any + r * a.d_sl * Elem<DT>::bytes, pack_lane<DT>(o));
+        } else if (FULL || r < rows) {
+            BufIO<kBwdLaneChannels * Elem<DT>::bytes>::template store<kAuxStream>(pack_lane<DT>(o), rd, voff, (uint32_t)r * ds);
+        }
         // row by row: interleaved, the eight rows of a slab hold ten more registers and gain nothing
         __builtin_amdgcn_sched_barrier(0);
         if (r > 0) {
@@ -499,10 +504,17 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 // of rows packed from documents of hundreds of tokens, takes the ordinary sweep after one ballot; only a slab with a
 // boundary in reach takes the sweep that gates each tap.  The walk kernel, which gates every row and reads two bytes
 // per lane, took 192 us at B 2, C 3456, L 8192, bf16, SiLU, this one 74 (profiled; the whole training call 233 us with it, 118 now).
-template <int DT, int W, bool MASK, bool ACT, bool STATES, bool SEQ = false>
+//
+// ANY: a channel count, a row pitch or an address off the 8-byte grid.  A lane's channels are independent of every other
+// lane's: each takes its two at their elements' alignment through a pointer of its own, the last of an odd count the row's
+// last two (the first of which the lane before computes as well, to the same bits).  Such calls took the walk kernel, us
+// with the reduction, bf16: B 8, C 961, L 1021 29.6 -> 20.9, with SiLU and a mask 41.9 -> 23.2; B 24, C 1695, L 170 with both
+// 33.5 -> 22.0; B 8, C 3455, L 1024 79.1 -> 61.5 (on the grid 36.6: a misaligned four-byte access touches two words).
+template <int DT, int W, bool MASK, bool ACT, bool STATES, bool SEQ = false, bool ANY = false>
 __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 {
     static_assert(!(STATES && SEQ), "seq_idx excludes states");
+    static_assert(!ANY || !(STATES || SEQ), "neither packed nor with states");
     constexpr int BY = Elem<DT>::bytes;
     constexpr int E = kBwdLaneChannels, VB = E * BY;
     constexpr int R = kBwdSlab, NW = kBwdWaves;
@@ -541,7 +553,8 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t cv = ct * 64u + lane;
     const bool active = cv < a.nvec;
-    const uint32_t c0 = (active ? cv : a.nvec - 1u) * E;   // idle lanes shadow the last group: loads need no predicate
+    // idle lanes shadow the last group: loads need no predicate
+    const uint32_t c0 = ANY ? (cv < a.nvec - 1u ? cv * E : a.C - E) : (active ? cv : a.nvec - 1u) * E;
 
     // The wave's rows are reached through buffer resources, one per tensor and tile: the lane is a 32-bit vector offset,
     // the row a scalar one.  (As 64-bit pointers per lane the nineteen row addresses of a tile alone held 38 registers.)
@@ -561,8 +574,13 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     const int ntiles = (int)(a.chunk / (uint32_t)(R * NW));
 
     RawTaps<E> rawt;
-    fetch_taps<W, E>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c0, rawt);
+    fetch_taps<W, E, ANY>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c0, rawt);
     float w[E][W], bias[E];
+    // a row of x or dout at this lane's channels
+    auto load_row = [](const char *p) {
+        if constexpr (ANY) return load_any<VB, false>(p);
+        else return BwdIO<DT>::template load<false>(p);
+    };
     if constexpr (MASK || SEQ) {
         for (uint32_t i = threadIdx.x; i < a.chunk + 6u; i += 64u * NW) {
             int64_t t = t_chunk - 3 + (int64_t)i;
@@ -591,7 +609,7 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
         if (wv == NW - 1) {
 #pragma unroll
             for (int j = 0; j < 3; ++j)
-                if (te + j <= Lm1) GE[j] = BwdIO<DT>::template load<false>(gb + (te + j) * gs);
+                if (te + j <= Lm1) GE[j] = load_row(gb + (te + j) * gs);
         }
         decode_taps<DT, W, E>(rawt, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
 #pragma unroll
@@ -611,12 +629,12 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 #pragma unroll
             for (int j = 0; j < 6; ++j) {
                 const int64_t t = te - 3 + j;
-                XE[j] = BwdIO<DT>::template load<false>(xb + (t < Lm1 ? t : Lm1) * xs);
+                XE[j] = load_row(xb + (t < Lm1 ? t : Lm1) * xs);
             }
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 const int64_t t = te + j;
-                GE[j] = BwdIO<DT>::template load<false>(gb + (t < Lm1 ? t : Lm1) * gs);
+                GE[j] = load_row(gb + (t < Lm1 ? t : Lm1) * gs);
             }
             if constexpr (MASK) {
 #pragma unroll
@@ -674,14 +692,23 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             const uint32_t rr = r < rows ? (uint32_t)r : (rows > 0 ? (uint32_t)(rows - 1) : 0u);
-            X[r] = IO::template load<kAuxStream>(rx, voff, (rr + 3u) * xs32);
-            G[r] = IO::template load<kAuxStream>(rg, voff, rr * gs32);
+            if constexpr (ANY) {
+                const int64_t t = rows > 0 ? t0 + rr : Lm1;      // (a slab without rows: the sequence's last row, never used)
+                X[r] = load_any<VB, true>(xb + t * xs);
+                G[r] = load_any<VB, true>(gb + t * gs);
+            } else {
+                X[r] = IO::template load<kAuxStream>(rx, voff, (rr + 3u) * xs32);
+                G[r] = IO::template load<kAuxStream>(rg, voff, rr * gs32);
+            }
         }
 #pragma unroll
         for (int j = 0; j < 3; ++j) H[j] = BwdIO<DT>::zero();
         if (wv == 0 && t0 > 0) {     // (t0 is a multiple of the tile: all three rows exist)
 #pragma unroll
-            for (int j = 0; j < 3; ++j) H[j] = IO::template load<kAuxPlain>(rx, voff, (uint32_t)j * xs32);
+            for (int j = 0; j < 3; ++j) {
+                if constexpr (ANY) H[j] = load_any<VB, false>(xb + ((t0 <= Lm1 ? t0 : Lm1 + 1) - 3 + j) * xs);
+                else H[j] = IO::template load<kAuxPlain>(rx, voff, (uint32_t)j * xs32);
+            }
         }
         uint32_t mm[R + 3];   // mask of steps t0-3 .. t0+R-1 (bits, in scalar registers: one LDS read, then lane by lane)
 #pragma unroll
@@ -820,10 +847,15 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
             for (int j = 0; j < R + 6; ++j) q[j] = __builtin_amdgcn_readlane(q_lane, j);
             bwd_sweep<DT, W, MASK, ACT, false, false, R, E, SEQ>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
                                                                  nullptr, 0, q);
-        } else if (rows == R)
-            bwd_sweep<DT, W, MASK, ACT, true, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows);
-        else
-            bwd_sweep<DT, W, MASK, ACT, false, false, R, E>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows);
+        } else {
+            char *dany = ANY && active ? a.dx + ((int64_t)b * a.d_sb + c0) * BY + t0 * ds : nullptr;
+            if (rows == R)
+                bwd_sweep<DT, W, MASK, ACT, true, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
+                                                                           nullptr, 0, nullptr, dany);
+            else
+                bwd_sweep<DT, W, MASK, ACT, false, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
+                                                                            nullptr, 0, nullptr, dany);
+        }
     }
 
     if (STATES && a.dinit && ch == 0 && wv == 0 && active) {
@@ -1660,6 +1692,13 @@ template <int DT, int W, bool MASK> void launch_bwd_m(const BwdPlan &pl, hipStre
     } else if (pl.kind == BWD_BLC_VEC)
     {
         const bool states = pl.args.init != nullptr || pl.args.dfin != nullptr;
+        if constexpr (W == 4) {
+            if (pl.any) {
+                if (pl.args.act) hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, true, false, false, true>), g, b, 0, s, pl.args);
+                else hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, false, false, false, true>), g, b, 0, s, pl.args);
+                return;
+            }
+        }
         if (pl.args.seq) {
             if (pl.args.act) hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, true, false, true>), g, b, 0, s, pl.args);
             else hipLaunchKernelGGL((canon_bwd_blc_kernel<DT, W, MASK, false, false, true>), g, b, 0, s, pl.args);

@@ -461,6 +461,33 @@ template <> struct VecIO<4> {
     }
 };
 
+// A lane's piece of a row at any address an element may have: 4, 8 or 16 bytes
+template <int VB, bool NT> __device__ __forceinline__ typename VecIO<VB>::type load_any(const void *p)
+{
+    if constexpr (VB == 16) {
+        return load_vec_any<NT>(p);
+    } else if constexpr (VB == 8) {
+        u32x2_any_t v;
+        if constexpr (NT) v = __builtin_nontemporal_load((const u32x2_any_t *)p);
+        else v = *(const u32x2_any_t *)p;
+        return make_uint2(v.x, v.y);
+    } else {
+        if constexpr (NT) return __builtin_nontemporal_load((const u32_any_t *)p);
+        else return *(const u32_any_t *)p;
+    }
+}
+template <int VB> __device__ __forceinline__ void store_any(void *p, const typename VecIO<VB>::type &v)   // (streamed)
+{
+    if constexpr (VB == 16) {
+        store_vec_any<true>(p, v);
+    } else if constexpr (VB == 8) {
+        const u32x2_any_t q = {v.x, v.y};
+        __builtin_nontemporal_store(q, (u32x2_any_t *)p);
+    } else {
+        __builtin_nontemporal_store(v, (u32_any_t *)p);
+    }
+}
+
 // Buffer accesses: address = resource base + vector offset + scalar offset, the sum checked against the
 // resource's size (measured on this hardware: the scalar offset counts; an access beyond the size loads zeros
 // and stores nothing).  A resource therefore spans every row its wave touches, and lanes that must not access
@@ -767,7 +794,8 @@ template <int NC> struct RawTaps {
     uint32_t b[NC];
 };
 
-template <int W, int NC>
+// (ANY: c0 may be any channel, otherwise a multiple of NC)
+template <int W, int NC, bool ANY = false>
 __device__ __forceinline__ void fetch_taps(const void *weight, const void *bias, int64_t w_sc, int64_t w_sk,
                                            int w_dtype, bool vec, uint32_t c0, RawTaps<NC> &r)
 {
@@ -794,7 +822,7 @@ __device__ __forceinline__ void fetch_taps(const void *weight, const void *bias,
             const uint4 *p = (const uint4 *)((const uint2 *)weight + c0);   // c0 is a multiple of NC
 #pragma unroll
             for (int e = 0; e < NC; e += 2) {
-                const uint4 q = p[e / 2];
+                const uint4 q = ANY ? load_vec_any<false>(p + e / 2) : p[e / 2];
                 r.w[e][0] = q.x; r.w[e][1] = q.y;
                 r.w[e + 1][0] = q.z; r.w[e + 1][1] = q.w;
             }

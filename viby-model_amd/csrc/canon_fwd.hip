@@ -523,7 +523,8 @@ __device__ __forceinline__ void blc_request(const BlcLead &h, const BlcWave<VB> 
 // two-byte store per channel behind each, the end of the launch came eight memory round trips later: B 1, C 640, L 77
 // 5.9 -> 4.0 us, masked B 8, C 640, L 1024 10.0 -> 7.2, q / k / v at B 16, L 1024 17.1 -> 14.6.  One channel after the
 // other, in raw bits: with everything unpacked at once the kernel needed 171 registers, not 81.
-template <int DT, bool MASK, int VB>
+// ANY: the wave's lanes lie at any channel (`g` then holds no buffer offsets).
+template <int DT, bool MASK, int VB, bool ANY = false>
 __device__ __forceinline__ void blc_capture(const FwdArgs &a, const BlcLead &h, const BlcWave<VB> &g, const uint32_t cshift)
 {
     constexpr int E = VB / Elem<DT>::bytes, BY = Elem<DT>::bytes, N = 8;
@@ -535,7 +536,10 @@ __device__ __forceinline__ void blc_capture(const FwdArgs &a, const BlcLead &h, 
         const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void *)xw, 0, (int)((N - 1) * g.xs + g.nl * VB), kBufFlags);
         typename V::type row[N];
 #pragma unroll
-        for (int j = 0; j < N; ++j) row[j] = BufIO<VB>::template load<kAuxPlain>(r, g.voff, (uint32_t)j * g.xs);
+        for (int j = 0; j < N; ++j) {
+            if constexpr (ANY) row[j] = load_any<VB, false>(h.x + ((int64_t)g.b * h.x_sb + g.c0) * BY + (first + j) * a.x_sl * BY);
+            else row[j] = BufIO<VB>::template load<kAuxPlain>(r, g.voff, (uint32_t)j * g.xs);
+        }
         if constexpr (MASK) {
             float m[N];
             load_mask_rows_wave<N>(a.mask, (int64_t)g.b * a.m_sb, first, a.L, a.m_sl, a.mask_dtype, (int)g.lane, m);
@@ -572,7 +576,7 @@ __device__ __forceinline__ void blc_capture(const FwdArgs &a, const BlcLead &h, 
 #pragma unroll
         for (int e = 0; e < E; ++e) v[e] = 0.0f;
         if (t >= 0) {
-            V::template unpack<DT>(V::template load<false>(xb + t * (int64_t)g.xs), v);
+            V::template unpack<DT>(ANY ? load_any<VB, false>(xb + t * a.x_sl * BY) : V::template load<false>(xb + t * (int64_t)g.xs), v);
             if constexpr (MASK) {
                 const float mm = load_mask(a.mask, g.b * a.m_sb + t * a.m_sl, a.mask_dtype);
 #pragma unroll
@@ -917,6 +921,129 @@ __global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_seq_kernel(const Fw
     blc_block_linear<DT, W, R, MASK, false, true, kBlcVecBytes>(a, blockIdx.x);
 }
 
+// Channel-contiguous rows off the 8-byte grid: a channel count, a row pitch or an address that is no multiple of 8 bytes.
+// A lane's channels are independent of every other lane's, so all that changes against the kernel above is where they
+// lie: a lane takes E adjacent channels at their elements' alignment, the one that would pass the end of a row the row's last
+// E (some of which the lane before computes as well, to the same bits).  The waves share nothing: each reads its three
+// rows of history itself (hits in L2, the block order is that of the plain kernel) and its taps.
+// Such calls took the strided kernel, whose lanes read two bytes each (us, bf16): B 8, C 961, L 1021 23.5 -> 10.8, with
+// SiLU and a mask 27.3 -> 11.7; B 24, C 1695, L 170 masked with a captured state 27.9 -> 11.1; B 8, C 3455, L 1024
+// 72.3 -> 28.5 (C 3456, on the grid: 19.5; a misaligned 8-byte access touches three words).  Bound by bandwidth.
+template <int DT, int W, bool MASK, bool EAGER>
+__device__ __forceinline__ void blc_any_rows(const FwdArgs &a, const float (&w)[kBlcVecBytes / Elem<DT>::bytes][W],
+                                             const float (&bias)[kBlcVecBytes / Elem<DT>::bytes],
+                                             float (&hist)[3][kBlcVecBytes / Elem<DT>::bytes],
+                                             const typename VecIO<kBlcVecBytes>::type (&X)[kBlcRows], const float (&m)[kBlcRows + 3],
+                                             char *out, int rows)
+{
+    constexpr int VB = kBlcVecBytes, E = VB / Elem<DT>::bytes;
+    const int64_t os = a.o_sl * Elem<DT>::bytes;
+#pragma unroll
+    for (int r = 0; r < kBlcRows; ++r) {
+        if (r >= rows) break;      // wave uniform
+        float xr[E], xm[E], o[E];
+        VecIO<VB>::template unpack<DT>(X[r], xr);
+#pragma unroll
+        for (int e = 0; e < E; ++e) {
+            xm[e] = MASK ? mul_round<DT>(xr[e], m[3 + r]) : xr[e];
+            float acc = bias[e];
+            if constexpr (W == 4) acc = fmaf(w[e][0], hist[0][e], acc);
+            if constexpr (W >= 3) acc = fmaf(w[e][W - 3], hist[1][e], acc);
+            acc = fmaf(w[e][W - 2], hist[2][e], acc);
+            acc = fmaf(w[e][W - 1], xm[e], acc);
+            o[e] = acc;
+            hist[0][e] = hist[1][e];
+            hist[1][e] = hist[2][e];
+            hist[2][e] = xm[e];
+        }
+        activate<DT, E>(o, a.act != 0, EAGER);
+        if (a.res_mode == CANON_RESIDUAL_UNMASKED) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[e] += xr[e];
+        } else if (a.res_mode == CANON_RESIDUAL_MASKED) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) o[e] += xm[e];
+        }
+        if (out) store_any<VB>(out + r * os, VecIO<VB>::template pack<DT>(o));
+    }
+}
+
+template <int DT, int W, bool MASK>
+__global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_any_kernel(const FwdArgs a)
+{
+    constexpr int VB = kBlcVecBytes, BY = Elem<DT>::bytes, E = VB / BY, R = kBlcRows;
+    using V = VecIO<VB>;
+    // block -> tile as in the plain kernel
+    const uint32_t jq = blockIdx.x >> 3;
+    const uint32_t jg = fdiv(jq, a.div_nseg);
+    const uint32_t q = jg * 8u + (blockIdx.x & 7u);
+    if (q >= a.ntasks) return;
+    const uint32_t qr = fdiv(q, a.div_nct);
+    const uint32_t ct = q - qr * a.nct;
+    BlcWave<VB> g;
+    g.b = fdiv(qr, a.div_ntt);
+    const uint32_t tt = (qr - g.b * a.nseg) * a.chunk + (jq - jg * a.chunk);
+    g.lane = threadIdx.x & 63u;
+    g.wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    g.t0 = ((int64_t)tt * kBlcWaves + g.wv) * R;
+    if (g.t0 >= (int64_t)a.L) return;
+    g.rows = (int64_t)a.L - g.t0 < R ? (int)((int64_t)a.L - g.t0) : R;
+    const uint32_t cv = ct * 64u + g.lane;
+    g.active = cv < a.nvec;
+    g.c0 = cv < a.nvec - 1u ? cv * E : a.C - E;    // the row's last E channels for the last group (idle lanes shadow it)
+
+    const char *xb = a.x + ((int64_t)g.b * a.x_sb + g.t0 * a.x_sl) * BY;     // the slab's first row
+    const int64_t xs = a.x_sl * BY;
+    const uint32_t voff = g.c0 * BY;
+    typename V::type X[R], H[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        H[j] = V::zero();
+        if (j >= 3 - (W - 1) && g.t0 > 0) H[j] = load_any<VB, false>(xb + (j - 3) * xs + voff);   // (t0 is a multiple of R > 3)
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        X[r] = load_any<VB, true>(xb + (r < g.rows ? r : g.rows - 1) * xs + voff);   // past the end: the last row again, never used
+    RawTaps<E> raw;
+    fetch_taps<W, E, true>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, g.c0, raw);
+    float m[R + 3];
+#pragma unroll
+    for (int j = 0; j < R + 3; ++j) m[j] = 1.0f;
+    if constexpr (MASK) load_mask_rows_wave<R + 3>(a.mask, (int64_t)g.b * a.m_sb, g.t0 - 3, a.L, a.m_sl, a.mask_dtype, (int)g.lane, m);
+
+    float hist[3][E];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        V::template unpack<DT>(H[j], hist[j]);
+        if constexpr (MASK) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) hist[j][e] = mul_round<DT>(hist[j][e], m[j]);
+        }
+    }
+    if (g.t0 == 0 && a.init) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            if (j < 3 - (W - 1)) continue;
+#pragma unroll
+            for (int e = 0; e < E; ++e)
+                hist[j][e] = load1<DT>(a.init, g.b * a.i_sb + (int64_t)(g.c0 + e) * a.i_sc + (int64_t)(a.S_in - 3 + j) * a.i_ss);
+        }
+    }
+    float w[E][W], bias[E];
+    decode_taps<DT, W, E>(raw, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
+    char *out = g.active ? a.out + ((int64_t)g.b * a.o_sb + g.t0 * a.o_sl + g.c0) * BY : nullptr;
+    if (a.eager) blc_any_rows<DT, W, MASK, true>(a, w, bias, hist, X, m, out, g.rows);
+    else blc_any_rows<DT, W, MASK, false>(a, w, bias, hist, X, m, out, g.rows);
+
+    if (a.fin && g.t0 + g.rows == (int64_t)a.L) {
+        const BlcLead h = {a.x, a.x_sb, 0u, a.L, a.nvec};
+        g.cv0 = 0;
+        g.nl = 0;
+        g.xs = 0;
+        blc_capture<DT, MASK, VB, true>(a, h, g, 0u);
+    }
+}
+
 // fb1..fb3: the first blocks of parts 1..3 once more as leading scalars, which arrive in registers with the wave:
 // the block knows its part at once and reads that part's arguments in one round instead of two.
 template <int DT, int W, int R, bool MASK, bool BIG>
@@ -1110,6 +1237,7 @@ template <int DT, int W, bool MASK, bool BIG> void launch_fwd_vec(const FwdPlan 
         if (pl.ragged) hipLaunchKernelGGL((canon_fwd_bcl_short_kernel<DT, W, MASK, true>), dim3(pl.grid), dim3(256), 0, s, pl.args);
         else hipLaunchKernelGGL((canon_fwd_bcl_short_kernel<DT, W, MASK, false>), dim3(pl.grid), dim3(256), 0, s, pl.args);
     }
+    else if (pl.kind == FWD_BLC_ANY) hipLaunchKernelGGL((canon_fwd_blc_any_kernel<DT, W, MASK>), dim3(pl.grid), dim3(kBlcThreads), 0, s, pl.args);
     else if (pl.kind == FWD_BCL) launch_bcl<DT, W, MASK, BIG>(pl, s);
     else {
         const FwdArgs &a = pl.args;

@@ -201,13 +201,16 @@ constexpr int kBwdLaneChannels = 2;         // adjacent channels per lane in the
 constexpr uint32_t kBwdChunk = CANON_BWD_CHUNK;   // most time steps a block of it walks while the scratch has room for the sets
 constexpr int kBwdWaves = 4;
 constexpr int kBwdMaxChunk = 32 * kBwdSlab * kBwdWaves;   // ... and at all
-enum FwdKind { FWD_BCL, FWD_BCL_SHORT, FWD_BLC, FWD_GENERIC };
+enum FwdKind { FWD_BCL, FWD_BCL_SHORT, FWD_BLC, FWD_BLC_ANY, FWD_GENERIC };
 #ifndef CANON_BCL_MAX_U
 #define CANON_BCL_MAX_U 4
 #endif
 constexpr int kBclMaxVectorsPerLane = CANON_BCL_MAX_U;   // most 16-byte vectors a lane of the time-contiguous kernel takes (1, 2 or 4)
 enum UpdKind { UPD_VEC, UPD_GENERIC };
 
+// shortest sequences of channel-contiguous rows off the 8-byte grid that the tiled backward takes; us against the walk
+// kernel: B 32 C 961 L 4 6.7 / 6.0, L 8 7.0 / 6.7, L 14 7.2 / 8.5; C 3455 L 10 10.8 / 10.0; B 2 C 67 L 5 6.4 / 5.8, L 14 6.4 / 7.4
+constexpr uint32_t kBwdAnyMinSteps = 12;
 constexpr uint32_t kBclShortMaxVectors = 32;   // longest time-contiguous rows that share waves
 
 constexpr uint32_t kGenericChunk = 8;   // time steps per thread in the scalar kernel
@@ -278,6 +281,7 @@ struct BwdPlan {
     int U;
     bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
     bool short_rows;   // bcl: several rows share a wave
+    bool any;    // blc: channels, row pitches or addresses off the 8-byte grid
     bool walk_too;   // a call that the walk kernel takes instead when the scratch is too small for this kernel's sets
     BwdArgs args;
     uint32_t grid;
