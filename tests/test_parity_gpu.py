@@ -607,6 +607,25 @@ def test_seq_idx_matches_oracle_and_separate_calls(cc, dtype):
                 assert torch.equal(bits(packed[bi:bi + 1, :, lo:hi]), bits(alone)), (bi, lo, hi)
 
 
+@pytest.mark.parametrize("dtype,L", [(torch.bfloat16, 3041), (torch.float32, 1519), (torch.bfloat16, 4861)])
+def test_seq_idx_in_large_launches(cc, dtype, L):
+    """Packed rows from 40 MB of traffic on (slabs of four steps) and from 64 MB on (written-through stores): boundaries
+    at every step of a slab, slabs within one sequence, a sequence's last slab that is not full; with a mask, eight steps."""
+    g = torch.Generator().manual_seed(73)
+    C = 3456
+    x = torch.randn(1, C, L, generator=g).to(dtype)
+    w, b = (torch.randn(C, 4, generator=g) * 0.3).to(dtype), (torch.randn(C, generator=g) * 0.1).to(dtype)
+    seq = torch.cumsum((torch.rand(1, L, generator=g) < torch.linspace(0, 0.3, L)).int(), 1).int()
+    xg = x.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)
+    mask = right_padded_mask([L - 5], L)
+    for act, res, m in [(None, False, None), ("silu", "masked", None), (None, "masked", mask)]:
+        got = cc.causal_conv1d_fn(xg, w.to(DEV), b.to(DEV), seq_idx=seq.to(DEV), activation=act,
+                                  attention_mask=None if m is None else m.to(DEV), residual=res)
+        want = co.conv1d_fwd_seq(x, w, b, seq, mask=m, activation=act, residual=res)
+        xm = x if m is None else (x.float() * m[:, None, :].float()).to(dtype)
+        assert_parity(got, want, exact=act is None, what=f"{dtype} {L} {act} {res}", res=xm if res else None)
+
+
 def test_seq_idx_constant_is_no_seq_idx(cc):
     g = torch.Generator().manual_seed(72)
     x = torch.randn(8, 3456, 256, generator=g).bfloat16().to(DEV).transpose(1, 2).contiguous().transpose(1, 2)

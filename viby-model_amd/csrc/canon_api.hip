@@ -92,7 +92,7 @@ Extent extent_of(const void *base, int64_t B, int64_t C, int64_t L, int64_t sb, 
 // Time steps per wave of the channel-contiguous prefill for a problem that moves `bytes` (see kBlcRowsShort).
 static int blc_rows_for(const canon_conv1d_fwd_params *p, uint64_t bytes)
 {
-    return (!p->mask && !p->seq_idx && p->width == 4 && bytes >= kBlcShortSlabBytes) ? kBlcRowsShort : kBlcRows;
+    return (!p->mask && p->width == 4 && bytes >= kBlcShortSlabBytes) ? kBlcRowsShort : kBlcRows;
 }
 
 // blc_rows: time steps per wave of the channel-contiguous kernel; 0 = chosen here from the call's own size

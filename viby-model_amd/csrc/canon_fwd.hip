@@ -673,7 +673,7 @@ __device__ __forceinline__ void blc_block_body(const ARGS &args, const BlcLead &
     const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void *)ow, 0, (int)orec, kBufFlags);
 
     float m[R], mh[3];
-    int32_t sq[SEQ ? R + 3 : 1];   // sequence index of rows t0-3 .. t0+R-1
+    int32_t seq_lane = 0;          // SEQ: sequence index of row t0-3 + lane
     RawTaps<E> raw;
     TapWords<WDT, E> tw;
     const uint32_t g = wt * 64u + lane;                         // thread within the tile's group of waves
@@ -687,13 +687,11 @@ __device__ __forceinline__ void blc_block_body(const ARGS &args, const BlcLead &
 #pragma unroll
     for (int r = 0; r < R; ++r) m[r] = 0.0f;
 #pragma unroll
-    for (int j = 0; j < (SEQ ? R + 3 : 1); ++j) sq[j] = 0;
-#pragma unroll
     for (int j = 0; j < 3; ++j) mh[j] = 0.0f;
     if (rows > 0) {
         if constexpr (MODE == TAPS_ANY)
             fetch_taps<W, E>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c0, raw);
-        if constexpr (SEQ) load_seq_rows_wave<R + 3>(a.seq, (int64_t)b * a.q_sb, t0 - 3, a.L, a.q_sl, lane, sq);
+        if constexpr (SEQ) seq_lane = load_seq_lanes<R + 3>(a.seq, (int64_t)b * a.q_sb, t0 - 3, a.L, a.q_sl, lane);
         if constexpr (MASK) {
             // mask of the three rows before the slab and of the slab, last so that nothing is issued after its wait
             float mm[R + 3];
@@ -758,19 +756,21 @@ __device__ __forceinline__ void blc_block_body(const ARGS &args, const BlcLead &
     float w[E][W], bias[E];
     if constexpr (MODE == TAPS_ANY) decode_taps<DT, W, E>(raw, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
     else decode_taps_contiguous<DT, WDT, E>(tw, a.bias != nullptr, w, bias);
-    if constexpr (SEQ) {
+    // Packed sequences: a slab whose rows, the three before it included, carry one index (nearly every one: documents are
+    // hundreds of tokens long) is an ordinary slab; in the others rows t-3, t-2, t-1 count only if they carry row t's index.
+    if (!SEQ || __builtin_amdgcn_ballot_w64(seq_lane != __builtin_amdgcn_readfirstlane(seq_lane)) == 0) {
+        blc_rows_dispatch<DT, W, R, MASK, BIG, VB>(a, w, bias, hist, X, m, ro, voff, os, rows);
+    } else if constexpr (SEQ) {
+        int32_t sq[R + 3];
+#pragma unroll
+        for (int j = 0; j < R + 3; ++j) sq[j] = __builtin_amdgcn_readlane(seq_lane, j);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             if (r >= rows) continue;
-            // rows t-3, t-2, t-1 count only if they carry the index of row t; sequence boundaries are rare,
-            // so the all-kept case takes the plain code
             const int32_t cur = sq[3 + r];
-            const bool k0 = sq[r] == cur, k1 = sq[r + 1] == cur, k2 = sq[r + 2] == cur;
-            if (k0 && k1 && k2) blc_row_buf<DT, W, MASK, BIG, VB>(a, w, bias, hist, X[r], m[r], ro, voff, (uint32_t)r * os);
-            else blc_row_buf<DT, W, MASK, BIG, VB>(a, w, bias, hist, X[r], m[r], ro, voff, (uint32_t)r * os, k0, k1, k2);
+            blc_row_buf<DT, W, MASK, BIG, VB>(a, w, bias, hist, X[r], m[r], ro, voff, (uint32_t)r * os, sq[r] == cur, sq[r + 1] == cur,
+                                              sq[r + 2] == cur);
         }
-    } else {
-        blc_rows_dispatch<DT, W, R, MASK, BIG, VB>(a, w, bias, hist, X, m, ro, voff, os, rows);
     }
 
     if (a.fin && t0 + rows == (int64_t)a.L) blc_capture<DT, MASK, VB>(a, h, wave, cshift);
@@ -810,7 +810,7 @@ __device__ __forceinline__ void blc_block(const ARGS &a, const BlcLead &h, const
 // so the launch still sweeps memory in address order.
 //
 // ... with the blocks numbered in one dimension (block = (column group * chunk + tile of the group) * 8 + XCD)
-template <int DT, int W, int R, bool MASK, bool BIG, bool SEQ = false, int VB = kBlcVecBytes>
+template <int DT, int W, int R, bool MASK, bool BIG, int VB = kBlcVecBytes>
 __device__ __forceinline__ void blc_block_linear(const FwdArgs &a, const uint32_t blk)
 {
     const uint32_t jq = blk >> 3;
@@ -823,7 +823,7 @@ __device__ __forceinline__ void blc_block_linear(const FwdArgs &a, const uint32_
     const uint32_t tt = (qr - b * a.nseg) * a.chunk + (jq - jg * a.chunk);
     if (tt >= a.ntt) return;
     const BlcLead h = {a.x, a.x_sb, (uint32_t)(a.x_sl * Elem<DT>::bytes), a.L, a.nvec};
-    blc_block<DT, W, R, MASK, BIG, SEQ, VB>(ArgsHere{a}, h, (uint32_t)a.tap_mode, b, ct, tt);
+    blc_block<DT, W, R, MASK, BIG, false, VB>(ArgsHere{a}, h, (uint32_t)a.tap_mode, b, ct, tt);
 }
 
 // ... and the same in the plain kernel from leading scalar arguments: fourteen dwords, the most that arrive in
@@ -845,7 +845,11 @@ struct BlcSegment {
 };
 static_assert(offsetof(BlcSegment, a) == 14 * 4, "fourteen leading dwords, then the argument block");
 
-template <int DT, int W, int R, bool MASK, bool BIG>
+// SEQ: the same over packed variable-length sequences (seq_idx).  Such calls read their argument block first, gated every
+// row by itself and kept eight-step slabs in large launches; us, bf16: B 2, C 3456, L 8192 39.6 -> 36.4 (SiLU 40.5 -> 38.5,
+// with eight-step slabs 38.3; 36.5 at the plain copy's rate), L 2048 with SiLU 15.1 -> 13.3, B 2, C 2144, L 1718 9.7 -> 7.8,
+// fp32 L 4096 with SiLU 42.0 -> 35.8.
+template <int DT, int W, int R, bool MASK, bool BIG, bool SEQ = false>
 __global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_kernel(CANON_BLC_LEAD(CANON_LEAD_PARAM) const FwdArgs a)
 {
     const uint32_t lg = packed & 3u, nct = packed >> 16;
@@ -862,7 +866,7 @@ __global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_kernel(CANON_BLC_LE
 #ifdef CANON_NO_LATE_ARGS
     // build switch: the argument block read the ordinary way, at the top of the kernel (for a toolchain whose
     // kernel-argument segment is not laid out like BlcSegment: costs speed, not correctness)
-    blc_block<DT, W, R, MASK, BIG>(ArgsHere{a}, h, (packed >> 2) & 3u, b, ct, tt);
+    blc_block<DT, W, R, MASK, BIG, SEQ>(ArgsHere{a}, h, (packed >> 2) & 3u, b, ct, tt);
     return;
 #endif
     ArgsLate late;
@@ -870,7 +874,7 @@ __global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_kernel(CANON_BLC_LE
     late.weight = (const void *)((uint64_t)w_lo | (uint64_t)(wb_hi & 0xFFFFu) << 32);
     late.bias = (const void *)((uint64_t)b_lo | (uint64_t)(wb_hi >> 16) << 32);
     late.part = 0u;
-    blc_block<DT, W, R, MASK, BIG>(late, h, (packed >> 2) & 3u, b, ct, tt);
+    blc_block<DT, W, R, MASK, BIG, SEQ>(late, h, (packed >> 2) & 3u, b, ct, tt);
 }
 
 // Two tensors of the same shape, each dense ([B, L, C] with nothing between rows or sequences), in ONE launch of the
@@ -913,13 +917,6 @@ __global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_pair_kernel(CANON_B
     blc_block<DT, W, R, MASK, BIG>(late, h, (packed >> 2) & 3u, b, ct, tt);
 }
 #endif  // CANON_NO_LATE_ARGS
-
-// the same over packed variable-length sequences (seq_idx)
-template <int DT, int W, int R, bool MASK>
-__global__ __launch_bounds__(kBlcThreads) void canon_fwd_blc_seq_kernel(const FwdArgs a)
-{
-    blc_block_linear<DT, W, R, MASK, false, true, kBlcVecBytes>(a, blockIdx.x);
-}
 
 // Channel-contiguous rows off the 8-byte grid: a channel count, a row pitch or an address that is no multiple of 8 bytes.
 // A lane's channels are independent of every other lane's, so all that changes against the kernel above is where they
@@ -1246,19 +1243,21 @@ template <int DT, int W, bool MASK, bool BIG> void launch_fwd_vec(const FwdPlan 
         const uint32_t packed = lg | (uint32_t)a.tap_mode << 2 | a.div_nct.s1 << 4 | a.div_nct.s2 << 5 | a.div_ntt.s1 << 10 |
                                 a.div_ntt.s2 << 11 | a.nct << 16;
         const uint64_t wp = (uint64_t)(uintptr_t)a.weight, bp = (uint64_t)(uintptr_t)a.bias;
-#define CANON_BLC_LAUNCH(RR)                                                                                             \
-    hipLaunchKernelGGL((canon_fwd_blc_kernel<DT, W, RR, MASK, BIG>), dim3(pl.grid), dim3(kBlcThreads), 0, s, a.x,        \
+#define CANON_BLC_LAUNCH(RR, SEQ)                                                                                        \
+    hipLaunchKernelGGL((canon_fwd_blc_kernel<DT, W, RR, MASK, BIG, SEQ>), dim3(pl.grid), dim3(kBlcThreads), 0, s, a.x,        \
                        (uint32_t)(a.x_sb / (kBlcVecBytes / Elem<DT>::bytes)), (uint32_t)(a.x_sl * Elem<DT>::bytes), a.L, a.nvec, \
                        a.ntasks, a.div_nct.m, a.nseg, a.div_ntt.m, packed, (uint32_t)wp, (uint32_t)bp,                 \
                        (uint32_t)(wp >> 32) | (uint32_t)(bp >> 32) << 16, a)
         // (short slabs are planned for unmasked width-4 launches only)
         if constexpr (W == 4 && !MASK) {
             if (pl.rows == kBlcRowsShort) {
-                CANON_BLC_LAUNCH(kBlcRowsShort);
+                if (a.seq) CANON_BLC_LAUNCH(kBlcRowsShort, true);
+                else CANON_BLC_LAUNCH(kBlcRowsShort, false);
                 return;
             }
         }
-        CANON_BLC_LAUNCH(kBlcRows);
+        if (a.seq) CANON_BLC_LAUNCH(kBlcRows, true);
+        else CANON_BLC_LAUNCH(kBlcRows, false);
 #undef CANON_BLC_LAUNCH
     }
 }
@@ -1267,11 +1266,6 @@ template <int DT, int W, bool MASK, bool BIG> void launch_fwd_vec(const FwdPlan 
 template <int DT, int W> void launch_fwd_w(const FwdPlan &pl, hipStream_t s)
 {
     const bool mask = pl.args.mask != nullptr;
-    if (pl.args.seq) {   // only the channel-contiguous kernel is planned with seq_idx
-        if (mask) hipLaunchKernelGGL((canon_fwd_blc_seq_kernel<DT, W, kBlcRows, true>), dim3(pl.grid), dim3(kBlcThreads), 0, s, pl.args);
-        else hipLaunchKernelGGL((canon_fwd_blc_seq_kernel<DT, W, kBlcRows, false>), dim3(pl.grid), dim3(kBlcThreads), 0, s, pl.args);
-        return;
-    }
     // the variants for large launches (stores written through, see store_policy) exist for width 4 only
     if (W == 4 && pl.args.nt) {
         if (mask) launch_fwd_vec<DT, W, true, W == 4>(pl, s);

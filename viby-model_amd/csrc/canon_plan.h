@@ -216,7 +216,7 @@ constexpr uint32_t kBclShortMaxVectors = 32;   // longest time-contiguous rows t
 constexpr uint32_t kGenericChunk = 8;   // time steps per thread in the scalar kernel
 constexpr int kBlcRows = CANON_BLC_ROWS;   // time steps per wave in the channel-contiguous kernel
 // ... and in its unmasked width-4 launches that move at least kBlcShortSlabBytes (single tensor or pair): measured
-// 2-8 % faster there (B 8, C 3456, bf16: 19.9 -> 19.45 us, with SiLU 20.85 -> 19.86 us; B 16, C 640: 10.2 -> 9.4 us),
+// 2-8 % faster there, packed sequences included (B 8, C 3456, bf16: 19.9 -> 19.45 us, with SiLU 20.85 -> 19.86 us; B 16, C 640: 10.2 -> 9.4 us),
 // 5-16 % slower below that size (B 8, C 640 / 960: 5.3 -> 6.2 / 6.7 -> 7.8 us) and 0-4 % slower with a padding mask
 #ifndef CANON_BLC_ROWS_SHORT
 #define CANON_BLC_ROWS_SHORT 4
