@@ -199,3 +199,119 @@ def test_another_stream_and_a_captured_graph(cc):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(bits(out), bits(want)), i
+
+
+@pytest.mark.parametrize("layout", ["channel", "time"])
+def test_training_call(cc, monkeypatch, layout):
+    """The native autograd node against the Python one: gradients of every subset of the inputs, a gradient of the output in
+    another layout or expanded, a graph walked twice, saved-tensor hooks; and what is refused stays refused with the same
+    words (a saved input written to, a graph walked a second time, transforms, forward mode, double backward)."""
+    g = torch.Generator(device=DEV).manual_seed(4)
+    B, C, L = 2, 24, 70
+    x0 = torch.randn(B, L, C, device=DEV, generator=g).bfloat16()
+    x0 = x0.transpose(1, 2) if layout == "channel" else x0.transpose(1, 2).contiguous()
+    d0 = torch.randn(B, C, L, device=DEV, generator=g).bfloat16()
+    m = torch.ones(B, L, dtype=torch.int64, device=DEV)
+    m[1, 50:] = 0
+    seq = torch.arange(L, device=DEV, dtype=torch.int32).div(9, rounding_mode="floor").int().repeat(B, 1)
+    for wtype in (torch.bfloat16, torch.float32):
+        w0, b0 = torch.randn(C, 4, device=DEV, generator=g).to(wtype), torch.randn(C, device=DEV, generator=g).to(wtype)
+
+        def leaves(which=(1, 1, 1)):
+            return [t.detach().clone(memory_format=torch.preserve_format).requires_grad_(bool(r)) for t, r in zip((x0, w0, b0), which)]
+
+        for which in ((1, 1, 1), (1, 0, 0), (0, 1, 0), (0, 0, 1), (0, 1, 1)):
+            for options in (dict(), dict(attention_mask=m, activation="silu", residual=True), dict(seq_idx=seq, residual="unmasked")):
+                def grads(d=d0):
+                    t = leaves(which)
+                    y = cc.causal_conv1d_fn(*t, **options)
+                    return (y.detach(), *torch.autograd.grad(y, [v for v in t if v.requires_grad], d))
+                assert_same(*both(cc, monkeypatch, grads), (which, list(options)))
+        for d in (d0.transpose(1, 2).contiguous().transpose(1, 2), d0[:1, :1, :1].expand(B, C, L)):
+            assert_same(*both(cc, monkeypatch, lambda: grads(d)), "dout")
+
+        def twice():
+            x, w, b = leaves()
+            y = cc.causal_conv1d_fn(x, w, b, activation="silu")
+            first = torch.autograd.grad(y, (x, w, b), d0, retain_graph=True)
+            return first, torch.autograd.grad(y, (x, w, b), d0)
+        assert_same(*both(cc, monkeypatch, twice), "twice")
+
+        packed = []
+
+        def hooked():
+            packed.clear()
+            x, w, b = leaves()
+            with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(1) or t.cpu(), lambda t: t.to(DEV)):
+                y = cc.causal_conv1d_fn(x, w, b, attention_mask=m)
+            return torch.autograd.grad(y, (w, b), d0), len(packed)
+        (got, n), (want, n_want) = both(cc, monkeypatch, hooked)
+        assert_same(got, want, "hooks")
+        assert n == n_want == 4
+
+        def written():
+            x, w, b = leaves()
+            y = cc.causal_conv1d_fn(x, w, b)
+            with torch.no_grad():
+                w.add_(1)
+            return torch.autograd.grad(y, (x, w, b), d0)
+
+        def freed():
+            x, w, b = leaves()
+            y = cc.causal_conv1d_fn(x, w, b)
+            torch.autograd.grad(y, (x, w, b), d0)
+            return torch.autograd.grad(y, (x, w, b), d0)
+
+        def transform():
+            x, w, b = leaves((0, 0, 0))
+            return torch.func.grad(lambda v: cc.causal_conv1d_fn(v, w, b).float().sum())(x)
+
+        def mapped():
+            x, w, b = leaves((0, 1, 1))
+            return torch.func.vmap(lambda v: cc.causal_conv1d_fn(v, w, b))(torch.stack([x, x]))
+
+        def forward_mode():
+            x, w, b = leaves()
+            with torch.autograd.forward_ad.dual_level():
+                dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+                return cc.causal_conv1d_fn(dual, w, b).sum()
+
+        def second():
+            x, w, b = leaves()
+            y = cc.causal_conv1d_fn(x, w, b, activation="silu")
+            gx, = torch.autograd.grad(y, x, d0, create_graph=True)
+            return torch.autograd.grad(gx.float().sum(), x)
+        for call in (written, freed, transform, mapped, forward_mode, second):
+            got, want = both(cc, monkeypatch, call)
+            assert isinstance(got, str) and isinstance(want, str), (call.__name__, got, want)
+            assert got.split(":")[0] == want.split(":")[0], (call.__name__, got, want)
+
+
+def test_blocks_of_the_layer(cc, monkeypatch):
+    """CanonLayer's block call: one tensor and parts, with and without a cache, a continued state, masks, x that is not
+    dense; outputs, their strides and the cached states as through the functions."""
+    from causal_conv1d.canon import CanonLayer
+    g = torch.Generator(device=DEV).manual_seed(5)
+    for n, dtype in enumerate([torch.bfloat16, torch.float32, torch.float16]):
+        dims, B, T = ((16, 8, 8), (12, 12), (33,))[n], 3, 21
+        C = sum(dims)
+        config = types.SimpleNamespace(canon_kernel=4, canon_bias=n != 1, canon_activation=n == 0)
+        layer = CanonLayer(C, config, "b", rounding=("fused", "eager")[n == 2]).to(DEV, dtype).requires_grad_(False)
+        x = torch.randn(B, T, C, device=DEV, generator=g).to(dtype)
+        forms = [x, x.transpose(1, 2).contiguous().transpose(1, 2), torch.cat([x, x], -1)[..., 1:1 + C], x[:, :2]]
+        for xs in forms:
+            mask = torch.ones(B, xs.shape[1] + 5, dtype=torch.int64, device=DEV)
+            mask[1, -3:] = 0
+            for m in (None, mask, mask[:, 5:]):
+                def one():
+                    cache = types.SimpleNamespace(_max_layers=2)
+                    y = layer(xs, m), layer(xs, m, cache, 1), layer(xs, m, cache, 1)
+                    return y, cache.canon_cache_b[1]
+
+                def parts():
+                    cache = types.SimpleNamespace(_max_layers=2)
+                    p = xs.split(dims, -1)
+                    y = layer.forward_parts(p, m), layer.forward_parts(list(p), m, cache, 0), layer.forward_parts(p, m, cache, 0)
+                    return y, cache.canon_cache_b[0]
+                for call in (one, parts):
+                    assert_same(*both(cc, monkeypatch, call), (dtype, xs.stride(), call.__name__))

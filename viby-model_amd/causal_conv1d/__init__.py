@@ -270,7 +270,8 @@ def causal_conv1d_fn(
                      conv, after SiLU and after the residual add, which
                      reproduces the eager bf16/fp16 module bit for bit).
     """
-    # a plain call is checked and launched in one native step; None: anything else, errors included, from here on
+    # a plain call is checked and launched (and, with gradients, recorded) in one native step; None: anything else, errors
+    # included, from here on
     if not torch.compiler.is_compiling() and x.is_cuda and not (return_final_states and final_states_out is None):
         out = _lib.native().try_fwd(x, weight, bias, seq_idx, initial_states, final_states_out, activation,
                                     attention_mask, residual, rounding)
@@ -506,39 +507,26 @@ def causal_conv1d_update(
                 ``model/model.py:385-396``).
     """
     # A serving loop makes this call 72 times per generated token with the same shapes, strides, types and flags:
-    # such a call, once it has passed every check below, is recognised by that signature and launched from a
-    # prepared argument block with only the five addresses filled in.
-    if cache_seqlens is None and conv_state_indices is None and not (
-            torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad or conv_state.requires_grad
-                                         or (bias is not None and bias.requires_grad)
-                                         or (token_mask is not None and token_mask.requires_grad))):
-        key = (x.shape, x.stride(), x.dtype, x.device, conv_state.shape, conv_state.stride(), conv_state.dtype,
-               conv_state.device, weight.shape, weight.stride(), weight.dtype, weight.device,
-               None if bias is None else (bias.shape, bias.stride(), bias.dtype, bias.device),
-               None if token_mask is None else (token_mask.shape, token_mask.stride(), token_mask.dtype, token_mask.device),
-               activation, residual, rounding)
-        known = _known_updates()
-        p = known.get(key)
-        if p is not None and not torch.compiler.is_compiling():
-            out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-            p.x, p.out, p.conv_state, p.weight = x.data_ptr(), out.data_ptr(), conv_state.data_ptr(), weight.data_ptr()
-            if bias is not None:
-                p.bias = bias.data_ptr()
-            if token_mask is not None:
-                p.token_mask = token_mask.data_ptr()
-            rc = _call(_lib.lib().canon_conv1d_update, x.device, ctypes.byref(p))
-            if rc:
-                _lib.check(rc, "causal_conv1d_update")
-            return out
-    else:
-        key = None
-        if not torch.compiler.is_compiling() and x.is_cuda and (cache_seqlens is not None or conv_state_indices is not None):
-            out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices,
-                                                 token_mask, residual, rounding)
-            if out is not None:
+    # such a call, once it has passed every check below, is recognised by that signature (bytes that the native module
+    # forms) and launched from a prepared argument block with only the addresses filled in.
+    key = None
+    if cache_seqlens is None and conv_state_indices is None:
+        if not torch.compiler.is_compiling() and x.is_cuda:
+            out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, None, None, token_mask, residual,
+                                                 rounding, _known_updates())
+            if type(out) is bytes:
+                key = out
+            elif out is not None:
                 if type(out) is int:
                     _lib.check(out, "causal_conv1d_update")
                 return out
+    elif not torch.compiler.is_compiling() and x.is_cuda:
+        out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices,
+                                             token_mask, residual, rounding)
+        if out is not None:
+            if type(out) is int:
+                _lib.check(out, "causal_conv1d_update")
+            return out
     act = _activation_flag(activation)
     res = _residual_mode(residual)
     rnd = _round_mode(rounding)
@@ -600,7 +588,7 @@ def causal_conv1d_update(
         if (key is not None and not squeeze_back and out.numel()
                 and (bias is None or (bias.dtype == weight.dtype and bias.is_contiguous()))):
             # the call went through: remember its signature with an argument block whose sizes, strides and flags are set
-            _remember_update(key, _fill_update(x2, out, conv_state, weight, bias, token_mask, act, res, rnd))
+            _remember_update(key, bytes(_fill_update(x2, out, conv_state, weight, bias, token_mask, act, res, rnd)))
     return out.unsqueeze(-1) if squeeze_back else out
 
 
@@ -621,7 +609,7 @@ def _canon_decode_step(x: torch.Tensor, conv_state: torch.Tensor, taps: torch.Te
                                 residual="unmasked", rounding=rounding).unsqueeze(1)
 
 
-# signature of a checked decode call -> its prepared argument block; per thread, because the block is written to
+# signature of a checked decode call -> its argument block (bytes); per thread, so that a lookup needs no lock
 _KNOWN_UPDATES_MAX = 256
 _update_tls = threading.local()
 
@@ -634,7 +622,7 @@ def _known_updates() -> dict:
         return _update_tls.known
 
 
-def _remember_update(key, block) -> None:
+def _remember_update(key: bytes, block: bytes) -> None:
     """Keep at most _KNOWN_UPDATES_MAX signatures per thread: the oldest one makes room (a model has a handful of
     distinct decode calls; a program that keeps producing new ones must not lose the fast path for good)."""
     known = _known_updates()

@@ -12,10 +12,16 @@
 
 #include <ATen/ATen.h>
 #include <ATen/TensorSubclassLikeUtils.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPFunctions.h>
+#include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/version.h>
 
 #include "canon_conv1d.h"
@@ -23,9 +29,6 @@
 namespace {
 
 using at::Tensor;
-
-PyObject *g_raw_stream = nullptr;   // torch._C._cuda_getCurrentRawStream
-PyObject *g_get_device = nullptr;   // torch._C._cuda_getDevice
 
 int dtype_code(at::ScalarType t)
 {
@@ -94,28 +97,19 @@ int round_mode(PyObject *o)
 // The current stream of the tensor's device, which has to be the current device (false without an exception: it is not).
 bool stream_of(const Tensor &x, void **stream)
 {
-    const int dev = x.get_device();
-    PyObject *current = PyObject_CallNoArgs(g_get_device);
-    if (!current) throw python_error();
-    const long now = PyLong_AsLong(current);
-    Py_DECREF(current);
-    if (now != dev) return false;
-    PyObject *index = PyLong_FromLong(dev);
-    PyObject *raw = PyObject_CallOneArg(g_raw_stream, index);
-    Py_DECREF(index);
-    if (!raw) throw python_error();
-    *stream = PyLong_AsVoidPtr(raw);
-    Py_DECREF(raw);
+    const c10::DeviceIndex dev = (c10::DeviceIndex)x.get_device();
+    if (c10::hip::current_device() != dev) return false;
+    *stream = (void *)c10::hip::getCurrentHIPStream(dev).stream();
     return true;
 }
 
 template <typename F> int without_gil(F &&call)
 {
-    int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = call();
-    Py_END_ALLOW_THREADS
-    return rc;
+    struct Released {
+        PyThreadState *thread = PyEval_SaveThread();
+        ~Released() { PyEval_RestoreThread(thread); }   // (also when an allocation throws)
+    } released;
+    return call();
 }
 
 void *address(const Tensor *t) { return t ? t->data_ptr() : nullptr; }
@@ -215,6 +209,73 @@ bool fwd_args_ok(const Tensor &x, int64_t B, int64_t C, int64_t L, const Tensor 
     return true;
 }
 
+// The autograd node of a plain call (neither states nor anything a transform adds): forward and backward are one fused
+// launch each, nothing but the inputs is saved, and the backward runs in the engine's thread without the interpreter.
+// As a Python function, which the engine's thread has to take the interpreter's lock for, a training step that the host
+// bounds took 87-95 us (B 16, C 640, L 511, y.detach() and torch.autograd.grad included), with this node 65-67.
+int run_bwd(const Tensor &x, Tensor dout, const Tensor &weight, const Tensor *bias, const Tensor *mask, const Tensor &dweight,
+            const Tensor *dbias, int act, int res, const Tensor *seq, const Tensor *init, const Tensor *dinit, const Tensor *dfin,
+            void *stream, Tensor &dx);
+int run_fwd(const Tensor &x, const Tensor &weight, const Tensor *bias, const Tensor *mask, const Tensor *seq, int act, int res, int rnd,
+            void *stream, Tensor &out);
+
+[[noreturn]] void refuse(int rc, const char *what)
+{
+    const std::string message = std::string(what) + ": " + canon_conv1d_last_error();
+    if (rc == CANON_ERR_INVALID_ARGUMENT) C10_THROW_ERROR(ValueError, message);
+    if (rc == CANON_ERR_UNSUPPORTED) C10_THROW_ERROR(NotImplementedError, message);
+    C10_THROW_ERROR(Error, message);
+}
+
+struct CanonConv : torch::autograd::Function<CanonConv> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias,
+                          const std::optional<Tensor> &mask, const std::optional<Tensor> &seq, int64_t act, int64_t res, int64_t rnd,
+                          void *stream)
+    {
+        Tensor out;
+        const int rc = run_fwd(x, weight, bias ? &*bias : nullptr, mask ? &*mask : nullptr, seq ? &*seq : nullptr, (int)act, (int)res,
+                               (int)rnd, stream, out);
+        if (rc != CANON_OK) refuse(rc, "causal_conv1d_fn");
+        ctx->save_for_backward({x, weight, bias.value_or(Tensor()), mask.value_or(Tensor()), seq.value_or(Tensor())});
+        ctx->saved_data["flags"] = act | res << 1;
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, const torch::autograd::variable_list &grads)
+    {
+        const at::NoGradGuard no_grad;
+        const torch::autograd::variable_list saved = ctx->get_saved_variables();
+        const Tensor &x = saved[0], &weight = saved[1];
+        const auto given = [&](int i) { return saved[i].defined() ? &saved[i] : nullptr; };
+        const int64_t flags = ctx->saved_data["flags"].toInt();
+        Tensor dout = grads[0].defined() ? grads[0] : at::zeros_like(x);
+        if (dout.scalar_type() != x.scalar_type()) dout = dout.to(x.scalar_type());
+        const c10::DeviceGuard device(x.device());
+        const at::TensorOptions options = weight.options();
+        Tensor dx, dweight = at::empty(weight.sizes(), options), dbias;
+        if (given(2)) dbias = at::empty({weight.size(0)}, options);
+        const int rc = run_bwd(x, std::move(dout), weight, given(2), given(3), dweight, given(2) ? &dbias : nullptr, (int)(flags & 1),
+                               (int)(flags >> 1), given(4), nullptr, nullptr, nullptr,
+                               (void *)c10::hip::getCurrentHIPStream((c10::DeviceIndex)x.get_device()).stream(), dx);
+        if (rc != CANON_OK) refuse(rc, "causal_conv1d_fn backward");
+        return {dx, dweight, dbias, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    }
+};
+
+// Whether the node above sees all there is to see: no functorch level, no tracer, no forward-mode tangent (the Python
+// function's ways with those, errors included, are what callers know).
+bool plain_autograd(std::initializer_list<const Tensor *> inputs)
+{
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || torch::jit::tracer::isTracing())
+        return false;
+    for (const Tensor *t : inputs)
+        if (t && t->_fw_grad(0).defined()) return false;
+    return true;
+}
+
+std::optional<Tensor> optional_of(const Tensor *t) { return t ? std::optional<Tensor>(*t) : std::nullopt; }
+
 // What _narrow_mask does: a wide integer mask of a large call is converted, for this call, to x's type, unless the
 // channel-contiguous vector kernels take it (`kept` holds it until the launch is enqueued).
 constexpr int64_t kNarrowMinElements = 1 << 24;
@@ -243,14 +304,19 @@ PyObject *try_fwd(PyObject *, PyObject *const *args, Py_ssize_t n)
                       plain(args[4], &init) && plain(args[5], &fin) && plain(args[7], &mask) && x);
     const int act = activation_flag(args[6]), res = residual_mode(args[8]), rnd = round_mode(args[9]);
     CANON_NONE_UNLESS(act >= 0 && res >= 0 && rnd >= 0 && x->dim() == 3);
-    CANON_NONE_UNLESS(!c10::GradMode::is_enabled() || !(wants_grad(x) || wants_grad(weight) || wants_grad(bias) || wants_grad(init)));
+    const bool grad = c10::GradMode::is_enabled() && (wants_grad(x) || wants_grad(weight) || wants_grad(bias) || wants_grad(init));
+    CANON_NONE_UNLESS(!grad || (!init && !fin && plain_autograd({x, weight, bias})));
     CANON_NONE_UNLESS(fwd_args_ok(*x, x->size(0), x->size(1), x->size(2), weight, bias, mask, init, fin));
     CANON_NONE_UNLESS(!seq || (!init && !fin && seq->dim() == 2 && seq->size(0) == x->size(0) && seq->size(1) == x->size(2) &&
                                seq->scalar_type() == at::kInt && seq->device() == x->device()));
     void *stream;
     CANON_NONE_UNLESS(stream_of(*x, &stream));
-    Tensor out = at::empty_like(*x), narrowed;
+    Tensor narrowed;
     mask = narrow(mask, *x, x->numel(), narrowed);
+    if (grad)
+        return THPVariable_Wrap(CanonConv::apply(*x, *weight, optional_of(bias), optional_of(mask), optional_of(seq), (int64_t)act,
+                                                 (int64_t)res, (int64_t)rnd, stream));
+    Tensor out = at::empty_like(*x);
     const canon_conv1d_fwd_params p = fwd_params(*x, out, *weight, bias, mask, init, fin, seq, act, res, rnd);
     const int rc = without_gil([&] { return canon_conv1d_fwd(&p, stream); });
     if (rc != CANON_OK) return PyLong_FromLong(rc);
@@ -258,11 +324,85 @@ PyObject *try_fwd(PyObject *, PyObject *const *args, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// The block call of CanonLayer (inference), from the layer's own (batch, seqlen, dim) tensors, one or several parts, without
+// a view of any of them: try_fwd_parts(x | (x, ..), taps, bias, history, slots, activation, mask, residual, rounding, True)
+//   -> (output | outputs, new state of that many slots or None) | status code | None
+PyObject *layer_block(PyObject *const *args)
+{
+    PyObject *const one[1] = {args[0]};
+    const bool tuple = PyTuple_CheckExact(args[0]);
+    PyObject *const *items = tuple ? &PyTuple_GET_ITEM(args[0], 0) : one;
+    const Py_ssize_t np = tuple ? PyTuple_GET_SIZE(args[0]) : 1;
+    CANON_NONE_UNLESS(np >= 1 && np <= CANON_CONV1D_MAX_PARTS);
+    const Tensor *xs[CANON_CONV1D_MAX_PARTS], *weight, *bias, *init, *mask;
+    int64_t dim = 0;
+    bool grad = false;
+    for (Py_ssize_t i = 0; i < np; ++i) {
+        // (dense: the output then has x's strides, whichever way round its last two dimensions are named)
+        CANON_NONE_UNLESS(plain(items[i], &xs[i]) && xs[i] && xs[i]->dim() == 3 && xs[i]->is_non_overlapping_and_dense());
+        CANON_NONE_UNLESS(xs[i]->scalar_type() == xs[0]->scalar_type() && xs[i]->device() == xs[0]->device() &&
+                          xs[i]->size(0) == xs[0]->size(0) && xs[i]->size(1) == xs[0]->size(1));
+        dim += xs[i]->size(2);
+        grad |= xs[i]->requires_grad();
+    }
+    CANON_NONE_UNLESS(plain(args[1], &weight) && plain(args[2], &bias) && plain(args[3], &init) && plain(args[6], &mask));
+    const int act = activation_flag(args[5]), res = residual_mode(args[7]), rnd = round_mode(args[8]);
+    const long slots = PyLong_AsLong(args[4]);
+    CANON_NONE_UNLESS(act >= 0 && res >= 0 && rnd >= 0 && slots >= 0);
+    CANON_NONE_UNLESS(!c10::GradMode::is_enabled() || !(grad || wants_grad(weight) || wants_grad(bias) || wants_grad(init)));
+    const Tensor &x0 = *xs[0];
+    const int64_t B = x0.size(0), L = x0.size(1);
+    CANON_NONE_UNLESS(fwd_args_ok(x0, B, dim, L, weight, bias, mask, init, nullptr));
+    void *stream;
+    CANON_NONE_UNLESS(stream_of(x0, &stream));
+    const Tensor view = x0.transpose(1, 2);
+    Tensor narrowed, state, outs[CANON_CONV1D_MAX_PARTS];
+    mask = narrow(mask, view, B * dim * L, narrowed);
+    if (slots > 0) state = at::empty({B, dim, slots}, x0.options());
+    canon_conv1d_part parts[CANON_CONV1D_MAX_PARTS];
+    for (Py_ssize_t i = 0; i < np; ++i) {
+        outs[i] = at::empty_like(*xs[i]);
+        parts[i] = part_of(*xs[i], outs[i]);
+        std::swap(parts[i].x_stride_c, parts[i].x_stride_l);
+        std::swap(parts[i].out_stride_c, parts[i].out_stride_l);
+        parts[i].channels = xs[i]->size(2);
+    }
+    canon_conv1d_fwd_params p = fwd_params(view, outs[0], *weight, bias, mask, init, slots > 0 ? &state : nullptr, nullptr, act, res, rnd);
+    p.channels = dim;
+    if (np == 1) {
+        p.out_stride_c = parts[0].out_stride_c;
+        p.out_stride_l = parts[0].out_stride_l;
+    } else {
+        p.x = p.out = nullptr;
+    }
+    const int rc = without_gil([&] { return np == 1 ? canon_conv1d_fwd(&p, stream) : canon_conv1d_fwd_parts(&p, parts, (int32_t)np, stream); });
+    if (rc != CANON_OK) return PyLong_FromLong(rc);
+    PyObject *out;
+    if (tuple) {
+        out = PyTuple_New(np);
+        if (!out) return nullptr;
+        for (Py_ssize_t i = 0; i < np; ++i) PyTuple_SET_ITEM(out, i, THPVariable_Wrap(std::move(outs[i])));
+    } else {
+        out = THPVariable_Wrap(std::move(outs[0]));
+    }
+    PyObject *result = PyTuple_New(2);
+    if (!result) return nullptr;
+    PyTuple_SET_ITEM(result, 0, out);
+    if (slots > 0) {
+        PyTuple_SET_ITEM(result, 1, THPVariable_Wrap(std::move(state)));
+    } else {
+        Py_INCREF(Py_None);
+        PyTuple_SET_ITEM(result, 1, Py_None);
+    }
+    return result;
+}
+
 // try_fwd_parts((x, ..), weight, bias, initial_states, final_states, activation, attention_mask, residual, rounding)
 //   -> tuple of outputs | status code | None
 PyObject *try_fwd_parts(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
+    if (n == 10 && no_mode()) return layer_block(args);
     CANON_NONE_UNLESS(n == 9 && no_mode() && (PyTuple_CheckExact(args[0]) || PyList_CheckExact(args[0])));
     const Py_ssize_t np = PySequence_Fast_GET_SIZE(args[0]);
     CANON_NONE_UNLESS(np >= 1 && np <= CANON_CONV1D_MAX_PARTS);
@@ -304,11 +444,66 @@ PyObject *try_fwd_parts(PyObject *, PyObject *const *args, Py_ssize_t n)
     END_HANDLE_TH_ERRORS
 }
 
+// The plain decode step of a signature that has been through every check before (see causal_conv1d_update): `known` maps
+// signatures to argument blocks in which only the addresses are missing (with the signature a tuple of Python's sizes and
+// strides and the launch through ctypes, B 256, C 3456: 10.4 us a call, here 6.5).  try_update_modes(x, conv_state, weight, bias,
+// activation, None, None, token_mask, residual, rounding, known) -> output | status code | the signature, which the table
+// does not hold (nothing was done) | None
+PyObject *known_update(PyObject *const *args)
+{
+    const Tensor *x, *state, *weight, *bias, *mask;
+    CANON_NONE_UNLESS(plain(args[0], &x) && plain(args[1], &state) && plain(args[2], &weight) && plain(args[3], &bias) &&
+                      plain(args[7], &mask) && x && state && weight && PyDict_CheckExact(args[10]));
+    const int act = activation_flag(args[4]), res = residual_mode(args[8]), rnd = round_mode(args[9]);
+    CANON_NONE_UNLESS(act >= 0 && res >= 0 && rnd >= 0 && x->dim() == 2 && state->dim() == 3 && weight->dim() == 2 && x->is_cuda());
+    CANON_NONE_UNLESS(!c10::GradMode::is_enabled() ||
+                      !(wants_grad(x) || wants_grad(state) || wants_grad(weight) || wants_grad(bias) || wants_grad(mask)));
+    int64_t key[32] = {act | res << 4 | rnd << 8, x->get_device()};
+    int at = 2;
+    for (const Tensor *t : {x, state, weight, bias, mask}) {
+        if (!t) {
+            key[at++] = -1;
+            continue;
+        }
+        CANON_NONE_UNLESS(t->dim() <= 3 && t->device() == x->device());
+        key[at++] = (int64_t)t->scalar_type() | t->dim() << 8;
+        for (int64_t i = 0; i < t->dim(); ++i) {
+            key[at++] = t->size(i);
+            key[at++] = t->stride(i);
+        }
+    }
+    void *stream;
+    CANON_NONE_UNLESS(stream_of(*x, &stream));
+    PyObject *signature = PyBytes_FromStringAndSize((const char *)key, at * sizeof(key[0]));
+    if (!signature) return nullptr;
+    PyObject *block = PyDict_GetItemWithError(args[10], signature);   // (borrowed)
+    if (!block) {
+        if (!PyErr_Occurred()) return signature;
+        Py_DECREF(signature);
+        return nullptr;
+    }
+    Py_DECREF(signature);
+    CANON_NONE_UNLESS(PyBytes_CheckExact(block) && PyBytes_GET_SIZE(block) == sizeof(canon_conv1d_update_params));
+    canon_conv1d_update_params p;
+    memcpy(&p, PyBytes_AS_STRING(block), sizeof(p));
+    Tensor out = at::empty(x->sizes(), x->options());
+    p.x = x->data_ptr();
+    p.out = out.data_ptr();
+    p.conv_state = state->data_ptr();
+    p.weight = weight->data_ptr();
+    p.bias = address(bias);
+    p.token_mask = address(mask);
+    const int rc = without_gil([&] { return canon_conv1d_update(&p, stream); });
+    if (rc != CANON_OK) return PyLong_FromLong(rc);
+    return THPVariable_Wrap(std::move(out));
+}
+
 // try_update_modes(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices, token_mask, residual,
 //   rounding) -> output | status code | None: the decode step over a ring buffer or a state pool, x (batch, dim)
 PyObject *try_update_modes(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
+    if (n == 11 && no_mode()) return known_update(args);
     CANON_NONE_UNLESS(n == 10 && no_mode());
     const Tensor *x, *state, *weight, *bias, *seqlens, *indices, *mask;
     CANON_NONE_UNLESS(plain(args[0], &x) && plain(args[1], &state) && plain(args[2], &weight) && plain(args[3], &bias) &&
@@ -409,11 +604,33 @@ PyObject *launch_bwd(PyObject *, PyObject *const *args, Py_ssize_t n)
     CANON_NONE_UNLESS(plain(args[0], &xp) && plain(args[1], &gp) && plain(args[2], &wp) && plain(args[3], &bias) &&
                       plain(args[4], &mask) && plain(args[5], &dwp) && plain(args[6], &dbias) && plain(args[9], &seq) &&
                       plain(args[10], &init) && plain(args[11], &dinit) && plain(args[12], &dfin) && xp && gp && wp && dwp);
-    const Tensor &x = *xp, &weight = *wp, &dweight = *dwp;
+    const long act = small_int(args[7]), res = small_int(args[8]);
     void *stream;
-    CANON_NONE_UNLESS(stream_of(x, &stream));
-    Tensor dx = at::empty_like(x);
-    Tensor dout = *gp;
+    CANON_NONE_UNLESS(stream_of(*xp, &stream));
+    Tensor dx;
+    const int rc = without_gil([&] {
+        return run_bwd(*xp, *gp, *wp, bias, mask, *dwp, dbias, (int)act, (int)res, seq, init, dinit, dfin, stream, dx);
+    });
+    if (rc != CANON_OK) return PyLong_FromLong(rc);
+    return THPVariable_Wrap(std::move(dx));
+    END_HANDLE_TH_ERRORS
+}
+
+int run_fwd(const Tensor &x, const Tensor &weight, const Tensor *bias, const Tensor *mask, const Tensor *seq, int act, int res, int rnd,
+            void *stream, Tensor &out)
+{
+    out = at::empty_like(x);
+    const canon_conv1d_fwd_params p = fwd_params(x, out, weight, bias, mask, nullptr, nullptr, seq, act, res, rnd);
+    return without_gil([&] { return canon_conv1d_fwd(&p, stream); });
+}
+
+// The backward launch of checked arguments (dout and dfin of x's type) into dweight / dbias and a dx in x's layout, with a
+// scratch of this call alone.  Callable without the interpreter's lock.
+int run_bwd(const Tensor &x, Tensor dout, const Tensor &weight, const Tensor *bias, const Tensor *mask, const Tensor &dweight,
+            const Tensor *dbias, int act, int res, const Tensor *seq, const Tensor *init, const Tensor *dinit, const Tensor *dfin,
+            void *stream, Tensor &dx)
+{
+    dx = at::empty_like(x);
     if (dout.strides() != x.strides()) {
         // x's own layout keeps the vector kernels (empty_like: x's strides where x is dense)
         Tensor copy = at::empty_like(x);
@@ -427,7 +644,7 @@ PyObject *launch_bwd(PyObject *, PyObject *const *args, Py_ssize_t n)
     p.w_dtype = dtype_code(weight.scalar_type());
     p.grad_dtype = dtype_code(dweight.scalar_type());
     p.width = (int32_t)weight.size(1);
-    p.activation = (int32_t)small_int(args[7]); p.residual_mode = (int32_t)small_int(args[8]);
+    p.activation = act; p.residual_mode = res;
     p.batch = x.size(0); p.channels = x.size(1); p.seqlen = x.size(2);
     p.x = x.data_ptr();
     p.x_stride_b = x.stride(0); p.x_stride_c = x.stride(1); p.x_stride_l = x.stride(2);
@@ -464,14 +681,11 @@ PyObject *launch_bwd(PyObject *, PyObject *const *args, Py_ssize_t n)
     p.dweight = dweight.data_ptr();
     p.dbias = address(dbias);
     const int64_t bytes = canon_conv1d_bwd_workspace_bytes(&p);
-    if (bytes < 0) return PyLong_FromLong(CANON_ERR_INVALID_ARGUMENT);
+    if (bytes < 0) return CANON_ERR_INVALID_ARGUMENT;
     Tensor workspace = at::empty({bytes > 16 ? bytes : 16}, x.options().dtype(at::kByte));
     p.workspace = workspace.data_ptr();
     p.workspace_bytes = workspace.numel();
-    const int rc = without_gil([&] { return canon_conv1d_bwd(&p, stream); });
-    if (rc != CANON_OK) return PyLong_FromLong(rc);
-    return THPVariable_Wrap(std::move(dx));
-    END_HANDLE_TH_ERRORS
+    return canon_conv1d_bwd(&p, stream);
 }
 
 #define CANON_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
@@ -483,12 +697,6 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 PyMODINIT_FUNC PyInit__native()
 {
-    PyObject *torch_c = PyImport_ImportModule("torch._C");
-    if (!torch_c) return nullptr;
-    g_raw_stream = PyObject_GetAttrString(torch_c, "_cuda_getCurrentRawStream");
-    g_get_device = PyObject_GetAttrString(torch_c, "_cuda_getDevice");
-    Py_DECREF(torch_c);
-    if (!g_raw_stream || !g_get_device) return nullptr;
     // (torch's C++ interface is another one in every release: the loader compares this before it calls anything)
     PyObject *m = PyModule_Create(&module);
     if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
