@@ -31,7 +31,7 @@ namespace canon {
 __device__ __forceinline__ float silu_grad(float z)
 {
     const float s = __builtin_amdgcn_rcpf(1.0f + __expf(-z));
-    return s * (1.0f + z * (1.0f - s));
+    return fmaf(s, fmaf(-z, s, z), s);   // s + s * z * (1 - s)
 }
 
 template <int DT, int W, bool MASK, int R, bool SEQ>
@@ -296,8 +296,7 @@ __global__ __launch_bounds__(256) void canon_bwd_walk_kernel(const BwdArgs a)
 // of a channel stay in registers through the sweep, about thirty of them, so
 // the channels a lane owns decide how many waves a CU holds: with four
 // channels (8 bytes of a 16-bit row) 170-200 registers, two blocks per CU;
-// with two 82-100 (16-bit types, neither states nor packed rows; 93-107 with
-// packed rows, 100-123 with states; fp32 94-110, 104-123, 113-130), four or
+// with two 81-97 without an activation, up to 128 with SiLU or states, four or
 // five.  And chunks of 128 steps where the grid alone
 // would allow up to 1024: a CU then has new blocks to start while others drain,
 // for one partial set (20 bytes per channel) per 768 bytes of rows read and
@@ -386,7 +385,9 @@ __device__ __forceinline__ void bwd_dz_gated(const float (*w)[W], const float *b
 // first channel of slot 0) where it is needed: at most S_out steps per sequence.
 // SEQ: rows of several packed sequences in reach; q[j] is the sequence index of slab row j - 3 (rows -3 .. R+2).
 // ANY: dx is written through the lane's own pointer `any` (nullptr: a lane without channels), rows a.d_sl apart.
-template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E, bool SEQ = false, bool ANY = false>
+// RES: the residual's gradient is added to dx (1) or is not (0), with nothing between that sum and the store; -1: as the
+// arguments say.
+template <int DT, int W, bool MASK, bool ACT, bool FULL, bool FIN, int R, int E, bool SEQ = false, bool ANY = false, int RES = -1>
 __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W], const float *bias, const BwdVec<DT> *X,
                                           const BwdVec<DT> *H, const BwdVec<DT> *G, const uint32_t *mm, const float (*dzh)[E],
                                           float (*dzf)[E], float (*dw)[W], float *dbs, __amdgpu_buffer_rsrc_t rd, uint32_t voff,
@@ -399,8 +400,8 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
     // The residual's gradient is added before the mask multiply (masked residual) or after it (unmasked); with
     // nothing in between the two are the same sum.  Real branches (the empty asm keeps the compiler from turning
     // them into an add and a select per element and mode: 12 of 75 VALU instructions per row).
-    const bool res_pre = a.res_mode == CANON_RESIDUAL_MASKED || (!MASK && !FIN && a.res_mode == CANON_RESIDUAL_UNMASKED);
-    const bool res_post = a.res_mode == CANON_RESIDUAL_UNMASKED && !res_pre;
+    const bool res_pre = RES >= 0 ? RES == 1 : a.res_mode == CANON_RESIDUAL_MASKED || (!MASK && !FIN && a.res_mode == CANON_RESIDUAL_UNMASKED);
+    const bool res_post = RES < 0 && a.res_mode == CANON_RESIDUAL_UNMASKED && !res_pre;
 #pragma unroll
     for (int r = R - 1; r >= 0; --r) {
         float g[E], dz[E], o[E];
@@ -452,7 +453,7 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
             dzf[0][e] = dz[e];
         }
         if (res_pre) {
-            asm volatile("");
+            if constexpr (RES < 0) asm volatile("");
 #pragma unroll
             for (int e = 0; e < E; ++e) o[e] += g[e];
         }
@@ -476,7 +477,8 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
             for (int e = 0; e < E; ++e) o[e] += g[e];
         }
         if constexpr (ANY) {
-            if ((FULL || r < rows) && any) store_any<kBwdLaneChannels * Elem<DT>::bytes>(any + r * a.d_sl * Elem<DT>::bytes, pack_lane<DT>(o));
+            if ((FULL || r < rows) && any)
+                store_any<kBwdLaneChannels * Elem<DT>::bytes>(any + r * a.d_sl * Elem<DT>::bytes, pack_lane<DT>(o));
         } else if (FULL || r < rows) {
             BufIO<kBwdLaneChannels * Elem<DT>::bytes>::template store<kAuxStream>(pack_lane<DT>(o), rd, voff, (uint32_t)r * ds);
         }
@@ -511,13 +513,16 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
 // with the reduction, bf16: B 8, C 961, L 1021 29.6 -> 20.9, with SiLU and a mask 41.9 -> 23.2; B 24, C 1695, L 170 with both
 // 33.5 -> 22.0; B 8, C 3455, L 1024 79.1 -> 61.5 (on the grid 36.6: a misaligned four-byte access touches two words).
 template <int DT, int W, bool MASK, bool ACT, bool STATES, bool SEQ = false, bool ANY = false>
-__global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
+__global__ __launch_bounds__(256, ACT ? 4 : 1) void canon_bwd_blc_kernel(const BwdArgs a)
 {
     static_assert(!(STATES && SEQ), "seq_idx excludes states");
     static_assert(!ANY || !(STATES || SEQ), "neither packed nor with states");
     constexpr int BY = Elem<DT>::bytes;
     constexpr int E = kBwdLaneChannels, VB = E * BY;
     constexpr int R = kBwdSlab, NW = kBwdWaves;
+    // which instances take whole slabs through a sweep without branches, and request their first tile ahead of the staged
+    // mask and indices (both below): the others hold 82-95 registers and lose a wave per SIMD, or time, to it
+    constexpr bool kStraight = !STATES && (ACT || !(MASK || SEQ)), kAllAtOnce = ACT || !(MASK || SEQ);
     // With an activation: tailx / headdz, two barriers per tile (dz of a slab's head needs the previous
     // wave's tail first).  Without one dz IS dout, so the head is handed over as raw rows (headg) together
     // with the tail, one barrier per tile, both double-buffered (a fast wave publishes the next tile while
@@ -532,6 +537,10 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     union Shared {
         Exchange x;
         float red[NW - 1][5 * E][64];                 // dweight / dbias sums of waves 1..3
+        // Four blocks a CU instead of the five their registers allow: unmasked launches without an activation, B 8 / 16 / 32,
+        // C 3456, L 1024, bf16: 36.2 / 64.0 / 120.5 -> 35.4 / 63.3 / 119.7 us a call (three: 38.5 / 64.6 / 122; with a mask
+        // four are 0.4 % slower).
+        char room[!ACT && !MASK && !SEQ && !STATES ? 33 * 1024 : 16];
     };
     __shared__ Shared shared;
     auto &tailx = shared.x.tailx;
@@ -573,14 +582,72 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
     const int64_t t_chunk = (int64_t)ch * a.chunk;
     const int ntiles = (int)(a.chunk / (uint32_t)(R * NW));
 
-    RawTaps<E> rawt;
-    fetch_taps<W, E, ANY>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c0, rawt);
-    float w[E][W], bias[E];
     // a row of x or dout at this lane's channels
     auto load_row = [](const char *p) {
         if constexpr (ANY) return load_any<VB, false>(p);
         else return BwdIO<DT>::template load<false>(p);
     };
+    auto rows_from = [&](int64_t t0) {      // steps of the slab at t0 that exist (wave uniform)
+        const int64_t left = (int64_t)a.L - t0;
+        return left >= R ? R : (left > 0 ? (int)left : 0);
+    };
+    // All rows of x and dout of a tile's slab and, for the first wave, the three rows of x before it.  (Requesting the next
+    // tile's rows while this one is worked on was measured three times (before, and after, this tile's rows are waited for;
+    // with two register sets taken in turn and wait counts that leave the next tile's loads in flight): 3-5 % slower, 40-60
+    // more registers.)  The x resource starts three rows before the slab; a row past the end of the sequence is the slab's last
+    // row again, loaded and never used, and a slab without rows has resources without a range.
+    BwdVec<DT> X[R], G[R], H[3];
+    auto request = [&](int it) {
+        const int64_t t0 = t_chunk + ((int64_t)it * NW + wv) * R;
+        const int rows = rows_from(t0);
+        const uint32_t xrec = rows == 0 ? 0u : (uint32_t)(R + 2) * xs32 + nl * VB;
+        const uint32_t grec = rows == 0 ? 0u : (uint32_t)(R - 1) * gs32 + nl * VB;
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(xb0 + (t0 - 3) * xs), 0, (int)xrec, kBufFlags);
+        const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void *)(gb0 + t0 * gs), 0, (int)grec, kBufFlags);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint32_t rr = r < rows ? (uint32_t)r : (rows > 0 ? (uint32_t)(rows - 1) : 0u);
+            if constexpr (ANY) {
+                const int64_t t = rows > 0 ? t0 + rr : Lm1;      // (a slab without rows: the sequence's last row, never used)
+                X[r] = load_any<VB, true>(xb + t * xs);
+                G[r] = load_any<VB, true>(gb + t * gs);
+            } else {
+                X[r] = IO::template load<kAuxStream>(rx, voff, (rr + 3u) * xs32);
+                G[r] = IO::template load<kAuxStream>(rg, voff, rr * gs32);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) H[j] = BwdIO<DT>::zero();
+        if (wv == 0 && t0 > 0) {     // (t0 is a multiple of the tile: all three rows exist)
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                if constexpr (ANY) H[j] = load_any<VB, false>(xb + ((t0 <= Lm1 ? t0 : Lm1 + 1) - 3 + j) * xs);
+                else H[j] = IO::template load<kAuxPlain>(rx, voff, (uint32_t)j * xs32);
+            }
+        }
+    };
+
+    // Everything the block reads before its second tile is requested here, before the first wait: taps, the rows just past
+    // the chunk (last wave), the first tile, the staged mask and indices.  One after the other, each behind the barrier or
+    // the wait of the one before, they were three memory round trips: B 8, C 640, L 1024, bf16 12.6 -> 12.2 us a call,
+    // B 8, C 3456 with SiLU 39.6 -> 38.5; with a mask and no activation 24.0 -> 24.25 (B 16, C 960), so not there.
+    RawTaps<E> rawt;
+    fetch_taps<W, E, ANY>(a.weight, a.bias, a.w_sc, a.w_sk, a.w_dtype, a.w_vec != 0, c0, rawt);
+    const int64_t te = t_chunk + (int64_t)a.chunk;   // first step after the chunk (at least 32)
+    BwdVec<DT> XE[ACT ? 6 : 1], GE[3];               // rows te-3 .. te+2 of x (with an activation), te .. te+2 of dout
+#pragma unroll
+    for (int j = 0; j < (ACT ? 6 : 1); ++j) XE[j] = BwdIO<DT>::zero();
+#pragma unroll
+    for (int j = 0; j < 3; ++j) GE[j] = BwdIO<DT>::zero();
+    if (wv == NW - 1 && te <= Lm1) {
+        if constexpr (ACT) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) XE[j] = load_row(xb + (te - 3 + j < Lm1 ? te - 3 + j : Lm1) * xs);
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) GE[j] = load_row(gb + (te + j < Lm1 ? te + j : Lm1) * gs);
+    }
+    if constexpr (kAllAtOnce) request(ntiles - 1);
     if constexpr (MASK || SEQ) {
         for (uint32_t i = threadIdx.x; i < a.chunk + 6u; i += 64u * NW) {
             int64_t t = t_chunk - 3 + (int64_t)i;
@@ -590,62 +657,31 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
         }
         __syncthreads();
     }
+    if constexpr (!kAllAtOnce) request(ntiles - 1);
 
     // The tiles are walked from the last to the first, so the dz of the three steps after a tile
     // are the head of the tile done just before (still in headdz[0]).  For the chunk's last tile
     // the last wave computes them here, from six rows of x and three of dout, and leaves them
     // in that slot itself.
     float dzf[3][E];   // dzf[j] = dz[t + 1 + j] for the step t being processed
-#pragma unroll
-    for (int j = 0; j < 3; ++j)
-#pragma unroll
-        for (int e = 0; e < E; ++e) dzf[j][e] = 0.0f;
+    float w[E][W], bias[E];
+    decode_taps<DT, W, E>(rawt, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
     if constexpr (!ACT) {
         // no activation: the three dz after the chunk are three rows of dout, kept by the last wave
-        const int64_t te = t_chunk + (int64_t)a.chunk;
-        BwdVec<DT> GE[3];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) GE[j] = BwdIO<DT>::zero();
-        if (wv == NW - 1) {
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                if (te + j <= Lm1) GE[j] = load_row(gb + (te + j) * gs);
-        }
-        decode_taps<DT, W, E>(rawt, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
-#pragma unroll
-        for (int j = 0; j < 3; ++j) unpack_lane<DT>(GE[j], dzf[j]);
+        for (int j = 0; j < 3; ++j) unpack_lane<DT>(te + j <= Lm1 ? GE[j] : BwdIO<DT>::zero(), dzf[j]);
     } else {
-        const int64_t te = t_chunk + (int64_t)a.chunk;   // first step after the chunk (at least 32)
-        BwdVec<DT> XE[6], GE[3];
-        uint32_t me[6];
 #pragma unroll
-        for (int j = 0; j < 6; ++j) {
-            XE[j] = BwdIO<DT>::zero();
-            me[j] = kMaskOne;
-        }
+        for (int j = 0; j < 3; ++j)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) GE[j] = BwdIO<DT>::zero();
-        if (wv == NW - 1 && te <= Lm1) {
-#pragma unroll
-            for (int j = 0; j < 6; ++j) {
-                const int64_t t = te - 3 + j;
-                XE[j] = load_row(xb + (t < Lm1 ? t : Lm1) * xs);
-            }
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const int64_t t = te + j;
-                GE[j] = load_row(gb + (t < Lm1 ? t : Lm1) * gs);
-            }
-            if constexpr (MASK) {
-#pragma unroll
-                for (int j = 0; j < 6; ++j) me[j] = f_bits(smask[a.chunk + j]);   // steps te-3 .. te+2
-            }
-        }
-        decode_taps<DT, W, E>(rawt, a.w_dtype, a.w_vec != 0, a.bias != nullptr, w, bias);
+            for (int e = 0; e < E; ++e) dzf[j][e] = 0.0f;
         if (wv == NW - 1) {
             float xt[6][E];
 #pragma unroll
-            for (int j = 0; j < 6; ++j) unpack_lane<DT>(bwd_mask_row<DT, MASK>(XE[j], me[j], te - 3 + j <= Lm1), xt[j]);
+            for (int j = 0; j < 6; ++j) {
+                const uint32_t m = MASK ? f_bits(smask[a.chunk + j]) : kMaskOne;   // steps te-3 .. te+2
+                unpack_lane<DT>(bwd_mask_row<DT, MASK>(XE[j], m, te - 3 + j <= Lm1), xt[j]);
+            }
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
                 float g[E], d[E];
@@ -674,48 +710,18 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
 
     for (int it = ntiles - 1; it >= 0; --it) {
         const int64_t t0 = t_chunk + ((int64_t)it * NW + wv) * R;
-        const int64_t left = (int64_t)a.L - t0;
-        const int rows = left >= R ? R : (left > 0 ? (int)left : 0);   // wave uniform
-
-        // ---- all loads of the tile.  Requesting the next tile's rows while this one is worked on was measured
-        // three times (before, and after, this tile's rows are waited for; with two register sets taken in turn
-        // and wait counts that leave the next tile's loads in flight): 3-5 % slower, 40-60 more registers.
-        // (the x resource starts three rows before the slab; a row past the end of the sequence is the slab's last row
-        // again, loaded and never used, and a slab without rows has resources without a range)
-        const uint32_t xrec = rows == 0 ? 0u : (uint32_t)(R + 2) * xs32 + nl * VB;
-        const uint32_t grec = rows == 0 ? 0u : (uint32_t)(R - 1) * gs32 + nl * VB;
+        const int rows = rows_from(t0);
         const uint32_t drec = rows == 0 ? 0u : (uint32_t)(R - 1) * ds32 + nl * VB;
-        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(xb0 + (t0 - 3) * xs), 0, (int)xrec, kBufFlags);
-        const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc((void *)(gb0 + t0 * gs), 0, (int)grec, kBufFlags);
         const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc((void *)(db0 + t0 * ds), 0, (int)drec, kBufFlags);
-        BwdVec<DT> X[R], G[R], H[3];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const uint32_t rr = r < rows ? (uint32_t)r : (rows > 0 ? (uint32_t)(rows - 1) : 0u);
-            if constexpr (ANY) {
-                const int64_t t = rows > 0 ? t0 + rr : Lm1;      // (a slab without rows: the sequence's last row, never used)
-                X[r] = load_any<VB, true>(xb + t * xs);
-                G[r] = load_any<VB, true>(gb + t * gs);
-            } else {
-                X[r] = IO::template load<kAuxStream>(rx, voff, (rr + 3u) * xs32);
-                G[r] = IO::template load<kAuxStream>(rg, voff, rr * gs32);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 3; ++j) H[j] = BwdIO<DT>::zero();
-        if (wv == 0 && t0 > 0) {     // (t0 is a multiple of the tile: all three rows exist)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                if constexpr (ANY) H[j] = load_any<VB, false>(xb + ((t0 <= Lm1 ? t0 : Lm1 + 1) - 3 + j) * xs);
-                else H[j] = IO::template load<kAuxPlain>(rx, voff, (uint32_t)j * xs32);
-            }
-        }
+        if (it != ntiles - 1) request(it);
+        bool plain_mask = true;   // every row of the slab and the three before it are valid tokens: x * 1 is x
         uint32_t mm[R + 3];   // mask of steps t0-3 .. t0+R-1 (bits, in scalar registers: one LDS read, then lane by lane)
 #pragma unroll
         for (int j = 0; j < R + 3; ++j) mm[j] = kMaskOne;
         if constexpr (MASK) {
             const uint32_t first = ((uint32_t)it * NW + wv) * R;   // index of step t0 - 3 in smask
             const uint32_t m_lane = f_bits(smask[first + (uint32_t)(lane < R + 2 ? lane : R + 2)]);
+            plain_mask = __builtin_amdgcn_ballot_w64(m_lane != kMaskOne) == 0;
 #pragma unroll
             for (int j = 0; j < R + 3; ++j) mm[j] = (uint32_t)__builtin_amdgcn_readlane((int)m_lane, j);
         }
@@ -744,12 +750,12 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
         }
 
         // ---- rows become xm (masked, zero where they do not exist), once ----------------
-        if (MASK || rows < R) {
+        if (!plain_mask || rows < R) {
 #pragma unroll
             for (int r = 0; r < R; ++r) X[r] = bwd_mask_row<DT, MASK>(X[r], mm[3 + r], r < rows);
         }
         if constexpr (MASK) {
-            if (wv == 0) {
+            if (wv == 0 && !plain_mask) {
 #pragma unroll
                 for (int j = 0; j < 3; ++j) H[j] = bwd_mask_row<DT, MASK>(H[j], mm[j], true);   // zero already when t < 0
             }
@@ -849,12 +855,25 @@ __global__ __launch_bounds__(256) void canon_bwd_blc_kernel(const BwdArgs a)
                                                                  nullptr, 0, q);
         } else {
             char *dany = ANY && active ? a.dx + ((int64_t)b * a.d_sb + c0) * BY + t0 * ds : nullptr;
-            if (rows == R)
-                bwd_sweep<DT, W, MASK, ACT, true, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
-                                                                           nullptr, 0, nullptr, dany);
-            else
-                bwd_sweep<DT, W, MASK, ACT, false, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows,
-                                                                            nullptr, 0, nullptr, dany);
+            // Whole slabs of valid tokens, which most are, take a sweep without a branch in it: with the residual's and the
+            // mask's branches in every row, each a break in the instruction stream, the launches with SiLU were bound by the
+            // sweep.  us a call, both changes: C 3456, L 1024, bf16, SiLU B 8 39.5 -> 38.1, with a mask B 32 138.2 -> 133.3;
+            // packed rows with SiLU B 2, L 8192 72.5 -> 69.6, B 1, L 4000 25.7 -> 24.2; fp32 B 24, C 2848, L 385 70.6 -> 66.9;
+            // (up to 128 registers with SiLU, four waves per SIMD; held to 96 and five it spills: 43-198 us in place of 38-134)
+            if (kStraight && rows == R && plain_mask) {
+                if (a.res_mode != CANON_RESIDUAL_NONE)
+                    bwd_sweep<DT, W, false, ACT, true, false, R, E, false, ANY, 1>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff,
+                                                                                   ds32, rows, nullptr, 0, nullptr, dany);
+                else
+                    bwd_sweep<DT, W, false, ACT, true, false, R, E, false, ANY, 0>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff,
+                                                                                   ds32, rows, nullptr, 0, nullptr, dany);
+            } else if (rows == R) {
+                bwd_sweep<DT, W, MASK, ACT, true, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32,
+                                                                           rows, nullptr, 0, nullptr, dany);
+            } else {
+                bwd_sweep<DT, W, MASK, ACT, false, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32,
+                                                                            rows, nullptr, 0, nullptr, dany);
+            }
         }
     }
 
