@@ -553,6 +553,18 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
             assert torch.equal(torch.isfinite(dw), torch.isfinite(dws)), (bad, back, "silu")
 
 
+@pytest.mark.parametrize("sets", [1, 7, 8, 9, 31, 32, 33, 64, 65, 127, 128, 129, 130, 257])
+def test_reduction_over_any_number_of_partial_sets(cc, sets):
+    """One partial set per batch row: counts around the rounds in which a slice of the reduction requests its sets."""
+    g = torch.Generator().manual_seed(sets)
+    x, dout = torch.randn(sets, 12, 20, generator=g), torch.randn(sets, 12, 20, generator=g)
+    w, b = torch.randn(12, 4, generator=g), torch.randn(12, generator=g)
+    _, rdw, rdb, _ = conv1d_grads(x, w, b, dout, None, "silu", False)
+    _, dw, db, _ = gpu_grads(cc, x, w, b, dout, "blc", None, "silu", False)
+    check(dw, rdw, torch.float32, "dweight", sum_terms=sets * 20)
+    check(db, rdb, torch.float32, "dbias", sum_terms=sets * 20)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_backward_of_channel_contiguous_rows_off_the_8_byte_grid(cc, dtype):
     """Channel counts that are no multiple of 8 bytes, and slices of wider rows: from one lane's two channels on, around a

@@ -1372,6 +1372,11 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_short_kernel(const char *x_
 // (c, j) columns; its 8 slices each sum every 8th set in set order (fp64), then the slices are added
 // in slice order.  Reads are 128 contiguous bytes per set and slice.
 //
+// U sets a slice are requested together, added in set order: what bounds the kernel is the round trips in a row, not the
+// bytes.  Four loads in flight and the sets past the last whole round one by one -> sixteen from 65 sets on, four below, us of the whole
+// call: B 8 C 640 L 1024 12.2 -> 11.4, B 16 C 640 L 511 SiLU masked 16.2 -> 15.4, packed rows B 2 C 3456 L 8192 72.1 -> 70.5, B 1
+// C 160 L 896 8.1 -> 7.6.  (Sixteen at B 1 and B 4, C 3456, 8 and 32 sets: 10.0 -> 10.4, 20.9 -> 21.4.)
+//
 // The sum is stored as the caller's gradient type: converting fp32 sums to 16-bit parameters' type in two further
 // launches took a training step at B 16, C 640, L 511 (of 33 us on the device) 3.5 us and their host time.
 template <typename T> __global__ __launch_bounds__(256) void canon_zero_kernel(T *p, uint32_t n)
@@ -1387,7 +1392,7 @@ __device__ __forceinline__ void store_grad(void *p, uint32_t i, float v, int dty
     else store1<CANON_DTYPE_F16>(p, i, v);
 }
 
-__global__ __launch_bounds__(256) void canon_bwd_reduce_kernel(const float *partial, void *dweight, void *dbias,
+template <uint32_t U> __global__ __launch_bounds__(256) void canon_bwd_reduce_kernel(const float *partial, void *dweight, void *dbias,
                                                               uint32_t C, uint32_t nsets, int W, int dtype)
 {
     __shared__ double part[8][32];
@@ -1396,16 +1401,13 @@ __global__ __launch_bounds__(256) void canon_bwd_reduce_kernel(const float *part
     const uint32_t i = blockIdx.x * 32u + col;   // (c, j), j in 0..4
     double acc = 0.0;
     if (i < ncols) {
-        uint32_t s = slice;
-        for (; s + 24u < nsets; s += 32u) {   // four loads in flight, added in set order
-            const float v0 = partial[(int64_t)s * ncols + i], v1 = partial[(int64_t)(s + 8u) * ncols + i];
-            const float v2 = partial[(int64_t)(s + 16u) * ncols + i], v3 = partial[(int64_t)(s + 24u) * ncols + i];
-            acc += (double)v0;
-            acc += (double)v1;
-            acc += (double)v2;
-            acc += (double)v3;
+        for (uint32_t s = slice; s < nsets; s += 8u * U) {
+            float v[U];   // (past the last set: the round's first again, not added)
+#pragma unroll
+            for (uint32_t k = 0; k < U; ++k) v[k] = partial[(int64_t)(s + 8u * k < nsets ? s + 8u * k : s) * ncols + i];
+#pragma unroll
+            for (uint32_t k = 0; k < U; ++k) acc += s + 8u * k < nsets ? (double)v[k] : 0.0;
         }
-        for (; s < nsets; s += 8u) acc += (double)partial[(int64_t)s * ncols + i];
     }
     part[slice][col] = acc;
     __syncthreads();
@@ -1680,6 +1682,13 @@ __global__ __launch_bounds__(256) void canon_update_bwd_vec_kernel(const UpdBwdA
 // ---------------------------------------------------------------------------
 namespace {
 
+void launch_reduce(const float *partial, void *dweight, void *dbias, uint32_t C, uint32_t nsets, int W, int dtype, hipStream_t s)
+{
+    const dim3 g((C * 5u + 31u) / 32u), b(256);
+    if (nsets > 64u) hipLaunchKernelGGL((canon_bwd_reduce_kernel<16>), g, b, 0, s, partial, dweight, dbias, C, nsets, W, dtype);
+    else hipLaunchKernelGGL((canon_bwd_reduce_kernel<4>), g, b, 0, s, partial, dweight, dbias, C, nsets, W, dtype);
+}
+
 template <int DT, int W, bool MASK, bool RAGGED> void launch_bwd_bcl(const BwdPlan &pl, hipStream_t s)
 {
     const dim3 g(pl.grid), b(256);
@@ -1754,8 +1763,7 @@ void launch_bwd(const BwdPlan &pl, int x_dtype, hipStream_t s)
     case CANON_DTYPE_BF16: launch_bwd<CANON_DTYPE_BF16>(pl, s); break;
     default: launch_bwd<CANON_DTYPE_F16>(pl, s); break;
     }
-    hipLaunchKernelGGL(canon_bwd_reduce_kernel, dim3((pl.args.C * 5u + 31u) / 32u), dim3(256), 0, s,
-                       pl.args.partial, pl.args.dweight, pl.args.dbias, pl.args.C, pl.args.nsets, pl.args.W, pl.args.grad_dtype);
+    launch_reduce(pl.args.partial, pl.args.dweight, pl.args.dbias, pl.args.C, pl.args.nsets, pl.args.W, pl.args.grad_dtype, s);
 }
 
 void launch_update_bwd(const UpdBwdPlan &pl, int x_dtype, hipStream_t s)
@@ -1785,8 +1793,7 @@ void launch_update_bwd(const UpdBwdPlan &pl, int x_dtype, hipStream_t s)
         }
     }
     if (pl.args.partial)
-        hipLaunchKernelGGL(canon_bwd_reduce_kernel, dim3((pl.args.C * 5u + 31u) / 32u), dim3(256), 0, s, pl.args.partial,
-                           pl.args.dweight, pl.args.dbias, pl.args.C, pl.args.ngroups, pl.args.W, CANON_DTYPE_F32);
+        launch_reduce(pl.args.partial, pl.args.dweight, pl.args.dbias, pl.args.C, pl.args.ngroups, pl.args.W, CANON_DTYPE_F32, s);
 }
 
 // Asking for a kernel's attributes makes the runtime load this file's code object onto the current device.
