@@ -765,7 +765,7 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         // Chunks of kBwdChunk steps, shorter where the grid would not have one and a half blocks per CU.  A scratch with
         // no room for their partial sets (a caller's own, or the library's static one) gets the longest chunks that fill
         // the grid.
-        BwdChunks ch = bwd_chunks(a.B, a.L, nct, kBwdChunk);
+        BwdChunks ch = bwd_chunks(a.B, a.L, nct, p->x_dtype == CANON_DTYPE_F32 ? kBwdChunkWide : kBwdChunk);
         plan->workspace_bytes = (int64_t)a.B * ch.n * set_bytes;
         const int64_t room = check_pointers ? p->workspace_bytes : scratch;
         if (room >= 0 && plan->workspace_bytes > room) {

@@ -199,6 +199,10 @@ constexpr int kBwdLaneChannels = 2;         // adjacent channels per lane in the
 #define CANON_BWD_CHUNK 128
 #endif
 constexpr uint32_t kBwdChunk = CANON_BWD_CHUNK;   // most time steps a block of it walks while the scratch has room for the sets
+// ... and of fp32, whose rows are twice the bytes a partial set is set against (us a call with chunks of 128 / 64 steps: B 8
+// C 3456 L 1024 64.3 / 62.4, B 24 C 2848 L 385 SiLU masked 67.0 / 62.9, B 16 C 3456 L 512 masked 66.6 / 63.8, packed B 2 L 4096
+// SiLU 64.8 / 62.5, C 640 and 960 equal; bf16 with 64: packed SiLU 72 / 81, B 16 C 960 masked 24.0 / 26.9)
+constexpr uint32_t kBwdChunkWide = CANON_BWD_CHUNK / 2;
 constexpr int kBwdWaves = 4;
 constexpr int kBwdMaxChunk = 32 * kBwdSlab * kBwdWaves;   // ... and at all
 enum FwdKind { FWD_BCL, FWD_BCL_SHORT, FWD_BLC, FWD_BLC_ANY, FWD_GENERIC };
