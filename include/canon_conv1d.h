@@ -388,7 +388,7 @@ int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *stream);
 
 /* Scratch bytes canon_conv1d_bwd works with for these sizes, strides and pointer
  * alignments (less is accepted where fewer partial sets can be cut: a set per sequence and chunk is 20 bytes per
- * channel, a chunk of the channel-contiguous kernel 64 to 128 time steps where there is room, up to 1024 where not); with x, dout or dx missing (NULL) the figure also covers the
+ * channel, a chunk of the channel-contiguous kernel 64 to 128 time steps (32 to 64 in fp32) where there is room, up to 1024 where not); with x, dout or dx missing (NULL) the figure also covers the
  * kernel a misaligned pointer would select.  Negative if the arguments are
  * rejected. */
 int64_t canon_conv1d_bwd_workspace_bytes(const canon_conv1d_bwd_params *p);

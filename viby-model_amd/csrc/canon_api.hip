@@ -179,7 +179,7 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     const bool ptr_ok = aligned16(p->x) && aligned16(p->out);
     // packed sequences: the channel-contiguous kernel has a variant (the index is uniform per time row);
     // time-contiguous rows take the strided kernel
-    // shorter rows leave most of a wave idle: measured slower than the strided kernel below 16 vectors
+    // (the shortest rows of this family by name; rows of up to kBclShortMaxVectors share waves, below)
     const uint32_t kBclMinVectors = 16;
     const bool bcl_rows = !p->seq_idx && ptr_ok && a.x_sl == 1 && a.o_sl == 1 && a.L / E >= kBclMinVectors;
     // every row starts on a 16-byte boundary and is a whole number of vectors ...
@@ -678,10 +678,10 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     // whole vectors on 16-byte boundaries ...
     const bool rows_aligned = rows_any && ptrs16 && a.L % E == 0 && a.L / E >= 16 && a.x_sb % E == 0 && a.x_sc % E == 0 &&
                               a.g_sb % E == 0 && a.g_sc % E == 0 && a.d_sb % E == 0 && a.d_sc % E == 0;
-    // ... or not: the kernel's ragged variant (elements at their own alignment), for rows of at least kRaggedMinSteps.
-    // A wave per row costs the same whatever the row's length, the walk kernel, whose lanes lie a row apart, pays for
-    // every step: measured at 30720 rows, bf16: L 24 15.6 against 10.2 us, L 64 16.1 against 30.0, L 120 16.6 against
-    // 62.8, L 500 20.0 against 272; fp32 with mask and SiLU: L 30 17.6 against 19.6 us.
+    // ... or not: the kernel's ragged variant (elements at their own alignment).  A wave per row costs the same whatever the
+    // row's length, the walk kernel, whose lanes lie a row apart, pays for every step: measured at 30720 rows, bf16, L 500
+    // 20.0 against 272 us.  (Rows of up to kBclShortMaxVectors share waves, below; the least length here is that of the family
+    // by name.)
     constexpr uint32_t kRaggedMinSteps = 40;
     const int64_t unit = rows_aligned ? E : 1;
     const uintptr_t elem_mask = (uintptr_t)elem_bytes(p->x_dtype) - 1;
