@@ -553,6 +553,42 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
             assert torch.equal(torch.isfinite(dw), torch.isfinite(dws)), (bad, back, "silu")
 
 
+@pytest.mark.parametrize("sets", [10, 9, 5, 3, 2, 1])
+def test_fp32_backward_in_scratch_for_fewer_sets(cc, sets):
+    """96 sequences of 640 steps in fp32: ten chunks each where there is room, chunks twice as long (and so on) where not:
+    the same dx bits, sums in another order."""
+    import ctypes
+
+    from causal_conv1d import _lib
+    B, C, L = 96, 1024, 640
+    g = torch.Generator(device=DEV).manual_seed(6)
+    x, dout = (torch.randn(B, L, C, device=DEV, generator=g).transpose(1, 2) for _ in range(2))
+    w, b = torch.randn(C, 4, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+
+    def call(nbytes):
+        dx, dw, db = torch.empty_like(x), torch.empty(C, 4, device=DEV), torch.empty(C, device=DEV)
+        p = _lib.BwdParams(struct_size=ctypes.sizeof(_lib.BwdParams), width=4, activation=1, batch=B, channels=C, seqlen=L)
+        for name, t in (("x", x), ("dout", dout), ("dx", dx)):
+            setattr(p, name, t.data_ptr())
+            for axis, stride in zip("bcl", t.stride()):
+                setattr(p, f"{name}_stride_{axis}", stride)
+        p.weight, p.w_stride_c, p.w_stride_k, p.bias = w.data_ptr(), 4, 1, b.data_ptr()
+        p.dweight, p.dbias = dw.data_ptr(), db.data_ptr()
+        need = _lib.lib().canon_conv1d_bwd_workspace_bytes(ctypes.byref(p))
+        space = torch.empty(nbytes or need, dtype=torch.uint8, device=DEV)
+        p.workspace, p.workspace_bytes = space.data_ptr(), space.numel()
+        rc = _lib.lib().canon_conv1d_bwd(ctypes.byref(p), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, _lib.lib().canon_conv1d_last_error()
+        torch.cuda.synchronize()
+        return need, dx, dw, db
+    want = call(0)
+    assert want[0] == 10 * B * C * 20
+    got = call(sets * B * C * 20)
+    assert torch.equal(got[1], want[1])
+    for a, c in zip(got[2:], want[2:]):
+        assert (a - c).abs().max().item() <= 1e-4 * c.abs().max().item()
+
+
 @pytest.mark.parametrize("sets", [1, 7, 8, 9, 31, 32, 33, 64, 65, 127, 128, 129, 130, 257])
 def test_reduction_over_any_number_of_partial_sets(cc, sets):
     """One partial set per batch row: counts around the rounds in which a slice of the reduction requests its sets."""

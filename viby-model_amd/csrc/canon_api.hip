@@ -763,15 +763,16 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         const uint32_t nct = (nvec + 63) / 64;
         const int64_t set_bytes = (int64_t)a.C * 5 * (int64_t)sizeof(float);
         // Chunks of kBwdChunk steps, shorter where the grid would not have one and a half blocks per CU.  A scratch with
-        // no room for their partial sets (a caller's own, or the library's static one) gets the longest chunks that fill
-        // the grid.
-        BwdChunks ch = bwd_chunks(a.B, a.L, nct, p->x_dtype == CANON_DTYPE_F32 ? kBwdChunkWide : kBwdChunk);
+        // no room for their partial sets (a caller's own, or the library's static one) gets chunks twice as long, and so on,
+        // until the sets fit.
+        const uint32_t usual = p->x_dtype == CANON_DTYPE_F32 ? kBwdChunkWide : kBwdChunk;
+        BwdChunks ch = bwd_chunks(a.B, a.L, nct, usual);
         plan->workspace_bytes = (int64_t)a.B * ch.n * set_bytes;
         const int64_t room = check_pointers ? p->workspace_bytes : scratch;
-        if (room >= 0 && plan->workspace_bytes > room) {
-            const BwdChunks longest = bwd_chunks(a.B, a.L, nct, kBwdMaxChunk);
-            if ((int64_t)a.B * longest.n * set_bytes <= room) {
-                ch = longest;
+        for (uint32_t longest = 2 * usual; room >= 0 && plan->workspace_bytes > room && longest <= (uint32_t)kBwdMaxChunk; longest *= 2) {
+            const BwdChunks fewer = bwd_chunks(a.B, a.L, nct, longest);
+            if ((int64_t)a.B * fewer.n * set_bytes <= room) {
+                ch = fewer;
                 plan->workspace_bytes = (int64_t)a.B * ch.n * set_bytes;
             }
         }
