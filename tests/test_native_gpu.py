@@ -180,6 +180,20 @@ def test_refused_calls(cc, monkeypatch):
         assert_same(native, general, n)
 
 
+def test_decode_call_of_the_wrong_rank(cc, monkeypatch):
+    """A bias or a token mask of another rank than one is refused before its sizes enter the call's signature, whose length
+    is that of the ranks that are taken (a bias and a mask of three dimensions each would not fit it)."""
+    x, w, b = torch.randn(2, 8, device=DEV), torch.randn(8, 4, device=DEV), torch.randn(8, device=DEV)
+    state, mask = torch.randn(2, 8, 3, device=DEV), torch.ones(2, device=DEV)
+    for bias in (b, b[None, :], b[None, :, None], b[0]):
+        for m in (None, mask, mask[:, None], mask[:, None, None], mask[0]):
+            native, general = both(cc, monkeypatch, lambda: cc.causal_conv1d_update(x, state.clone(), w, bias, token_mask=m))
+            assert_same(native, general, (bias.shape, None if m is None else m.shape))
+            assert isinstance(native, str) == (bias.dim() != 1 or (m is not None and m.dim() != 1))
+            if bias.dim() != 1:
+                assert native == f"ValueError: Expected 1D bias tensor, got {bias.dim()}D"
+
+
 def test_another_stream_and_a_captured_graph(cc):
     x = torch.randn(2, 64, 256, device=DEV).bfloat16()
     w = torch.randn(64, 4, device=DEV).bfloat16()

@@ -458,14 +458,16 @@ PyObject *known_update(PyObject *const *args)
     CANON_NONE_UNLESS(act >= 0 && res >= 0 && rnd >= 0 && x->dim() == 2 && state->dim() == 3 && weight->dim() == 2 && x->is_cuda());
     CANON_NONE_UNLESS(!c10::GradMode::is_enabled() ||
                       !(wants_grad(x) || wants_grad(state) || wants_grad(weight) || wants_grad(bias) || wants_grad(mask)));
-    int64_t key[32] = {act | res << 4 | rnd << 8, x->get_device()};
+    CANON_NONE_UNLESS((!bias || bias->dim() == 1) && (!mask || mask->dim() == 1));
+    // two entries, then a type and a size and stride per dimension: x 2, state 3, weight 2, bias 1, mask 1 (checked above)
+    int64_t key[2 + 5 + 2 * (2 + 3 + 2 + 1 + 1)] = {act | res << 4 | rnd << 8, x->get_device()};
     int at = 2;
     for (const Tensor *t : {x, state, weight, bias, mask}) {
         if (!t) {
             key[at++] = -1;
             continue;
         }
-        CANON_NONE_UNLESS(t->dim() <= 3 && t->device() == x->device());
+        CANON_NONE_UNLESS(t->device() == x->device());
         key[at++] = (int64_t)t->scalar_type() | t->dim() << 8;
         for (int64_t i = 0; i < t->dim(); ++i) {
             key[at++] = t->size(i);
