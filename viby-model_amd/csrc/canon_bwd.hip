@@ -441,10 +441,11 @@ __device__ __forceinline__ void bwd_sweep(const BwdArgs &a, const float (*w)[W],
             // Steps past the end of the sequence have a dz of zero, but their window holds the sequence's last inputs, and
             // 0 * Inf is NaN: the window is zero as well (selects), or the sums are left out (a branch).  By register
             // count: the branch costs the ordinary instances five registers and with SiLU (95 -> 100) a wave per SIMD;
-            // the gated sweep holds 107 with it, 128 with the selects.
-            if (!SEQ || r < rows) {
+            // the gated sweep holds 107 with it, 128 with the selects, but at width 3 117-122 with the selects and up to 130
+            // (fp16: four waves hold 128) with the branch.
+            if (!SEQ || W == 3 || r < rows) {
 #pragma unroll
-                for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], FULL || SEQ || r < rows ? xv[(4 - W) + k][e] : 0.0f, dw[e][k]);
+                for (int k = 0; k < W - 1; ++k) dw[e][k] = fmaf(dz[e], FULL || (SEQ && W != 3) || r < rows ? xv[(4 - W) + k][e] : 0.0f, dw[e][k]);
                 dw[e][W - 1] = fmaf(dz[e], xw[3][e], dw[e][W - 1]);
             }
             dbs[e] += dz[e];
@@ -522,8 +523,19 @@ __global__ __launch_bounds__(256, ACT ? 4 : 1) void canon_bwd_blc_kernel(const B
     constexpr int R = kBwdSlab, NW = kBwdWaves;
     // which instances take whole slabs through a sweep without branches, and request their first tile ahead of the staged
     // mask and indices (both below): the others hold 82-95 registers and lose a wave per SIMD, or time, to it (ANY with a mask
-    // and SiLU, B 8, C 961, L 1021: 24.1 us with its first tile ahead of the mask, 23.3 behind it)
-    constexpr bool kStraight = !STATES && (ACT || !(MASK || SEQ)), kAllAtOnce = !(ANY && MASK) && (ACT || !(MASK || SEQ));
+    // and SiLU, B 8, C 961, L 1021: 24.1 us with its first tile ahead of the mask, 23.3 behind it).
+    // kTight: fp16 with SiLU at widths 3 and 4.  Its conversions keep more values alive: with both it spilled 20 registers,
+    // 49 with a mask, 62-67 packed, at the 128 that four waves leave it.  With the residual's branch in the sweep's rows
+    // (which is what ends each row's live values) and the first tile behind the mask it holds 98-121; us a call before both /
+    // with both as they are elsewhere / so: B 8, C 640, L 1024 15.3 / 20.6 / 13.8, with a mask 17.3 / 29.8 / 15.0; B 8, C 3456
+    // 41.3 / 73.8 / 40.1, with a mask 44.9 / 118 / 42.4; B 32 134 / 252 / 131, with a mask 145 / 439 / 140; packed B 2,
+    // C 3456, L 8192 75 / 161 / 72.3, with a mask 83.5 / 165 / 77.0.  (Ordinary sweeps instead: 43.1 at B 8, masked.)
+    // Packed rows with a mask keep the branch in every type: bf16 held 128 and spilled one, now 109: 78.0 -> 77.2 (81.9 before
+    // the straight sweep).
+    constexpr bool kTight = ACT && !ANY && W > 2 && DT == CANON_DTYPE_F16;
+    constexpr bool kStraight = !STATES && (ACT || !(MASK || SEQ));
+    constexpr bool kAllAtOnce = !(ANY && MASK) && !kTight && (ACT || !(MASK || SEQ));
+    constexpr bool kResBranch = kTight || (SEQ && MASK);
     // With an activation: tailx / headdz, two barriers per tile (dz of a slab's head needs the previous
     // wave's tail first).  Without one dz IS dout, so the head is handed over as raw rows (headg) together
     // with the tail, one barrier per tile, both double-buffered (a fast wave publishes the next tile while
@@ -722,7 +734,8 @@ __global__ __launch_bounds__(256, ACT ? 4 : 1) void canon_bwd_blc_kernel(const B
         if constexpr (MASK) {
             const uint32_t first = ((uint32_t)it * NW + wv) * R;   // index of step t0 - 3 in smask
             const uint32_t m_lane = f_bits(smask[first + (uint32_t)(lane < R + 2 ? lane : R + 2)]);
-            plain_mask = __builtin_amdgcn_ballot_w64(m_lane != kMaskOne) == 0;
+            // (kTight with states, at its 128 registers, looks at every row of the slab by itself: one spilled with this flag)
+            plain_mask = !(STATES && kTight) && __builtin_amdgcn_ballot_w64(m_lane != kMaskOne) == 0;
 #pragma unroll
             for (int j = 0; j < R + 3; ++j) mm[j] = (uint32_t)__builtin_amdgcn_readlane((int)m_lane, j);
         }
@@ -862,12 +875,12 @@ __global__ __launch_bounds__(256, ACT ? 4 : 1) void canon_bwd_blc_kernel(const B
             // packed rows with SiLU B 2, L 8192 72.5 -> 69.6, B 1, L 4000 25.7 -> 24.2; fp32 B 24, C 2848, L 385 70.6 -> 66.9;
             // (up to 128 registers with SiLU, four waves per SIMD; held to 96 and five it spills: 43-198 us in place of 38-134)
             if (kStraight && rows == R && plain_mask) {
-                if (a.res_mode != CANON_RESIDUAL_NONE)
+                if (!kResBranch && a.res_mode != CANON_RESIDUAL_NONE)
                     bwd_sweep<DT, W, false, ACT, true, false, R, E, false, ANY, 1>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff,
                                                                                    ds32, rows, nullptr, 0, nullptr, dany);
                 else
-                    bwd_sweep<DT, W, false, ACT, true, false, R, E, false, ANY, 0>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff,
-                                                                                   ds32, rows, nullptr, 0, nullptr, dany);
+                    bwd_sweep<DT, W, false, ACT, true, false, R, E, false, ANY, kResBranch ? -1 : 0>(
+                        a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32, rows, nullptr, 0, nullptr, dany);
             } else if (rows == R) {
                 bwd_sweep<DT, W, MASK, ACT, true, false, R, E, false, ANY>(a, w, bias, X, H, G, mm, dzh, dzf, dw, dbs, rd, voff, ds32,
                                                                            rows, nullptr, 0, nullptr, dany);
