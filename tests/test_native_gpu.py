@@ -301,6 +301,69 @@ def test_training_call(cc, monkeypatch, layout):
             assert got.split(":")[0] == want.split(":")[0], (call.__name__, got, want)
 
 
+@pytest.mark.parametrize("activation", [None, "silu"])
+def test_a_graph_of_the_backward(cc, monkeypatch, activation):
+    """create_graph=True: the gradients themselves are as without, and a loss that differentiates one of them again is refused,
+    also where another term of it has a gradient of its own; one that does not depend on the variable asked for is not."""
+    g = torch.Generator(device=DEV).manual_seed(6)
+    B, C, L, S = 2, 24, 40, 4
+    x0, t0 = torch.randn(B, C, L, device=DEV, generator=g), torch.randn(B, C, device=DEV, generator=g)
+    w0, b0 = torch.randn(C, 4, device=DEV, generator=g), torch.randn(C, device=DEV, generator=g)
+    s0 = torch.randn(B, C, S, device=DEV, generator=g)
+
+    def fn(x, w, b, s):
+        return [cc.causal_conv1d_fn(x, w, b, activation=activation)]
+
+    def packed(x, w, b, s):
+        return [cc.causal_conv1d_fn(x, w, b, torch.zeros(B, L, dtype=torch.int32, device=DEV), activation=activation)]
+
+    def states(x, w, b, s):
+        return cc.causal_conv1d_fn(x, w, b, initial_states=s, final_states_out=torch.empty(B, C, S, device=DEV), activation=activation)
+
+    def parts(x, w, b, s):
+        ys, fin = cc.causal_conv1d_fn_parts(x.split([8, 16], 1), w, b, initial_states=s, activation=activation,
+                                            final_states_out=torch.empty(B, C, S, device=DEV))
+        return [*ys, fin]
+
+    def update(x, w, b, s):
+        s = s * 1
+        return [cc.causal_conv1d_update(x[..., 0], s, w, b, activation), s]
+
+    def update_parts(x, w, b, s):
+        s = s * 1
+        return [*cc.causal_conv1d_update_parts(x[..., 0].split([8, 16], 1), s, w, b, activation), s]
+
+    for call in (fn, packed, states, parts, update, update_parts):
+        n = 3 if call in (fn, packed) else 4
+
+        def leaves():
+            return [t.clone().requires_grad_() for t in (x0, w0, b0, s0)]
+
+        def first(create_graph):
+            t = leaves()
+            loss = sum(y.square().sum() for y in call(*t))
+            return torch.autograd.grad(loss, t[:n], create_graph=create_graph)
+        for plain, again in zip(both(cc, monkeypatch, lambda: first(False)), both(cc, monkeypatch, lambda: first(True))):
+            assert_same([v.detach() for v in again], list(plain), call.__name__)
+
+        # the gradient of a linear loss in variable i, squared, beside a term of its own: its derivative in variable j
+        for i in range(n):
+            for j in range(n):
+                def mixed(second=True):
+                    t = leaves()
+                    y = call(*t)
+                    gi, = torch.autograd.grad(sum(v.sum() for v in y), t[i], create_graph=True)
+                    loss = sum(v.square().sum() for v in t) + (gi.square().sum() if second else 0)
+                    return torch.autograd.grad(loss, t[j])
+                # without an activation y is bilinear: dx and the state's gradient depend on the taps, the taps' on x and state
+                depends = activation is not None or (i in (0, 3) and j == 1) or (i == 1 and j in (0, 3))
+                for got in both(cc, monkeypatch, mixed):
+                    if depends:
+                        assert isinstance(got, str) and "its gradients cannot be differentiated" in got, (call.__name__, i, j, got)
+                    else:
+                        assert_same(got, mixed(second=False), (call.__name__, i, j))
+
+
 def test_blocks_of_the_layer(cc, monkeypatch):
     """CanonLayer's block call: one tensor and parts, with and without a cache, a continued state, masks, x that is not
     dense; outputs, their strides and the cached states as through the functions."""

@@ -310,7 +310,7 @@ def causal_conv1d_fn(
         return result, final_states
     if _wants_grad(x, weight, bias, initial_states):
         result = _CanonConvFn.apply(x, weight, bias, attention_mask, final_states, act, res, rnd, seq_idx,
-                                    initial_states)
+                                    initial_states, _origin(initial_states))
     else:
         result = _launch_fwd(x, weight, bias, attention_mask, initial_states, final_states, act, res, rnd, seq_idx)
         if final_states is not None:
@@ -337,6 +337,38 @@ def _wants_grad(*tensors) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
+class _Final(torch.autograd.Function):
+    """Hands a gradient on; a walk that comes back through it to one of ``sources`` ends in an error."""
+
+    @staticmethod
+    def forward(ctx, grad, *sources):
+        return grad.view_as(grad)
+
+    @staticmethod
+    def backward(ctx, *_):
+        raise RuntimeError(_SECOND_ORDER)
+
+
+# (canon_native.cpp's node says the same)
+_SECOND_ORDER = "causal_conv1d: the backward is a fused kernel without a derivative of its own: its gradients cannot be differentiated"
+
+
+def _final(act, by_linear, everything, *grads):
+    """The gradients of a backward for its caller.  Where a graph of the backward was asked for (``create_graph=True``) they
+    depend on tensors the kernel read, and that graph ends here: without a node that says so, a loss made of such a
+    gradient and of something else would lose the gradient's share without a word.  Without an activation the backward
+    is linear: ``by_linear`` then holds, per gradient, the tensors it depends on (with one, on ``everything``)."""
+    if not torch.is_grad_enabled():
+        return grads
+    return tuple(None if g is None else _Final.apply(g, *(t for t in (everything if act else of) if t is not None))
+                 for g, of in zip(grads, by_linear, strict=True))
+
+
+def _origin(state: Optional[torch.Tensor]):
+    """An empty tensor with ``state``'s place in the graph (in a list: no input of the node), for nodes that keep a copy."""
+    return [state[:0].clone()] if state is not None and state.requires_grad else []
+
+
 class _CanonConvFn(torch.autograd.Function):
     """Autograd node of the prefill: forward and backward are one fused launch each
     (the backward recomputes the pre-activation from x, nothing but the inputs is saved).
@@ -344,13 +376,14 @@ class _CanonConvFn(torch.autograd.Function):
     (causal_conv1d_mps/autograd.py:13-160, 162-338)."""
 
     @staticmethod
-    def forward(ctx, x, weight, bias, mask, final_states, act, res, rnd, seq_idx=None, initial_states=None):
+    def forward(ctx, x, weight, bias, mask, final_states, act, res, rnd, seq_idx=None, initial_states=None, origin=()):
         out = _launch_fwd(x, weight, bias, mask, initial_states, final_states, act, res, rnd, seq_idx)
         # a copy of the (small) initial state: callers keep it in a cache tensor they overwrite right after
         # the call (CanonLayer copies the new state into it, decode steps shift it in place)
         ctx.save_for_backward(x, weight, bias, mask, seq_idx,
                               initial_states.detach().clone() if initial_states is not None else None)
         ctx.flags = (act, res)
+        ctx.origin = origin
         ctx.set_materialize_grads(False)
         if final_states is not None:
             # filled in place and differentiable: a gradient that arrives through the captured state (the next
@@ -372,7 +405,9 @@ class _CanonConvFn(torch.autograd.Function):
         if initial_states is not None and ctx.needs_input_grad[9]:
             dinit = torch.empty_like(initial_states)
         dx = _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx, initial_states, dinit, dfinal)
-        return dx, dweight, dbias, None, None, None, None, None, None, dinit
+        dx, dweight, dbias, dinit = _final(act, ((dout, dfinal, weight), (dout, x, *ctx.origin), (dout,), (dout, dfinal, weight)),
+                                           (dout, dfinal, x, weight, bias, *ctx.origin), dx, dweight, dbias, dinit)
+        return dx, dweight, dbias, None, None, None, None, None, None, dinit, None
 
 
 def _launch_bwd(x, dout, weight, bias, mask, dweight, dbias, act, res, seq_idx=None, initial_states=None,
@@ -579,7 +614,7 @@ def causal_conv1d_update(
         conv_state.copy_(new_state)
     elif wants_grad:
         out, _ = _CanonUpdateFn.apply(x2, conv_state, weight, bias, token_mask, act, res, cache_seqlens, conv_state_indices,
-                                      rnd)
+                                      rnd, _origin(conv_state))
     elif torch.compiler.is_compiling():
         out = torch.ops.canon_conv1d.update(x2, conv_state, weight, bias, token_mask, cache_seqlens, conv_state_indices,
                                             act, res, rnd)
@@ -660,13 +695,14 @@ class _CanonUpdateFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x2, conv_state, weight, bias, token_mask, act, res, cache_seqlens=None, conv_state_indices=None,
-                rnd=0):
+                rnd=0, origin=()):
         before = conv_state.detach().clone()
         out = _launch_update(x2, conv_state, weight, bias, token_mask, cache_seqlens, conv_state_indices, act, res, rnd)
         ctx.mark_dirty(conv_state)
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(x2, before, weight, bias, token_mask, cache_seqlens, conv_state_indices)
         ctx.flags = (act, res)
+        ctx.origin = origin
         return out, conv_state
 
     @staticmethod
@@ -679,8 +715,11 @@ class _CanonUpdateFn(torch.autograd.Function):
         want_params = ctx.needs_input_grad[2] or (bias is not None and ctx.needs_input_grad[3])
         dx, dstate, dweight, dbias = _launch_update_bwd(x2, before, weight, bias, token_mask, dout, dstate_out, act, res,
                                                         want_state, want_params, cache_seqlens, conv_state_indices)
-        return (dx, dstate, dweight.to(weight.dtype) if dweight is not None else None,
-                dbias.to(bias.dtype) if dbias is not None else None, None, None, None, None, None, None)
+        dx, dstate, dweight, dbias = _final(
+            act, ((dout, dstate_out, weight), (dout, dstate_out, weight), (dout, x2, *ctx.origin), (dout,)),
+            (dout, dstate_out, x2, weight, bias, *ctx.origin), dx, dstate,
+            dweight.to(weight.dtype) if dweight is not None else None, dbias.to(bias.dtype) if dbias is not None else None)
+        return dx, dstate, dweight, dbias, None, None, None, None, None, None, None
 
 
 def _launch_update_bwd(x2, before, weight, bias, token_mask, dout, dstate_out, act, res, want_state=True,
@@ -843,7 +882,8 @@ def causal_conv1d_fn_parts(
         if final_states is not None:
             final_states.copy_(fin)
     elif wants_grad:
-        result = _CanonConvPartsFn.apply(weight, bias, attention_mask, final_states, act, res, rnd, initial_states, *xs)
+        result = _CanonConvPartsFn.apply(weight, bias, attention_mask, final_states, act, res, rnd, initial_states,
+                                         _origin(initial_states), *xs)
         outs = tuple(result[:len(xs)])
     else:
         outs = _launch_fwd_parts(xs, weight, bias, attention_mask, initial_states, final_states, act, res, rnd)
@@ -870,12 +910,13 @@ class _CanonConvPartsFn(torch.autograd.Function):
     differentiable (a gradient arriving through it flows back into the inputs) and so is the initial state."""
 
     @staticmethod
-    def forward(ctx, weight, bias, mask, final_states, act, res, rnd, initial_states, *xs):
+    def forward(ctx, weight, bias, mask, final_states, act, res, rnd, initial_states, origin, *xs):
         outs = _launch_fwd_parts(xs, weight, bias, mask, initial_states, final_states, act, res, rnd)
         # (a copy of the small initial state: callers keep it in a cache tensor they overwrite right after the call)
         ctx.save_for_backward(weight, bias, mask, initial_states.detach().clone() if initial_states is not None else None,
                               *xs)
         ctx.flags = (act, res, final_states is not None)
+        ctx.origin = origin
         ctx.set_materialize_grads(False)
         if final_states is not None:
             ctx.mark_dirty(final_states)
@@ -906,7 +947,10 @@ class _CanonConvPartsFn(torch.autograd.Function):
                                    dinit[:, c0:c1] if dinit is not None else None,
                                    dfinal[:, c0:c1] if dfinal is not None else None))
             c0 = c1
-        return dweight, dbias, None, None, None, None, None, dinit, *dxs
+        dweight, dbias, dinit, *dxs = _final(
+            act, ((*douts, *xs, *ctx.origin), douts, (*grads, weight), *((*grads, weight) for _ in xs)),
+            (*grads, *xs, weight, bias, *ctx.origin), dweight, dbias, dinit, *dxs)
+        return dweight, dbias, None, None, None, None, None, dinit, None, *dxs
 
 
 def causal_conv1d_update_parts(
@@ -959,7 +1003,8 @@ def causal_conv1d_update_parts(
     if torch.compiler.is_compiling():
         return tuple(torch.ops.canon_conv1d.update_parts(xs, conv_state, weight, bias, token_mask, act, res, rnd))
     if wants_grad:
-        return tuple(_CanonUpdatePartsFn.apply(conv_state, weight, bias, token_mask, act, res, rnd, *xs)[:len(xs)])
+        return tuple(_CanonUpdatePartsFn.apply(conv_state, weight, bias, token_mask, act, res, rnd, _origin(conv_state),
+                                               *xs)[:len(xs)])
     return _launch_update_parts(xs, conv_state, weight, bias, token_mask, act, res, rnd)
 
 
@@ -969,13 +1014,14 @@ class _CanonUpdatePartsFn(torch.autograd.Function):
     rows of weight / bias.  The state is modified in place and differentiable, as in ``_CanonUpdateFn``."""
 
     @staticmethod
-    def forward(ctx, conv_state, weight, bias, token_mask, act, res, rnd, *xs):
+    def forward(ctx, conv_state, weight, bias, token_mask, act, res, rnd, origin, *xs):
         before = conv_state.detach().clone()
         outs = _launch_update_parts(xs, conv_state, weight, bias, token_mask, act, res, rnd)
         ctx.mark_dirty(conv_state)
         ctx.set_materialize_grads(False)
         ctx.save_for_backward(before, weight, bias, token_mask, *xs)
         ctx.flags = (act, res)
+        ctx.origin = origin
         return (*outs, conv_state)
 
     @staticmethod
@@ -1002,7 +1048,10 @@ class _CanonUpdatePartsFn(torch.autograd.Function):
             c0 = c1
         dweight = torch.cat(dws, dim=0).to(weight.dtype) if want_params else None
         dbias = torch.cat(dbs, dim=0).to(bias.dtype) if want_params and bias is not None else None
-        return (dstate, dweight, dbias, None, None, None, None, *dxs)
+        dstate, dweight, dbias, *dxs = _final(
+            act, ((*grads, weight), (*douts, *xs, *ctx.origin), douts, *((*grads, weight) for _ in xs)),
+            (*grads, *xs, weight, bias, *ctx.origin), dstate, dweight, dbias, *dxs)
+        return (dstate, dweight, dbias, None, None, None, None, None, *dxs)
 
 
 def _launch_update_parts(xs, conv_state, weight, bias, token_mask, act, res, rnd):

@@ -20,6 +20,8 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/version.h>
@@ -227,6 +229,20 @@ int run_fwd(const Tensor &x, const Tensor &weight, const Tensor *bias, const Ten
     C10_THROW_ERROR(Error, message);
 }
 
+// A gradient for a caller that asked for a graph of the backward (create_graph): it depends on `sources`, and a walk from it
+// to one of them ends in an error.  (Without a node that says so, a loss made of such a gradient and of something else would
+// lose the gradient's share without a word.  As _final in the Python nodes.)
+void refuse_second_order(const Tensor &grad, std::initializer_list<Tensor> sources)
+{
+    torch::autograd::edge_list edges;
+    for (const Tensor &t : sources)
+        if (t.defined() && t.requires_grad()) edges.push_back(torch::autograd::impl::gradient_edge(t));
+    if (!grad.defined() || edges.empty()) return;
+    torch::autograd::set_history(grad, std::make_shared<torch::autograd::Error>(
+        "causal_conv1d: the backward is a fused kernel without a derivative of its own: its gradients cannot be differentiated",
+        std::move(edges)));
+}
+
 struct CanonConv : torch::autograd::Function<CanonConv> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias,
                           const std::optional<Tensor> &mask, const std::optional<Tensor> &seq, int64_t act, int64_t res, int64_t rnd,
@@ -244,6 +260,7 @@ struct CanonConv : torch::autograd::Function<CanonConv> {
 
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, const torch::autograd::variable_list &grads)
     {
+        const bool graph_wanted = c10::GradMode::is_enabled();   // (create_graph)
         const at::NoGradGuard no_grad;
         const torch::autograd::variable_list saved = ctx->get_saved_variables();
         const Tensor &x = saved[0], &weight = saved[1];
@@ -259,6 +276,14 @@ struct CanonConv : torch::autograd::Function<CanonConv> {
                                (int)(flags >> 1), given(4), nullptr, nullptr, nullptr,
                                (void *)c10::hip::getCurrentHIPStream((c10::DeviceIndex)x.get_device()).stream(), dx);
         if (rc != CANON_OK) refuse(rc, "causal_conv1d_fn backward");
+        if (graph_wanted) {
+            // (without an activation the backward is linear in each of these)
+            const bool act = flags & 1;
+            const Tensor none;
+            refuse_second_order(dx, {grads[0], weight, act ? x : none, act ? saved[2] : none});
+            refuse_second_order(dweight, {grads[0], x, act ? weight : none, act ? saved[2] : none});
+            refuse_second_order(dbias, {grads[0], act ? x : none, act ? weight : none, act ? saved[2] : none});
+        }
         return {dx, dweight, dbias, Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
     }
 };
