@@ -194,6 +194,36 @@ def test_decode_call_of_the_wrong_rank(cc, monkeypatch):
                 assert native == f"ValueError: Expected 1D bias tensor, got {bias.dim()}D"
 
 
+def test_decode_signatures_without_the_native_module(cc, monkeypatch):
+    """Where the native module declines (another device than the current one, a module built for another torch) a decode call
+    that was checked once is launched from its argument block as well, and no other call is."""
+    x, w, b = torch.randn(2, 8, device=DEV), torch.randn(8, 4, device=DEV), torch.randn(8, device=DEV)
+    state, mask = torch.randn(2, 8, 4, device=DEV), torch.tensor([1.0, 0.5], device=DEV)
+    calls = [lambda s: cc.causal_conv1d_update(x, s, w), lambda s: cc.causal_conv1d_update(x, s, w, b, "silu", token_mask=mask, residual=True),
+             lambda s: cc.causal_conv1d_update(x.t().contiguous().t(), s, w, b, rounding="eager")]
+    monkeypatch.setattr(cc._update_tls, "known", {}, raising=False)
+    states = [[state.clone() for _ in calls] for _ in range(2)]
+    want = [[call(s) for call, s in zip(calls, row)] for row in states for _ in range(2)]
+    assert len(cc._known_updates()) == len(calls) and all(type(key) is bytes for key in cc._known_updates())   # (the module's own)
+    monkeypatch.setattr(cc._update_tls, "known", {})
+    monkeypatch.setattr(cc._lib, "native", cc._lib._OtherTorch)
+    launch, checked = cc._launch_update, []
+    monkeypatch.setattr(cc, "_launch_update", lambda *a: checked.append(1) or launch(*a))
+    again = [[state.clone() for _ in calls] for _ in range(2)]
+    got = [[call(s) for call, s in zip(calls, row)] for row in again for _ in range(2)]
+    assert_same(got, want, "outputs")
+    assert_same(again, states, "states")
+    assert len(checked) == len(calls) == len(cc._known_updates())
+    calls[0](state.half().float()[:, :, 1:])                                   # another stride of the state
+    cc.causal_conv1d_update(x[..., None], state, w)                            # another rank of x
+    with torch.enable_grad():
+        cc.causal_conv1d_update(x, state.clone(), w.clone().requires_grad_())  # gradients
+    assert len(checked) == len(calls) + 3
+    for bad in (lambda: cc.causal_conv1d_update(x, state, w, activation=["relu"]), lambda: cc.causal_conv1d_update(x, state, w[:7])):
+        with pytest.raises((ValueError, NotImplementedError)):
+            bad()
+
+
 def test_another_stream_and_a_captured_graph(cc):
     x = torch.randn(2, 64, 256, device=DEV).bfloat16()
     w = torch.randn(64, 4, device=DEV).bfloat16()

@@ -543,8 +543,10 @@ def causal_conv1d_update(
     """
     # A serving loop makes this call 72 times per generated token with the same shapes, strides, types and flags:
     # such a call, once it has passed every check below, is recognised by that signature (bytes that the native module
-    # forms) and launched from a prepared argument block with only the addresses filled in.
+    # forms) and launched from a prepared argument block with only the addresses filled in.  Where the module declines (x on
+    # another device than the current one, a module built for another torch) the same is done here (``_known_update``).
     key = None
+    declined = False
     if cache_seqlens is None and conv_state_indices is None:
         if not torch.compiler.is_compiling() and x.is_cuda:
             out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, None, None, token_mask, residual,
@@ -555,6 +557,8 @@ def causal_conv1d_update(
                 if type(out) is int:
                     _lib.check(out, "causal_conv1d_update")
                 return out
+            else:
+                declined = True
     elif not torch.compiler.is_compiling() and x.is_cuda:
         out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices,
                                              token_mask, residual, rounding)
@@ -565,6 +569,10 @@ def causal_conv1d_update(
     act = _activation_flag(activation)
     res = _residual_mode(residual)
     rnd = _round_mode(rounding)
+    if declined and not _wants_grad(x, weight, bias, conv_state, token_mask):
+        key, out = _known_update(x, conv_state, weight, bias, token_mask, act, res, rnd)
+        if out is not None:
+            return out
     squeeze_back = False
     if x.dim() == 3:
         if x.shape[2] != 1:
@@ -657,7 +665,25 @@ def _known_updates() -> dict:
         return _update_tls.known
 
 
-def _remember_update(key: bytes, block: bytes) -> None:
+def _known_update(x, conv_state, weight, bias, token_mask, act, res, rnd):
+    """The signature of a plain decode call, and the output where its argument block is known (then it is launched)."""
+    tensors = (x, conv_state, weight, bias, token_mask)
+    key = (act, res, rnd, *(None if t is None else (t.shape, t.stride(), t.dtype, t.device) for t in tensors))
+    block = _known_updates().get(key)
+    if block is None:
+        return key, None
+    p = UpdateParams.from_buffer_copy(block)
+    out = torch.empty(x.shape, dtype=x.dtype, device=x.device)
+    p.x, p.out, p.conv_state, p.weight = x.data_ptr(), out.data_ptr(), conv_state.data_ptr(), weight.data_ptr()
+    p.bias = bias.data_ptr() if bias is not None else None
+    p.token_mask = token_mask.data_ptr() if token_mask is not None else None
+    rc = _call(_lib.lib().canon_conv1d_update, x.device, ctypes.byref(p))
+    if rc:
+        _lib.check(rc, "causal_conv1d_update")
+    return key, out
+
+
+def _remember_update(key, block: bytes) -> None:
     """Keep at most _KNOWN_UPDATES_MAX signatures per thread: the oldest one makes room (a model has a handful of
     distinct decode calls; a program that keeps producing new ones must not lose the fast path for good)."""
     known = _known_updates()
