@@ -388,25 +388,33 @@ int canon_conv1d_bwd_static(const canon_conv1d_bwd_params *p, void *stream);
 
 /* Scratch bytes canon_conv1d_bwd works with for these sizes, strides and pointer
  * alignments (less is accepted where fewer partial sets can be cut: a set per sequence and chunk is 20 bytes per
- * channel, a chunk of the channel-contiguous kernel 64 to 128 time steps (32 to 64 in fp32) where there is room, up to 1024 where not); with x, dout or dx missing (NULL) the figure also covers the
- * kernel a misaligned pointer would select.  Negative if the arguments are
- * rejected. */
+ * channel, a chunk of the channel-contiguous kernel 64 to 128 time steps (32 to 64 in fp32) where there is room, up to
+ * 1024 where not); with x, dout or dx missing (NULL) the figure also covers the kernel a misaligned pointer would
+ * select.  Negative if the arguments are rejected. */
 int64_t canon_conv1d_bwd_workspace_bytes(const canon_conv1d_bwd_params *p);
 int64_t canon_conv1d_update_bwd_workspace_bytes(const canon_conv1d_update_bwd_params *p);
 
 /*
- * Name of the kernel family the call above would launch for these arguments
- * ("bcl_vec", "bcl_vec_short", "blc_vec", "blc_vec_seq", "generic", "update_vec", "update_generic"), or NULL
+ * Name of the kernel family the call above would launch for these arguments, or NULL
  * if the arguments are rejected.  Launches nothing.  Lets a caller or a test
- * assert that a layout takes the fast path.
+ * assert that a layout takes the fast path.  Prefill:
+ *   "bcl_vec"               time-contiguous rows of more than 32 vectors of 16 bytes
+ *   "bcl_vec_short"         ... of 1 to 32 whole vectors on 16-byte boundaries, several rows to a wave
+ *   "bcl_vec_short_ragged"  ... of any length from one vector on up to 32, at their elements' alignment
+ *   "blc_vec"               channel-contiguous rows on the 8-byte grid ("blc_vec_seq" with seq_idx)
+ *   "blc_vec_any"           ... off that grid: a channel count, a stride or an address that is no multiple of 8 bytes
+ *   "generic"               the strided kernel
+ * Decode: "update_vec", "update_generic".
  */
 const char *canon_conv1d_fwd_plan(const canon_conv1d_fwd_params *p);
 /* Waves per block of that launch (time-contiguous rows: 8 in unmasked launches of at least 16384 waves, 1 with a
  * mask, else 4; 4 for the other vector kernels and the strided one), 0 for an empty problem, -1 if rejected. */
 int canon_conv1d_fwd_plan_waves(const canon_conv1d_fwd_params *p);
 const char *canon_conv1d_update_plan(const canon_conv1d_update_params *p);
-/* "bwd_blc_vec" | "bwd_blc_vec_seq" | "bwd_bcl_vec" | "bwd_bcl_vec_ragged" | "bwd_generic": with a workspace given the
- * kernel that runs in that many bytes, without one the kernel that runs where there is room for its partial sets */
+/* "bwd_blc_vec" | "bwd_blc_vec_seq" | "bwd_blc_vec_any" (off the 8-byte grid) | "bwd_bcl_vec_short" (time-contiguous rows of
+ * 1 to 32 vectors) | "bwd_bcl_vec" | "bwd_bcl_vec_ragged" (longer ones, on 16-byte boundaries or not) | "bwd_generic" (the
+ * walk kernel): with a workspace given the kernel that runs in that many bytes, without one the kernel that runs where
+ * there is room for its partial sets */
 const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p);
 /* "blc_vec_pair" (two dense tensors of one shape: one launch of the single-tensor code), "blc_vec_parts" /
  * "update_vec_parts" (one launch over a table of parts) or "per_part" (one launch per part) */

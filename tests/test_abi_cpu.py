@@ -121,29 +121,38 @@ def test_fwd_plan_picks_the_vector_kernels_for_dense_layouts():
     # as long as x and out share their strides
     assert plan(fwd_params(L=1023)) == "bcl_vec"
     assert plan(fwd_params(L=1023, out_stride_c=1024, out_stride_b=3456 * 1024)) == "generic"
-    # ragged channel counts, misaligned base pointers -> strided kernel
-    assert plan(fwd_params(C=3457, layout="blc")) == "generic"
+    # ragged channel counts -> the tiles at the elements' own alignment, long rows on misaligned base pointers -> strided kernel
+    assert plan(fwd_params(C=3457, layout="blc")) == "blc_vec_any"
+    assert plan(fwd_params(C=3, layout="blc")) == "generic"                # ... less than a lane's channels
+    assert plan(fwd_params(layout="blc", x=FAKE_X + 2)) == "blc_vec_any"
+    assert plan(fwd_params(layout="blc", x=FAKE_X + 1)) == "generic"       # ... not even on an element
     assert plan(fwd_params(x=FAKE_X + 2)) == "generic"
     # the channel-contiguous kernel takes the tap addresses (48 bits each), the batch stride in lane vectors (32 bits)
-    # and the number of channel tiles (16 bits) among its leading scalar arguments: beyond those, the strided kernel
-    assert plan(fwd_params(layout="blc", weight=FAKE_W | 1 << 48)) == "generic"
+    # and the number of channel tiles (16 bits) among its leading scalar arguments: beyond those, the tiles that read their
+    # arguments the ordinary way
+    assert plan(fwd_params(layout="blc", weight=FAKE_W | 1 << 48)) == "blc_vec_any"
     assert plan(fwd_params(layout="blc", bias=FAKE_W + 4096)) == "blc_vec"
-    assert plan(fwd_params(layout="blc", bias=1 << 50)) == "generic"
+    assert plan(fwd_params(layout="blc", bias=1 << 50)) == "blc_vec_any"
     assert plan(fwd_params(B=1, C=65535 * 256, L=8, layout="blc")) == "blc_vec"
-    assert plan(fwd_params(B=1, C=65536 * 256, L=8, layout="blc")) == "generic"
-    assert plan(fwd_params(B=2, C=8, L=8, layout="blc", x_stride_b=4 << 32, out_stride_b=4 << 32)) == "generic"
+    assert plan(fwd_params(B=1, C=65536 * 256, L=8, layout="blc")) == "blc_vec_any"
+    assert plan(fwd_params(B=2, C=8, L=8, layout="blc", x_stride_b=4 << 32, out_stride_b=4 << 32)) == "blc_vec_any"
+    # neither dimension contiguous: the strided kernel
+    assert plan(fwd_params(layout="blc", x_stride_c=2, x_stride_l=2 * 3456, x_stride_b=2 * 3456 * 1024)) == "generic"
+    assert plan(fwd_params(layout="blc", out_stride_c=2, out_stride_l=2 * 3456, out_stride_b=2 * 3456 * 1024)) == "generic"
     # the eager module's rounding points are register arithmetic: the same kernels
     assert plan(fwd_params(round_mode=1)) == "bcl_vec"
     assert plan(fwd_params(round_mode=1, layout="blc")) == "blc_vec"
-    # rows too short for a wave of their own: several rows per wave, as long as they are whole aligned vectors
+    # rows too short for a wave of their own: several rows per wave, whole aligned vectors or not
     assert plan(fwd_params(L=64)) == "bcl_vec_short"
     assert plan(fwd_params(L=8)) == "bcl_vec_short"
     assert plan(fwd_params(L=120)) == "bcl_vec_short"
     assert plan(fwd_params(L=128)) == "bcl_vec_short" and plan(fwd_params(L=256)) == "bcl_vec_short"
     assert plan(fwd_params(L=264)) == "bcl_vec"
-    assert plan(fwd_params(L=255)) == "bcl_vec"                            # ... not whole vectors, but long enough
-    assert plan(fwd_params(L=60)) == "generic"                             # ... not whole vectors
-    assert plan(fwd_params(L=4)) == "generic"
+    assert plan(fwd_params(L=257)) == "bcl_vec"
+    assert plan(fwd_params(L=255)) == "bcl_vec_short_ragged"               # ... not whole vectors
+    assert plan(fwd_params(L=60)) == "bcl_vec_short_ragged" and plan(fwd_params(L=9)) == "bcl_vec_short_ragged"
+    assert plan(fwd_params(L=64, x=FAKE_X + 2)) == "bcl_vec_short_ragged"  # ... not aligned
+    assert plan(fwd_params(L=7)) == "generic" and plan(fwd_params(L=4)) == "generic"      # ... not even one vector
     assert plan(fwd_params(L=64, round_mode=1)) == "bcl_vec_short"
     # strided but aligned rows (a channel slice of a bigger tensor) stay vectorised
     assert plan(fwd_params(C=128, x_stride_b=4096 * 1024, x_stride_c=1024)) == "bcl_vec"
@@ -374,17 +383,24 @@ def test_bwd_plan_and_workspace():
     ws = L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(p))
     assert 0 < ws <= 20 << 20 and ws % (3456 * 5 * 4) == 0        # whole partial sets, bounded scratch
     assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl"))) == b"bwd_bcl_vec"
-    # time-contiguous rows off the 16-byte vectors: the row kernel's ragged variant from 40 steps on, the walk kernel below
-    for length, want in ((1023, b"bwd_bcl_vec_ragged"), (1024, b"bwd_bcl_vec"), (41, b"bwd_bcl_vec_ragged"),
-                         (40, b"bwd_bcl_vec_ragged"), (39, b"bwd_generic"), (32, b"bwd_generic"), (128, b"bwd_bcl_vec"),
-                         (127, b"bwd_bcl_vec_ragged"), (120, b"bwd_bcl_vec_ragged")):
+    # time-contiguous rows of up to 32 vectors share waves, longer ones off the 16-byte vectors take the row kernel's ragged
+    # variant, rows below one vector the walk kernel
+    for length, want in ((1023, b"bwd_bcl_vec_ragged"), (1024, b"bwd_bcl_vec"), (257, b"bwd_bcl_vec_ragged"), (264, b"bwd_bcl_vec"),
+                         (256, b"bwd_bcl_vec_short"), (255, b"bwd_bcl_vec_short"), (39, b"bwd_bcl_vec_short"),
+                         (8, b"bwd_bcl_vec_short"), (7, b"bwd_generic")):
         assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl", L=length))) == want, length
-    assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(C=3457))) == b"bwd_generic"
+    # off the 8-byte grid: the tiles at the elements' own alignment, at width 4 from 12 steps on; else the walk kernel
+    for over, want in ((dict(C=3457), b"bwd_blc_vec_any"), (dict(C=3457, L=12), b"bwd_blc_vec_any"), (dict(C=3457, L=11), b"bwd_generic"),
+                       (dict(C=3457, width=3), b"bwd_generic"), (dict(x=FAKE_X + 2), b"bwd_blc_vec_any"), (dict(x=FAKE_X + 1), b"bwd_generic"),
+                       (dict(C=3457, dfinal_state=FAKE_X + 0x900000, final_len=4), b"bwd_generic")):
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(**over))) == want, over
+    # neither dimension contiguous: the walk kernel
+    assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(x_stride_c=2, x_stride_l=6912, x_stride_b=6912 * 1024))) == b"bwd_generic"
     # channel-contiguous: one row for every step (a stride of zero) is a layout like any other; rows further apart than a
-    # buffer resource reaches, or in falling order, take the walk kernel
+    # buffer resource reaches, or in falling order, are addressed by 64-bit pointers
     for over, want in ((dict(x_stride_l=0), b"bwd_blc_vec"), (dict(dout_stride_l=0), b"bwd_blc_vec"),
-                       (dict(x_stride_l=0, dout_stride_l=0), b"bwd_blc_vec"), (dict(x_stride_l=-3456), b"bwd_generic"),
-                       (dict(dout_stride_l=1 << 27), b"bwd_generic"), (dict(dx_stride_l=1 << 26), b"bwd_blc_vec")):
+                       (dict(x_stride_l=0, dout_stride_l=0), b"bwd_blc_vec"), (dict(x_stride_l=-3456), b"bwd_blc_vec_any"),
+                       (dict(dout_stride_l=1 << 27), b"bwd_blc_vec_any"), (dict(dx_stride_l=1 << 26), b"bwd_blc_vec")):
         assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(**over))) == want, over
     # packed sequences: the channel-contiguous kernel gates taps by sequence index, time-contiguous rows go to the walk kernel
     for layout, over, want in (("blc", {}, b"bwd_blc_vec_seq"), ("blc", dict(C=3457), b"bwd_generic"), ("bcl", {}, b"bwd_generic"),
@@ -461,9 +477,9 @@ def test_bwd_workspace_query_covers_misaligned_pointers():
         q = bwd_params(layout="bcl", **over)
         assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == b"bwd_generic"
         assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q)) == _demanded_workspace(q), over
-    for over in (dict(x=FAKE_X + 4), dict(dx=FAKE_STATE + 2)):          # channel-contiguous: 8-byte boundaries
+    for over in (dict(x=FAKE_X + 4), dict(dx=FAKE_STATE + 2)):          # channel-contiguous: off the 8-byte boundaries
         q = bwd_params(**over)
-        assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == b"bwd_generic"
+        assert L.canon_conv1d_bwd_plan(ctypes.byref(q)) == b"bwd_blc_vec_any"
         assert L.canon_conv1d_bwd_workspace_bytes(ctypes.byref(q)) == _demanded_workspace(q), over
     # sizes asked for before the tensors exist (NULL pointers): enough for whichever kernel the call will take
     for layout in ("bcl", "blc"):

@@ -470,8 +470,8 @@ def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
                 xg = buf[offset:].view(B, C, L + 1)[..., :L]
             xg = xg.detach().requires_grad_()
             # (a slice of longer rows is no dense tensor: dout and dx are rows of their own length, which may be whole vectors)
-            assert plan_of(xg, W) == ("bwd_generic" if L < 40 else
-                                      "bwd_bcl_vec" if L % E == 0 and L >= 16 * E and not offset else "bwd_bcl_vec_ragged")
+            assert plan_of(xg, W) == ("bwd_generic" if L < E else "bwd_bcl_vec_short" if L <= 32 * E else
+                                      "bwd_bcl_vec" if L % E == 0 and not offset else "bwd_bcl_vec_ragged")
             wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
             out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
             grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))
@@ -504,7 +504,8 @@ def dweight_of(x, dout, W, seq_idx=None):
 @pytest.mark.parametrize("route,B,C,L", [
     ("bcl", 2, 6, 45), ("bcl", 2, 6, 1021), ("bcl", 3, 1030, 1021),        # rows that end inside a vector, 1 and 2 vectors a lane
     ("bcl", 2, 6, 40), ("bcl", 2, 6, 136), ("bcl", 2, 6, 520), ("bcl", 2, 1030, 1536), ("bcl", 2, 6, 1024),   # idle lanes, none
-    ("bcl", 2, 6, 23), ("blc", 2, 7, 45),                                  # the walk kernel
+    ("bcl", 2, 6, 23), ("blc", 2, 7, 45), ("blc", 2, 7, 101),              # rows that share waves, tiles off the 8-byte grid
+    ("bcl", 2, 6, 3), ("blc", 2, 7, 11), ("strided", 2, 6, 45),            # the walk kernel
     ("blc", 2, 8, 3), ("blc", 2, 24, 45), ("blc", 2, 24, 40), ("blc", 2, 24, 64), ("blc", 2, 136, 1021),   # partial and empty slabs, none
     ("packed", 2, 24, 45), ("packed", 2, 24, 40), ("packed", 2, 136, 1021), ("packed", 2, 7, 45), ("state", 2, 24, 45)])
 def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, route, B, C, L):
@@ -518,12 +519,15 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
         seq[0, L // 2:] = 1
         seq[1, L - 2:] = 1
     probe = torch.empty(B, C, L, dtype=dtype, device=DEV)
-    if route != "bcl":
+    if route == "strided":
+        probe = probe.permute(2, 1, 0).contiguous().permute(2, 1, 0)
+    elif route != "bcl":
         probe = probe.transpose(1, 2).contiguous().transpose(1, 2)
-    E = 16 // dtype.itemsize
+    E, grid = 16 // dtype.itemsize, C * dtype.itemsize % 8 == 0
     assert plan_of(probe, W, None if seq is None else seq.to(DEV)) == (
-        "bwd_generic" if (L < 40 if route == "bcl" else C * dtype.itemsize % 8) else "bwd_blc_vec_seq" if route == "packed" else
-        "bwd_blc_vec" if route != "bcl" else "bwd_bcl_vec" if L % E == 0 and L >= 16 * E else "bwd_bcl_vec_ragged")
+        "bwd_generic" if route == "strided" or (route == "bcl" and L < E) or (route == "packed" and not grid) or (route == "blc" and not grid and L < 12) else
+        ("bwd_blc_vec_seq" if route == "packed" else "bwd_blc_vec" if grid else "bwd_blc_vec_any") if route != "bcl" else
+        "bwd_bcl_vec_short" if L <= 32 * E else "bwd_bcl_vec" if L % E == 0 else "bwd_bcl_vec_ragged")
     for bad, back in ((float("inf"), 1), (float("-inf"), 2), (float("nan"), 1), (float("nan"), 3), (float("inf"), 4)):
         x = torch.randn(B, C, L, generator=g).to(dtype)
         if back <= L:
@@ -624,6 +628,8 @@ def test_backward_of_channel_contiguous_rows_off_the_8_byte_grid(cc, dtype):
         xg = wide[..., off:].transpose(1, 2)
         xg.copy_(x)
         xg = xg.detach().requires_grad_()
+        # (one channel is a time-contiguous row)
+        assert plan_of(xg, 4) == ("bwd_bcl_vec_short" if C == 1 else "bwd_generic" if L < 12 else "bwd_blc_vec_any"), (C, L)
         wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
         out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
         dg = dout.to(DEV).transpose(1, 2).contiguous().transpose(1, 2)
@@ -660,6 +666,7 @@ def test_backward_of_short_rows_of_any_length_and_alignment(cc, dtype):
         xg = buf[off:].view(B, C, L + off)[..., :L]
         xg.copy_(x)
         xg = xg.detach().requires_grad_()
+        assert plan_of(xg, W) == "bwd_bcl_vec_short", L
         wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
         out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
         grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))

@@ -222,13 +222,14 @@ def test_edge_shapes_and_strides(cc, dtype):
     xg = big.to(DEV)[1:3, 5:25, 3:280:2]
     want = co.conv1d_fwd(big[1:3, 5:25, 3:280:2], w, None, activation="silu")
     got = run_fwd(cc, xg, w, None, act="silu")
+    assert cc.kernel_plan_fwd(xg, w.to(DEV)) == "generic"
     assert_parity(got, want, exact=False, what="edge/strided view")
-    # dense but misaligned (base pointer off by one element) -> scalar kernel, same answer
+    # dense but misaligned (base pointer off by one element) -> rows at their elements' alignment, same answer
     flat = torch.randn(2 * 16 * 256 + 1, generator=g).to(dtype)
     xv = flat[1:].view(2, 16, 256)
     w = torch.randn(16, 4, generator=g).to(dtype)
     xg = flat.to(DEV)[1:].view(2, 16, 256)
-    assert cc.kernel_plan_fwd(xg, w.to(DEV)) == "generic"
+    assert cc.kernel_plan_fwd(xg, w.to(DEV)) == ("generic" if dtype.itemsize == 4 else "bcl_vec_short_ragged")   # (64 or 32 vectors)
     assert_parity(run_fwd(cc, xg, w, None), co.conv1d_fwd(xv, w), exact=True, what="edge/misaligned")
 
 
@@ -686,7 +687,7 @@ def test_time_contiguous_rows_off_the_16_byte_grid(cc, dtype):
             want = co.conv1d_fwd(x, w, b, mask=m, activation=act, residual=res,
                                  initial_state=init if st else None, final_state_len=8 if st else None)
             xg = x.to(DEV)
-            assert cc.kernel_plan_fwd(xg, w.to(DEV)) == "bcl_vec", (B, C, L)
+            assert cc.kernel_plan_fwd(xg, w.to(DEV)) == ("bcl_vec" if L > 32 * E else "bcl_vec_short_ragged"), (B, C, L)
             got = run_fwd(cc, xg, w, b, act=act, mask=m, residual=res, init=init if st else None, S_out=8 if st else None)
             what = f"edge/{dtype}/{B}x{C}x{L}/W{W}/{act}/{res}/mask{m is not None}/state{st}"
             xm = x if m is None else (x.float() * m[:, None, :].float()).to(dtype)
@@ -776,6 +777,7 @@ def test_channel_contiguous_rows_off_the_8_byte_grid(cc, dtype):
         wide = torch.zeros(B, L, C + off, dtype=dtype, device=DEV)
         xg = wide[..., off:].transpose(1, 2)
         xg.copy_(x)
+        assert cc.kernel_plan_fwd(xg, w.to(DEV)) == "blc_vec_any", (C, L)
         for rounding in ("fused", "eager"):
             want, want_fs = co.conv1d_fwd(x, w, b, mask=mask, activation=act, residual=res, initial_state=init, final_state_len=S_out,
                                           round_mode=int(rounding == "eager"))
@@ -810,6 +812,7 @@ def test_short_rows_of_any_length_and_alignment(cc, dtype):
         buf = torch.zeros(off + B * C * (L + off), dtype=dtype, device=DEV)
         xg = buf[off:].view(B, C, L + off)[..., :L]
         xg.copy_(x)
+        assert cc.kernel_plan_fwd(xg, w.to(DEV)) == ("bcl_vec_short" if L % E == 0 and not off else "bcl_vec_short_ragged"), L
         for rounding in ("fused", "eager"):
             want, want_fs = co.conv1d_fwd(x, w, b, mask=mask, activation=act, residual=res, initial_state=init, final_state_len=8,
                                           round_mode=int(rounding == "eager"))
@@ -1013,7 +1016,7 @@ def test_randomised_shapes_layouts_and_options(cc):
         added = None if not res else (x if res == "unmasked" else xm)      # the term the sum may cancel against
         assert_parity(got, want, exact=act is None, what=what, res=added)
     # the draw reaches every kernel family
-    assert set(plans) >= {"bcl_vec", "bcl_vec_short", "blc_vec", "blc_vec_seq", "generic"}, plans
+    assert set(plans) == {"bcl_vec", "bcl_vec_short", "bcl_vec_short_ragged", "blc_vec", "blc_vec_seq", "blc_vec_any", "generic"}, plans
 
 
 def test_randomised_large_channel_contiguous_launches(cc):

@@ -1337,7 +1337,8 @@ def short_conv_update(
 # ---------------------------------------------------------------------------
 def kernel_plan_fwd(x, weight, bias=None, activation=None, attention_mask=None, residual=False,
                     rounding="fused", initial_states=None, final_states_out=None, seq_idx=None) -> str:
-    """Kernel family ``causal_conv1d_fn`` would launch: 'bcl_vec', 'blc_vec', 'blc_vec_seq' or 'generic'."""
+    """Kernel family ``causal_conv1d_fn`` would launch: 'bcl_vec', 'bcl_vec_short', 'bcl_vec_short_ragged', 'blc_vec',
+    'blc_vec_seq', 'blc_vec_any' or 'generic' (see ``include/canon_conv1d.h``)."""
     out = torch.empty_like(x)
     p = _fill_fwd(x, out, weight, _prep_bias(weight, bias), attention_mask, initial_states, final_states_out,
                   _activation_flag(activation), _residual_mode(residual), _round_mode(rounding), seq_idx)

@@ -170,7 +170,6 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     plan->wpb = 4;
     plan->grid = 0;
     plan->kind = FWD_GENERIC;
-    plan->name = "generic";
     if (empty) return CANON_OK;
 
     const int E = 16 / elem_bytes(p->x_dtype);
@@ -179,9 +178,8 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     const bool ptr_ok = aligned16(p->x) && aligned16(p->out);
     // packed sequences: the channel-contiguous kernel has a variant (the index is uniform per time row);
     // time-contiguous rows take the strided kernel
-    // (the shortest rows of this family by name; rows of up to kBclShortMaxVectors share waves, below)
-    const uint32_t kBclMinVectors = 16;
-    const bool bcl_rows = !p->seq_idx && ptr_ok && a.x_sl == 1 && a.o_sl == 1 && a.L / E >= kBclMinVectors;
+    // (rows of up to kBclShortMaxVectors share waves, below)
+    const bool bcl_rows = !p->seq_idx && ptr_ok && a.x_sl == 1 && a.o_sl == 1 && (a.L + E - 1) / E > kBclShortMaxVectors;
     // every row starts on a 16-byte boundary and is a whole number of vectors ...
     const bool bcl_aligned = a.L % E == 0 && a.x_sb % E == 0 && a.x_sc % E == 0 && a.o_sb % E == 0 && a.o_sc % E == 0;
     // ... or x and out share one geometry (the kernel's ragged variant, accesses at the elements' own alignment)
@@ -211,8 +209,6 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
     if (!p->seq_idx && a.x_sl == 1 && a.o_sl == 1 && (short_aligned || elem_ok) && a.L >= (uint32_t)E &&
         (a.L + E - 1) / E <= kBclShortMaxVectors && rows < (1ull << 31)) {
         const uint32_t nvec = (a.L + E - 1) / E;
-        // (the families keep their names: whole vectors, rows of at least sixteen, neither)
-        plan->name = short_aligned ? "bcl_vec_short" : bcl_ok ? "bcl_vec" : "generic";
         plan->ragged = !short_aligned;
         if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
         const uint64_t nwaves = (rows + 64u / nvec - 1) / (64u / nvec);
@@ -243,7 +239,6 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         const uint64_t ntasks = rows * nseg;
         if (ntasks < (1ull << 31)) {
             plan->kind = FWD_BCL;
-            plan->name = "bcl_vec";
             plan->U = U;
             plan->ragged = !bcl_aligned;
             if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
@@ -277,7 +272,6 @@ int plan_fwd(const canon_conv1d_fwd_params *p, FwdPlan *plan, int blc_rows = 0)
         const uint64_t nblocks = (ncols + 7) / 8 * 8 * group;
         if (nblocks < (1ull << 31) - 8) {
             plan->kind = blc_any ? FWD_BLC_ANY : FWD_BLC;
-            plan->name = blc_any ? "generic" : p->seq_idx ? "blc_vec_seq" : "blc_vec";   // (the family keeps its name)
             a.nvec = nvec; a.nct = nct; a.ntt = ntt; a.ntasks = (uint32_t)ncols;
             a.nseg = ngroups; a.chunk = group;
             a.div_nct = make_fastdiv(nct); a.div_ntt = make_fastdiv(ngroups); a.div_nseg = make_fastdiv(group);
@@ -659,7 +653,6 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
     a.grad_dtype = p->grad_dtype;
     a.w_vec = p->width == 4 && p->w_stride_k == 1 && p->w_stride_c == 4 && aligned16(p->weight);
     plan->kind = BWD_GENERIC;
-    plan->name = "bwd_generic";
     plan->U = 1;
     plan->ragged = plan->short_rows = plan->any = plan->walk_too = false;
     plan->grid = 0;
@@ -680,12 +673,10 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
                               a.g_sb % E == 0 && a.g_sc % E == 0 && a.d_sb % E == 0 && a.d_sc % E == 0;
     // ... or not: the kernel's ragged variant (elements at their own alignment).  A wave per row costs the same whatever the
     // row's length, the walk kernel, whose lanes lie a row apart, pays for every step: measured at 30720 rows, bf16, L 500
-    // 20.0 against 272 us.  (Rows of up to kBclShortMaxVectors share waves, below; the least length here is that of the family
-    // by name.)
-    constexpr uint32_t kRaggedMinSteps = 40;
+    // 20.0 against 272 us.  (Rows of up to kBclShortMaxVectors share waves, below.)
     const int64_t unit = rows_aligned ? E : 1;
     const uintptr_t elem_mask = (uintptr_t)elem_bytes(p->x_dtype) - 1;
-    const bool rows = rows_any && (rows_aligned || (a.L >= kRaggedMinSteps && (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0)) &&
+    const bool rows = rows_any && (rows_aligned || ((a.L + E - 1) / E > kBclShortMaxVectors && (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0)) &&
                       // the kernel receives the batch and channel strides of x and dout as 32-bit leading scalars
                       a.x_sb >= 0 && a.x_sc >= 0 && a.g_sb >= 0 && a.g_sc >= 0 &&
                       (uint64_t)(a.x_sb / unit) < (1ull << 32) && (uint64_t)(a.x_sc / unit) < (1ull << 32) &&
@@ -699,7 +690,6 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         const uint32_t nvec = (a.L + E - 1) / E;
         const uint64_t waves = (nrows + 64u / nvec - 1) / (64u / nvec);
         plan->kind = BWD_BCL_VEC;
-        plan->name = rows_aligned ? "bwd_bcl_vec" : rows ? "bwd_bcl_vec_ragged" : "bwd_generic";   // (the families keep their names)
         plan->short_rows = true;
         a.m_vec = p->mask && p->mask_stride_l == 1;
         a.nvec = nvec; a.chunk = (65536u + nvec - 1) / nvec; a.nthreads = (uint32_t)nrows;
@@ -730,7 +720,6 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
             plan->ragged = plan->walk_too = !rows_aligned;
             if (plan->ragged) a.m_vec = p->mask && p->mask_stride_l == 1;   // wide mask loads at any alignment
             plan->kind = BWD_BCL_VEC;
-            plan->name = plan->ragged ? "bwd_bcl_vec_ragged" : "bwd_bcl_vec";
             plan->U = U;
             // field use in this kernel family: nthreads = wave tasks, nchunk = segments per row
             a.nvec = nvec; a.nchunk = (uint32_t)nseg; a.nthreads = (uint32_t)ntasks;
@@ -779,7 +768,6 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         const uint64_t blocks = (uint64_t)a.B * ch.n * nct;
         if (blocks < (1ull << 31)) {
             plan->kind = BWD_BLC_VEC;
-            plan->name = any ? "bwd_generic" : packed ? "bwd_blc_vec_seq" : "bwd_blc_vec";   // (the family keeps its name)
             plan->any = any;
             plan->walk_too = packed || any;
             a.nvec = nvec; a.nct = nct; a.chunk = ch.len; a.nchunk = ch.n;
@@ -793,7 +781,6 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
         }
     }
     plan->kind = BWD_GENERIC;
-    plan->name = "bwd_generic";
     a.nvec = a.C;
     // time steps per lane: about 8 waves per CU, a multiple of the look-ahead, and few enough
     // partial sets that the scratch stays below ~16 MB
@@ -1127,14 +1114,24 @@ CANON_API const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p)
     BwdPlan pl;
     const int rc = p && p->workspace ? plan_bwd_in(p, &pl, p->workspace_bytes) : plan_bwd(p, &pl, false);
     if (rc != CANON_OK) return nullptr;
-    return pl.name;
+    switch (pl.kind) {
+    case BWD_BLC_VEC: return pl.any ? "bwd_blc_vec_any" : pl.args.seq ? "bwd_blc_vec_seq" : "bwd_blc_vec";
+    case BWD_BCL_VEC: return pl.short_rows ? "bwd_bcl_vec_short" : pl.ragged ? "bwd_bcl_vec_ragged" : "bwd_bcl_vec";
+    default: return "bwd_generic";
+    }
 }
 
 CANON_API const char *canon_conv1d_fwd_plan(const canon_conv1d_fwd_params *p)
 {
     FwdPlan pl;
     if (plan_fwd(p, &pl) != CANON_OK) return nullptr;
-    return pl.name;
+    switch (pl.kind) {
+    case FWD_BCL: return "bcl_vec";
+    case FWD_BCL_SHORT: return pl.ragged ? "bcl_vec_short_ragged" : "bcl_vec_short";
+    case FWD_BLC: return pl.args.seq ? "blc_vec_seq" : "blc_vec";
+    case FWD_BLC_ANY: return "blc_vec_any";
+    default: return "generic";
+    }
 }
 
 CANON_API int canon_conv1d_fwd_plan_waves(const canon_conv1d_fwd_params *p)

@@ -249,7 +249,6 @@ constexpr uint32_t kBclBigLaunch = 16384;
 
 struct FwdPlan {
     FwdKind kind;
-    const char *name;   // what canon_conv1d_fwd_plan answers
     int U;
     bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
     uint32_t wpb; // bcl: waves per block
@@ -281,7 +280,6 @@ struct UpdPartsPlan {
 
 struct BwdPlan {
     BwdKind kind;
-    const char *name;   // what canon_conv1d_bwd_plan answers
     int U;
     bool ragged; // bcl: rows are no whole number of vectors or do not start on 16-byte boundaries
     bool short_rows;   // bcl: several rows share a wave
