@@ -21,7 +21,8 @@ def both(cc, monkeypatch, call):
     """call() through the native module and without it: the two results, or the two exceptions as text."""
     results = []
     none = types.SimpleNamespace(**{name: (lambda *a: None) for name in
-                                    ("try_fwd", "try_fwd_parts", "try_update_modes", "try_decode_step", "launch_fwd", "launch_bwd")})
+                                    ("try_fwd", "try_fwd_parts", "try_layer_block", "try_known_update", "try_update_modes",
+                                     "try_decode_step", "launch_fwd", "launch_bwd")})
     for native in (cc._lib.native(), none):
         with monkeypatch.context() as m:
             m.setattr(cc._lib, "native", lambda native=native: native)

@@ -549,8 +549,8 @@ def causal_conv1d_update(
     declined = False
     if cache_seqlens is None and conv_state_indices is None:
         if not torch.compiler.is_compiling() and x.is_cuda:
-            out = _lib.native().try_update_modes(x, conv_state, weight, bias, activation, None, None, token_mask, residual,
-                                                 rounding, _known_updates())
+            out = _lib.native().try_known_update(x, conv_state, weight, bias, activation, token_mask, residual, rounding,
+                                                 _known_updates())
             if type(out) is bytes:
                 key = out
             elif out is not None:

@@ -120,7 +120,7 @@ class CanonLayer(nn.Module):
         if torch.compiler.is_compiling():
             return None
         slots = 0 if not use_cache else state.size(-1) if state is not None else self._state_len()
-        done = _lib.native().try_fwd_parts(x, taps, self.bias_param, history, slots, act, mask, "masked", self.rounding, True)
+        done = _lib.native().try_layer_block(x, taps, self.bias_param, history, slots, act, mask, "masked", self.rounding)
         if type(done) is int:
             _lib.check(done, "causal_conv1d_fn")
         return done

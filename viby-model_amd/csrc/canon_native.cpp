@@ -350,10 +350,12 @@ PyObject *try_fwd(PyObject *, PyObject *const *args, Py_ssize_t n)
 }
 
 // The block call of CanonLayer (inference), from the layer's own (batch, seqlen, dim) tensors, one or several parts, without
-// a view of any of them: try_fwd_parts(x | (x, ..), taps, bias, history, slots, activation, mask, residual, rounding, True)
+// a view of any of them: try_layer_block(x | (x, ..), taps, bias, history, slots, activation, mask, residual, rounding)
 //   -> (output | outputs, new state of that many slots or None) | status code | None
-PyObject *layer_block(PyObject *const *args)
+PyObject *try_layer_block(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
+    HANDLE_TH_ERRORS
+    CANON_NONE_UNLESS(n == 9 && no_mode());
     PyObject *const one[1] = {args[0]};
     const bool tuple = PyTuple_CheckExact(args[0]);
     PyObject *const *items = tuple ? &PyTuple_GET_ITEM(args[0], 0) : one;
@@ -420,6 +422,7 @@ PyObject *layer_block(PyObject *const *args)
         PyTuple_SET_ITEM(result, 1, Py_None);
     }
     return result;
+    END_HANDLE_TH_ERRORS
 }
 
 // try_fwd_parts((x, ..), weight, bias, initial_states, final_states, activation, attention_mask, residual, rounding)
@@ -427,7 +430,6 @@ PyObject *layer_block(PyObject *const *args)
 PyObject *try_fwd_parts(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    if (n == 10 && no_mode()) return layer_block(args);
     CANON_NONE_UNLESS(n == 9 && no_mode() && (PyTuple_CheckExact(args[0]) || PyList_CheckExact(args[0])));
     const Py_ssize_t np = PySequence_Fast_GET_SIZE(args[0]);
     CANON_NONE_UNLESS(np >= 1 && np <= CANON_CONV1D_MAX_PARTS);
@@ -471,15 +473,17 @@ PyObject *try_fwd_parts(PyObject *, PyObject *const *args, Py_ssize_t n)
 
 // The plain decode step of a signature that has been through every check before (see causal_conv1d_update): `known` maps
 // signatures to argument blocks in which only the addresses are missing (with the signature a tuple of Python's sizes and
-// strides and the launch through ctypes, B 256, C 3456: 10.4 us a call, here 6.5).  try_update_modes(x, conv_state, weight, bias,
-// activation, None, None, token_mask, residual, rounding, known) -> output | status code | the signature, which the table
-// does not hold (nothing was done) | None
-PyObject *known_update(PyObject *const *args)
+// strides and the launch through ctypes, B 256, C 3456: 10.4 us a call, here 6.5).  try_known_update(x, conv_state, weight, bias,
+// activation, token_mask, residual, rounding, known) -> output | status code | the signature, which the table does not hold
+// (nothing was done) | None
+PyObject *try_known_update(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
+    HANDLE_TH_ERRORS
+    CANON_NONE_UNLESS(n == 9 && no_mode());
     const Tensor *x, *state, *weight, *bias, *mask;
     CANON_NONE_UNLESS(plain(args[0], &x) && plain(args[1], &state) && plain(args[2], &weight) && plain(args[3], &bias) &&
-                      plain(args[7], &mask) && x && state && weight && PyDict_CheckExact(args[10]));
-    const int act = activation_flag(args[4]), res = residual_mode(args[8]), rnd = round_mode(args[9]);
+                      plain(args[5], &mask) && x && state && weight && PyDict_CheckExact(args[8]));
+    const int act = activation_flag(args[4]), res = residual_mode(args[6]), rnd = round_mode(args[7]);
     CANON_NONE_UNLESS(act >= 0 && res >= 0 && rnd >= 0 && x->dim() == 2 && state->dim() == 3 && weight->dim() == 2 && x->is_cuda());
     CANON_NONE_UNLESS(!c10::GradMode::is_enabled() ||
                       !(wants_grad(x) || wants_grad(state) || wants_grad(weight) || wants_grad(bias) || wants_grad(mask)));
@@ -503,7 +507,7 @@ PyObject *known_update(PyObject *const *args)
     CANON_NONE_UNLESS(stream_of(*x, &stream));
     PyObject *signature = PyBytes_FromStringAndSize((const char *)key, at * sizeof(key[0]));
     if (!signature) return nullptr;
-    PyObject *block = PyDict_GetItemWithError(args[10], signature);   // (borrowed)
+    PyObject *block = PyDict_GetItemWithError(args[8], signature);   // (borrowed)
     if (!block) {
         if (!PyErr_Occurred()) return signature;
         Py_DECREF(signature);
@@ -523,6 +527,7 @@ PyObject *known_update(PyObject *const *args)
     const int rc = without_gil([&] { return canon_conv1d_update(&p, stream); });
     if (rc != CANON_OK) return PyLong_FromLong(rc);
     return THPVariable_Wrap(std::move(out));
+    END_HANDLE_TH_ERRORS
 }
 
 // try_update_modes(x, conv_state, weight, bias, activation, cache_seqlens, conv_state_indices, token_mask, residual,
@@ -530,7 +535,6 @@ PyObject *known_update(PyObject *const *args)
 PyObject *try_update_modes(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
-    if (n == 11 && no_mode()) return known_update(args);
     CANON_NONE_UNLESS(n == 10 && no_mode());
     const Tensor *x, *state, *weight, *bias, *seqlens, *indices, *mask;
     CANON_NONE_UNLESS(plain(args[0], &x) && plain(args[1], &state) && plain(args[2], &weight) && plain(args[3], &bias) &&
@@ -716,8 +720,9 @@ int run_bwd(const Tensor &x, Tensor dout, const Tensor &weight, const Tensor *bi
 }
 
 #define CANON_METHOD(name) {#name, (PyCFunction)(void (*)(void))name, METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {CANON_METHOD(try_fwd), CANON_METHOD(try_fwd_parts), CANON_METHOD(try_update_modes), CANON_METHOD(try_decode_step),
-                         CANON_METHOD(launch_fwd), CANON_METHOD(launch_bwd), {nullptr, nullptr, 0, nullptr}};
+PyMethodDef methods[] = {CANON_METHOD(try_fwd), CANON_METHOD(try_fwd_parts), CANON_METHOD(try_layer_block), CANON_METHOD(try_known_update),
+                         CANON_METHOD(try_update_modes), CANON_METHOD(try_decode_step), CANON_METHOD(launch_fwd), CANON_METHOD(launch_bwd),
+                         {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
