@@ -350,6 +350,9 @@ def test_backward_of_packed_sequences(cc, dtype, layout):
     ("channel", 96, 1024, 200, False, 96),       # ... nor a caller's own scratch of one set per sequence
     ("packed", 96, 1024, 640, True, None),
     ("packed", 96, 1024, 200, False, 96),
+    ("off grid", 96, 1023, 640, True, None),
+    ("off grid", 96, 1023, 200, False, 96),      # ... one set per sequence
+    ("off grid", 200, 1023, 1100, False, 200),   # ... where the longest chunks still take two: the walk kernel's
     ("time", 132, 1000, 2100, False, 132)])      # rows of two segments, scratch for the walk kernel's one chunk per row
 def test_backward_with_a_scratch_for_fewer_partial_sets(cc, kind, B, C, L, static, scratch):
     """A scratch too small for the sets of the kernel's usual split gets fewer sets, not a refusal: same dx bits, sums
@@ -382,14 +385,15 @@ def test_backward_with_a_scratch_for_fewer_partial_sets(cc, kind, B, C, L, stati
         return p, dx, dw, db, space
 
     lib, stream = _lib.lib(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-    usual = {"channel": b"bwd_blc_vec", "packed": b"bwd_blc_vec_seq", "time": b"bwd_bcl_vec_ragged"}[kind]
+    usual = {"channel": b"bwd_blc_vec", "packed": b"bwd_blc_vec_seq", "off grid": b"bwd_blc_vec_any", "time": b"bwd_bcl_vec_ragged"}[kind]
+    walks = kind == "time" or (kind == "off grid" and L > 1024)
     need = lib.canon_conv1d_bwd_workspace_bytes(ctypes.byref(params(16)[0]))
     small = scratch * C * 20 if scratch else 16
     assert need > (8 << 20 if static else small)
     full, few = params(need), params(small)
     assert lib.canon_conv1d_bwd_plan(ctypes.byref(full[0])) == usual
     if not static:
-        assert lib.canon_conv1d_bwd_plan(ctypes.byref(few[0])) == (b"bwd_generic" if kind == "time" else usual)
+        assert lib.canon_conv1d_bwd_plan(ctypes.byref(few[0])) == (b"bwd_generic" if walks else usual)
     assert lib.canon_conv1d_bwd(ctypes.byref(full[0]), stream) == 0
     call = lib.canon_conv1d_bwd_static if static else lib.canon_conv1d_bwd
     assert call(ctypes.byref(few[0]), stream) == 0, lib.canon_conv1d_last_error()
