@@ -389,6 +389,16 @@ def test_bwd_plan_and_workspace():
                          (256, b"bwd_bcl_vec_short"), (255, b"bwd_bcl_vec_short"), (39, b"bwd_bcl_vec_short"),
                          (8, b"bwd_bcl_vec_short"), (7, b"bwd_generic")):
         assert L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl", L=length))) == want, length
+    # ... of 16 to 32 vectors (off the vectors with a mask from 40 steps on) not in launches of few rows
+    for length, act, mask, most, want in (
+            (128, 0, 0, 2560, b"bwd_bcl_vec"), (256, 0, 0, 5120, b"bwd_bcl_vec"), (128, 1, 0, 1280, b"bwd_bcl_vec"),
+            (256, 1, 1, 2560, b"bwd_bcl_vec"), (128, 0, 1, 1280, b"bwd_bcl_vec"), (129, 0, 0, 1280, b"bwd_bcl_vec_ragged"),
+            (255, 1, 0, 1280, b"bwd_bcl_vec_ragged"), (41, 0, 1, 1024, b"bwd_bcl_vec_ragged"), (119, 1, 1, 1024, b"bwd_bcl_vec_ragged"),
+            (120, 1, 1, 0, b""), (119, 1, 0, 0, b""), (39, 1, 1, 0, b""), (8, 0, 0, 0, b"")):
+        over = dict(mask=FAKE_X + 0x400000, mask_dtype=2, mask_stride_b=length, mask_stride_l=1) if mask else {}
+        for rows in (1, most or 1, most + 1):
+            got = L.canon_conv1d_bwd_plan(ctypes.byref(bwd_params(layout="bcl", B=1, C=rows, L=length, activation=act, **over)))
+            assert got == (want if rows <= most else b"bwd_bcl_vec_short"), (length, act, mask, rows)
     # off the 8-byte grid: the tiles at the elements' own alignment, at width 4 from 12 steps on; else the walk kernel
     for over, want in ((dict(C=3457), b"bwd_blc_vec_any"), (dict(C=3457, L=12), b"bwd_blc_vec_any"), (dict(C=3457, L=11), b"bwd_generic"),
                        (dict(C=3457, width=3), b"bwd_generic"), (dict(x=FAKE_X + 2), b"bwd_blc_vec_any"), (dict(x=FAKE_X + 1), b"bwd_generic"),

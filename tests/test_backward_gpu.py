@@ -37,7 +37,20 @@ def gpu_grads(cc, x_cpu, w, b, dout_cpu, layout, mask=None, act=None, residual=F
     return xg.grad, wg.grad, (bg.grad if bg is not None else None), out.detach()
 
 
-def plan_of(x, W=4, seq_idx=None):
+def time_plan(B, C, L, dtype, act=None, aligned=True, mask=None):
+    """The kernel of a time-contiguous backward: rows of up to 32 vectors share waves, not so few of 16 or more (with a mask off
+    the vectors of 40 steps) that the launch is one wave's life."""
+    E = 16 // dtype.itemsize
+    nvec, whole = -(-L // E), aligned and L % E == 0 and L >= 16 * E
+    if L < E:
+        return "bwd_generic"
+    masked = mask is not None
+    few = (B * C <= (80 if act or masked else 160) * nvec if whole else
+           B * C <= 1280 if nvec >= 16 else L >= 40 and masked and L % E != 0 and B * C <= 1024)
+    return "bwd_bcl_vec_short" if nvec <= 32 and not few else "bwd_bcl_vec" if whole else "bwd_bcl_vec_ragged"
+
+
+def plan_of(x, W=4, seq_idx=None, act=None, mask=None):
     """The kernel that the backward of a plain call on x runs (dout and dx in x's layout)."""
     import ctypes
 
@@ -45,11 +58,13 @@ def plan_of(x, W=4, seq_idx=None):
     code = _lib.DTYPE_CODE[x.dtype]
     others = [torch.empty_like(x) for _ in range(2)]
     p = _lib.BwdParams(struct_size=ctypes.sizeof(_lib.BwdParams), x_dtype=code, w_dtype=code, width=W, batch=x.shape[0],
-                       channels=x.shape[1], seqlen=x.shape[2])
+                       channels=x.shape[1], seqlen=x.shape[2], activation=int(act is not None))
     for name, t in zip(("x", "dout", "dx"), (x, *others)):
         setattr(p, name, t.data_ptr())
         for axis, stride in zip("bcl", t.stride()):
             setattr(p, f"{name}_stride_{axis}", stride)
+    if mask is not None:
+        p.mask, p.mask_dtype, p.mask_stride_b, p.mask_stride_l = mask.data_ptr(), _lib.MASK_CODE[mask.dtype], *mask.stride()
     if seq_idx is not None:
         p.seq_idx, p.seq_stride_b, p.seq_stride_l = seq_idx.data_ptr(), *seq_idx.stride()
     return _lib.lib().canon_conv1d_bwd_plan(ctypes.byref(p)).decode()
@@ -474,8 +489,7 @@ def test_backward_of_ragged_time_contiguous_rows(cc, dtype):
                 xg = buf[offset:].view(B, C, L + 1)[..., :L]
             xg = xg.detach().requires_grad_()
             # (a slice of longer rows is no dense tensor: dout and dx are rows of their own length, which may be whole vectors)
-            assert plan_of(xg, W) == ("bwd_generic" if L < E else "bwd_bcl_vec_short" if L <= 32 * E else
-                                      "bwd_bcl_vec" if L % E == 0 and not offset else "bwd_bcl_vec_ragged")
+            assert plan_of(xg, W, act=act, mask=mask) == time_plan(B, C, L, dtype, act, not offset, mask)
             wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
             out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
             grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))
@@ -531,7 +545,7 @@ def test_non_finite_inputs_at_the_end_of_a_row_stay_in_their_taps(cc, dtype, rou
     assert plan_of(probe, W, None if seq is None else seq.to(DEV)) == (
         "bwd_generic" if route == "strided" or (route == "bcl" and L < E) or (route == "packed" and not grid) or (route == "blc" and not grid and L < 12) else
         ("bwd_blc_vec_seq" if route == "packed" else "bwd_blc_vec" if grid else "bwd_blc_vec_any") if route != "bcl" else
-        "bwd_bcl_vec_short" if L <= 32 * E else "bwd_bcl_vec" if L % E == 0 else "bwd_bcl_vec_ragged")
+        time_plan(B, C, L, dtype))
     for bad, back in ((float("inf"), 1), (float("-inf"), 2), (float("nan"), 1), (float("nan"), 3), (float("inf"), 4)):
         x = torch.randn(B, C, L, generator=g).to(dtype)
         if back <= L:
@@ -656,6 +670,8 @@ def test_backward_of_short_rows_of_any_length_and_alignment(cc, dtype):
     lengths = [E, E + 1, 2 * E - 1, 2 * E, *(3 * E + j for j in range(1, E)), 9 * E + 2, 10 * E + 1, 16 * E + 1, 21 * E - 1, 21 * E, 32 * E - 1, 32 * E]
     for n, L in enumerate(lengths):
         B, C, W, off = (1, 2, 3)[n % 3], (13, 67, 130)[n % 3], 4 - n % 3, (0, 3)[n % 2]
+        if L >= 9 * E:
+            B, C = 3, 1720 + n         # (few of the longer rows take a wave each)
         act, res, mtype = (None, "silu")[n % 4 >= 2], (False, "masked", "unmasked")[n % 3], masks[n % len(masks)]
         x, dout = torch.randn(B, C, L, generator=g).to(dtype), torch.randn(B, C, L, generator=g).to(dtype)
         w = (torch.randn(C, W, generator=g) * 0.5).to(dtype)
@@ -670,7 +686,7 @@ def test_backward_of_short_rows_of_any_length_and_alignment(cc, dtype):
         xg = buf[off:].view(B, C, L + off)[..., :L]
         xg.copy_(x)
         xg = xg.detach().requires_grad_()
-        assert plan_of(xg, W) == "bwd_bcl_vec_short", L
+        assert plan_of(xg, W, act=act, mask=mask) == "bwd_bcl_vec_short", L
         wg, bg = w.to(DEV).requires_grad_(), b.to(DEV).requires_grad_() if b is not None else None
         out = cc.causal_conv1d_fn(xg, wg, bg, activation=act, attention_mask=None if mask is None else mask.to(DEV), residual=res)
         grads = torch.autograd.grad(out, [t for t in (xg, wg, bg) if t is not None], dout.to(DEV))

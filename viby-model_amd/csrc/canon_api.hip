@@ -673,21 +673,33 @@ int plan_bwd(const canon_conv1d_bwd_params *p, BwdPlan *plan, bool check_pointer
                               a.g_sb % E == 0 && a.g_sc % E == 0 && a.d_sb % E == 0 && a.d_sc % E == 0;
     // ... or not: the kernel's ragged variant (elements at their own alignment).  A wave per row costs the same whatever the
     // row's length, the walk kernel, whose lanes lie a row apart, pays for every step: measured at 30720 rows, bf16, L 500
-    // 20.0 against 272 us.  (Rows of up to kBclShortMaxVectors share waves, below.)
+    // 20.0 against 272 us.
+    constexpr uint32_t kRaggedMinSteps = 40;
     const int64_t unit = rows_aligned ? E : 1;
     const uintptr_t elem_mask = (uintptr_t)elem_bytes(p->x_dtype) - 1;
-    const bool rows = rows_any && (rows_aligned || ((a.L + E - 1) / E > kBclShortMaxVectors && (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0)) &&
+    const bool rows = rows_any && (rows_aligned || (a.L >= kRaggedMinSteps && (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0)) &&
                       // the kernel receives the batch and channel strides of x and dout as 32-bit leading scalars
                       a.x_sb >= 0 && a.x_sc >= 0 && a.g_sb >= 0 && a.g_sc >= 0 &&
                       (uint64_t)(a.x_sb / unit) < (1ull << 32) && (uint64_t)(a.x_sc / unit) < (1ull << 32) &&
                       (uint64_t)(a.g_sb / unit) < (1ull << 32) && (uint64_t)(a.g_sc / unit) < (1ull << 32);
     const uint64_t nrows = (uint64_t)a.B * a.C;
-    // rows of at most 32 vectors, down to one: several to a wave (canon_bwd_bcl_short_kernel), at any alignment
-    if (rows_any && a.L >= (uint32_t)E && (a.L + E - 1) / E <= kBclShortMaxVectors &&
+    // rows of at most 32 vectors, down to one: several to a wave (canon_bwd_bcl_short_kernel), at any alignment.  Not so few
+    // that the launch is one wave's life, which is longer with two to four rows in it: such launches keep a wave per row, in
+    // the number that both measured alike.  us a call, wave per row / shared, bf16: L 128, 640 rows 5.08 / 5.63, 2560 rows
+    // 5.86 / 5.87, 5120 rows 6.60 / 6.11; L 256, 640 rows 5.17 / 5.82, 5120 rows 6.60 / 6.91, 10240 rows 8.78 / 7.99; with
+    // SiLU and a mask L 128 and L 256, 640 rows 5.67 / 5.96 and 5.76 / 6.26, 1280 rows 6.18 / 6.16 and 6.29 / 6.29, 2560 rows
+    // 6.93 / 6.24 and 7.02 / 7.05; with a mask alone L 128, 2560 rows 6.44 / 6.11; off the vectors L 129, 640 rows 5.89 /
+    // 6.15, 2560 rows 6.61 / 6.36, with a mask 1280 rows 6.77 / 7.33, and with a mask (whose last vector moves as well) down to
+    // L 41, 640 rows 6.20 / 6.62, L 119, 1280 rows 6.73 / 6.59 (with SiLU alone 5.92 / 5.68); fp32 L 128, 640 rows 5.18 / 5.65,
+    // 5120 rows 6.61 / 6.69.
+    const uint32_t row_vecs = (a.L + E - 1) / E;
+    const bool few_rows = rows && (rows_aligned ? nrows <= (a.act || p->mask ? 80ull : 160ull) * row_vecs
+                                                : row_vecs >= 16 ? nrows <= 1280 : p->mask && a.L % E != 0 && nrows <= 1024);
+    if (rows_any && !few_rows && a.L >= (uint32_t)E && row_vecs <= kBclShortMaxVectors &&
         (((uintptr_t)p->x | (uintptr_t)p->dout | (uintptr_t)p->dx) & elem_mask) == 0 &&
         a.x_sb >= 0 && a.x_sc >= 0 && a.g_sb >= 0 && a.g_sc >= 0 &&      // (32-bit leading scalars, as below)
         std::max({a.x_sb, a.x_sc, a.g_sb, a.g_sc}) < (1ll << 32)) {
-        const uint32_t nvec = (a.L + E - 1) / E;
+        const uint32_t nvec = row_vecs;
         const uint64_t waves = (nrows + 64u / nvec - 1) / (64u / nvec);
         plan->kind = BWD_BCL_VEC;
         plan->short_rows = true;

@@ -1227,8 +1227,8 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_kernel(const char *x_base, 
 // then hold nothing, or below 40 steps the walk kernel.  us per call with the reduction, bf16: B 31, C 2848, L 82 with a
 // mask 54.4 -> 25.7; B 32, C 3456: L 13 (SiLU, mask) 14.6 -> 11.0, L 39 (SiLU) 48.8 -> 14.6, L 64 47.6 -> 14.8, L 128
 // 41.0 -> 23.2, L 129 53.3 -> 31.5 (45.5 with rows in the next power of two of lanes), L 255 57 -> 44, L 256 43.5 -> 40.6
-// (27.4 at the plain copy's rate); a launch of a few rows (B 3, C 96, L 209, SiLU, mask) is one wave's life, which is
-// 0.7 us longer with two rows in it.
+// (27.4 at the plain copy's rate).  A launch of a few rows is one wave's life, which is longer with two to four rows in it
+// (B 3, C 96, L 209, SiLU, mask 6.35 -> 7.3): those of 16 vectors and more keep a wave each (few_rows in the planning).
 template <int DT, int W, bool MASK>
 __global__ __launch_bounds__(256) void canon_bwd_bcl_short_kernel(const char *x_base, const char *g_base, uint32_t x_sb32,
                                                                   uint32_t x_sc32, uint32_t g_sb32, uint32_t g_sc32,
