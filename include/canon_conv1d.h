@@ -412,9 +412,9 @@ const char *canon_conv1d_fwd_plan(const canon_conv1d_fwd_params *p);
 int canon_conv1d_fwd_plan_waves(const canon_conv1d_fwd_params *p);
 const char *canon_conv1d_update_plan(const canon_conv1d_update_params *p);
 /* "bwd_blc_vec" | "bwd_blc_vec_seq" | "bwd_blc_vec_any" (off the 8-byte grid) | "bwd_bcl_vec_short" (time-contiguous rows of
- * 1 to 32 vectors) | "bwd_bcl_vec" | "bwd_bcl_vec_ragged" (longer ones and few of 16 to 32, on 16-byte boundaries or not) |
- * "bwd_generic" (the walk kernel): with a workspace given the kernel that runs in that many bytes, without one the kernel that runs where
- * there is room for its partial sets */
+ * 1 to 32 vectors) | "bwd_bcl_vec" | "bwd_bcl_vec_ragged" (longer ones, and launches of few of these, on 16-byte boundaries
+ * or not) | "bwd_generic" (the strided kernel): with a workspace given the kernel that runs in that many bytes, without one
+ * the kernel that runs where there is room for its partial sets */
 const char *canon_conv1d_bwd_plan(const canon_conv1d_bwd_params *p);
 /* "blc_vec_pair" (two dense tensors of one shape: one launch of the single-tensor code), "blc_vec_parts" /
  * "update_vec_parts" (one launch over a table of parts) or "per_part" (one launch per part) */

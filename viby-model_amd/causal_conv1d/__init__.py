@@ -122,8 +122,10 @@ def _narrow_mask(mask: torch.Tensor, x: torch.Tensor, numel: int) -> torch.Tenso
     ``model/model.py:455``; the reference wrapper casts the mask the same way,
     ``causal_conv1d_mps/__init__.py:244-247``).  Read as it is / converted, bf16, us: time-contiguous B 16 C 640 L 1024
     11.0 / 12.4, B 4 C 960 L 4096 17.7 / 16.5, B 8 C 3456 L 1024 24.0 / 24.4 (training in fp32 104.7 / 100.0), B 32
-    86.1 / 75.2; strided kernels (B 32 C 3455) 311 / 301, training 754 / 690.  The channel-contiguous vector kernels
-    read an entry once per wave: 73.0 / 76.8 at B 32 C 3456, so they get the mask as it is.
+    86.1 / 75.2.  The channel-contiguous vector kernels read an entry once per wave: 73.0 / 76.8 at B 32 C 3456, so on the
+    8-byte grid they get the mask as it is.  Off that grid it is converted as well, and need not be where the tiles at the
+    elements' own alignment run: their kernel takes the same time with either mask (B 32 C 3455 102, backward 234), the call
+    104.6 with the conversion, 100.4 with a mask that was bf16 before.
     The result belongs to this call alone: a copy kept for the next one would not follow what another stream, a
     captured graph or a write past the version counter does to the mask.  (``canon_native.cpp`` has the same rule.)
     """

@@ -993,7 +993,7 @@ CANON_API int canon_conv1d_bwd(const canon_conv1d_bwd_params *p, void *stream)
     pl.walk_too = false;
     int rc = plan_bwd(p, &pl, true);
     if (rc != CANON_OK && pl.walk_too && p->workspace && aligned16(p->workspace)) {
-        // packed or ragged rows: the walk kernel cuts long rows into fewer partial sets where there are many channels,
+        // packed, ragged or off-grid rows: the walk kernel cuts long rows into fewer partial sets where there are many channels,
         // so a scratch that is too small for the plan's kernel may still hold its sets
         BwdPlan walk;
         if (plan_bwd(p, &walk, false, true) == CANON_OK && p->workspace_bytes >= walk.workspace_bytes) {

@@ -552,7 +552,10 @@ __global__ __launch_bounds__(256, ACT ? 4 : 1) void canon_bwd_blc_kernel(const B
         float red[NW - 1][5 * E][64];                 // dweight / dbias sums of waves 1..3
         // Four blocks a CU instead of the five their registers allow: unmasked launches without an activation, B 8 / 16 / 32,
         // C 3456, L 1024, bf16: 36.2 / 64.0 / 120.5 -> 35.4 / 63.3 / 119.7 us a call (three: 38.5 / 64.6 / 122; with a mask
-        // four are 0.4 % slower).
+        // four are 0.4 % slower).  The other instances it holds for, five -> four, B 8 and B 32: fp16 36.5 and 121.0 -> 36.5
+        // and 119.9; width 3 36.3 and 121.8 -> 36.6 and 119.9, width 2 36.2 and 123.6 -> 35.9 and 120.3 (fp16 alike); fp32 of
+        // widths 2 and 3, B 16 119.3 -> 118.5 (width 4 has four by its registers); off the grid, C 3455 60.9 and 232 -> 61.5
+        // and 230; C 640 and 960 within 0.3 % throughout.
         char room[!ACT && !MASK && !SEQ && !STATES ? 33 * 1024 : 16];
     };
     __shared__ Shared shared;
@@ -1388,8 +1391,9 @@ __global__ __launch_bounds__(256) void canon_bwd_bcl_short_kernel(const char *x_
 //
 // U sets a slice are requested together, added in set order: what bounds the kernel is the round trips in a row, not the
 // bytes.  Four loads in flight and the sets past the last whole round one by one -> sixteen from 65 sets on, four below, us of the whole
-// call: B 8 C 640 L 1024 12.2 -> 11.4, B 16 C 640 L 511 SiLU masked 16.2 -> 15.4, packed rows B 2 C 3456 L 8192 72.1 -> 70.5, B 1
-// C 160 L 896 8.1 -> 7.6.  (Sixteen at B 1 and B 4, C 3456, 8 and 32 sets: 10.0 -> 10.4, 20.9 -> 21.4.)
+// call: B 8 C 640 L 1024 12.2 -> 11.5, B 16 C 640 L 511 SiLU masked 16.2 -> 15.4, B 4 C 640 9.2 -> 8.5, B 1 C 160 L 896 6.2 ->
+// 5.7; from C 3456 on, packed rows included, within 0.5 %.  (Sixteen at B 1 and B 4, C 3456, 8 and 32 sets: 10.0 -> 10.4,
+// 20.9 -> 21.4.)
 //
 // The sum is stored as the caller's gradient type: converting fp32 sums to 16-bit parameters' type in two further
 // launches took a training step at B 16, C 640, L 511 (of 33 us on the device) 3.5 us and their host time.

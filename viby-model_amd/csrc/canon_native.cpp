@@ -1,6 +1,6 @@
 // causal_conv1d._native: the host path of the prefill, the pool / ring decode step and the backward, from torch tensors
 // to the C ABI, without a Python statement per field.  Filled through ctypes the argument block of a prefill took
-// 7 of the 18 us such a call needed on the host (CanonLayer, B 1, C 640, L 77: now 12 us, of which the kernel is 4).
+// 7 of the 18 us such a call needed on the host (CanonLayer, B 1, C 640, L 77: now 10.5 us, of which the kernel is 4).
 //
 // The functions come in two kinds.  launch_*: the arguments were checked by the caller; the output (a status code where
 // the launch failed) is returned, or None where the tensors are not plain.  try_*: the public calls' own arguments; they
